@@ -212,7 +212,11 @@ int mstf_scale_softmax_f16(void* stream, const mstf_half* s, mstf_half* p, int64
  *   out[bq, :] = softmax_t( fp16(q[bq].Ktilde[t]) / sqrt(d) ) . Vtilde[t, :]     over the `tokens` cached tokens
  * q, out: [Bq, head_dim] fp16 (head_dim 128, groups <= 8).  Scores and probabilities stay on chip.
  * lse_out (nullable) [Bq, 2] fp32 receives (max, sum of exp(w - max)) per row, so a caller that keeps a
- * dense local window can combine that window's attention with this result under one softmax. */
+ * dense local window can combine that window's attention with this result under one softmax.
+ * Workspace: a call demands 520 bytes per query row and 512 tokens (and per row and 64 tokens of a window, where there is
+ * one), rounded up to 256 - the more, the larger the call, so that a workspace made for the largest serves all others.  The
+ * queries answer up to eight times that for a call of few token blocks (at most 3.2 MB), whose wavefronts then share blocks;
+ * with less it goes without, slower and to the same results. */
 size_t mstf_decode_attention_workspace_bytes(int tokens, int head_dim, int Bq, int groups);
 int mstf_decode_attention_f16(void* stream, const uint64_t* k_bmp, const mstf_half* k_nz, const uint32_t* k_idx,
                               const uint32_t* k_nz_off, const uint64_t* v_bmp, const mstf_half* v_nz,
@@ -240,7 +244,8 @@ int mstf_decode_attention_static_f16(void* stream, const uint64_t* k_bmp, const 
  * partial: per token split s and query row: workspace = float part_o[Bq][ns][head_dim] followed by
  *   float part_ml[Bq][ns][2] = (max, sum of exp(w - max)), part_o un-normalised;
  *   ns = mstf_decode_attention_splits(tokens, head_dim, Bq, groups) <= ceil(tokens / 512): a split covers 512
- *   tokens while every 64-token block can have a resident wavefront of its own, an even share of more beyond.
+ *   tokens while every 64-token block can have a resident wavefront of its own, an even share of more beyond
+ *   (workspace: as above, a slot per query row and 512 tokens).
  * merge: log-sum-exp combine of the ns splits into out (fp16) and, if given, lse_out. */
 int mstf_decode_attention_splits(int tokens, int head_dim, int Bq, int groups);
 int mstf_decode_attention_partial_f16(void* stream, const uint64_t* k_bmp, const mstf_half* k_nz, const uint32_t* k_idx,

@@ -722,8 +722,7 @@ using namespace mstf;
 extern "C" size_t mstf_decode_attention_workspace_bytes(int tokens, int head_dim, int Bq, int groups)
 {
     if (tokens <= 0 || head_dim != kFusedD || Bq <= 0 || groups <= 0 || tokens % 64 != 0 || Bq % groups != 0) return 0;
-    const int ns = fused_nsplit_room(tokens, Bq / groups, groups);
-    return round_up((size_t)Bq * ns * (head_dim + 2) * sizeof(float), 256);
+    return fused_workspace_room(tokens, 0, Bq, groups);
 }
 
 // How the compressed tokens of a launch are dealt out: whether wavefronts share blocks, blocks per wavefront, split slots per
@@ -735,9 +734,9 @@ struct DecodePlan {
 };
 // pooled: the token count is in device memory, at most `tokens` - as many splits as any count needs, and the kernel works
 // out the shares itself (deal: the workgroups per head that fill the chip).  window: blocks of the dense window that the
-// same launch takes.  share: whether wavefronts may share blocks (the two-phase entry points hand out splits of 512 tokens
-// or more).
-static DecodePlan decode_plan(int tokens, int Bq, int groups, bool pooled, int window = 0, bool share = true)
+// same launch takes.  share: whether wavefronts may share blocks (not where the workspace lacks the room for their slots; the
+// two-phase entry points hand out splits of 512 tokens or more).
+static DecodePlan decode_plan(int tokens, int Bq, int groups, bool pooled, int window, bool share)
 {
     const int Bkv = Bq / groups;
     if (share && fused_shares_blocks(tokens, Bkv, groups, Bkv * ((window + kShare - 1) / kShare)))
@@ -761,8 +760,7 @@ static int decode_check(const void* k_bmp, const void* k_nz, const void* k_idx, 
         !aligned_to(q, 16))
         return MSTF_EALIGN;
     if (workspace_bytes == kWorkspaceIsOurs) return MSTF_OK;  // the library's own buffer: nothing of the caller's to check
-    const size_t need = mstf_decode_attention_workspace_bytes(tokens, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(tokens, 0, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     return MSTF_OK;
 }
@@ -882,8 +880,7 @@ extern "C" int mstf_decode_attention_merge_f16(void* stream, const void* workspa
     if (!out) return MSTF_EINVAL;
     if (tokens <= 0 || Bq <= 0 || groups <= 0 || Bq % groups != 0) return MSTF_EINVAL;
     if (head_dim != kFusedD || tokens % 64 != 0 || groups > 8) return MSTF_EUNSUPPORTED;
-    const size_t need = mstf_decode_attention_workspace_bytes(tokens, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(tokens, 0, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16) || !aligned_to(out, 2) || (lse_out && !aligned_to(lse_out, 4))) return MSTF_EALIGN;
     return merge_splits(as_stream(stream), workspace, out, lse_out, decode_plan(tokens, Bq, groups, false, 0, false).ns, head_dim,
                         Bq);
@@ -904,7 +901,8 @@ extern "C" int mstf_decode_attention_f16(void* stream, const uint64_t* k_bmp, co
     // (up to 512 tokens one launch without a merge: sharing would make it two, 10.1 -> 7.8 us from a graph but 11.1 -> 14.4
     // launched call by call)
     const bool one_launch = fused_nsplit(tokens) == 1 && !lse_out;
-    const DecodePlan plan = decode_plan(tokens, Bq, groups, false, 0, !one_launch);
+    const DecodePlan plan = decode_plan(tokens, Bq, groups, false, 0,
+                                        !one_launch && fused_share_fits(tokens, 0, Bq, workspace_bytes));
     const int write_final = (!plan.shared && plan.ns == 1 && !lse_out) ? 1 : 0;
     rc = decode_launch(as_stream(stream), plan, k_bmp, k_nz, k_idx, k_nz_off, v_bmp, v_nz, v_idx, v_nz_off, q, out, tokens,
                        head_dim, Bq, groups, workspace, write_final);
@@ -954,11 +952,10 @@ extern "C" int mstf_decode_attention_static_f16(void* stream, const uint64_t* k_
     // sizes first, on the host alone: a problem whose partials do not fit is refused before anything touches the GPU
     if (tokens <= 0 || Bq <= 0 || groups <= 0 || Bq % groups != 0) return MSTF_EINVAL;
     if (head_dim != kFusedD || tokens % 64 != 0 || groups > 8) return MSTF_EUNSUPPORTED;
-    // (a launch whose wavefronts share blocks has more splits; where they do not fit it goes without sharing)
-    const auto bytes = [&](int ns) { return round_up((size_t)Bq * ns * (head_dim + 2) * sizeof(float), 256); };
-    if (bytes(fused_nsplit(tokens)) > kStaticScratchBytes) return MSTF_ETOOLARGE;
-    const bool share = bytes(fused_nsplit_room(tokens, Bq / groups, groups)) <= kStaticScratchBytes &&
-                       (fused_nsplit(tokens) > 1 || lse_out);
+    if (fused_workspace_need(tokens, 0, Bq) > kStaticScratchBytes) return MSTF_ETOOLARGE;
+    static_assert(fused_slot_bytes(4 * fused_share_launch(4)) <= kStaticScratchBytes &&
+                      fused_slot_bytes(8 * fused_share_launch(8)) <= kStaticScratchBytes, "room for every launch that shares blocks");
+    const bool share = fused_nsplit(tokens) > 1 || lse_out;
     void* ws = nullptr;
     int rc = decode_check(k_bmp, k_nz, k_idx, k_nz_off, v_bmp, v_nz, v_idx, v_nz_off, q, tokens, head_dim, Bq, groups,
                           nullptr, kWorkspaceIsOurs);
@@ -980,8 +977,7 @@ extern "C" size_t mstf_decode_attention_window_workspace_bytes(int tokens, int m
     if (tokens < 0 || max_window <= 0 || head_dim != kFusedD || Bq <= 0 || groups <= 0 || tokens % 64 != 0 ||
         Bq % groups != 0)
         return 0;
-    const int nst = (tokens > 0 ? fused_nsplit_room(tokens, Bq / groups, groups) : 0) + window_blocks(max_window);
-    return round_up((size_t)Bq * nst * (head_dim + 2) * sizeof(float), 256);
+    return fused_workspace_room(tokens, max_window, Bq, groups);
 }
 
 extern "C" int mstf_decode_attention_window_f16(void* stream, const uint64_t* k_bmp, const mstf_half* k_nz,
@@ -1000,10 +996,10 @@ extern "C" int mstf_decode_attention_window_f16(void* stream, const uint64_t* k_
     if (!aligned_to(q, 16) || !aligned_to(k_win, 16) || !aligned_to(v_win, 16) || !aligned_to(out, 2) ||
         (lse_out && !aligned_to(lse_out, 4)) || (win_len_dev && !aligned_to(win_len_dev, 4)))
         return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_window_workspace_bytes(tokens, win_len, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
-    const DecodePlan plan = tokens > 0 ? decode_plan(tokens, Bq, groups, false) : DecodePlan{false, 1, 0, 0};
+    const bool share = fused_share_fits(tokens, win_len, Bq, workspace_bytes);
+    const DecodePlan plan = tokens > 0 ? decode_plan(tokens, Bq, groups, false, 0, share) : DecodePlan{false, 1, 0, 0};
     const int ns = plan.ns, nst = ns + window_blocks(win_len);
     int rc;
     if (tokens > 0) {
@@ -1038,11 +1034,11 @@ extern "C" int mstf_decode_attention_window_pool_f16(void* stream, const uint64_
     if (!aligned_to(q, 16) || !aligned_to(k_win, 16) || !aligned_to(v_win, 16) || !aligned_to(out, 2) ||
         (lse_out && !aligned_to(lse_out, 4)) || (win_len_dev && !aligned_to(win_len_dev, 4)) || !aligned_to(tokens_dev, 4))
         return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_window_workspace_bytes(max_tokens, win_len, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(max_tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     // (planned with the window, though its blocks are a launch of their own here: as mstf_decode_step_pool_f16 does it)
-    const DecodePlan plan = decode_plan(max_tokens, Bq, groups, true, window_blocks(win_len));
+    const DecodePlan plan = decode_plan(max_tokens, Bq, groups, true, window_blocks(win_len),
+                                        fused_share_fits(max_tokens, win_len, Bq, workspace_bytes));
     const int ns = plan.ns, nst = ns + window_blocks(win_len);
     int rc = decode_check(k_bmp, k_nz, k_idx, k_nz_off, v_bmp, v_nz, v_idx, v_nz_off, q, max_tokens, head_dim, Bq, groups,
                           workspace, workspace_bytes);
@@ -1082,13 +1078,13 @@ extern "C" int mstf_decode_step_pool_f16(void* stream, const uint64_t* k_bmp, co
         (lse_out && !aligned_to(lse_out, 4)) || (win_len_dev && !aligned_to(win_len_dev, 4)) ||
         !aligned_to(tokens_dev, 4) || !aligned_to(overflow, 4))
         return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_window_workspace_bytes(max_tokens, win_len, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(max_tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     int rc = decode_check(k_bmp, k_nz, k_idx, k_nz_off, v_bmp, v_nz, v_idx, v_nz_off, q_in, max_tokens, head_dim, Bq, groups,
                           workspace, workspace_bytes);
     if (rc != MSTF_OK) return rc;
-    const DecodePlan plan = decode_plan(max_tokens, Bq, groups, true, window_blocks(win_len));
+    const DecodePlan plan = decode_plan(max_tokens, Bq, groups, true, window_blocks(win_len),
+                                        fused_share_fits(max_tokens, win_len, Bq, workspace_bytes));
     const int nst = plan.ns + window_blocks(win_len);
     StepArgs sa = {};
     sa.q_in = reinterpret_cast<const _Float16*>(q_in);

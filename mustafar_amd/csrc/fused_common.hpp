@@ -100,15 +100,34 @@ constexpr BlockRange fused_blocks_of(int nblk, int deal, int split, int wave)
 // 512 12.8 -> 9.8, 1024 12.9 -> 11.6 us; two wavefronts per block at 1536 and 2048 blocks 13.9 -> 14.2 and 13.8 -> 14.6.
 // The merge has a split per block then, eight times as many: beyond 128 blocks per head its round trips outweigh the gain
 // (3 heads x 256 blocks 14.6 -> 15.3, 1 x 512 17.0 -> 20.2).
+constexpr int kShareMaxBlocks = 128;                                            // token blocks of a head
+constexpr int fused_share_launch(int groups) { return groups <= 4 ? 1024 : 768; }  // of all heads
 constexpr bool fused_shares_blocks(int tokens, int Bkv, int groups, int extra = 0)
 {
-    return tokens <= 128 * 64 && (long long)Bkv * (tokens / 64) + extra <= (groups <= 4 ? 1024 : 768);
+    return tokens <= kShareMaxBlocks * 64 && (long long)Bkv * (tokens / 64) + extra <= fused_share_launch(groups);
 }
-// Split slots per query row that a workspace for up to `tokens` tokens has room for: one per kFusedWaves blocks, or one per
-// block where wavefronts may share blocks.
-constexpr int fused_nsplit_room(int tokens, int Bkv, int groups)
+
+constexpr int window_blocks(int win_len) { return (win_len + 63) / 64; }
+// Bytes of `slots` split slots: kFusedD outputs and (max, sum) each, fp32.
+constexpr size_t fused_slot_bytes(size_t slots) { return (slots * (kFusedD + 2) * sizeof(float) + 255) / 256 * 256; }
+// What a call over `tokens` compressed tokens and a window demands of its workspace: a slot per query row, kFusedWaves blocks
+// and window block.  Grows with every argument, so that a workspace made for the largest call serves the others.
+constexpr size_t fused_workspace_need(int tokens, int window, int Bq)
 {
-    return fused_shares_blocks(tokens, Bkv, groups) ? tokens / 64 : fused_nsplit(tokens);
+    return fused_slot_bytes((size_t)Bq * (fused_nsplit(tokens) + window_blocks(window)));
+}
+// Whether a workspace has room for wavefronts to share blocks, a slot per block; without it a call goes without sharing (the
+// results are the same numbers).
+constexpr bool fused_share_fits(int tokens, int window, int Bq, size_t workspace_bytes)
+{
+    return fused_slot_bytes((size_t)Bq * (tokens / 64 + window_blocks(window))) <= workspace_bytes;
+}
+// The size that the queries answer: what the call demands, or has use for where its wavefronts may share blocks.
+constexpr size_t fused_workspace_room(int tokens, int window, int Bq, int groups)
+{
+    return fused_shares_blocks(tokens, Bq / groups, groups)
+               ? fused_slot_bytes((size_t)Bq * (tokens / 64 + window_blocks(window)))
+               : fused_workspace_need(tokens, window, Bq);
 }
 
 // Launches the merge of ns split slots per query row out of a workspace in the layout of the fused kernels
@@ -121,7 +140,6 @@ int merge_splits(hipStream_t st, const void* workspace, mstf_half* out, float* l
 int window_launch(hipStream_t st, const mstf_half* k_win, const mstf_half* v_win, const mstf_half* q, void* workspace,
                   int win_len, const int32_t* win_len_dev, int win_stride, int head_dim, int Bq, int groups, int nst,
                   int split0);
-constexpr int window_blocks(int win_len) { return (win_len + 63) / 64; }
 
 // Reductions over the sixteen lanes 4b+j (b = 0..15) that hold column j, without LDS round trips: inside a row of
 // sixteen lanes by two rotations (DPP row_ror 4 and 8, folded into the combining instruction), across the four rows by

@@ -407,8 +407,7 @@ static int decode_attention_quant_impl(void* stream, const uint64_t* k_bmp, cons
                          tokens, head_dim, Bq, groups, bit, capacity, dequant_mode);
     if (rc != MSTF_OK) return rc;
     if (!aligned_to(out, 2) || (lse_out && !aligned_to(lse_out, 4))) return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_workspace_bytes(tokens, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(tokens, 0, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
     const int ns = quant_nsplit(tokens, Bq / groups, groups, bit, group_size);
@@ -463,8 +462,7 @@ extern "C" int mstf_decode_attention_window_quant(
     if (!aligned_to(q, 16) || !aligned_to(k_win, 16) || !aligned_to(v_win, 16) || !aligned_to(out, 2) ||
         (lse_out && !aligned_to(lse_out, 4)) || (win_len_dev && !aligned_to(win_len_dev, 4)))
         return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_window_workspace_bytes(tokens, win_len, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
     int rc, ns = 0;
@@ -504,8 +502,7 @@ extern "C" int mstf_decode_attention_window_quant_pool(
         return MSTF_EALIGN;
     // rows of the per-tile arrays start tile_capacity entries apart: the two-byte ones keep their four-byte alignment
     if (tile_capacity % 2 != 0) return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_window_workspace_bytes(max_tokens, win_len, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(max_tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
     int rc = quant_check(k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
@@ -550,8 +547,7 @@ extern "C" int mstf_decode_step_quant_pool(
         (lse_out && !aligned_to(lse_out, 4)) || (win_len_dev && !aligned_to(win_len_dev, 4)) ||
         !aligned_to(tokens_dev, 4) || !aligned_to(overflow, 4))
         return MSTF_EALIGN;
-    const size_t need = mstf_decode_attention_window_workspace_bytes(max_tokens, win_len, head_dim, Bq, groups);
-    if (!workspace || workspace_bytes < need) return MSTF_EWORKSPACE;
+    if (!workspace || workspace_bytes < fused_workspace_need(max_tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     int rc = quant_check(k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros,
                          q_in, max_tokens, head_dim, Bq, groups, bit, capacity, dequant_mode);

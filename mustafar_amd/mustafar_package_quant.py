@@ -138,7 +138,7 @@ def decode_attention_quant(key_side, value_side, q, num_key_value_groups, bit, d
     tokens = kb.shape[1] * 64 // D
     L = lib()
     o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
-    ws = ops.workspace(q.device, L.mstf_decode_attention_workspace_bytes(tokens, D, Bq, num_key_value_groups), ws)
+    ws = ops.workspace(q.device, ops.attention_workspace_least(tokens, 0, Bq), ws)
     group_size = _group_size(kb, ks, kz)
     if _group_size(vb, vs, vz) != group_size:
         raise RuntimeError("key side and value side must use the same group size.")
@@ -173,8 +173,7 @@ def decode_attention_window_quant(key_side, value_side, q, k_win, v_win, win_len
                 vo.data_ptr(), vs.data_ptr(), vz.data_ptr()]
     else:
         tokens, ptrs = 0, [None] * 10
-    ws = ops.workspace(q.device, L.mstf_decode_attention_window_workspace_bytes(tokens, int(win_len), D, Bq,
-                                                                                int(num_key_value_groups)), ws)
+    ws = ops.workspace(q.device, ops.attention_workspace_least(tokens, int(win_len), Bq), ws)
     check(L.mstf_decode_attention_window_quant(
         ops._stream(), *ptrs, q.contiguous().data_ptr(), k_win.data_ptr(), v_win.data_ptr(),
         int(win_len), win_len_dev.data_ptr() if win_len_dev is not None else None, int(k_win.shape[1]), o.data_ptr(),
@@ -195,8 +194,7 @@ def decode_attention_window_quant_pool(k_pool, v_pool, q, k_win, v_win, win_len,
     Bq = q.numel() // D
     L = lib()
     o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
-    ws = ops.workspace(q.device, L.mstf_decode_attention_window_workspace_bytes(k_pool.max_tokens, int(win_len), D, Bq,
-                                                                                int(num_key_value_groups)), ws)
+    ws = ops.workspace(q.device, ops.attention_workspace_least(k_pool.max_tokens, int(win_len), Bq), ws)
     ptrs = []
     for p in (k_pool, v_pool):
         ptrs += [p.bmp_store.data_ptr(), p.packed.data_ptr(), p.off_store.data_ptr(), p.scales_store.data_ptr(),
@@ -235,8 +233,7 @@ def decode_step_quant_pool(k_pool, v_pool, q_in, k_in, v_in, k_win, v_win, win_l
     L = lib()
     Bq = bs * n_q
     o = torch.empty((Bq, D), dtype=torch.float16, device=q_in.device) if out is None else out
-    ws = ops.workspace(q_in.device, L.mstf_decode_attention_window_workspace_bytes(k_pool.max_tokens, int(win_len), D, Bq,
-                                                                                   n_q // n_kv), ws)
+    ws = ops.workspace(q_in.device, ops.attention_workspace_least(k_pool.max_tokens, int(win_len), Bq), ws)
     ptrs = []
     for p in (k_pool, v_pool):
         ptrs += [p.bmp_store.data_ptr(), p.packed.data_ptr(), p.off_store.data_ptr(), p.scales_store.data_ptr(),

@@ -18,7 +18,7 @@ class Workspace:
     call BEFORE capturing and passes it as `ws=`: the buffer then never moves, and calls on different streams with
     different workspaces are independent.  `get` hands out the buffer if it is large enough; growing replaces it but
     keeps the old buffers alive (a captured graph may still point at them), and growing while the current stream is
-    being captured is an error."""
+    being captured is an error - unless it holds the least that an attention call does with, if slower."""
 
     def __init__(self, device, nbytes=1 << 20):
         self.device = torch.device(device)
@@ -38,7 +38,11 @@ class Workspace:
             self._bufs.append(torch.empty(int(nbytes), dtype=torch.uint8, device=self.device))
         return self.tensor
 
-    def get(self, nbytes):
+    def get(self, nbytes, call=None):
+        """call: (tokens, window, rows) of an attention call, which nbytes is the best size for."""
+        if (call is not None and attention_workspace_least(*call) <= self.tensor.numel() < nbytes
+                and torch.cuda.is_current_stream_capturing()):
+            return self.tensor
         return self.reserve(nbytes)
 
 
@@ -66,18 +70,26 @@ def read_word(t):
     return own[2].value
 
 
-def workspace(device, nbytes, ws=None):
+def attention_workspace_least(tokens, window, rows):
+    """Bytes that an attention call over `tokens` compressed tokens and a window demands of its workspace."""
+    return (rows * (-(-tokens // 512) + -(-window // 64)) * 520 + 255) // 256 * 256
+
+
+def workspace(device, nbytes, ws=None, call=None):
     """The scratch tensor for a call that needs nbytes: the caller's Workspace (`ws`) or, for the mirrors of the
     reference's operators, which have no such argument, a default one per (device, stream) - so two streams never
-    share a buffer unless the caller passes the same Workspace to both."""
+    share a buffer unless the caller passes the same Workspace to both.  call: see Workspace.get."""
     if ws is not None:
-        return ws.get(nbytes) if isinstance(ws, Workspace) else ws
+        if not isinstance(ws, Workspace):
+            return ws
+        t = ws.tensor
+        return t if t.numel() >= nbytes else ws.get(nbytes, call)
     device = torch.device(device)
     key = (device.type, device.index if device.index is not None else torch.cuda.current_device(), _stream())
     w = _WS.get(key)
     if w is None:
         w = _WS[key] = Workspace(device)
-    return w.get(nbytes)
+    return w.get(nbytes, call)
 
 
 def kth_from_sparsity(sparsity, head_dim):
@@ -272,7 +284,7 @@ def decode_attention(ck, cv, q, groups, out=None, lse=None, ws=None):
     Bq = q.numel() // D
     L = lib()
     o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
-    ws = workspace(q.device, L.mstf_decode_attention_workspace_bytes(ck.tokens, D, Bq, groups), ws)
+    ws = workspace(q.device, L.mstf_decode_attention_workspace_bytes(ck.tokens, D, Bq, groups), ws, (ck.tokens, 0, Bq))
     check(L.mstf_decode_attention_f16(_stream(), ck.bmp.data_ptr(), ck.nz.data_ptr(), ck.idx.data_ptr(),
                                       ck.nz_off.data_ptr(), cv.bmp.data_ptr(), cv.nz.data_ptr(), cv.idx.data_ptr(),
                                       cv.nz_off.data_ptr(), q.data_ptr(), o.data_ptr(),
@@ -309,7 +321,8 @@ def decode_attention_window(ck, cv, q, k_win, v_win, win_len, groups, out=None, 
     tokens = ck.tokens if ck is not None else 0
     L = lib()
     o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
-    ws = workspace(q.device, L.mstf_decode_attention_window_workspace_bytes(tokens, int(win_len), D, Bq, groups), ws)
+    ws = workspace(q.device, L.mstf_decode_attention_window_workspace_bytes(tokens, int(win_len), D, Bq, groups), ws,
+                   (tokens, int(win_len), Bq))
     cp = [t.data_ptr() for t in (ck.bmp, ck.nz, ck.idx, ck.nz_off, cv.bmp, cv.nz, cv.idx, cv.nz_off)] if tokens else [None] * 8
     check(L.mstf_decode_attention_window_f16(_stream(), *cp, q.data_ptr(), k_win.data_ptr(), v_win.data_ptr(), int(win_len),
                                              win_len_dev.data_ptr() if win_len_dev is not None else None,
@@ -332,7 +345,8 @@ def decode_attention_window_pool(k_pool, v_pool, q, k_win, v_win, win_len, group
     L = lib()
     o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
     ws = workspace(q.device, L.mstf_decode_attention_window_workspace_bytes(k_pool.max_tokens, int(win_len), D, Bq,
-                                                                           groups), ws)
+                                                                           groups), ws,
+                   (k_pool.max_tokens, int(win_len), Bq))
     cp = [t.data_ptr() for t in (k_pool.bmp_store, k_pool.nz, k_pool.idx_store, k_pool.nz_off, v_pool.bmp_store, v_pool.nz,
                                  v_pool.idx_store, v_pool.nz_off)]
     check(L.mstf_decode_attention_window_pool_f16(_stream(), *cp, q.data_ptr(), k_win.data_ptr(), v_win.data_ptr(),
@@ -370,7 +384,8 @@ def decode_step_pool(k_pool, v_pool, q_in, k_in, v_in, k_win, v_win, win_len, co
     Bq = bs * n_q
     o = torch.empty((Bq, D), dtype=torch.float16, device=q_in.device) if out is None else out
     ws = workspace(q_in.device, L.mstf_decode_attention_window_workspace_bytes(k_pool.max_tokens, int(win_len), D, Bq,
-                                                                              n_q // n_kv), ws)
+                                                                              n_q // n_kv), ws,
+                   (k_pool.max_tokens, int(win_len), Bq))
     cp = [t.data_ptr() for t in (k_pool.bmp_store, k_pool.nz, k_pool.idx_store, k_pool.nz_off, v_pool.bmp_store, v_pool.nz,
                                  v_pool.idx_store, v_pool.nz_off)]
     check(L.mstf_decode_step_pool_f16(
@@ -427,7 +442,7 @@ def decode_attention_partial(ck, cv, q, groups, ws=None):
     D = ck.head_dim
     Bq = q.numel() // D
     L = lib()
-    ws = workspace(q.device, L.mstf_decode_attention_workspace_bytes(ck.tokens, D, Bq, groups), ws)
+    ws = workspace(q.device, attention_workspace_least(ck.tokens, 0, Bq), ws)
     check(L.mstf_decode_attention_partial_f16(_stream(), ck.bmp.data_ptr(), ck.nz.data_ptr(), ck.idx.data_ptr(),
                                               ck.nz_off.data_ptr(), cv.bmp.data_ptr(), cv.nz.data_ptr(),
                                               cv.idx.data_ptr(), cv.nz_off.data_ptr(), q.data_ptr(), ck.tokens, D, Bq,

@@ -85,6 +85,22 @@ def test_argument_validation_returns_before_any_launch(lib):
     assert L.mstf_compress_quant_workspace_bytes(0, 64, 128) == 0
 
 
+def test_attention_workspaces():
+    """The queries never answer less than the calls demand, a slot of 520 bytes per row and 512 tokens or window block
+    (which grows with the call), and the bindings ask a workspace for no more than that where it cannot grow."""
+    from mustafar_amd import _lib, ops
+    L = _lib.lib()
+    for g in range(1, 9):
+        for t in (64, 512, 4096, 8128, 8192, 8256, 16384, 65536):
+            for h in (1, 2, 7, 8, 9, 16, 17, 64, 256, 1100):
+                least = -(-h * g * -(-t // 512) * 520 // 256) * 256
+                assert ops.attention_workspace_least(t, 0, h * g) == least <= L.mstf_decode_attention_workspace_bytes(t, 128, h * g, g)
+                for w in (1, 64, 65, 512, 20480):
+                    least = -(-h * g * (-(-t // 512) + -(-w // 64)) * 520 // 256) * 256
+                    assert ops.attention_workspace_least(t, w, h * g) == least <= \
+                        L.mstf_decode_attention_window_workspace_bytes(t, w, 128, h * g, g)
+
+
 def test_host_helpers():
     from mustafar_amd import ops
     assert [ops.kth_from_sparsity(s, 128) for s in (0.5, 0.7, 0.9, 0.0)] == [64, 89, 115, 1]

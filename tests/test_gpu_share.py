@@ -65,3 +65,58 @@ def test_pooled_step_equals_the_calls_it_fuses(bs, n_kv, groups, tokens, bit):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.equal(one, two)
     n = int(wlen)
     assert torch.equal(kb[:, :n], a._kbuf[:, :n]) and torch.equal(vb[:, :n], a._vbuf[:, :n])
+
+
+@pytest.mark.parametrize("heads,groups,tokens", [(8, 4, 512), (8, 4, 4096), (2, 8, 4096), (17, 4, 3840)])
+def test_a_workspace_without_room_for_sharing_serves_the_call(heads, groups, tokens):
+    """The least a call demands - a slot per 512 tokens and row, what a workspace made for a longer context or more rows
+    may come to - gives the same numbers as the size the query answers."""
+    from mustafar_amd import compression_quant as cq, mustafar_package_quant as mpq, ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(tokens + groups)
+    K, V = kv(gen, heads, tokens)
+    ck, cv = ops.compress(K, False, kth=89), ops.compress(V, True, kth=89)
+    rows, n = heads * groups, -(-tokens // 512)
+    q = torch.randn((rows, D), generator=gen, device="cuda", dtype=torch.float16)
+
+    def least(slots):
+        return torch.empty(-(-rows * slots * 520 // 256) * 256, dtype=torch.uint8, device="cuda")
+    lse, lse2 = (torch.empty((rows, 2), device="cuda") for _ in range(2))
+    assert torch.equal(ops.decode_attention(ck, cv, q, groups, lse=lse, ws=least(n)),
+                       ops.decode_attention(ck, cv, q, groups, lse=lse2)) and torch.equal(lse, lse2)
+    ws = ops.decode_attention_partial(ck, cv, q, groups, ws=least(n))
+    assert torch.equal(ops.decode_attention_merge(ws, tokens, D, rows, groups), ops.decode_attention(ck, cv, q, groups))
+    kw, vw = kv(gen, heads, 320)
+    assert torch.equal(ops.decode_attention_window(ck, cv, q, kw, vw, 300, groups, ws=least(n + 5)),
+                       ops.decode_attention_window(ck, cv, q, kw, vw, 300, groups))
+    k, v = cq.convert_key_batched_quant(K, True, 2, kth=89), cq.convert_value_batched_quant(V, 2, kth=89)
+    assert torch.equal(mpq.decode_attention_quant(k, v, q, groups, 2, ws=least(n)),
+                       mpq.decode_attention_quant(k, v, q, groups, 2))
+    with pytest.raises(RuntimeError):
+        ops.decode_attention(ck, cv, q, groups, ws=least(n)[:-256])
+
+
+def test_a_workspace_reserved_for_the_longest_context_holds_in_a_capture():
+    """`Workspace` sized before the capture for 8256 tokens of 8 heads, which do not share; the shorter calls, which would
+    like more room than that, are captured with it."""
+    from mustafar_amd import ops
+    from mustafar_amd._lib import lib
+    heads, groups = 8, 4
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    ws = ops.Workspace("cuda", lib().mstf_decode_attention_workspace_bytes(8256, D, heads * groups, groups))
+    assert ws.tensor.numel() < lib().mstf_decode_attention_workspace_bytes(8192, D, heads * groups, groups)
+    q = torch.randn((heads * groups, D), generator=gen, device="cuda", dtype=torch.float16)
+    sides = []
+    for tokens in (1024, 8192):
+        K, V = kv(gen, heads, tokens)
+        sides.append((ops.compress(K, False, kth=89), ops.compress(V, True, kth=89)))
+    want = [ops.decode_attention(k, v, q, groups) for k, v in sides]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = [ops.decode_attention(k, v, q, groups, ws=ws) for k, v in sides]
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
