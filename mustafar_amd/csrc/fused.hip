@@ -439,7 +439,10 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_kernel(const 
 // The same over `blocks` slots of one token block each, with nsplit - blocks ordinary splits (the window's) behind them.
 // First the groups make eight blocks each into what the workgroup combine of the fused kernel makes of them, a split of
 // 512 tokens, left in LDS; then these splits are merged in the order and by the groups of decode_merge_kernel, so that the
-// results are the same numbers.  Dynamic LDS: 130 floats per split of 512 tokens or window block.
+// results are the same numbers.  Dynamic LDS: 130 floats for each of the first kMergeKept units (a split of 512 tokens or a
+// window block); the window blocks behind those - the window may have any length - are read from their slots.
+constexpr int kMergeKept = 64;
+static_assert(kMergeKept % kMergeRun == 0 && kMergeKept >= kShareMaxBlocks / kFusedWaves, "whole runs, all made units");
 constexpr int merge_blocks_units(int nsplit, int blocks) { return (blocks + kFusedWaves - 1) / kFusedWaves + nsplit - blocks; }
 __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel(const float* __restrict__ part_o,
                                                                                  const float* __restrict__ part_ml,
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
 {
     constexpr int G = kMergeRun, W = kFusedWaves;
     __shared__ MergeLds sh;
-    extern __shared__ float unit[];  // [units][128] outputs, [units][2] (max, sum)
+    extern __shared__ float unit[];  // [kept][128] outputs, [kept][2] (max, sum)
     const size_t row = blockIdx.x;
     const int t = (int)threadIdx.x & 127;
     const int group = (int)threadIdx.x >> 7;
@@ -457,8 +460,9 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
     const float2* ml = reinterpret_cast<const float2*>(part_ml) + row * nsplit;
     const float* po = part_o + row * nsplit * D + c;
     const int whole = (blocks + W - 1) / W, units = merge_blocks_units(nsplit, blocks);
-    float2* unit_ml = reinterpret_cast<float2*>(unit + (size_t)units * 128);
-    for (int u = group; u < units; u += (int)blockDim.x >> 7) {
+    const int kept = units < kMergeKept ? units : kMergeKept;
+    float2* unit_ml = reinterpret_cast<float2*>(unit + (size_t)kept * 128);
+    for (int u = group; u < kept; u += (int)blockDim.x >> 7) {
         float M = -INFINITY, so = 0.f, sl = 0.f;
         if (u < whole) {
             float m[W], l[W], o[W];
@@ -494,13 +498,24 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
     if (group < groups) {
         for (int s0 = group * G; s0 < units; s0 += groups * G) {
             float m[G], l[G], o[G];
+            if (s0 < kept) {
 #pragma unroll
-            for (int k = 0; k < G; k++) {
-                const int i = s0 + k < units ? s0 + k : units - 1;
-                const float2 v = unit_ml[i];
-                m[k] = v.x;
-                l[k] = v.y;
-                o[k] = unit[i * 128 + t];
+                for (int k = 0; k < G; k++) {
+                    const int i = s0 + k < units ? s0 + k : units - 1;
+                    const float2 v = unit_ml[i];
+                    m[k] = v.x;
+                    l[k] = v.y;
+                    o[k] = unit[i * 128 + t];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < G; k++) {
+                    const int i = blocks - whole + (s0 + k < units ? s0 + k : units - 1);
+                    const float2 v = ml[i];
+                    m[k] = v.x;
+                    l[k] = v.y;
+                    o[k] = po[(size_t)i * D];
+                }
             }
             merge_run(s, m, l, o, units - s0);
         }
@@ -823,8 +838,9 @@ int mstf::merge_splits(hipStream_t st, const void* workspace, mstf_half* out, fl
     if (blocks > 0) {
         const int units = merge_blocks_units(ns, blocks);
         const int threads = 128 * (units < kMergeGroups ? units : kMergeGroups);
-        hipLaunchKernelGGL(decode_merge_blocks_kernel, dim3((unsigned)Bq), dim3(threads), (size_t)units * 130 * sizeof(float),
-                           st, part_o, part_ml, oh, lse_out, ns, blocks, head_dim);
+        const size_t kept = (size_t)(units < kMergeKept ? units : kMergeKept);
+        hipLaunchKernelGGL(decode_merge_blocks_kernel, dim3((unsigned)Bq), dim3(threads), kept * 130 * sizeof(float), st,
+                           part_o, part_ml, oh, lse_out, ns, blocks, head_dim);
     } else {
         const int runs = (ns + kMergeRun - 1) / kMergeRun;
         const int threads = 128 * (runs < kMergeGroups ? runs : kMergeGroups);

@@ -120,3 +120,40 @@ def test_a_workspace_reserved_for_the_longest_context_holds_in_a_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+# window rows: splits of 512 tokens and window blocks on both sides of the 64 that the merge keeps in LDS, and far beyond
+@pytest.mark.parametrize("heads,groups,tokens,window", [(1, 4, 512, 63 * 64), (1, 4, 512, 63 * 64 + 1), (3, 2, 8192, 48 * 64 + 5),
+                                                        (1, 8, 64, 6000), (2, 4, 512, 20480)])
+def test_a_long_window_behind_shared_blocks(heads, groups, tokens, window):
+    from mustafar_amd import ops
+    from mustafar_amd.cache import CompressedPool, append_pair
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(window + groups)
+    K, V = kv(gen, heads, tokens)
+    kw, vw = kv(gen, heads, window)
+    rows = heads * groups
+    proj = torch.randn((1, (rows + 2 * heads) * D), generator=gen, device="cuda", dtype=torch.float16)
+    q, k_in, v_in = proj[:, :rows * D], proj[:, rows * D:(rows + heads) * D], proj[:, (rows + heads) * D:]
+    kw[:, -1], vw[:, -1] = k_in.view(heads, D), v_in.view(heads, D)
+    q = q.contiguous().view(rows, D)
+    ck, cv = ops.compress(K, False, kth=89), ops.compress(V, True, kth=89)
+    one, two, three = (torch.empty((rows, 2), device="cuda") for _ in range(3))
+    got = ops.decode_attention_window(ck, cv, q, kw, vw, window, groups, lse=one)
+    least = torch.empty(ops.attention_workspace_least(tokens, window, rows), dtype=torch.uint8, device="cuda")
+    assert torch.equal(got, ops.decode_attention_window(ck, cv, q, kw, vw, window, groups, lse=two, ws=least))
+    assert torch.equal(one, two)
+    # the step over pools of the same tokens, which appends the last row of the window itself
+    kp, vp = CompressedPool(heads, D, tokens, False, "cuda"), CompressedPool(heads, D, tokens, True, "cuda")
+    append_pair(kp, vp, K, V, 89, 89)
+    kb, vb = kw.clone(), vw.clone()
+    kb[:, -1], vb[:, -1] = 0, 0
+    step = ops.decode_step_pool(kp, vp, q.view(1, -1), k_in, v_in, kb, vb, window, lse=three)
+    assert torch.equal(step.view(rows, D), got) and torch.equal(one, three)
+    assert torch.equal(kb, kw) and torch.equal(vb, vw)
+    keys = torch.cat([ops.prune_rows(K, 89), kw], 1).float().repeat_interleave(groups, 0)
+    values = torch.cat([ops.prune_rows(V, 89), vw], 1).float().repeat_interleave(groups, 0)
+    s = torch.matmul(keys, q.float().view(rows, D, 1))[..., 0].half()
+    want = torch.matmul(torch.softmax((s / D ** 0.5).float(), -1).view(rows, 1, -1), values)[:, 0]
+    # weights and outputs rounded to fp16, a score rounded to the neighbouring fp16 value now and then (test_gpu_deal.py)
+    assert float((got.float() - want).norm(dim=-1).div(want.norm(dim=-1)).max()) < 5e-3
