@@ -182,7 +182,9 @@ int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value
  * K = head_dim (128), Bq = query heads x batch, groups = query heads per KV head.
  * n_rows = 8 reproduces the reference operator (its N is hard-wired to 8, mustafar_wrapper.cu:125);
  * n_rows = 1 is the decode fast path without the 7 padding rows.
- * Every compressed byte is read once per KV head, not once per query head. */
+ * Every compressed byte is read once per KV head, not once per query head.
+ * Absent elements are zeros that are multiplied: an infinite weight gives NaN with them.  With eight rows per KV head or more
+ * it gives an infinity with a kept element; with one to four the element's neighbours make that a NaN, too. */
 int mstf_key_spmv_f16(void* stream, const uint64_t* bmp, const mstf_half* nz, const uint32_t* idx,
                       const uint32_t* nz_off, const mstf_half* Bm, mstf_half* C, int M, int K, int Bq, int groups,
                       int n_rows);

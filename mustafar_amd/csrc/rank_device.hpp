@@ -167,13 +167,15 @@ __device__ __forceinline__ RankTable rank_table(const char* room, int lane)
         [wa] "v"(wa), [woff] "i"(WOFF)
 #define MSTF_RLOAD "s_load_dwordx16 %[nm], %[nb], %[boff]\n\t"
 
-// Batch G into acc[m][P] for at most eight accumulators, by 4x4x4 products: the register pair (t0, 0, t2, 0) and the
-// pair (0, t1, 0, t3) both against the weights (w0 .. w3) of the lane's four tiles, so that no vector instruction packs.
+// Batch G into acc[m][P] for at most eight accumulators, by 4x4x4 products.  Four: the register pair (t0, 0, t2, 0) and
+// the pair (0, t1, 0, t3) both against the weights (w0 .. w3) of the lane's four tiles, so that no vector instruction
+// packs - and an infinite weight makes a NaN of a tile's neighbour as it does of an absent element, 0 x inf.  Eight: the
+// pairs are merged first, two vector instructions for two products less; only absent elements meet a zero then.
 //   mv      : the batch's eight bitmaps;  PREFETCH: those of the coming batch are requested at nbm + BOFF bytes
 //   I0, IS  : immediate offset of the batch's first tile and bytes between two tiles (0, 0: `at` is the full address)
 //   wa, wb  : LDS address of w[lane & 3][4 * (lane >> 5)] of the first tile of the stage, for the accumulators 0 .. 3
 //             and (NM = 2) 4 .. 7;  WOFF: + bytes to the batch's first tile
-// The order of the products keeps two of one accumulator at least two instructions apart, and the statement ends
+// Two products of one accumulator are at least two instructions apart, and the statement ends
 // with the wait states that an ordinary vector instruction needs before it may read a sum.
 template <int NM, bool PREFETCH, int G, int BOFF, int I0, int IS, int WOFF>
 __device__ __forceinline__ void rank_batch(const u32x16_t& mv, u32x16_t& nxt, const uint64_t* nbm, const RankAddr& a,
@@ -188,9 +190,10 @@ __device__ __forceinline__ void rank_batch(const u32x16_t& mv, u32x16_t& nxt, co
     MSTF_RM("p1", MSTF_GV6_7, "w") "s_nop 4"
 #define MSTF_RTWO                                                                                                     \
     MSTF_RCLEAR "ds_read_b64 %[w], %[wa] offset:%[woff]\n\tds_read_b64 %[w2], %[wb] offset:%[woff]\n\t" MSTF_RGATHER  \
-    MSTF_RM("p0", MSTF_GV0_1, "w") MSTF_RM("q0", MSTF_GV0_1, "w2") "s_waitcnt lgkmcnt(0)\n\t"                         \
-    MSTF_RM("p1", MSTF_GV4_5, "w") MSTF_RM("q1", MSTF_GV4_5, "w2") MSTF_RM("p0", MSTF_GV2_3, "w")                     \
-    MSTF_RM("q0", MSTF_GV2_3, "w2") MSTF_RM("p1", MSTF_GV6_7, "w") MSTF_RM("q1", MSTF_GV6_7, "w2") "s_nop 4"
+    "v_or_b32 " MSTF_GV0 ", " MSTF_GV0 ", " MSTF_GV2 "\n\tv_or_b32 " MSTF_GV1 ", " MSTF_GV1 ", " MSTF_GV3 "\n\t"        \
+    "s_nop 1\n\t" MSTF_RM("p0", MSTF_GV0_1, "w") MSTF_RM("q0", MSTF_GV0_1, "w2") "s_waitcnt lgkmcnt(0)\n\t"          \
+    "v_or_b32 " MSTF_GV4 ", " MSTF_GV4 ", " MSTF_GV6 "\n\tv_or_b32 " MSTF_GV5 ", " MSTF_GV5 ", " MSTF_GV7 "\n\t"        \
+    "s_nop 1\n\t" MSTF_RM("p1", MSTF_GV4_5, "w") MSTF_RM("q1", MSTF_GV4_5, "w2") "s_nop 4"
     if constexpr (NM == 1) {
         if constexpr (PREFETCH)
             asm volatile(MSTF_RLOAD MSTF_RONE
