@@ -444,6 +444,8 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_kernel(const 
 constexpr int kMergeKept = 64;
 static_assert(kMergeKept % kMergeRun == 0 && kMergeKept >= kShareMaxBlocks / kFusedWaves, "whole runs, all made units");
 constexpr int merge_blocks_units(int nsplit, int blocks) { return (blocks + kFusedWaves - 1) / kFusedWaves + nsplit - blocks; }
+// LONG: there are units behind the kept ones.
+template <bool LONG>
 __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel(const float* __restrict__ part_o,
                                                                                  const float* __restrict__ part_ml,
                                                                                  _Float16* __restrict__ out,
@@ -460,7 +462,7 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
     const float2* ml = reinterpret_cast<const float2*>(part_ml) + row * nsplit;
     const float* po = part_o + row * nsplit * D + c;
     const int whole = (blocks + W - 1) / W, units = merge_blocks_units(nsplit, blocks);
-    const int kept = units < kMergeKept ? units : kMergeKept;
+    const int kept = LONG ? kMergeKept : units;
     float2* unit_ml = reinterpret_cast<float2*>(unit + (size_t)kept * 128);
     for (int u = group; u < kept; u += (int)blockDim.x >> 7) {
         float M = -INFINITY, so = 0.f, sl = 0.f;
@@ -498,7 +500,7 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
     if (group < groups) {
         for (int s0 = group * G; s0 < units; s0 += groups * G) {
             float m[G], l[G], o[G];
-            if (s0 < kept) {
+            if (!LONG || s0 < kept) {
 #pragma unroll
                 for (int k = 0; k < G; k++) {
                     const int i = s0 + k < units ? s0 + k : units - 1;
@@ -838,9 +840,10 @@ int mstf::merge_splits(hipStream_t st, const void* workspace, mstf_half* out, fl
     if (blocks > 0) {
         const int units = merge_blocks_units(ns, blocks);
         const int threads = 128 * (units < kMergeGroups ? units : kMergeGroups);
-        const size_t kept = (size_t)(units < kMergeKept ? units : kMergeKept);
-        hipLaunchKernelGGL(decode_merge_blocks_kernel, dim3((unsigned)Bq), dim3(threads), kept * 130 * sizeof(float), st,
-                           part_o, part_ml, oh, lse_out, ns, blocks, head_dim);
+        const bool rest = units > kMergeKept;
+        hipLaunchKernelGGL((rest ? decode_merge_blocks_kernel<true> : decode_merge_blocks_kernel<false>), dim3((unsigned)Bq),
+                           dim3(threads), (size_t)(rest ? kMergeKept : units) * 130 * sizeof(float), st, part_o, part_ml, oh,
+                           lse_out, ns, blocks, head_dim);
     } else {
         const int runs = (ns + kMergeRun - 1) / kMergeRun;
         const int threads = 128 * (runs < kMergeGroups ? runs : kMergeGroups);
