@@ -142,7 +142,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
     const char* wsrc = reinterpret_cast<const char*>(Bm + ((size_t)kv * rows_per_kv + row0) * D);
     char* my = lds + (kShared ? kRowsLds : 0) + wave * kWaveLds;
     char* wl = kShared ? lds : my + kQ;             // the rows; what lies behind row NW - 1 stays unwritten
-    const uint32_t wbytes = (uint32_t)NW * D * 2u;
 
     Sums sums;
     sums.clear();
@@ -151,16 +150,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
     const uint32_t wrow = Sums::waddr(lds_addr(wl), rbytes, lane);
     auto stage_rows = [=](int n) {
         if (n != 0) return;  // the query rows are staged once per task
-        constexpr int kPieces = (NW * kMaxD * 2 + 1023) / 1024, kMine = kShared ? kPieces / 4 : kPieces;
-        static_assert(!kShared || kPieces % 4 == 0, "the four wavefronts fetch equal shares");
-#pragma unroll
-        for (int k = 0; k < kMine; k++) {
-            const int i = kShared ? wave * kMine + k : k;
-            const uint32_t o = (uint32_t)(i * 64 + lane) * 16u;
-            uint32_t from = o;
-            if (kShared) from ^= weight_swizzle((int)(o / rbytes), (int)rbytes / 16) * 16u;
-            if (o < wbytes) dma16(wsrc + from, wl + i * 1024);
-        }
+        stage_key_rows<NW, 4, kShared>(wsrc, rbytes, wl, wave, lane);
     };
     if (kShared && tb >= nblk) {  // (wave-uniform) no block left, but a share of the rows
         stage_rows(0);
@@ -364,8 +354,9 @@ static int key_spmv_quant_impl(void* stream, const uint64_t* bmp, const uint32_t
     const _Float16* b = reinterpret_cast<const _Float16*>(Bm);
     _Float16* c = reinterpret_cast<_Float16*>(C);
     const QArgs a = {bmp, packed, tile_off, scales, zeros, dequant_mode, group_size};
+    const bool lines = aligned_to(C, 16);     // (the rows of a wide pass leave as whole lines)
     for (int row0 = 0; row0 < rows_per_kv;) {
-        const int nw = pick_nw(rows_per_kv - row0);
+        const int nw = pick_nw(rows_per_kv - row0, lines);
         switch (nw) {
             case 32: launch_key_q_bit<32>(bit, st, a, b, c, M, K, Bkv, rows_per_kv, row0); break;
             case 16: launch_key_q_bit<16>(bit, st, a, b, c, M, K, Bkv, rows_per_kv, row0); break;
@@ -426,9 +417,11 @@ static int value_spmv_quant_impl(void* stream, const uint64_t* bmp, const uint32
     _Float16* c = reinterpret_cast<_Float16*>(C);
     float* part = reinterpret_cast<float*>(workspace);
     const QArgs a = {bmp, packed, tile_off, scales, zeros, dequant_mode, group_size};
+    const bool pieces = aligned_to(P, 16);    // (a wide pass fetches the weights in pieces of sixteen bytes)
+    const int most = pieces ? kAnySplits : splits_that_fit(workspace ? workspace_bytes : 0, M, Bq, n_rows);
     for (int row0 = 0; row0 < rows_per_kv;) {
-        const int nw = pick_nw(rows_per_kv - row0);
-        const ValuePlan pl = plan_value(K, M, Bkv, nw);
+        const int nw = pick_nw(rows_per_kv - row0, pieces);
+        const ValuePlan pl = plan_value(K, M, Bkv, nw, most);
         switch (nw) {
             case 32: launch_value_q_bit<32, 4>(bit, st, pl, a, p, c, part, K, M, Bkv, rows_per_kv, row0); break;
             case 16: launch_value_q_bit<16, 4>(bit, st, pl, a, p, c, part, K, M, Bkv, rows_per_kv, row0); break;

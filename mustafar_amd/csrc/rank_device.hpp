@@ -422,6 +422,35 @@ __device__ __forceinline__ void stage_rows_wide(const _Float16* src, size_t stri
     }
 }
 
+// Requests the NW query rows of a key product, rbytes each and contiguous at src, into [row][rbytes] at dst.  SHARED: the
+// WAVES wavefronts of the workgroup fetch equal shares, and the sixteen-byte pieces go where weight_swizzle wants them.
+// Rows that do not start at a multiple of sixteen bytes come four bytes a lane.
+template <int NW, int WAVES, bool SHARED>
+__device__ __forceinline__ void stage_key_rows(const char* src, uint32_t rbytes, char* dst, int wave, int lane)
+{
+    constexpr int kPieces = (NW * 128 * 2 + 1023) / 1024, kMine = SHARED ? (kPieces + WAVES - 1) / WAVES : kPieces;
+    static_assert(!SHARED || kPieces % WAVES == 0 || kMine == 1, "equal shares, or a piece each for some wavefronts");
+    const uint32_t bytes = (uint32_t)NW * rbytes;
+    auto from = [=](uint32_t o) {
+        return SHARED ? o ^ weight_swizzle((int)(o / rbytes), (int)rbytes / 16) * 16u : o;
+    };
+    const bool whole = ((uintptr_t)src & 15u) == 0;  // (wave-uniform)
+#pragma unroll
+    for (int k = 0; k < kMine; k++) {
+        const int i = SHARED ? wave * kMine + k : k;
+        if (__builtin_expect(whole, 1)) {
+            const uint32_t o = (uint32_t)(i * 64 + lane) * 16u;
+            if (o < bytes) dma16(src + from(o), dst + i * 1024);
+        } else {
+#pragma unroll 1
+            for (int part = 0; part < 4; part++) {
+                const uint32_t o = (uint32_t)(i * 1024 + part * 256 + lane * 4);
+                if (o < bytes) dma4(src + from(o), dst + i * 1024 + part * 256);
+            }
+        }
+    }
+}
+
 // Walks `nsubs` sub-chunks of one KV head with a two-deep pipeline: while sub-chunk n is being
 // decompressed out of one LDS buffer, sub-chunk n+1 streams from HBM into the other.
 //   tile_of(n)    : first tile of sub-chunk n

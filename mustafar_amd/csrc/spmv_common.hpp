@@ -47,12 +47,12 @@ __global__ __launch_bounds__(256) void value_merge_kernel(const float* __restric
     C[row * D + d] = (_Float16)s;
 }
 
-// Largest accumulator count with an instantiated kernel that fits in `left`.
-inline int pick_nw(int left)
+// Largest accumulator count with an instantiated kernel that fits in `left`; wide: whether more than eight may be taken.
+inline int pick_nw(int left, bool wide = true)
 {
     const int opts[] = {32, 16, 8, 4, 2, 1};
     for (int o : opts)
-        if (o <= left) return o;
+        if (o <= left && (wide || o <= 8)) return o;
     return 1;
 }
 
@@ -72,7 +72,9 @@ struct ValuePlan {
     int nsplit;  // workgroups along the token axis
 };
 
-inline ValuePlan plan_value(int Lc, int D, int Bkv, int nw)
+// most: splits that there is room for.
+constexpr int kAnySplits = 0x7FFFFFFF;
+inline ValuePlan plan_value(int Lc, int D, int Bkv, int nw, int most_splits = kAnySplits)
 {
     ValuePlan p;
     const int nblk = Lc / 64;
@@ -104,7 +106,8 @@ inline ValuePlan plan_value(int Lc, int D, int Bkv, int nw)
     long nb = (chunks + 4095) / 4096;
     if (nb < 1) nb = 1;
     if (nb > nblk) nb = nblk;
-    p.nbpw = (int)nb;
+    const long room = ((long)nblk + (long)p.waves * most_splits - 1) / ((long)p.waves * most_splits);
+    p.nbpw = (int)(nb > room ? nb : room);
     p.nsplit = (nblk + p.waves * p.nbpw - 1) / (p.waves * p.nbpw);
     return p;
 }
@@ -122,7 +125,14 @@ inline void launch_value_merge(hipStream_t st, const float* part, _Float16* C, i
                            rows_per_kv, row0, nw, total);
 }
 
-// Workspace of a token-split value product (fp32 partials), 0 when no pass splits.
+// Splits of a value product that a workspace has room for, at least the one that takes none.
+inline int splits_that_fit(size_t workspace_bytes, int head_dim, int Bq, int n_rows)
+{
+    const size_t fit = workspace_bytes / ((size_t)Bq * n_rows * head_dim * sizeof(float));
+    return fit < 1 ? 1 : (fit < 1024 ? (int)fit : 1024);
+}
+// Workspace of a token-split value product (fp32 partials), 0 when no pass splits.  (Passes of eight rows in the place of a
+// wide one, for unaligned weights, take no more splits than fit.)
 inline size_t value_workspace_bytes(int head_dim, int tokens, int Bq, int groups, int n_rows)
 {
     const int rows_per_kv = groups * n_rows;
