@@ -73,29 +73,47 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
         return *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(c.bmp + t) + touch8);
     };
 
-    size_t t_cur = tile_of(0);
+    size_t t_cur = tile_of(0), t_nxt = nsubs > 1 ? tile_of(1) : t_cur;
+    // The bounds of the coming stage: even lanes the first tile's offset, odd ones the last tile's and, with its bitmap, where
+    // its words end.  Requested in front of the stage before it, whose wait completes the loads (see walk_subs).
+    const uint32_t bnd4 = (uint32_t)(lane & 1) * ((kSubTiles - 1) * 4u);
+    struct Raw {
+        uint32_t off;
+        uint2 last;
+    };
+    auto bounds_of = [&](size_t t) {
+        Raw r;
+        r.off = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(c.off + t) + bnd4);
+        r.last = *reinterpret_cast<const uint2*>(c.bmp + t + kSubTiles - 1);
+        return r;
+    };
+    Raw bnd = bounds_of(t_nxt);
     uint32_t s_cur, e_cur;
     bounds(t_cur, s_cur, e_cur);
     uint2 touch = issue(0, t_cur, s_cur, e_cur);
-    size_t t_nxt = nsubs > 1 ? tile_of(1) : t_cur;
-    uint32_t s_nxt, e_nxt;
-    bounds(t_nxt, s_nxt, e_nxt);
     if constexpr (SHARED) {
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(touch.x), "+v"(touch.y)::"memory");
         __syncthreads();
     }
     for (int n = 0; n < nsubs; n++) {
         set_wave_priority_uniform(3u - ((uint32_t)n & 3u));  // falls from stage to stage (see set_wave_priority)
-        asm volatile("s_waitcnt vmcnt(0)" : "+v"(touch.x), "+v"(touch.y)::"memory");  // stage n has landed
+        // stage n has landed, and the bounds of the coming one
+        asm volatile("s_waitcnt vmcnt(0)"
+                     : "+v"(touch.x), "+v"(touch.y), "+v"(bnd.off), "+v"(bnd.last.x), "+v"(bnd.last.y)::"memory");
         const uint2 bits = touch;
-        if (n + 1 < nsubs) touch = issue(n + 1, t_nxt, s_nxt, e_nxt);
         const size_t t_now = t_cur;
         const uint32_t s_now = s_cur;
-        t_cur = t_nxt;
-        s_cur = s_nxt;
-        if (n + 2 < nsubs) {
-            t_nxt = tile_of(n + 2);
-            bounds(t_nxt, s_nxt, e_nxt);
+        if (n + 1 < nsubs) {
+            t_cur = t_nxt;
+            const uint32_t words = ((uint32_t)__builtin_popcount(bnd.last.x) + (uint32_t)__builtin_popcount(bnd.last.y) +
+                                    (uint32_t)F::kCap - 1u) >> F::kCapShift;
+            s_cur = (uint32_t)__builtin_amdgcn_readlane((int)bnd.off, 0);
+            e_cur = (uint32_t)__builtin_amdgcn_readlane((int)(bnd.off + words), 1);
+            touch = issue(n + 1, t_cur, s_cur, e_cur);
+            if (n + 2 < nsubs) {
+                t_nxt = tile_of(n + 2);
+                bnd = bounds_of(t_nxt);
+            }
         }
         dequant_stage<BIT, G32>(lds_addr(metabuf) + (uint32_t)(n & 1) * kMetaBytes,
                            lds_addr(wordbuf) + (uint32_t)(n & 1) * F::kWordBuf, lbase, s_now, bits, lane, mode);
