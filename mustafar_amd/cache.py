@@ -397,10 +397,17 @@ class SparseKVCache:
         self.kv_len = 0
         self.ws = None                      # ops.Workspace of this cache: never shared with another cache or stream
 
-    def _workspace(self, device):
+    def _workspace(self, device, heads=0, tokens=0):
+        """heads, tokens: what the first append brings.  The buffer is made for a decode step over that (or over all
+        max_tokens) at once: a first step that has to replace it makes the GPU wait for an allocation in every layer."""
         if self.ws is None:
-            self.ws = ops.Workspace(device)
+            step = self._step_workspace_bytes(max(self.max_tokens, tokens), heads * self.groups) if heads and self.fused else 0
+            self.ws = ops.Workspace(device, max(step, 1 << 20))
         return self.ws
+
+    def _step_workspace_bytes(self, tokens, rows):
+        return lib().mstf_decode_attention_window_workspace_bytes(tokens, self.residual_length + CHUNK, self.head_dim, rows,
+                                                                  self.groups)
 
     def _make_pools(self, heads, D, device):
         fk = self.pool_fraction if self.pool_fraction is not None else slab_fraction_for(self.kth_k, D)
@@ -427,7 +434,7 @@ class SparseKVCache:
         if self.max_tokens > 0:
             if self.k_pool is None:
                 self._make_pools(bs * n_kv, D, K.device)
-            ws = self._workspace(K.device)
+            ws = self._workspace(K.device, bs * n_kv, M)
             append_pair(self.k_pool, self.v_pool, K.reshape(bs * n_kv, M, D), V.reshape(bs * n_kv, M, D), self.kth_k,
                         self.kth_v, ws)
             self._pool_views()
@@ -446,7 +453,7 @@ class SparseKVCache:
 
     def _compress(self, K, V):
         bs, n_kv, L, D = K.shape
-        ws = self._workspace(K.device)
+        ws = self._workspace(K.device, bs * n_kv, L)
         ck = ops.compress(K.reshape(bs * n_kv, L, D), False, kth=self.kth_k, ws=ws)
         cv = ops.compress(V.reshape(bs * n_kv, L, D), True, kth=self.kth_v, ws=ws)
         return ck, cv
@@ -462,13 +469,13 @@ class SparseKVCache:
         if self.max_tokens > 0:
             if self.k_pool is None:
                 self._make_pools(bs * n_kv, D, kx.device)
-            ws = self._workspace(kx.device)
+            ws = self._workspace(kx.device, bs * n_kv, Lc)
             self.k_pool.append_proj(kx, self.kth_k, Lc, cos, sin, ws=ws)
             if Lc > 0:
                 self.v_pool.append_proj(vx, self.kth_v, Lc, ws=ws)
                 self._pool_views()
         else:
-            ws = self._workspace(kx.device)
+            ws = self._workspace(kx.device, bs * n_kv, Lc)
             ck, _ = ops.compress_proj(kx, False, self.kth_k, Lc, cos, sin, ws=ws)
             if Lc > 0:
                 cv, _ = ops.compress_proj(vx, True, self.kth_v, Lc, ws=ws)
@@ -493,6 +500,7 @@ class SparseKVCache:
             if self.max_tokens > 0 and self.k_pool is None:
                 # nothing compressed yet: the (empty) pools exist from the start, so the attention call never changes form
                 self._make_pools(bs * n_kv, D, K.device)
+            self._workspace(K.device, bs * n_kv, Lc)
             cap = max(self.residual_length + CHUNK, L - Lc)   # the window never holds more before a chunk leaves
             self._kbuf = torch.empty((bs * n_kv, cap, D), dtype=torch.float16, device=K.device)
             self._vbuf = torch.empty_like(self._kbuf)
@@ -668,6 +676,9 @@ class QuantSparseKVCache(SparseKVCache):
         self.bit, self.dequant_mode = bit, dequant_mode
         # self.k / self.v: 7-element lists [bitmaps, tile_offsets, packed, counts, units, scales, zeros]
 
+    def _step_workspace_bytes(self, tokens, rows):
+        return ops.attention_workspace_least(tokens, self.residual_length + CHUNK, rows)
+
     def _step_device(self, q_in, k_in, v_in, cos, sin):
         from . import mustafar_package_quant as mpq
         return mpq.decode_step_quant_pool(self.k_pool, self.v_pool, q_in, k_in, v_in, self._kbuf, self._vbuf,
@@ -688,7 +699,8 @@ class QuantSparseKVCache(SparseKVCache):
         """As SparseKVCache.prefill_proj for the rotation - the keys are rotated in place by the compressor's kernel,
         in the projection's own layout - while the quantised producer, which takes contiguous rows like the
         reference's, goes through prefill on the transposed views."""
-        ops.compress_proj(kx, False, self.kth_k, 0, cos, sin, ws=self._workspace(kx.device))      # M = 0: rotation only
+        ws = self._workspace(kx.device, kx.shape[0] * kx.shape[2], kx.shape[1] // 64 * 64)
+        ops.compress_proj(kx, False, self.kth_k, 0, cos, sin, ws=ws)      # M = 0: rotation only
         K, V = kx.transpose(1, 2), vx.transpose(1, 2)
         self.prefill(K, V)
         return K, V
@@ -696,7 +708,7 @@ class QuantSparseKVCache(SparseKVCache):
     def _compress(self, K, V):
         from . import compression_quant as cq
         bs, n_kv, M, D = K.shape
-        ws = self._workspace(K.device)   # the pruning runs inside the producer: one read of the dense rows
+        ws = self._workspace(K.device, bs * n_kv, M)   # the pruning runs inside the producer: one read of the dense rows
         return (list(cq.convert_key_batched_quant(K.reshape(bs * n_kv, M, D), return_metadata=True, bit=self.bit, ws=ws,
                                                   kth=self.kth_k)),
                 list(cq.convert_value_batched_quant(V.reshape(bs * n_kv, M, D), bit=self.bit, ws=ws, kth=self.kth_v)))
@@ -720,7 +732,7 @@ class QuantSparseKVCache(SparseKVCache):
             bs, n_kv, M, D = K.shape
             if self.k_pool is None:
                 self._make_pools(bs * n_kv, D, K.device)
-            ws = self._workspace(K.device)
+            ws = self._workspace(K.device, bs * n_kv, M)
             self.k_pool.append(K.reshape(bs * n_kv, M, D), self.kth_k, ws)
             self.v_pool.append(V.reshape(bs * n_kv, M, D), self.kth_v, ws)
             if not self.window_kernel:
