@@ -62,7 +62,7 @@ struct QuantKernargs {
     StepArgs st;
 };
 constexpr size_t kQuantStepArgsAt = offsetof(QuantKernargs, st);
-template <int NM, int BIT, bool G32, bool STEP = false>
+template <int NM, int BIT, bool G32, bool MULTI, bool STEP = false>
 __global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_eu(quant_occupancy<NM, BIT, G32>()))) void decode_attention_quant_kernel(
     const uint32_t* __restrict__ k_off, const uint32_t* __restrict__ v_off, const uint64_t* __restrict__ k_bmp,
     const uint64_t* __restrict__ v_bmp, size_t tstride, const int* __restrict__ tokens_dev, int nblk, int deal,
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_e
         nblk = valid < nblk ? valid : nblk;
         // the blocks a wavefront walks follow from the tokens that are there now, as a launch sized for exactly them
         // would choose; the workgroups behind the last block leave neutral partials
-        if (quant_multi<NM>()) deal = fused_deal(nblk, fused_splits(nblk, fused_fill_unpack(deal)));
+        if (MULTI) deal = fused_deal(nblk, fused_splits(nblk, fused_fill_unpack(deal)));
     }
     constexpr int D = kFusedD;
     constexpr int kQRow = kQuantQRow, kPRow = kQuantPRow;
@@ -96,7 +96,6 @@ __global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_e
     const int wave = wave_id();
     const int split = tokens_dev ? (int)blockIdx.y : (int)blockIdx.x;
     const int kv = tokens_dev ? (int)blockIdx.x : (int)blockIdx.y;
-    constexpr bool MULTI = quant_multi<NM>();
     BlockRange mine = {split * kFusedWaves + wave, 0};                // the token blocks of this wavefront
     if constexpr (MULTI) mine = fused_blocks_of(nblk, deal, split, wave);
     const int tb = mine.first, nb = MULTI ? mine.count : nblk - tb;   // (wave-uniform)
@@ -289,24 +288,25 @@ static void launch_decode_quant(hipStream_t st, dim3 grid, const uint64_t* k_bmp
                                 const uint16_t* v_scales, const uint16_t* v_zeros, const _Float16* q, _Float16* out,
                                 float* part_o, float* part_ml, int tokens, int groups, int ns, int write_final, float sq,
                                 int mode, int group_size, size_t tstride, const int32_t* tokens_dev, int deal,
-                                const StepArgs* step)
+                                bool one_block, const StepArgs* step)
 {
     const StepArgs sa = step ? *step : StepArgs{};
-    if (step)  // (group_size is 64 there: quant_launch has checked it)
-        hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, false, true>), grid, dim3(kFusedWaves * 64), 0, st, k_off,
-                           v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales,
-                           k_zeros, v_packed, v_off, v_scales, v_zeros, q, out, part_o, part_ml, groups, ns, write_final,
-                           sq, mode, sa);
-    else if (group_size == 32)
-        hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, true>), grid, dim3(kFusedWaves * 64), 0, st, k_off,
-                           v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales,
-                           k_zeros, v_packed, v_off, v_scales, v_zeros, q, out, part_o, part_ml, groups, ns, write_final,
-                           sq, mode, sa);
-    else
-        hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, false>), grid, dim3(kFusedWaves * 64), 0, st, k_off,
-                           v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales,
-                           k_zeros, v_packed, v_off, v_scales, v_zeros, q, out, part_o, part_ml, groups, ns, write_final,
-                           sq, mode, sa);
+#define MSTF_FQ_LAUNCH(...)                                                                                              \
+    hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, __VA_ARGS__>), grid, dim3(kFusedWaves * 64), 0, st, k_off, \
+                       v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales, k_zeros,   \
+                       v_packed, v_off, v_scales, v_zeros, q, out, part_o, part_ml, groups, ns, write_final, sq, mode, sa)
+    // With one block per wavefront the form for one, except for 2-bit codes of one group per tile: 280 to 1696 blocks, 70 - 75 %,
+    // fused attention in the form for several / for one: 4 bits 16.4 / 15.4 us (two groups per tile 18.4 / 17.7), 8 bits 17.8 /
+    // 17.5, 2 bits with two groups 17.4 / 16.5, but 2 bits with one 14.4 / 14.6 (4096 blocks: 17.9 / 18.3).
+    constexpr bool kMulti = quant_multi<NM>(), kOne = kMulti && BIT == 2;
+    if (step) {  // (group_size is 64 there: quant_launch has checked it)
+        if (one_block) MSTF_FQ_LAUNCH(false, kOne, true); else MSTF_FQ_LAUNCH(false, kMulti, true);
+    } else if (group_size == 32) {
+        if (one_block) MSTF_FQ_LAUNCH(true, false); else MSTF_FQ_LAUNCH(true, kMulti);
+    } else {
+        if (one_block) MSTF_FQ_LAUNCH(false, kOne); else MSTF_FQ_LAUNCH(false, kMulti);
+    }
+#undef MSTF_FQ_LAUNCH
 }
 
 }  // namespace mstf
@@ -364,8 +364,10 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
 {
     const int Bkv = Bq / groups;
     // (token count in device memory: the kernel deals the blocks out itself, from the number of workgroups that fill the chip)
-    const int deal = tokens_dev ? fused_fill_pack(fused_fill(Bkv, quant_resident(groups, bit, group_size)))
-                                : fused_deal(tokens / 64, ns);
+    const FusedFill fill = fused_fill(Bkv, quant_resident(groups, bit, group_size));
+    const int deal = tokens_dev ? fused_fill_pack(fill) : fused_deal(tokens / 64, ns);
+    // no wavefront has more than one block (and none has with fewer tokens, should their number be in device memory)
+    const bool one_block = fused_splits(tokens / 64, fill) == fused_nsplit(tokens);
     // step: the launch is a whole decode step; its window blocks are dealt out over the wavefronts of a head
     if (step && (group_size != 64 || window_blocks(step->win_len) > ns * kFusedWaves)) return MSTF_EUNSUPPORTED;
     // tile_stride / tokens_dev: a cache pre-allocated for `tokens` tokens that holds *tokens_dev of them (see the kernel)
@@ -383,7 +385,7 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
 #define MSTF_FQ(NMV, BITV)                                                                                             \
     launch_decode_quant<NMV, BITV>(st, grid, k_bmp, k_packed, k_tile_off, ks, kz, v_bmp, v_packed, v_tile_off, vs, vz, \
                                    qh, oh, part_o, part_ml, tokens, groups, nst, write_final, sq, dequant_mode, group_size, \
-                                   tstride, tokens_dev, deal, step)
+                                   tstride, tokens_dev, deal, one_block, step)
     if (groups <= 4) {
         if (bit == 2) MSTF_FQ(1, 2); else if (bit == 4) MSTF_FQ(1, 4); else MSTF_FQ(1, 8);
     } else {
