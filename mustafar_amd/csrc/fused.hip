@@ -100,7 +100,11 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
     // STEP: a wavefront that also has a block of the dense window to do keeps the highest issue priority through its
     // walk (it has the longest way to go; see set_wave_priority)
     uint32_t prio_boost = 0u;
-    if constexpr (STEP && !SHARE) prio_boost = step_window_boost(st, wave, split);
+    int order = wave;
+    if constexpr (STEP && !SHARE) {
+        order = fused_window_order(nblk, deal, split, wave);
+        prio_boost = step_window_boost(st, order, split);
+    }
     const int j = lane & 3;
     const size_t T = tstride;
     char* my = lds[wave];
@@ -324,7 +328,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
 
     if constexpr (STEP && !SHARE) {
         // The dense window: its 64-token blocks are dealt out over the wavefronts of the head's workgroups - block i to
-        // wavefront 7 - i / ns of split i % ns - which take them behind their compressed blocks, so the window costs no
+        // number i / ns (fused_window_order) of split i % ns - which take them behind their compressed blocks, so the window costs no
         // workgroup of its own (a ninth workgroup per head would find no free slot on a full chip and run behind the
         // others).  The query rows are still in LDS; the value buffers and the weight rows are free again.
         // (the step's arguments are fetched again here, through a pointer the compiler cannot see through: kept in
@@ -338,7 +342,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
         sw.cos = sp->cos, sw.sin = sp->sin, sw.rope_stride = sp->rope_stride;
         sw.k_win = sp->k_win, sw.v_win = sp->v_win, sw.win_len_dev = sp->win_len_dev, sw.overflow = sp->overflow;
         sw.win_len = sp->win_len, sw.win_stride = sp->win_stride, sw.n_kv = sp->n_kv, sw.ns = sp->ns;
-        const int wblk = step_window_block(sw.ns, wave, split);
+        const int wblk = step_window_block(sw.ns, order, split);
         if (wblk < (sw.win_len + 63) / 64) {
             if (!active) stage_query_rotated(ql, sw, kv, groups, lane);
             step_window_wave<NM>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, sqrt_d, lane);

@@ -31,18 +31,18 @@ struct StepArgs {
 };
 
 // Block of the dense window that a wavefront takes behind its compressed blocks: dealt out over the ns splits of a head
-// first, from the last wavefronts on, which have a compressed block less where the blocks do not divide evenly.
-__device__ __forceinline__ int step_window_block(int ns, int wave, int split)
+// first, then over the wavefronts of each (order: fused_window_order).
+__device__ __forceinline__ int step_window_block(int ns, int order, int split)
 {
-    return (kFusedWaves - 1 - wave) * ns + split;
+    return order * ns + split;
 }
 // 3 for a wavefront that step_window_wave gives a block of the dense window (step_window_block, of the rows that
 // are valid after this step), else 0: OR-ed into the issue priority of its walk over the compressed tokens.
-__device__ __forceinline__ uint32_t step_window_boost(const StepArgs& sa, int wave, int split)
+__device__ __forceinline__ uint32_t step_window_boost(const StepArgs& sa, int order, int split)
 {
     int wlen = sa.win_len_dev ? *sa.win_len_dev : sa.win_len;
     wlen = wlen < sa.win_len ? wlen : sa.win_len;
-    const int has = step_window_block(sa.ns, wave, split) < (wlen + 63) / 64;
+    const int has = step_window_block(sa.ns, order, split) < (wlen + 63) / 64;
     return (uint32_t)__builtin_amdgcn_readfirstlane(has ? 3 : 0);
 }
 
