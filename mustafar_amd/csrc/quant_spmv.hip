@@ -204,7 +204,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     const uint64_t* __restrict__ bmp, const uint32_t* packed, const uint32_t* __restrict__ tile_off,
     const uint32_t* tile_off_dma, const uint16_t* scales, const uint16_t* zeros, const _Float16* P,
     _Float16* __restrict__ C, float* __restrict__ part, int Lc, int D, int nblk, int nbpw, int nsplit, int rows_per_kv,
-    int row0, int mode, int nwg)
+    int row0, int mode, int nwg, uint32_t per_split)
 {
     using Sums = RowSums<NW>;
     constexpr int kWRow = kSubTiles * 2;
@@ -217,9 +217,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     const int nhalf = D / 64;
     const int logical = xcd_contiguous((int)blockIdx.x, nwg);
     if (logical >= nwg) return;  // (the whole workgroup: no barrier is left waiting)
-    const int half = logical % nhalf;
-    const int split = (logical / nhalf) % nsplit;
-    const int kv = logical / (nhalf * nsplit);
+    const ValueIndex at = value_index(logical, nhalf, nsplit, per_split);
+    const int half = at.half, split = at.split, kv = at.kv;
     const size_t T = (size_t)Lc * D / 64;
     const QCache c = {bmp, tile_off, tile_off_dma, scales, zeros, packed};
     const _Float16* wk = P + ((size_t)kv * rows_per_kv + row0) * Lc;
@@ -336,11 +335,11 @@ static void launch_value_q(hipStream_t st, const ValuePlan& pl, const QArgs& a, 
     if (a.group_size == 32)
         hipLaunchKernelGGL((value_spmv_quant_kernel<NW, WAVES, BIT, true>), dim3(xcd_grid(nwg)), dim3(WAVES * 64), 0,
                            st, a.bmp, a.packed, a.tile_off, a.tile_off, a.scales, a.zeros, P, C, part, Lc, D, Lc / 64,
-                           pl.nbpw, pl.nsplit, rows_per_kv, row0, a.mode, nwg);
+                           pl.nbpw, pl.nsplit, rows_per_kv, row0, a.mode, nwg, split_inverse(pl.nsplit));
     else
         hipLaunchKernelGGL((value_spmv_quant_kernel<NW, WAVES, BIT, false>), dim3(xcd_grid(nwg)), dim3(WAVES * 64), 0,
                            st, a.bmp, a.packed, a.tile_off, a.tile_off, a.scales, a.zeros, P, C, part, Lc, D, Lc / 64,
-                           pl.nbpw, pl.nsplit, rows_per_kv, row0, a.mode, nwg);
+                           pl.nbpw, pl.nsplit, rows_per_kv, row0, a.mode, nwg, split_inverse(pl.nsplit));
 }
 template <int NW, int WAVES>
 static void launch_value_q_bit(int bit, hipStream_t st, const ValuePlan& pl, const QArgs& a, const _Float16* P,

@@ -101,7 +101,8 @@ template <int NW, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(wide_rows(NW) ? 3 : 4))) void value_spmv_kernel(
     const uint64_t* __restrict__ bmp, const char* __restrict__ nz, const uint32_t* __restrict__ idx,
     const uint32_t* __restrict__ nz_off, const _Float16* __restrict__ P, _Float16* __restrict__ C,
-    float* __restrict__ part, int Lc, int D, int nblk, int nbpw, int nsplit, int p_rows_per_kv, int row0, int nwg)
+    float* __restrict__ part, int Lc, int D, int nblk, int nbpw, int nsplit, int p_rows_per_kv, int row0, int nwg,
+    uint32_t per_split)
 {
     using Sums = RowSums<NW>;
     constexpr int kWRow = kSubTiles * 2;          // bytes of one probability row per sub-chunk
@@ -115,9 +116,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(wide
     const int nhalf = D / 64;
     const int logical = xcd_contiguous((int)blockIdx.x, nwg);
     if (logical >= nwg) return;  // (the whole workgroup: no barrier is left waiting)
-    const int half = logical % nhalf;
-    const int split = (logical / nhalf) % nsplit;
-    const int kv = logical / (nhalf * nsplit);
+    const ValueIndex at = value_index(logical, nhalf, nsplit, per_split);
+    const int half = at.half, split = at.split, kv = at.kv;
     const size_t T = (size_t)Lc * D / 64;
     const uint64_t* bmk = bmp + (size_t)kv * T;
     const uint32_t* ixk = idx + (size_t)kv * (T + 1);
@@ -329,7 +329,7 @@ static void launch_value(hipStream_t st, const ValuePlan& pl, const uint64_t* bm
 {
     const int nwg = pl.nsplit * (D / 64) * Bkv;
     hipLaunchKernelGGL((value_spmv_kernel<NW, WAVES>), dim3(xcd_grid(nwg)), dim3(WAVES * 64), 0, st, bmp, nz, idx, nz_off, P,
-                       C, part, Lc, D, Lc / 64, pl.nbpw, pl.nsplit, rows_per_kv, row0, nwg);
+                       C, part, Lc, D, Lc / 64, pl.nbpw, pl.nsplit, rows_per_kv, row0, nwg, split_inverse(pl.nsplit));
 }
 
 }  // namespace mstf
