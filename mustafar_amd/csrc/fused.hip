@@ -102,7 +102,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
     uint32_t prio_boost = 0u;
     int order = wave;
     if constexpr (STEP && !SHARE) {
-        order = fused_window_order(nblk, deal, split, wave);
+        order = fused_window_order(nblk, deal, split, wave, (st.win_len + 63) / 64, st.ns);
         prio_boost = step_window_boost(st, order, split);
     }
     const int j = lane & 3;

@@ -99,10 +99,15 @@ constexpr BlockRange fused_blocks_of(int nblk, int deal, int split, int wave)
 // The wavefronts of a split in the order in which they take a block of the dense window behind their compressed ones: from the
 // last one on where those have a block less (128 heads x 60 blocks, 2 bits: 300 -> 264 us per eight layers; 64 x 60, 8 bits, four
 // layers: 150 -> 134), else from the first one on, which is the first to start (16 heads x 24 blocks, eight query heads, 8 bits:
-// 102 -> 98 us, 4 bits 93.5 -> 90).
-constexpr int fused_window_order(int nblk, int deal, int split, int wave)
+// 102 -> 98 us, 4 bits 93.5 -> 90).  Where the last ones have no block at all, but are too few for the split's share of the window
+// (window: its blocks, ns: splits of a head), the window's last block, the one with the new token's row, would come
+// to a wavefront that has one; from the first one on it does not (156 heads x 4 blocks, four layers: 98.4 -> 92.6 us with 2 bits,
+// 91.5 -> 85.9 fp16).
+constexpr int fused_window_order(int nblk, int deal, int split, int wave, int window, int ns)
 {
-    return fused_blocks_of_split(nblk, deal, split).count % kFusedWaves == 0 ? wave : kFusedWaves - 1 - wave;
+    const int n = fused_blocks_of_split(nblk, deal, split).count, left = n % kFusedWaves;
+    const bool last_first = left != 0 && (n > kFusedWaves || (kFusedWaves - left) * ns >= window);
+    return last_first ? kFusedWaves - 1 - wave : wave;
 }
 
 // Whether the four wavefronts of a workgroup share a token block instead of walking blocks of their own: with few blocks a

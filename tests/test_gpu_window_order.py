@@ -7,10 +7,12 @@ pytestmark = pytest.mark.gpu
 D = 128
 
 
-# (128 heads: with the capacities below neither format shares blocks; 4, 8, 12 and 16 compressed blocks per head)
+# (128 heads: with the capacities below neither format shares blocks; none to 16 compressed blocks per head; one split of four
+# blocks, whose idle wavefronts are fewer than the window's blocks)
 @pytest.mark.parametrize("bit", [0, 2, 8])
-@pytest.mark.parametrize("tokens", [256, 600, 767, 800, 1100, 1500])
-@pytest.mark.parametrize("groups,max_tokens", [(2, 1536), (8, 2560)])
+@pytest.mark.parametrize("tokens,groups,max_tokens",
+                         [(t, g, m) for t in (256, 600, 767, 800, 1100, 1500) for g, m in ((2, 1536), (8, 2560))] +
+                         [(t, 4, 512) for t in (256, 600, 767, 800)])
 def test_step_equals_the_calls(bit, tokens, groups, max_tokens):
     from mustafar_amd.cache import QuantSparseKVCache, SparseKVCache
     bs, n_kv = 16, 8
