@@ -102,8 +102,9 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
     uint32_t prio_boost = 0u;
     int order = wave;
     if constexpr (STEP && !SHARE) {
-        order = fused_window_order(nblk, deal, split, wave, (st.win_len + 63) / 64, st.ns);
-        prio_boost = step_window_boost(st, order, split);
+        const int rows = step_window_rows(st, step_window_count(st));
+        order = fused_window_order(nblk, deal, split, wave, rows, st.ns);
+        prio_boost = step_window_boost(st, order, split, rows);
     }
     const int j = lane & 3;
     const size_t T = tstride;
@@ -119,7 +120,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
             const int wblk = (split - st.wg0) * kShare + wave;
             if (wblk < (st.win_len + 63) / 64) {
                 stage_query_rotated(ql, st, kv, groups, lane);
-                step_window_wave<NM>(my, ql, pl, st, part_o, part_ml, kv, groups, nsplit, wblk, sqrt_d, lane);
+                step_window_wave<NM>(my, ql, pl, st, part_o, part_ml, kv, groups, nsplit, wblk, step_window_count(st), sqrt_d, lane);
             }
             return;  // (the whole workgroup: no barrier is left waiting)
         }
@@ -345,7 +346,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
         const int wblk = step_window_block(sw.ns, order, split);
         if (wblk < (sw.win_len + 63) / 64) {
             if (!active) stage_query_rotated(ql, sw, kv, groups, lane);
-            step_window_wave<NM>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, sqrt_d, lane);
+            step_window_wave<NM>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, step_window_count(sw), sqrt_d, lane);
         }
     }
     workgroup_combine<NM>(&lds[0][0], kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, split, nsplit, write_final,

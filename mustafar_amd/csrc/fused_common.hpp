@@ -99,14 +99,15 @@ constexpr BlockRange fused_blocks_of(int nblk, int deal, int split, int wave)
 // The wavefronts of a split in the order in which they take a block of the dense window behind their compressed ones: from the
 // last one on where those have a block less (128 heads x 60 blocks, 2 bits: 300 -> 264 us per eight layers; 64 x 60, 8 bits, four
 // layers: 150 -> 134), else from the first one on, which is the first to start (16 heads x 24 blocks, eight query heads, 8 bits:
-// 102 -> 98 us, 4 bits 93.5 -> 90).  Where the last ones have no block at all, but are too few for the split's share of the window
-// (window: its blocks, ns: splits of a head), the window's last block, the one with the new token's row, would come
-// to a wavefront that has one; from the first one on it does not (156 heads x 4 blocks, four layers: 98.4 -> 92.6 us with 2 bits,
-// 91.5 -> 85.9 fp16).
-constexpr int fused_window_order(int nblk, int deal, int split, int wave, int window, int ns)
+// 102 -> 98 us, 4 bits 93.5 -> 90).  Where the last ones have no block at all, they may still
+// be too few for the split's share of the window (rows: those there are, ns: splits of a head).  A short block - the window's
+// last one - then follows onto a wavefront with a compressed block, but a longer one would come to it with the new token's row
+// still behind it: from the first wavefront on the new row's block finds an idle one (156 heads x 4 blocks, four layers, 2 bits:
+// a window of 257 rows 77.7 us from the last one on, 100.6 from the first; 320 rows 95.9, 93.9; 429 98.4, 93.4; 511 103.8, 95.3).
+constexpr int fused_window_order(int nblk, int deal, int split, int wave, int rows, int ns)
 {
     const int n = fused_blocks_of_split(nblk, deal, split).count, left = n % kFusedWaves;
-    const bool last_first = left != 0 && (n > kFusedWaves || (kFusedWaves - left) * ns >= window);
+    const bool last_first = left != 0 && (n > kFusedWaves || rows <= ((kFusedWaves - left) * ns + split) * 64 + 32);
     return last_first ? kFusedWaves - 1 - wave : wave;
 }
 

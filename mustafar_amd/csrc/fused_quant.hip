@@ -271,12 +271,12 @@ __global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_e
         sw.cos = sp->cos, sw.sin = sp->sin, sw.rope_stride = sp->rope_stride;
         sw.k_win = sp->k_win, sw.v_win = sp->v_win, sw.win_len_dev = sp->win_len_dev, sw.overflow = sp->overflow;
         sw.win_len = sp->win_len, sw.win_stride = sp->win_stride, sw.n_kv = sp->n_kv, sw.ns = sp->ns;
-        const int window = (sw.win_len + 63) / 64;
-        const int order = fused_window_order(nblk, MULTI ? deal : kFusedWaves, split, wave, window, sw.ns);
+        const int count = step_window_count(sw);
+        const int order = fused_window_order(nblk, MULTI ? deal : kFusedWaves, split, wave, step_window_rows(sw, count), sw.ns);
         const int wblk = step_window_block(sw.ns, order, split);
-        if (wblk < window) {
+        if (wblk < (sw.win_len + 63) / 64) {
             if (!active) stage_query_rotated<kQRow>(ql, sw, kv, groups, lane);
-            step_window_wave<NM, kQRow, kPRow, 8>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, sqrt_d, lane);
+            step_window_wave<NM, kQRow, kPRow, 8>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, count, sqrt_d, lane);
         }
     }
     workgroup_combine<NM>(lds_all, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, split, nsplit, write_final, out,

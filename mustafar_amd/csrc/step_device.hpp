@@ -36,13 +36,14 @@ __device__ __forceinline__ int step_window_block(int ns, int order, int split)
 {
     return order * ns + split;
 }
-// 3 for a wavefront that step_window_wave gives a block of the dense window (step_window_block, of the rows that
-// are valid after this step), else 0: OR-ed into the issue priority of its walk over the compressed tokens.
-__device__ __forceinline__ uint32_t step_window_boost(const StepArgs& sa, int order, int split)
+// The count of valid rows after this step as it stands in memory, and as far as the launch is sized for it.
+__device__ __forceinline__ int step_window_count(const StepArgs& sa) { return sa.win_len_dev ? *sa.win_len_dev : sa.win_len; }
+__device__ __forceinline__ int step_window_rows(const StepArgs& sa, int count) { return count < sa.win_len ? count : sa.win_len; }
+// 3 for a wavefront that step_window_wave gives a block of the dense window (step_window_block, of the `rows` that are valid
+// after this step), else 0: OR-ed into the issue priority of its walk over the compressed tokens.
+__device__ __forceinline__ uint32_t step_window_boost(const StepArgs& sa, int order, int split, int rows)
 {
-    int wlen = sa.win_len_dev ? *sa.win_len_dev : sa.win_len;
-    wlen = wlen < sa.win_len ? wlen : sa.win_len;
-    const int has = step_window_block(sa.ns, order, split) < (wlen + 63) / 64;
+    const int has = step_window_block(sa.ns, order, split) < (rows + 63) / 64;
     return (uint32_t)__builtin_amdgcn_readfirstlane(has ? 3 : 0);
 }
 
@@ -72,7 +73,7 @@ __device__ __forceinline__ void stage_query_rotated(char* ql, const StepArgs& sa
 
 // One 64-token block (wblk) of the dense window of KV head kv, by one wavefront; leaves the block's (max, sum,
 // un-normalised output) in split slot sa.ns + wblk of every query row of the head, like a split of the compressed
-// tokens.  my: the wavefront's LDS (two value buffers of VROWS rows first), ql: the rotated query rows (QROW bytes
+// tokens.  wlen: step_window_count.  my: the wavefront's LDS (two value buffers of VROWS rows first), ql: the rotated query rows (QROW bytes
 // apart), pl: room for the block's weights (rows PROW bytes apart).
 //   key phase   : lane = token holds its whole key row in registers (sixteen 16-byte loads; the lane of the new row
 //                 reads the projection output instead, rotates it and stores it to the window), so the A operands of
@@ -81,15 +82,14 @@ __device__ __forceinline__ void stage_query_rotated(char* ql, const StepArgs& sa
 //                 from registers), lane = channel reads them column-wise.
 template <int NM, int QROW = kFusedD * 2, int PROW = 64 * 2, int VROWS = 16>
 __device__ __forceinline__ void step_window_wave(char* my, char* ql, char* pl, const StepArgs& sa, float* part_o,
-                                                 float* part_ml, int kv, int groups, int nst, int wblk, float sqrt_d,
-                                                 int lane)
+                                                 float* part_ml, int kv, int groups, int nst, int wblk, int wlen,
+                                                 float sqrt_d, int lane)
 {
     constexpr int D = kFusedD;
     constexpr int kPRow = PROW;
     constexpr int kVBuf = VROWS * D * 2;  // bytes of one of the two value buffers
     static_assert(VROWS == 16 || VROWS == 8, "value rows per LDS buffer");
     const int j = lane & 3;
-    int wlen = sa.win_len_dev ? *sa.win_len_dev : sa.win_len;
     const bool fits = wlen >= 1 && wlen <= sa.win_stride;
     if (!fits && sa.overflow && lane == 0 && wblk == 0) *sa.overflow = 1u;
     const int new_row = fits ? wlen - 1 : -1;

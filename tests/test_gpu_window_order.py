@@ -12,7 +12,7 @@ D = 128
 @pytest.mark.parametrize("bit", [0, 2, 8])
 @pytest.mark.parametrize("tokens,groups,max_tokens",
                          [(t, g, m) for t in (256, 600, 767, 800, 1100, 1500) for g, m in ((2, 1536), (8, 2560))] +
-                         [(t, 4, 512) for t in (256, 600, 767, 800)])
+                         [(t, 4, 512) for t in (256, 512, 543, 544, 600, 767, 800)])
 def test_step_equals_the_calls(bit, tokens, groups, max_tokens):
     from mustafar_amd.cache import QuantSparseKVCache, SparseKVCache
     bs, n_kv = 16, 8
