@@ -297,14 +297,14 @@ static void launch_decode_quant(hipStream_t st, dim3 grid, const uint64_t* k_bmp
     hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, __VA_ARGS__>), grid, dim3(kFusedWaves * 64), 0, st, k_off, \
                        v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales, k_zeros,   \
                        v_packed, v_off, v_scales, v_zeros, q, out, part_o, part_ml, groups, ns, write_final, sq, mode, sa)
-    // With one block per wavefront the form for one, except for 2-bit codes of one group per tile: 280 to 1696 blocks, 70 - 75 %,
-    // fused attention in the form for several / for one: 4 bits 16.4 / 15.4 us (two groups per tile 18.4 / 17.7), 8 bits 17.8 /
-    // 17.5, 2 bits with two groups 17.4 / 16.5, but 2 bits with one 14.4 / 14.6 (4096 blocks: 17.9 / 18.3).
-    constexpr bool kMulti = quant_multi<NM>(), kOne = kMulti && BIT == 2;
+    // With one block per wavefront the form for one where it is the faster one: 280 to 1696 blocks, 70 - 75 %, fused attention in
+    // the form for several / for one: 4 bits 16.4 / 15.4 us (two groups per tile 18.4 / 17.7), 8 bits 17.8 / 17.5 (20.1 / 20.6),
+    // 2 bits 14.4 / 14.6 (17.4 / 16.5; 4096 blocks, one group: 17.9 / 18.3).
+    constexpr bool kMulti = quant_multi<NM>(), kOne = kMulti && BIT == 2, kOneG32 = kMulti && BIT == 8;
     if (step) {  // (group_size is 64 there: quant_launch has checked it)
         if (one_block) MSTF_FQ_LAUNCH(false, kOne, true); else MSTF_FQ_LAUNCH(false, kMulti, true);
     } else if (group_size == 32) {
-        if (one_block) MSTF_FQ_LAUNCH(true, false); else MSTF_FQ_LAUNCH(true, kMulti);
+        if (one_block) MSTF_FQ_LAUNCH(true, kOneG32); else MSTF_FQ_LAUNCH(true, kMulti);
     } else {
         if (one_block) MSTF_FQ_LAUNCH(false, kOne); else MSTF_FQ_LAUNCH(false, kMulti);
     }
