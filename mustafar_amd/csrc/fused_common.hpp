@@ -22,7 +22,8 @@ constexpr int kFusedMaxBpw = 8;           // token blocks that a wavefront walks
 // that the chip holds at 24 heads x 511 blocks - or a part of the chip without work.  fp16, 70 %, launch + merge: 24 x 511
 // blocks 58.2 -> 45.1 us, 304 x 64 94.7 -> 66.3, 384 x 64 112 -> 70, 64 x 66 27.1 -> 26.0; 2 bits: 24 x 511 71.6 -> 52.0,
 // 1024 x 16 80.9 -> 56.2; a 2-bit decode step of 8 layers at 128 heads x 60 blocks + window 300 -> 264 us, where the
-// wavefronts with a block less now take the window's; one head of 4200 blocks 32.5 -> 34.8, its merge has twice the splits.)
+// wavefronts with a block less now take the window's; one head of 4200 blocks, whose merge got twice the splits, 32.5 -> 34.8,
+// 30.5 since the merge takes its runs in groups.)
 struct FusedFill {
     int once;  // workgroups per KV head up to which a launch takes eight blocks each
     int full;  // workgroups per KV head that fill the chip
