@@ -58,6 +58,16 @@ int mstf_probe_read(void* stream, const void* src, size_t bytes, uint32_t* sink,
  * uses meanwhile and that keep what they are given when the call fails; the caller's thread watches for it there.
  * Refused (MSTF_ELAUNCH) while the stream is being captured.  landing and value: host pointers. */
 int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* value);
+/* Totals that a producer's kernel stores to pinned host memory itself, before its values are all out (the calls ..._sized and
+ * ..._landing_f16 below): known on the host without a launch behind the kernel and a wait for its end.
+ * mstf_landing_take: a pair of such words for a call that returns without waiting; null when none is free (the caller then
+ * uses the call without landings).  mstf_landing_give hands it back, at any time, from any thread.
+ * mstf_landing_wait: waits for a word's value; MSTF_NOT_LANDED: the call was recorded into a graph or refused, and the total is
+ * in device memory only.  All ones: a workgroup gave up waiting. */
+#define MSTF_NOT_LANDED (INT64_MIN + 2)
+int64_t* mstf_landing_take(void);
+void mstf_landing_give(int64_t* pair);
+int mstf_landing_wait(void* stream, const int64_t* landing, int64_t* value);
 /* Test aid (no counterpart in the reference): the number of polls a workgroup of the one-pass producers
  * (mstf_compress_*, mstf_append_*, mstf_compress_*_quant*) spends on a wait before it gives up and marks the call.
  * polls < 0 restores the default (2^20).  Process-wide, read at every launch; nothing in the environment changes it.
@@ -133,6 +143,12 @@ int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, i
                          uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
                          uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
                          size_t workspace_bytes);
+/* The same with a pair of landings (mstf_landing_take): keys' total, values' total. */
+int mstf_compress_kv_landing_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k, int kth_v,
+                                 uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off, uint64_t* k_total_halfs, mstf_half* k_nz,
+                                 uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
+                                 uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
+                                 size_t workspace_bytes, int64_t* landings);
 int mstf_append_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k, int kth_v,
                        uint64_t* k_bmp, uint32_t* k_idx, const uint32_t* k_dst_off, const uint32_t* k_dst_limit,
                        mstf_half* k_nz, uint64_t* v_bmp, uint32_t* v_idx, const uint32_t* v_dst_off,
@@ -170,6 +186,12 @@ typedef struct mstf_proj_source {
 int mstf_compress_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                            uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, mstf_half* nz,
                            uint64_t nz_capacity_halfs, void* workspace, size_t workspace_bytes);
+/* The same (M > 0), waiting for the total: *value.  landing: 8 bytes of pinned host memory that no other call uses meanwhile.
+ * Refused (MSTF_ELAUNCH) while the stream is being captured. */
+int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
+                                 uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, mstf_half* nz,
+                                 uint64_t nz_capacity_halfs, void* workspace, size_t workspace_bytes, int64_t* landing,
+                                 int64_t* value);
 int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                          uint64_t* bmp, uint32_t* idx, const uint32_t* dst_off, const uint32_t* dst_limit,
                          mstf_half* nz, uint32_t* overflow, void* workspace, size_t workspace_bytes);
@@ -451,6 +473,12 @@ int mstf_compress_quant_grouped(void* stream, const mstf_half* x, int is_value, 
                                 int group_size, uint64_t* bmp, uint32_t* tile_off, uint32_t* counts, uint32_t* units,
                                 mstf_half* scales, mstf_half* zeros, uint64_t* total_words, uint32_t* packed,
                                 uint64_t packed_capacity_words, void* workspace, size_t workspace_bytes);
+/* mstf_compress_quant_grouped with `packed` given, waiting for the total: see mstf_compress_proj_sized_f16. */
+int mstf_compress_quant_sized(void* stream, const mstf_half* x, int is_value, int B, int M, int N, int kth, int bit,
+                              int group_size, uint64_t* bmp, uint32_t* tile_off, uint32_t* counts, uint32_t* units,
+                              mstf_half* scales, mstf_half* zeros, uint64_t* total_words, uint32_t* packed,
+                              uint64_t packed_capacity_words, void* workspace, size_t workspace_bytes, int64_t* landing,
+                              int64_t* value);
 int mstf_key_spmv_quant_grouped(void* stream, const uint64_t* bmp, const uint32_t* packed, const uint32_t* tile_off,
                                 const mstf_half* scales, const mstf_half* zeros, const mstf_half* Bm, mstf_half* C, int M,
                                 int K, int Bq, int groups, int n_rows, int bit, int capacity, int dequant_mode,

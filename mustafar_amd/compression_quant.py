@@ -11,11 +11,12 @@ from . import ops
 from ._lib import check, lib
 
 
-def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None):
+def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, sized=False):
     """One call of the producer.  room: int32 tensor that takes the packed words (tile offsets count from its start;
     a tile whose words would pass its end is not written, and the total then exceeds room.numel());
     default: a fresh buffer with room for the worst case.  Returns the per-tile arrays, the buffer and the word total
-    as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host."""
+    as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host.
+    sized: the total as an int instead."""
     assert inputs.is_cuda
     assert inputs.dim() == 3
     B, M, N = inputs.shape
@@ -45,10 +46,15 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None):
     else:
         cap_words = room.numel()
     assert room.dtype == torch.int32 and room.is_contiguous()
-    check(L.mstf_compress_quant_grouped(st, x.data_ptr(), int(bool(is_value)), B, M, N, int(kth), int(bit), int(group_size),
-                                        bmp.data_ptr(), tile_off.data_ptr(), counts.data_ptr(), units.data_ptr(),
-                                        scales.data_ptr(), zeros.data_ptr(), total.data_ptr(), room.data_ptr(), cap_words,
-                                        ws.data_ptr(), ws.numel()), "mstf_compress_quant_grouped")
+    args = (st, x.data_ptr(), int(bool(is_value)), B, M, N, int(kth), int(bit), int(group_size), bmp.data_ptr(),
+            tile_off.data_ptr(), counts.data_ptr(), units.data_ptr(), scales.data_ptr(), zeros.data_ptr(), total.data_ptr(),
+            room.data_ptr(), cap_words, ws.data_ptr(), ws.numel())
+    if sized:
+        own = ops._landing_word()
+        check(L.mstf_compress_quant_sized(*args, own[1], own[3]), "mstf_compress_quant_sized")
+        total = own[2].value
+    else:
+        check(L.mstf_compress_quant_grouped(*args), "mstf_compress_quant_grouped")
     return bmp, tile_off, room, counts, units, scales, zeros, total
 
 
@@ -61,7 +67,7 @@ def words_written(total):
 
 
 def _convert(inputs, is_value, bit, kth=0, group_size=64, ws=None):
-    bmp, tile_off, room, counts, units, scales, zeros, total = _produce(inputs, is_value, bit, kth, group_size, ws)
+    bmp, tile_off, room, counts, units, scales, zeros, total = _produce(inputs, is_value, bit, kth, group_size, ws, sized=True)
     # the used part is copied out so that the large buffer goes back to the allocator
     packed = room[:words_written(total)].clone()
     return bmp, tile_off, packed, counts, units, scales, zeros

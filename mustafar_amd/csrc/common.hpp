@@ -113,6 +113,13 @@ inline int check_launch()
     return MSTF_OK;
 }
 
+// A call's word in pinned host memory (runtime.hip).  ready: the word is told apart from every result, unless the stream is
+// being captured, which is refused (a recorded kernel would store to it at every replay).  wait: watches it, then the stream.
+constexpr int64_t kLandingEmpty = INT64_MIN + 1;
+int landing_ready(hipStream_t st, int64_t* landing, const int64_t* value);
+int landing_wait(hipStream_t st, const int64_t* landing, int64_t* value);
+int stream_recorded(hipStream_t st, bool* recorded);
+
 inline bool aligned_to(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 

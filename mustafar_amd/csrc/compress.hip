@@ -377,7 +377,7 @@ __device__ __forceinline__ void onepass_workgroup(
     uint64_t* __restrict__ bmp, uint32_t* __restrict__ idx, uint32_t* __restrict__ nz_off,
     uint64_t* __restrict__ total_halfs, const uint32_t* __restrict__ dst_off, const uint32_t* __restrict__ dst_limit,
     uint32_t* __restrict__ overflow, char* __restrict__ nz, uint64_t nz_capacity_halfs, uint64_t* state, int units,
-    int groups_total, uint32_t spin_limit)
+    int groups_total, uint32_t spin_limit, uint64_t* landing)
 {
     auto& bufs = lds.bufs;
     auto& wave_total = lds.wave_total;
@@ -470,6 +470,7 @@ __device__ __forceinline__ void onepass_workgroup(
         ok = ok && bases[w][2] != 0ull;
     }
     if (!ok && threadIdx.x == 0) mark_gave_up(gave_up, total_halfs, overflow);
+    if (landing && g != groups_total - 1 && threadIdx.x == 0) count_through(state + groups_total + 1, ok);
     const uint32_t base = (uint32_t)in_head + in_group;
     const uint32_t end = base + total;
 
@@ -503,6 +504,8 @@ __device__ __forceinline__ void onepass_workgroup(
             stream_image(img, bytesB, dst + bytesA, lane);
         }
     }
+    if (landing && g == groups_total - 1 && threadIdx.x == 0)
+        land_total(landing, 2ull * (H + in_head + group_total), ok, state + groups_total + 1, (uint32_t)groups_total - 1u, spin_limit);
     // The rotated rows last: in front of the search their stores stood between this unit's total and the units that wait
     // for it, and it waited for its own stores where it polls.  Keys of 128 heads x 4096 tokens, 70 %, rotated: 90.1 ->
     // 78.0 us (rocprofv3), with the compaction of the whole unit in front of the wait.  That one takes a values' launch
@@ -516,11 +519,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MSTF_COM
     const _Float16* __restrict__ x, ProjArgs proj, int M, int kth, uint64_t* __restrict__ bmp, uint32_t* __restrict__ idx,
     uint32_t* __restrict__ nz_off, uint64_t* __restrict__ total_halfs, const uint32_t* __restrict__ dst_off,
     const uint32_t* __restrict__ dst_limit, uint32_t* __restrict__ overflow, char* __restrict__ nz,
-    uint64_t nz_capacity_halfs, uint64_t* state, int units, int groups_total, uint32_t spin_limit)
+    uint64_t nz_capacity_halfs, uint64_t* state, int units, int groups_total, uint32_t spin_limit, uint64_t* landing)
 {
     __shared__ OnepassLds<W> lds;
     onepass_workgroup<IS_VALUE, W, SRC>(lds, (int)blockIdx.x, x, proj, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                        dst_limit, overflow, nz, nz_capacity_halfs, state, units, groups_total, spin_limit);
+                                        dst_limit, overflow, nz, nz_capacity_halfs, state, units, groups_total, spin_limit,
+                                        landing);
 }
 
 // Keys and values of the same tokens in one launch: workgroups 0 .. groups_total-1 compress the keys, the next
@@ -539,6 +543,7 @@ struct OnepassSide {
     char* nz;
     uint64_t nz_capacity_halfs;
     uint64_t* state;
+    uint64_t* landing;
 };
 template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void compress_onepass_kv_kernel(
@@ -549,11 +554,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
     if (g < groups_total)
         onepass_workgroup<false, W, kSrcMatrix>(lds, g, k.x, ProjArgs{}, M, k.kth, k.bmp, k.idx, k.nz_off, k.total_halfs,
                                                 k.dst_off, k.dst_limit, overflow, k.nz, k.nz_capacity_halfs, k.state, units,
-                                                groups_total, spin_limit);
+                                                groups_total, spin_limit, k.landing);
     else
         onepass_workgroup<true, W, kSrcMatrix>(lds, g - groups_total, v.x, ProjArgs{}, M, v.kth, v.bmp, v.idx, v.nz_off,
                                                v.total_halfs, v.dst_off, v.dst_limit, overflow, v.nz, v.nz_capacity_halfs,
-                                               v.state, units, groups_total, spin_limit);
+                                               v.state, units, groups_total, spin_limit, v.landing);
 }
 
 // ------------------------------------------------------------------------------- dense prune
@@ -605,7 +610,7 @@ static size_t compress_ws_bytes(int B, int M)
 template <bool IS_VALUE, int SRC = kSrcMatrix>
 static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& proj, int B, int M, int kth, uint64_t* bmp, uint32_t* idx,
                           uint32_t* nz_off, uint64_t* total_halfs, const uint32_t* dst_off, const uint32_t* dst_limit,
-                          uint32_t* overflow, mstf_half* nz, uint64_t cap, void* ws)
+                          uint32_t* overflow, mstf_half* nz, uint64_t cap, void* ws, uint64_t* landing = nullptr)
 {
     const int nblk = M / 64, units = B * nblk;
 #ifndef MSTF_ONEPASS_W
@@ -614,7 +619,7 @@ static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& pr
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
     uint64_t* state = reinterpret_cast<uint64_t*>(ws);
-    const int words = groups + 1;
+    const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
     const uint32_t spin_limit = onepass_spin_limit();
     hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),
                        dim3(256), 0, st, state, words, total_halfs, static_cast<uint64_t*>(nullptr));
@@ -623,7 +628,7 @@ static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& pr
 #define MSTF_OP(WV)                                                                                                   \
     hipLaunchKernelGGL((compress_onepass_kernel<IS_VALUE, WV, SRC>), dim3((unsigned)groups), dim3(64 * WV), 0, st, xh, proj, M, kth, \
                        bmp, idx, nz_off, total_halfs, dst_off, dst_limit, overflow, reinterpret_cast<char*>(nz), cap,  \
-                       state, units, groups, spin_limit)
+                       state, units, groups, spin_limit, landing)
     if (W == MSTF_ONEPASS_W)
         MSTF_OP(MSTF_ONEPASS_W);
     else if (W == 2)
@@ -640,7 +645,7 @@ static int launch_onepass_kv(hipStream_t st, OnepassSide k, OnepassSide v, int B
     const int nblk = M / 64, units = B * nblk;
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
-    const int words = groups + 1;
+    const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
     k.state = reinterpret_cast<uint64_t*>(ws);
     v.state = k.state + words;
     const uint32_t spin_limit = onepass_spin_limit();
@@ -754,7 +759,8 @@ static int append_impl(void* stream, const mstf_half* x, int B, int M, int N, in
 // (nz_off and *total_halfs are outputs), else the append contract (dst_off / dst_limit / overflow are inputs).
 static int proj_impl(void* stream, const mstf_proj_source* s, int is_value, int M, int N, int kth, uint64_t* bmp,
                      uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, const uint32_t* dst_off,
-                     const uint32_t* dst_limit, mstf_half* nz, uint64_t cap, uint32_t* overflow, void* ws, size_t ws_bytes)
+                     const uint32_t* dst_limit, mstf_half* nz, uint64_t cap, uint32_t* overflow, void* ws, size_t ws_bytes,
+                     uint64_t* landing = nullptr)
 {
     if (!s || !s->x || s->batch <= 0 || s->heads <= 0 || s->rows <= 0 || M < 0 || M > s->rows || kth < 0 || kth > N)
         return MSTF_EINVAL;
@@ -798,13 +804,13 @@ static int proj_impl(void* stream, const mstf_proj_source* s, int is_value, int 
         int rc;
         if (rope)
             rc = launch_onepass<false, kSrcRope>(st, nullptr, pa, B, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                                 dst_limit, overflow, nz, capacity, ws);
+                                                 dst_limit, overflow, nz, capacity, ws, landing);
         else if (is_value)
             rc = launch_onepass<true, kSrcView>(st, nullptr, pa, B, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                                dst_limit, overflow, nz, capacity, ws);
+                                                dst_limit, overflow, nz, capacity, ws, landing);
         else
             rc = launch_onepass<false, kSrcView>(st, nullptr, pa, B, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                                 dst_limit, overflow, nz, capacity, ws);
+                                                 dst_limit, overflow, nz, capacity, ws, landing);
         if (rc != MSTF_OK) return rc;
     }
     // the tokens behind the compressed ones are only rotated
@@ -893,6 +899,19 @@ extern "C" int mstf_compress_proj_f16(void* stream, const mstf_proj_source* src,
                      nz_capacity_halfs, nullptr, workspace, workspace_bytes);
 }
 
+extern "C" int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
+                                            uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs,
+                                            mstf_half* nz, uint64_t nz_capacity_halfs, void* workspace,
+                                            size_t workspace_bytes, int64_t* landing, int64_t* value)
+{
+    if (M <= 0) return MSTF_EINVAL;
+    int rc = landing_ready(as_stream(stream), landing, value);
+    if (rc != MSTF_OK) return rc;
+    rc = proj_impl(stream, src, is_value, M, N, kth, bmp, idx, nz_off, total_halfs, nullptr, nullptr, nz, nz_capacity_halfs,
+                   nullptr, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing));
+    return rc != MSTF_OK ? rc : landing_wait(as_stream(stream), landing, value);
+}
+
 extern "C" int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                                     uint64_t* bmp, uint32_t* idx, const uint32_t* dst_off, const uint32_t* dst_limit,
                                     mstf_half* nz, uint32_t* overflow, void* workspace, size_t workspace_bytes)
@@ -917,11 +936,11 @@ static int kv_side_check(const void* x, int B, int M, int N, int kth, const void
     return MSTF_OK;
 }
 
-extern "C" int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k,
-                                    int kth_v, uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off,
-                                    uint64_t* k_total_halfs, mstf_half* k_nz, uint64_t k_capacity_halfs, uint64_t* v_bmp,
-                                    uint32_t* v_idx, uint32_t* v_nz_off, uint64_t* v_total_halfs, mstf_half* v_nz,
-                                    uint64_t v_capacity_halfs, void* workspace, size_t workspace_bytes)
+static int compress_kv_impl(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k, int kth_v,
+                            uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off, uint64_t* k_total_halfs, mstf_half* k_nz,
+                            uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
+                            uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
+                            size_t workspace_bytes, uint64_t* k_landing, uint64_t* v_landing)
 {
     int rc = kv_side_check(k, B, M, N, kth_k, k_bmp, k_idx, k_nz);
     if (rc == MSTF_OK) rc = kv_side_check(v, B, M, N, kth_v, v_bmp, v_idx, v_nz);
@@ -932,10 +951,43 @@ extern "C" int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf
     if (!workspace || workspace_bytes < mstf_compress_kv_workspace_bytes(B, M, N)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 256)) return MSTF_EALIGN;
     OnepassSide ks = {reinterpret_cast<const _Float16*>(k), kth_k, k_bmp, k_idx, k_nz_off, k_total_halfs, nullptr, nullptr,
-                      reinterpret_cast<char*>(k_nz), k_capacity_halfs, nullptr};
+                      reinterpret_cast<char*>(k_nz), k_capacity_halfs, nullptr, k_landing};
     OnepassSide vs = {reinterpret_cast<const _Float16*>(v), kth_v, v_bmp, v_idx, v_nz_off, v_total_halfs, nullptr, nullptr,
-                      reinterpret_cast<char*>(v_nz), v_capacity_halfs, nullptr};
+                      reinterpret_cast<char*>(v_nz), v_capacity_halfs, nullptr, v_landing};
     return launch_onepass_kv(as_stream(stream), ks, vs, B, M, nullptr, workspace);
+}
+
+extern "C" int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k,
+                                    int kth_v, uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off,
+                                    uint64_t* k_total_halfs, mstf_half* k_nz, uint64_t k_capacity_halfs, uint64_t* v_bmp,
+                                    uint32_t* v_idx, uint32_t* v_nz_off, uint64_t* v_total_halfs, mstf_half* v_nz,
+                                    uint64_t v_capacity_halfs, void* workspace, size_t workspace_bytes)
+{
+    return compress_kv_impl(stream, k, v, B, M, N, kth_k, kth_v, k_bmp, k_idx, k_nz_off, k_total_halfs, k_nz, k_capacity_halfs,
+                            v_bmp, v_idx, v_nz_off, v_total_halfs, v_nz, v_capacity_halfs, workspace, workspace_bytes, nullptr,
+                            nullptr);
+}
+
+extern "C" int mstf_compress_kv_landing_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k,
+                                            int kth_v, uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off,
+                                            uint64_t* k_total_halfs, mstf_half* k_nz, uint64_t k_capacity_halfs,
+                                            uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off, uint64_t* v_total_halfs,
+                                            mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
+                                            size_t workspace_bytes, int64_t* landings)
+{
+    if (!landings || !aligned_to(landings, 8)) return MSTF_EINVAL;
+    // a recorded launch would store to the words at every replay, whoever has them by then
+    bool recorded = false;
+    int rc = stream_recorded(as_stream(stream), &recorded);
+    if (rc != MSTF_OK) return rc;
+    for (int i = 0; i < 2; i++) __atomic_store_n(landings + i, recorded ? MSTF_NOT_LANDED : kLandingEmpty, __ATOMIC_RELEASE);
+    uint64_t* l = recorded ? nullptr : reinterpret_cast<uint64_t*>(landings);
+    rc = compress_kv_impl(stream, k, v, B, M, N, kth_k, kth_v, k_bmp, k_idx, k_nz_off, k_total_halfs, k_nz, k_capacity_halfs,
+                          v_bmp, v_idx, v_nz_off, v_total_halfs, v_nz, v_capacity_halfs, workspace, workspace_bytes, l,
+                          l ? l + 1 : nullptr);
+    if (rc != MSTF_OK)
+        for (int i = 0; i < 2; i++) __atomic_store_n(landings + i, MSTF_NOT_LANDED, __ATOMIC_RELEASE);
+    return rc;
 }
 
 extern "C" int mstf_append_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k,
@@ -954,8 +1006,8 @@ extern "C" int mstf_append_kv_f16(void* stream, const mstf_half* k, const mstf_h
     if (!workspace || workspace_bytes < mstf_compress_kv_workspace_bytes(B, M, N)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 256)) return MSTF_EALIGN;
     OnepassSide ks = {reinterpret_cast<const _Float16*>(k), kth_k, k_bmp, k_idx, nullptr, nullptr, k_dst_off, k_dst_limit,
-                      reinterpret_cast<char*>(k_nz), ~0ull, nullptr};
+                      reinterpret_cast<char*>(k_nz), ~0ull, nullptr, nullptr};
     OnepassSide vs = {reinterpret_cast<const _Float16*>(v), kth_v, v_bmp, v_idx, nullptr, nullptr, v_dst_off, v_dst_limit,
-                      reinterpret_cast<char*>(v_nz), ~0ull, nullptr};
+                      reinterpret_cast<char*>(v_nz), ~0ull, nullptr, nullptr};
     return launch_onepass_kv(as_stream(stream), ks, vs, B, M, overflow, workspace);
 }

@@ -3,6 +3,7 @@
 
 #include <atomic>
 #include <chrono>
+#include <mutex>
 
 namespace mstf {
 static std::atomic<int> g_last_hip_error{0};
@@ -83,38 +84,120 @@ __global__ void publish_word_kernel(const int64_t* __restrict__ src, int64_t* la
 }
 }  // namespace mstf
 
-extern "C" int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* value)
+int mstf::stream_recorded(hipStream_t st, bool* recorded)
 {
-    if (!src || !landing || !value) return MSTF_EINVAL;
-    if (!mstf::aligned_to(src, 8) || !mstf::aligned_to(landing, 8)) return MSTF_EALIGN;
-    hipStream_t st = mstf::as_stream(stream);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(st, &capturing);
-    if (e == hipSuccess && capturing != hipStreamCaptureStatusNone) e = hipErrorStreamCaptureUnsupported;
+    const hipError_t e = hipStreamIsCapturing(st, &capturing);
     if (e != hipSuccess) {
-        mstf::set_last_hip_error((int)e);
+        set_last_hip_error((int)e);
         return MSTF_ELAUNCH;
     }
-    constexpr int64_t kNothing = INT64_MIN + 1;  // told apart from a result by waiting for the stream, should one equal it
-    __atomic_store_n(landing, kNothing, __ATOMIC_RELEASE);
-    hipLaunchKernelGGL(mstf::publish_word_kernel, dim3(1), dim3(1), 0, st, src, landing);
-    int rc = mstf::check_launch();
+    *recorded = capturing != hipStreamCaptureStatusNone;
+    return MSTF_OK;
+}
+
+int mstf::landing_ready(hipStream_t st, int64_t* landing, const int64_t* value)
+{
+    if (!landing || !value) return MSTF_EINVAL;
+    if (!aligned_to(landing, 8)) return MSTF_EALIGN;
+    bool recorded = false;
+    const int rc = stream_recorded(st, &recorded);
     if (rc != MSTF_OK) return rc;
+    if (recorded) {
+        set_last_hip_error((int)hipErrorStreamCaptureUnsupported);
+        return MSTF_ELAUNCH;
+    }
+    __atomic_store_n(landing, kLandingEmpty, __ATOMIC_RELEASE);
+    return MSTF_OK;
+}
+
+int mstf::landing_wait(hipStream_t st, const int64_t* landing, int64_t* value)
+{
     // Long waits (a full stream, an error that keeps the word from coming) are left to the runtime.
     constexpr auto kWatch = std::chrono::microseconds(500);
     const auto until = std::chrono::steady_clock::now() + kWatch;
-    int64_t v = kNothing;
+    int64_t v = kLandingEmpty;
     do {
-        for (int i = 0; i < 64 && v == kNothing; i++) v = __atomic_load_n(landing, __ATOMIC_ACQUIRE);
-    } while (v == kNothing && std::chrono::steady_clock::now() < until);
-    if (v == kNothing) {
-        e = hipStreamSynchronize(st);
+        for (int i = 0; i < 64 && v == kLandingEmpty; i++) v = __atomic_load_n(landing, __ATOMIC_ACQUIRE);
+    } while (v == kLandingEmpty && std::chrono::steady_clock::now() < until);
+    if (v == kLandingEmpty) {
+        bool recorded = false;
+        const int rc = stream_recorded(st, &recorded);
+        if (rc != MSTF_OK) return rc;
+        const hipError_t e = recorded ? hipErrorStreamCaptureUnsupported : hipStreamSynchronize(st);
         if (e != hipSuccess) {
-            mstf::set_last_hip_error((int)e);
+            set_last_hip_error((int)e);
             return MSTF_ELAUNCH;
         }
         v = __atomic_load_n(landing, __ATOMIC_ACQUIRE);
     }
     *value = v;
     return MSTF_OK;
+}
+
+extern "C" int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* value)
+{
+    if (!src || !landing || !value) return MSTF_EINVAL;
+    if (!mstf::aligned_to(src, 8) || !mstf::aligned_to(landing, 8)) return MSTF_EALIGN;
+    hipStream_t st = mstf::as_stream(stream);
+    int rc = mstf::landing_ready(st, landing, value);
+    if (rc != MSTF_OK) return rc;
+    hipLaunchKernelGGL(mstf::publish_word_kernel, dim3(1), dim3(1), 0, st, src, landing);
+    rc = mstf::check_launch();
+    return rc != MSTF_OK ? rc : mstf::landing_wait(st, landing, value);
+}
+
+extern "C" int mstf_landing_wait(void* stream, const int64_t* landing, int64_t* value)
+{
+    if (!landing || !value) return MSTF_EINVAL;
+    if (!mstf::aligned_to(landing, 8)) return MSTF_EALIGN;
+    return mstf::landing_wait(mstf::as_stream(stream), landing, value);
+}
+
+// ------------------------------------------------------------------ landings of calls that are not waited for
+// Pairs of words in one block of pinned memory, made with the first of them and kept: 1024 pairs, so that a program that holds
+// on to more results than that finds none free and reads its totals by mstf_read_word.  A pair that is given back while its
+// kernel has yet to store to it stays away from the others until it has.
+namespace mstf {
+static std::mutex g_landing_lock;
+static int64_t* g_landing_block = nullptr;
+static bool g_landing_failed = false;
+constexpr int kLandingPairs = 1024;
+static uint16_t g_landing_free[kLandingPairs];  // a ring: the one that was given back first is the first to be taken
+static int g_landing_head = 0, g_landing_count = 0;
+}  // namespace mstf
+
+extern "C" int64_t* mstf_landing_take(void)
+{
+    using namespace mstf;
+    std::lock_guard<std::mutex> hold(g_landing_lock);
+    if (!g_landing_block) {
+        void* p = nullptr;
+        if (g_landing_failed || hipHostMalloc(&p, kLandingPairs * 2 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+            g_landing_failed = true;
+            return nullptr;
+        }
+        g_landing_block = static_cast<int64_t*>(p);
+        for (int i = 0; i < kLandingPairs; i++) {
+            g_landing_block[2 * i] = g_landing_block[2 * i + 1] = MSTF_NOT_LANDED;
+            g_landing_free[i] = (uint16_t)i;
+        }
+        g_landing_count = kLandingPairs;
+    }
+    if (g_landing_count == 0) return nullptr;
+    int64_t* pair = g_landing_block + 2 * g_landing_free[g_landing_head];
+    for (int i = 0; i < 2; i++)
+        if (__atomic_load_n(pair + i, __ATOMIC_ACQUIRE) == kLandingEmpty) return nullptr;  // (and those behind it are younger)
+    g_landing_head = (g_landing_head + 1) % kLandingPairs;
+    g_landing_count--;
+    return pair;
+}
+
+extern "C" void mstf_landing_give(int64_t* pair)
+{
+    using namespace mstf;
+    std::lock_guard<std::mutex> hold(g_landing_lock);
+    if (!pair || !g_landing_block || pair < g_landing_block || pair >= g_landing_block + 2 * kLandingPairs) return;
+    g_landing_free[(g_landing_head + g_landing_count) % kLandingPairs] = (uint16_t)((pair - g_landing_block) / 2);
+    g_landing_count++;
 }

@@ -62,12 +62,36 @@ def read_word(t):
     if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.int64 and t.numel() == 1
             and t.device.index == torch._C._cuda_getDevice()):
         return int(t)
+    own = _landing_word()
+    check(lib().mstf_read_word(_stream(), t.data_ptr(), own[1], own[3]), "mstf_read_word")
+    return own[2].value
+
+
+def _landing_word():
+    """This thread's (pinned word, its address, result, its address) for the calls that wait for a word."""
     own = getattr(_LANDING, "own", None)
     if own is None:
         word, value = torch.empty(1, dtype=torch.int64, pin_memory=True), ctypes.c_int64()
         own = _LANDING.own = (word, word.data_ptr(), value, ctypes.addressof(value))
-    check(lib().mstf_read_word(_stream(), t.data_ptr(), own[1], own[3]), "mstf_read_word")
-    return own[2].value
+    return own
+
+
+class _LandingPair:
+    """The pinned words that a call which returns without waiting has its two totals stored to (mstf_landing_take)."""
+    __slots__ = ("pair", "stream", "_give")
+    NOT_LANDED = -(1 << 63) + 2
+
+    def __init__(self, pair, stream):
+        self.pair, self.stream, self._give = pair, stream, lib().mstf_landing_give
+
+    def read(self, side):
+        """The total, or None where the call was recorded into a graph."""
+        own = _landing_word()
+        check(lib().mstf_landing_wait(self.stream, self.pair + 8 * side, own[3]), "mstf_landing_wait")
+        return None if own[2].value == self.NOT_LANDED else own[2].value
+
+    def __del__(self):
+        self._give(self.pair)
 
 
 def attention_workspace_least(tokens, window, rows):
@@ -102,10 +126,11 @@ class CompressedKV:
 
     bmp int64 [B, T], idx int32 [B, T+1], nz fp16 flat, nz_off int32 [B] (16-byte units)."""
 
-    def __init__(self, bmp, idx, nz, nz_off, tokens, head_dim, is_value, total_halfs=None):
+    def __init__(self, bmp, idx, nz, nz_off, tokens, head_dim, is_value, total_halfs=None, landing=None):
         self.bmp, self.idx, self.nz, self.nz_off = bmp, idx, nz, nz_off
         self.tokens, self.head_dim, self.is_value = tokens, head_dim, is_value
         self.total_halfs = total_halfs
+        self._landing = landing     # _LandingPair that gets the total too
 
     @property
     def heads(self):
@@ -114,7 +139,9 @@ class CompressedKV:
     def used_halfs(self):
         """Number of fp16 values in use (reads the device-side total once).  The one-pass compressor reports a wait that
         ran out - which the dispatch order rules out - as a total of all ones: that raises here."""
-        n = read_word(self.total_halfs)
+        n = self._landing.read(int(self.is_value)) if self._landing is not None else None
+        if n is None:
+            n = read_word(self.total_halfs)
         if n < 0 or n > (1 << 62):
             raise RuntimeError("the compressor gave up waiting for an earlier workgroup; the packed values are incomplete")
         return n
@@ -194,11 +221,17 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
                     torch.empty((cap,), dtype=torch.float16, device=dev)))
     ws = workspace(dev, L.mstf_compress_kv_workspace_bytes(B, M, N), ws)
     (kb, ki, ko, kt, kn), (vb, vi, vo, vt, vn) = out
-    check(L.mstf_compress_kv_f16(_stream(), k.data_ptr(), v.data_ptr(), B, M, N, int(kth_k), int(kth_v), kb.data_ptr(),
-                                 ki.data_ptr(), ko.data_ptr(), kt.data_ptr(), kn.data_ptr(), cap, vb.data_ptr(),
-                                 vi.data_ptr(), vo.data_ptr(), vt.data_ptr(), vn.data_ptr(), cap, ws.data_ptr(),
-                                 ws.numel()), "mstf_compress_kv_f16")
-    return CompressedKV(kb, ki, kn, ko, M, N, False, kt), CompressedKV(vb, vi, vn, vo, M, N, True, vt)
+    st = _stream()
+    args = (st, k.data_ptr(), v.data_ptr(), B, M, N, int(kth_k), int(kth_v), kb.data_ptr(), ki.data_ptr(), ko.data_ptr(),
+            kt.data_ptr(), kn.data_ptr(), cap, vb.data_ptr(), vi.data_ptr(), vo.data_ptr(), vt.data_ptr(), vn.data_ptr(), cap,
+            ws.data_ptr(), ws.numel())
+    pair = L.mstf_landing_take()
+    landing = _LandingPair(pair, st) if pair else None
+    if landing is not None:
+        check(L.mstf_compress_kv_landing_f16(*args, pair), "mstf_compress_kv_landing_f16")
+    else:
+        check(L.mstf_compress_kv_f16(*args), "mstf_compress_kv_f16")
+    return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
 
 def proj_source(x, cos=None, sin=None, rot=None):
@@ -239,13 +272,20 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     total = torch.empty((1,), dtype=torch.int64, device=dev)
     nz = torch.empty((max(cap, 8),), dtype=torch.float16, device=dev)
     ws = workspace(dev, L.mstf_compress_workspace_bytes(B, max(M, 64), N), ws)
-    check(L.mstf_compress_proj_f16(_stream(), ctypes.byref(src), int(is_value), M, N, int(kth), bmp.data_ptr(),
-                                   idx.data_ptr(), nz_off.data_ptr(), total.data_ptr(), nz.data_ptr(), cap,
-                                   ws.data_ptr(), ws.numel()), "mstf_compress_proj_f16")
+    args = (_stream(), ctypes.byref(src), int(is_value), M, N, int(kth), bmp.data_ptr(), idx.data_ptr(), nz_off.data_ptr(),
+            total.data_ptr(), nz.data_ptr(), cap, ws.data_ptr(), ws.numel())
+    sized = capacity_halfs is None and M != 0
+    if sized:
+        own = _landing_word()
+        check(L.mstf_compress_proj_sized_f16(*args, own[1], own[3]), "mstf_compress_proj_sized_f16")
+    else:
+        check(L.mstf_compress_proj_f16(*args), "mstf_compress_proj_f16")
     if M == 0:
         return None, rot
-    if capacity_halfs is None:
-        n = read_word(total)
+    if sized:
+        n = own[2].value
+        if n < 0:
+            raise RuntimeError("the compressor gave up waiting for an earlier workgroup; the packed values are incomplete")
         return CompressedKV(bmp, idx, nz[:n], nz_off, M, N, is_value, n), rot
     return CompressedKV(bmp, idx, nz, nz_off, M, N, is_value, total), rot
 
