@@ -9,7 +9,10 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmustafar_hip.so")
 
+HOST_PATH = os.path.join(_HERE, "_host.so")
+
 _lib = None
+_host = None
 
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
@@ -116,6 +119,19 @@ def lib():
             fn.argtypes = args
         _lib = l
     return _lib
+
+
+def host():
+    """The native calls (csrc/host.cpp), which do in one call what the functions of this package do on the host."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError("_host.so is missing at %s: build it with `python -m mustafar_amd.build`" % HOST_PATH)
+        import torch  # noqa: F401  (the module's symbols)
+        from . import _host as module
+        _host = module
+    return _host
 
 
 def check(rc, what):

@@ -1,4 +1,4 @@
-"""Builds libmustafar_hip.so for gfx950 with hipcc (cross-compiles without a GPU)."""
+"""Builds libmustafar_hip.so for gfx950 with hipcc (cross-compiles without a GPU), and _host.so beside it."""
 import os
 import subprocess
 import sys
@@ -6,6 +6,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmustafar_hip.so")
+HOST = os.path.join(HERE, "_host.so")
 SOURCES = ["runtime.hip", "spmv.hip", "compress.hip", "quant.hip", "quant_spmv.hip", "fused.hip", "fused_quant.hip", "window_append.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -51,7 +52,25 @@ def build(verbose=False):
         for _, out in results:
             if out.strip():
                 print(out)
+    build_host(verbose)
     return LIB
+
+
+def build_host(verbose=False):
+    """The Python module of native calls, by the host compiler against torch's headers and the library above."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    import torch
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+    cmd += ["-isystem" + p for p in cpp_extension.include_paths()] + ["-I" + sysconfig.get_paths()["include"]]
+    cmd += [os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + HERE, "-l:libmustafar_hip.so", "-Wl,-rpath,$ORIGIN", "-L" + libs,
+            "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd))
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed on host.cpp:\n" + res.stdout)
 
 
 if __name__ == "__main__":

@@ -8,7 +8,7 @@ inputs: [B, M, N] fp16 on the GPU, already pruned (or pruned here: `kth`), M % 6
 import torch
 
 from . import ops
-from ._lib import check, lib
+from ._lib import host
 
 
 def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, sized=False):
@@ -17,45 +17,8 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, si
     default: a fresh buffer with room for the worst case.  Returns the per-tile arrays, the buffer and the word total
     as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host.
     sized: the total as an int instead."""
-    assert inputs.is_cuda
-    assert inputs.dim() == 3
-    B, M, N = inputs.shape
-    assert M % 64 == 0
-    if inputs.dtype != torch.float16:
-        raise RuntimeError("inputs must be float16")
-    x = inputs.contiguous()
-    dev = x.device
-    T = M * N // 64
-    L = lib()
-    bmp = torch.empty((B, T), dtype=torch.int64, device=dev)
-    tile_off = torch.empty((B, T), dtype=torch.int32, device=dev)
-    counts = torch.empty((B, T), dtype=torch.int32, device=dev)
-    units = torch.empty((B, T), dtype=torch.int32, device=dev)
-    if group_size not in (32, 64):
-        raise RuntimeError("group_size must be 32 or 64")
-    meta_shape = (B, T) if group_size == 64 else (B, T, 2)
-    scales = torch.empty(meta_shape, dtype=torch.float16, device=dev)
-    zeros = torch.empty(meta_shape, dtype=torch.float16, device=dev)
-    total = torch.empty((1,), dtype=torch.int64, device=dev)
-    ws = ops.workspace(dev, L.mstf_compress_quant_workspace_bytes(B, M, N), ws)
-    st = ops._stream()
-    # one pass with room for the worst case (every element kept: 64 // capacity words per tile)
-    cap_words = B * T * (64 * int(bit) // 32)
-    if room is None:
-        room = torch.empty((max(cap_words, 1),), dtype=torch.int32, device=dev)
-    else:
-        cap_words = room.numel()
-    assert room.dtype == torch.int32 and room.is_contiguous()
-    args = (st, x.data_ptr(), int(bool(is_value)), B, M, N, int(kth), int(bit), int(group_size), bmp.data_ptr(),
-            tile_off.data_ptr(), counts.data_ptr(), units.data_ptr(), scales.data_ptr(), zeros.data_ptr(), total.data_ptr(),
-            room.data_ptr(), cap_words, ws.data_ptr(), ws.numel())
-    if sized:
-        own = ops._landing_word()
-        check(L.mstf_compress_quant_sized(*args, own[1], own[3]), "mstf_compress_quant_sized")
-        total = own[2].value
-    else:
-        check(L.mstf_compress_quant_grouped(*args), "mstf_compress_quant_grouped")
-    return bmp, tile_off, room, counts, units, scales, zeros, total
+    return ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),
+                     int(group_size), room, ops._landing_word()[1] if sized else 0)
 
 
 def words_written(total):

@@ -9,7 +9,7 @@ import threading
 
 import torch
 
-from ._lib import check, lib
+from ._lib import check, host, lib
 
 class Workspace:
     """Scratch memory for the entry points that need it (split partials, compressor scans), owned by one caller.
@@ -116,6 +116,20 @@ def workspace(device, nbytes, ws=None, call=None):
     return w.get(nbytes, call)
 
 
+def _call(fn, ws, device, call, *args):
+    """One of the native calls (csrc/host.cpp), with the scratch memory at hand or, where it answers that it needs more,
+    with what `workspace` finds."""
+    if ws is None:
+        w = _WS.get((device.type, device.index, _stream())) if device.type == "cuda" else None
+        t = None if w is None else w._bufs[-1]
+    else:
+        t = ws._bufs[-1] if isinstance(ws, Workspace) else ws
+    r = fn(*args, t, 0)
+    if type(r) is int:
+        r = fn(*args, workspace(device, r, ws, call), 1)
+    return r
+
+
 def kth_from_sparsity(sparsity, head_dim):
     """Rank of the pruning threshold: max(1, int(target_sparsity * D)) as in dh_prune_key."""
     return max(1, int(sparsity * head_dim))
@@ -207,30 +221,11 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     identical outputs, less time - a launch of both sides runs less in lockstep than two launches of one side each.
     k, v: [B, M, N]; capacity_halfs (default: room for the dense rows) sizes both value buffers, the totals stay on
     the device.  Returns (CompressedKV of the keys, CompressedKV of the values)."""
-    assert k.is_cuda and v.is_cuda and k.dtype == v.dtype == torch.float16 and k.dim() == 3 and k.shape == v.shape
-    k, v = k.contiguous(), v.contiguous()
-    B, M, N = k.shape
-    T = M * N // 64
-    dev = k.device
-    L = lib()
-    cap = B * M * N if capacity_halfs is None else int(capacity_halfs)
-    out = []
-    for _ in range(2):
-        out.append((torch.empty((B, T), dtype=torch.int64, device=dev), torch.empty((B, T + 1), dtype=torch.int32, device=dev),
-                    torch.empty((B,), dtype=torch.int32, device=dev), torch.empty((1,), dtype=torch.int64, device=dev),
-                    torch.empty((cap,), dtype=torch.float16, device=dev)))
-    ws = workspace(dev, L.mstf_compress_kv_workspace_bytes(B, M, N), ws)
-    (kb, ki, ko, kt, kn), (vb, vi, vo, vt, vn) = out
-    st = _stream()
-    args = (st, k.data_ptr(), v.data_ptr(), B, M, N, int(kth_k), int(kth_v), kb.data_ptr(), ki.data_ptr(), ko.data_ptr(),
-            kt.data_ptr(), kn.data_ptr(), cap, vb.data_ptr(), vi.data_ptr(), vo.data_ptr(), vt.data_ptr(), vn.data_ptr(), cap,
-            ws.data_ptr(), ws.numel())
-    pair = L.mstf_landing_take()
-    landing = _LandingPair(pair, st) if pair else None
-    if landing is not None:
-        check(L.mstf_compress_kv_landing_f16(*args, pair), "mstf_compress_kv_landing_f16")
-    else:
-        check(L.mstf_compress_kv_f16(*args), "mstf_compress_kv_f16")
+    pair = lib().mstf_landing_take()
+    landing = _LandingPair(pair, _stream()) if pair else None
+    kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
+                                                   -1 if capacity_halfs is None else int(capacity_halfs), pair or 0)
+    M, N = k.shape[1:]
     return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
 
@@ -261,33 +256,15 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     """Prune and compress the first M tokens of x [batch, rows, heads, 128] where the projection left them, the keys
     rotated first when cos / sin are given (all rows are rotated and written to rot).  Heads are numbered
     batch * heads + head.  Returns (CompressedKV, rot)."""
-    src, rot = proj_source(x, cos, sin, rot)
-    B, N, dev = x.shape[0] * x.shape[2], x.shape[3], x.device
-    T = M * N // 64
-    L = lib()
-    cap = B * M * N if capacity_halfs is None else int(capacity_halfs)
-    bmp = torch.empty((B, T), dtype=torch.int64, device=dev)
-    idx = torch.empty((B, T + 1), dtype=torch.int32, device=dev)
-    nz_off = torch.empty((B,), dtype=torch.int32, device=dev)
-    total = torch.empty((1,), dtype=torch.int64, device=dev)
-    nz = torch.empty((max(cap, 8),), dtype=torch.float16, device=dev)
-    ws = workspace(dev, L.mstf_compress_workspace_bytes(B, max(M, 64), N), ws)
-    args = (_stream(), ctypes.byref(src), int(is_value), M, N, int(kth), bmp.data_ptr(), idx.data_ptr(), nz_off.data_ptr(),
-            total.data_ptr(), nz.data_ptr(), cap, ws.data_ptr(), ws.numel())
+    if cos is not None and rot is None:
+        rot = x
     sized = capacity_halfs is None and M != 0
-    if sized:
-        own = _landing_word()
-        check(L.mstf_compress_proj_sized_f16(*args, own[1], own[3]), "mstf_compress_proj_sized_f16")
-    else:
-        check(L.mstf_compress_proj_f16(*args), "mstf_compress_proj_f16")
+    bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
+                                           rot, -1 if capacity_halfs is None else int(capacity_halfs),
+                                           _landing_word()[1] if sized else 0)
     if M == 0:
         return None, rot
-    if sized:
-        n = own[2].value
-        if n < 0:
-            raise RuntimeError("the compressor gave up waiting for an earlier workgroup; the packed values are incomplete")
-        return CompressedKV(bmp, idx, nz[:n], nz_off, M, N, is_value, n), rot
-    return CompressedKV(bmp, idx, nz, nz_off, M, N, is_value, total), rot
+    return CompressedKV(bmp, idx, nz, nz_off, M, x.shape[3], is_value, n if sized else total), rot
 
 
 def key_spmv(ck, q, groups, n_rows=1, out=None):
@@ -319,18 +296,8 @@ def decode_attention(ck, cv, q, groups, out=None, lse=None, ws=None):
     """Fused key SpMV -> scale+softmax -> value SpMV over the compressed tokens, one query row per head.
 
     q: [Bq, D] fp16 -> out [Bq, D] fp16.  lse (optional fp32 [Bq, 2]) receives (max, sum) of every row."""
-    assert q.dtype == torch.float16 and q.is_contiguous()
-    D = ck.head_dim
-    Bq = q.numel() // D
-    L = lib()
-    o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
-    ws = workspace(q.device, L.mstf_decode_attention_workspace_bytes(ck.tokens, D, Bq, groups), ws, (ck.tokens, 0, Bq))
-    check(L.mstf_decode_attention_f16(_stream(), ck.bmp.data_ptr(), ck.nz.data_ptr(), ck.idx.data_ptr(),
-                                      ck.nz_off.data_ptr(), cv.bmp.data_ptr(), cv.nz.data_ptr(), cv.idx.data_ptr(),
-                                      cv.nz_off.data_ptr(), q.data_ptr(), o.data_ptr(),
-                                      lse.data_ptr() if lse is not None else None, ck.tokens, D, Bq, groups,
-                                      ws.data_ptr(), ws.numel()), "mstf_decode_attention_f16")
-    return o
+    return _call(host().decode_attention, ws, q.device, (ck.tokens, 0, q.numel() // ck.head_dim), ck.bmp, ck.nz, ck.idx, ck.nz_off,
+                 cv.bmp, cv.nz, cv.idx, cv.nz_off, q, groups, ck.tokens, ck.head_dim, out, lse)
 
 
 def decode_attention_static(ck, cv, q, groups, out=None, lse=None):
@@ -405,37 +372,11 @@ def decode_step_pool(k_pool, v_pool, q_in, k_in, v_in, k_win, v_win, win_len, co
     launch of the compressed tokens.  q_in [bs, n_q * D], k_in / v_in [bs, n_kv * D]: the projection outputs of the
     new token (views with a batch stride are fine); cos, sin [D] or [bs, D] or None; k_win, v_win
     [bs * n_kv, win_stride, D]; win_len bounds the count of valid rows after the step, win_len_dev holds it."""
-    D = k_win.shape[-1]
-    bs = k_in.shape[0]
-    n_kv, n_q = k_in.shape[-1] // D, q_in.shape[-1] // D
-    for t in (q_in, k_in, v_in):
-        assert t.dtype == torch.float16 and t.dim() == 2 and t.stride(1) == 1 and t.shape[0] == bs
-    assert k_win.dtype == torch.float16 and k_win.is_contiguous() and v_win.is_contiguous() and k_win.shape == v_win.shape
-    assert k_win.shape[0] == bs * n_kv and v_in.shape[-1] == n_kv * D and n_q % n_kv == 0
     assert k_pool.max_tokens == v_pool.max_tokens
-    rope_stride = 0
-    if cos is not None:
-        assert cos.dtype == torch.float16 and sin.dtype == torch.float16 and cos.shape == sin.shape
-        assert cos.shape[-1] == D and cos.stride(-1) == 1 and sin.stride(-1) == 1
-        if cos.dim() == 2 and cos.shape[0] > 1:
-            assert cos.shape[0] == bs and cos.stride(0) == sin.stride(0)
-            rope_stride = cos.stride(0)
-    L = lib()
-    Bq = bs * n_q
-    o = torch.empty((Bq, D), dtype=torch.float16, device=q_in.device) if out is None else out
-    ws = workspace(q_in.device, L.mstf_decode_attention_window_workspace_bytes(k_pool.max_tokens, int(win_len), D, Bq,
-                                                                              n_q // n_kv), ws,
-                   (k_pool.max_tokens, int(win_len), Bq))
-    cp = [t.data_ptr() for t in (k_pool.bmp_store, k_pool.nz, k_pool.idx_store, k_pool.nz_off, v_pool.bmp_store, v_pool.nz,
-                                 v_pool.idx_store, v_pool.nz_off)]
-    check(L.mstf_decode_step_pool_f16(
-        _stream(), *cp, q_in.data_ptr(), q_in.stride(0), k_in.data_ptr(), k_in.stride(0), v_in.data_ptr(), v_in.stride(0),
-        bs, n_q, n_kv, cos.data_ptr() if cos is not None else None, sin.data_ptr() if sin is not None else None,
-        rope_stride, k_win.data_ptr(), v_win.data_ptr(), k_win.shape[1], int(win_len),
-        win_len_dev.data_ptr() if win_len_dev is not None else None, overflow.data_ptr() if overflow is not None else None,
-        o.data_ptr(), lse.data_ptr() if lse is not None else None, k_pool.max_tokens, k_pool.tokens_dev.data_ptr(),
-        k_pool.tile_capacity, D, ws.data_ptr(), ws.numel()), "mstf_decode_step_pool_f16")
-    return o
+    return _call(host().decode_step, ws, q_in.device, (k_pool.max_tokens, int(win_len), q_in.numel() // k_win.shape[-1]),
+                 k_pool.bmp_store, k_pool.nz, k_pool.idx_store, k_pool.nz_off, v_pool.bmp_store, v_pool.nz, v_pool.idx_store,
+                 v_pool.nz_off, q_in, k_in, v_in, k_win, v_win, int(win_len), cos, sin, win_len_dev, overflow, out, lse,
+                 k_pool.max_tokens, k_pool.tokens_dev, k_pool.tile_capacity)
 
 
 def window_append(k_in, v_in, k_win, v_win, win_len, q_in=None, cos=None, sin=None, q_out=None, win_len_dev=None,
@@ -501,13 +442,7 @@ def decode_attention_merge(ws, tokens, head_dim, Bq, groups, out=None, lse=None)
 
 def scale_softmax(s, head_dim, out=None):
     """softmax(s / sqrt(head_dim), dtype=float32).to(float16) over the last axis."""
-    assert s.dtype == torch.float16 and s.stride(-1) == 1
-    L = s.shape[-1]
-    s2 = s.reshape(-1, L)
-    p = torch.empty_like(s2) if out is None else out.reshape(-1, L)
-    check(lib().mstf_scale_softmax_f16(_stream(), s2.data_ptr(), p.data_ptr(), s2.shape[0], L, s2.stride(0),
-                                       p.stride(0), int(head_dim)), "mstf_scale_softmax_f16")
-    return p.reshape(s.shape)
+    return host().scale_softmax(s, int(head_dim), out)
 
 
 def sqrt_head_dim(head_dim):
