@@ -65,6 +65,11 @@ int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* 
  * mstf_landing_wait: waits for a word's value; MSTF_NOT_LANDED: the call was recorded into a graph or refused, and the total is
  * in device memory only.  All ones: a workgroup gave up waiting. */
 #define MSTF_NOT_LANDED (INT64_MIN + 2)
+/* status (those calls; null: none): mstf_status_bytes(B, M, sides) bytes of device memory, 8-byte aligned, that hold zeros when
+ * the call begins and are used by nothing else meanwhile; the call leaves zeros, so that the next one may have them as they are
+ * (without, a launch in front clears words in the workspace).  After a total of all ones they have to be cleared.  sides: 2 for
+ * keys and values in one call. */
+size_t mstf_status_bytes(int B, int M, int sides);
 int64_t* mstf_landing_take(void);
 void mstf_landing_give(int64_t* pair);
 int mstf_landing_wait(void* stream, const int64_t* landing, int64_t* value);
@@ -143,12 +148,12 @@ int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, i
                          uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
                          uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
                          size_t workspace_bytes);
-/* The same with a pair of landings (mstf_landing_take): keys' total, values' total. */
+/* The same with a pair of landings (mstf_landing_take; null: none) - keys' total, values' total - and kept status words. */
 int mstf_compress_kv_landing_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k, int kth_v,
                                  uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off, uint64_t* k_total_halfs, mstf_half* k_nz,
                                  uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
                                  uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
-                                 size_t workspace_bytes, int64_t* landings);
+                                 size_t workspace_bytes, uint64_t* status, size_t status_bytes, int64_t* landings);
 int mstf_append_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k, int kth_v,
                        uint64_t* k_bmp, uint32_t* k_idx, const uint32_t* k_dst_off, const uint32_t* k_dst_limit,
                        mstf_half* k_nz, uint64_t* v_bmp, uint32_t* v_idx, const uint32_t* v_dst_off,
@@ -190,8 +195,8 @@ int mstf_compress_proj_f16(void* stream, const mstf_proj_source* src, int is_val
  * Refused (MSTF_ELAUNCH) while the stream is being captured. */
 int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                                  uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, mstf_half* nz,
-                                 uint64_t nz_capacity_halfs, void* workspace, size_t workspace_bytes, int64_t* landing,
-                                 int64_t* value);
+                                 uint64_t nz_capacity_halfs, void* workspace, size_t workspace_bytes, uint64_t* status,
+                                 size_t status_bytes, int64_t* landing, int64_t* value);
 int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                          uint64_t* bmp, uint32_t* idx, const uint32_t* dst_off, const uint32_t* dst_limit,
                          mstf_half* nz, uint32_t* overflow, void* workspace, size_t workspace_bytes);
@@ -477,8 +482,8 @@ int mstf_compress_quant_grouped(void* stream, const mstf_half* x, int is_value, 
 int mstf_compress_quant_sized(void* stream, const mstf_half* x, int is_value, int B, int M, int N, int kth, int bit,
                               int group_size, uint64_t* bmp, uint32_t* tile_off, uint32_t* counts, uint32_t* units,
                               mstf_half* scales, mstf_half* zeros, uint64_t* total_words, uint32_t* packed,
-                              uint64_t packed_capacity_words, void* workspace, size_t workspace_bytes, int64_t* landing,
-                              int64_t* value);
+                              uint64_t packed_capacity_words, void* workspace, size_t workspace_bytes, uint64_t* status,
+                              size_t status_bytes, int64_t* landing, int64_t* value);
 int mstf_key_spmv_quant_grouped(void* stream, const uint64_t* bmp, const uint32_t* packed, const uint32_t* tile_off,
                                 const mstf_half* scales, const mstf_half* zeros, const mstf_half* Bm, mstf_half* C, int M,
                                 int K, int Bq, int groups, int n_rows, int bit, int capacity, int dequant_mode,

@@ -39,6 +39,7 @@ SIGNATURES = {
     "mstf_version": (_i, []),
     "mstf_probe_read": (_i, [_vp, _vp, _sz, _vp, _i]),
     "mstf_read_word": (_i, [_vp, _vp, _vp, _vp]),
+    "mstf_status_bytes": (_sz, [_i, _i, _i]),
     "mstf_landing_take": (_vp, []),
     "mstf_landing_give": (None, [_vp]),
     "mstf_landing_wait": (_i, [_vp, _vp, _vp]),
@@ -55,11 +56,11 @@ SIGNATURES = {
     "mstf_compress_kv_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _vp, _vp, _vp, _vp,
                                   _u64, _vp, _sz]),
     "mstf_compress_kv_landing_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _vp, _vp, _vp,
-                                          _vp, _u64, _vp, _sz, _vp]),
+                                          _vp, _u64, _vp, _sz, _vp, _sz, _vp]),
     "mstf_append_kv_f16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                 _vp, _sz]),
     "mstf_compress_proj_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _sz]),
-    "mstf_compress_proj_sized_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _sz, _vp, _vp]),
+    "mstf_compress_proj_sized_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _sz, _vp, _sz, _vp, _vp]),
     "mstf_append_proj_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz]),
     "mstf_key_spmv_f16": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i]),
     "mstf_value_spmv_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
@@ -94,7 +95,7 @@ SIGNATURES = {
     "mstf_compress_quant_grouped": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _u64,
                                          _vp, _sz]),
     "mstf_compress_quant_sized": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _u64,
-                                       _vp, _sz, _vp, _vp]),
+                                       _vp, _sz, _vp, _sz, _vp, _vp]),
     "mstf_key_spmv_quant_grouped": (_i, [_vp] * 8 + [_i] * 9),
     "mstf_value_spmv_quant_grouped": (_i, [_vp] * 8 + [_i] * 9 + [_vp, _sz]),
     "mstf_decode_attention_quant_grouped": (_i, [_vp] * 14 + [_i] * 8 + [_vp, _sz]),

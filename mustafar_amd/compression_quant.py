@@ -17,15 +17,23 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, si
     default: a fresh buffer with room for the worst case.  Returns the per-tile arrays, the buffer and the word total
     as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host.
     sized: the total as an int instead."""
-    return ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),
-                     int(group_size), room, ops._landing_word()[1] if sized else 0)
+    own = ops._own_workspace(ws, inputs.device) if sized else None
+    out = ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),
+                    int(group_size), room, ops._landing_word()[1] if sized else 0,
+                    own.status(inputs.shape[0] * (inputs.shape[1] // 64) + 2) if own else None)
+    if sized and out[-1] < 0:
+        ops.gave_up(own, _GAVE_UP)
+    return out
+
+
+_GAVE_UP = "the quantised producer gave up waiting for an earlier workgroup; the packed words are incomplete"
 
 
 def words_written(total):
     """The producer's word total on the host (one read, as the reference's .item()); raises if the producer gave up."""
     n = ops.read_word(total)
     if n < 0:   # all ones: a workgroup of the one-pass producer gave up waiting (ruled out by the dispatch order)
-        raise RuntimeError("the quantised producer gave up waiting for an earlier workgroup; the packed words are incomplete")
+        raise RuntimeError(_GAVE_UP)
     return n
 
 

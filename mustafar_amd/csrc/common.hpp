@@ -119,6 +119,8 @@ constexpr int64_t kLandingEmpty = INT64_MIN + 1;
 int landing_ready(hipStream_t st, int64_t* landing, const int64_t* value);
 int landing_wait(hipStream_t st, const int64_t* landing, int64_t* value);
 int stream_recorded(hipStream_t st, bool* recorded);
+// Kept status words of a producer (mstf_status_bytes; null: none), compress.hip.
+int status_check(const uint64_t* status, size_t bytes, int64_t B, int M, int sides);
 
 inline bool aligned_to(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }

@@ -377,7 +377,7 @@ __device__ __forceinline__ void onepass_workgroup(
     uint64_t* __restrict__ bmp, uint32_t* __restrict__ idx, uint32_t* __restrict__ nz_off,
     uint64_t* __restrict__ total_halfs, const uint32_t* __restrict__ dst_off, const uint32_t* __restrict__ dst_limit,
     uint32_t* __restrict__ overflow, char* __restrict__ nz, uint64_t nz_capacity_halfs, uint64_t* state, int units,
-    int groups_total, uint32_t spin_limit, uint64_t* landing)
+    int groups_total, uint32_t spin_limit, const Handover& how)
 {
     auto& bufs = lds.bufs;
     auto& wave_total = lds.wave_total;
@@ -469,8 +469,8 @@ __device__ __forceinline__ void onepass_workgroup(
         in_head += bases[w][1];
         ok = ok && bases[w][2] != 0ull;
     }
-    if (!ok && threadIdx.x == 0) mark_gave_up(gave_up, total_halfs, overflow);
-    if (landing && g != groups_total - 1 && threadIdx.x == 0) count_through(state + groups_total + 1, ok);
+    if (!ok && threadIdx.x == 0) mark_gave_up(gave_up, how.kept ? nullptr : total_halfs, overflow);
+    if (how.counted() && g != groups_total - 1 && threadIdx.x == 0) count_through(state + groups_total + 1, ok);
     const uint32_t base = (uint32_t)in_head + in_group;
     const uint32_t end = base + total;
 
@@ -483,7 +483,7 @@ __device__ __forceinline__ void onepass_workgroup(
     if (lane == 0) {
         if (tb == nblk - 1) io[kD] = end;
         if (tb == 0 && nz_off) nz_off[b] = (uint32_t)(H >> 2);
-        if (u == units - 1 && total_halfs && ok)
+        if (u == units - 1 && total_halfs && ok && !how.kept)
             atomicMax(reinterpret_cast<unsigned long long*>(total_halfs), 2ull * (H + end));
     }
     const uint64_t head_half0 = dst_off ? 8ull * dst_off[b] : 2ull * H;
@@ -504,8 +504,8 @@ __device__ __forceinline__ void onepass_workgroup(
             stream_image(img, bytesB, dst + bytesA, lane);
         }
     }
-    if (landing && g == groups_total - 1 && threadIdx.x == 0)
-        land_total(landing, 2ull * (H + in_head + group_total), ok, state + groups_total + 1, (uint32_t)groups_total - 1u, spin_limit);
+    if (how.counted() && g == groups_total - 1)
+        hand_over(how, total_halfs, 2ull * (H + in_head + group_total), ok, state, groups_total, spin_limit, wave_total);
     // The rotated rows last: in front of the search their stores stood between this unit's total and the units that wait
     // for it, and it waited for its own stores where it polls.  Keys of 128 heads x 4096 tokens, 70 %, rotated: 90.1 ->
     // 78.0 us (rocprofv3), with the compaction of the whole unit in front of the wait.  That one takes a values' launch
@@ -519,12 +519,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MSTF_COM
     const _Float16* __restrict__ x, ProjArgs proj, int M, int kth, uint64_t* __restrict__ bmp, uint32_t* __restrict__ idx,
     uint32_t* __restrict__ nz_off, uint64_t* __restrict__ total_halfs, const uint32_t* __restrict__ dst_off,
     const uint32_t* __restrict__ dst_limit, uint32_t* __restrict__ overflow, char* __restrict__ nz,
-    uint64_t nz_capacity_halfs, uint64_t* state, int units, int groups_total, uint32_t spin_limit, uint64_t* landing)
+    uint64_t nz_capacity_halfs, uint64_t* state, int units, int groups_total, uint32_t spin_limit, Handover how)
 {
     __shared__ OnepassLds<W> lds;
     onepass_workgroup<IS_VALUE, W, SRC>(lds, (int)blockIdx.x, x, proj, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
                                         dst_limit, overflow, nz, nz_capacity_halfs, state, units, groups_total, spin_limit,
-                                        landing);
+                                        how);
 }
 
 // Keys and values of the same tokens in one launch: workgroups 0 .. groups_total-1 compress the keys, the next
@@ -543,7 +543,7 @@ struct OnepassSide {
     char* nz;
     uint64_t nz_capacity_halfs;
     uint64_t* state;
-    uint64_t* landing;
+    Handover how;
 };
 template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void compress_onepass_kv_kernel(
@@ -554,11 +554,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
     if (g < groups_total)
         onepass_workgroup<false, W, kSrcMatrix>(lds, g, k.x, ProjArgs{}, M, k.kth, k.bmp, k.idx, k.nz_off, k.total_halfs,
                                                 k.dst_off, k.dst_limit, overflow, k.nz, k.nz_capacity_halfs, k.state, units,
-                                                groups_total, spin_limit, k.landing);
+                                                groups_total, spin_limit, k.how);
     else
         onepass_workgroup<true, W, kSrcMatrix>(lds, g - groups_total, v.x, ProjArgs{}, M, v.kth, v.bmp, v.idx, v.nz_off,
                                                v.total_halfs, v.dst_off, v.dst_limit, overflow, v.nz, v.nz_capacity_halfs,
-                                               v.state, units, groups_total, spin_limit, v.landing);
+                                               v.state, units, groups_total, spin_limit, v.how);
 }
 
 // ------------------------------------------------------------------------------- dense prune
@@ -610,7 +610,8 @@ static size_t compress_ws_bytes(int B, int M)
 template <bool IS_VALUE, int SRC = kSrcMatrix>
 static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& proj, int B, int M, int kth, uint64_t* bmp, uint32_t* idx,
                           uint32_t* nz_off, uint64_t* total_halfs, const uint32_t* dst_off, const uint32_t* dst_limit,
-                          uint32_t* overflow, mstf_half* nz, uint64_t cap, void* ws, uint64_t* landing = nullptr)
+                          uint32_t* overflow, mstf_half* nz, uint64_t cap, void* ws, uint64_t* landing = nullptr,
+                          uint64_t* status = nullptr)
 {
     const int nblk = M / 64, units = B * nblk;
 #ifndef MSTF_ONEPASS_W
@@ -618,17 +619,20 @@ static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& pr
 #endif
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
-    uint64_t* state = reinterpret_cast<uint64_t*>(ws);
+    uint64_t* state = status ? status : reinterpret_cast<uint64_t*>(ws);
+    const Handover how = {landing, status != nullptr};
     const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
     const uint32_t spin_limit = onepass_spin_limit();
-    hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),
-                       dim3(256), 0, st, state, words, total_halfs, static_cast<uint64_t*>(nullptr));
-    int rc = check_launch();
-    if (rc != MSTF_OK) return rc;
+    if (!status) {
+        hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),
+                           dim3(256), 0, st, state, words, total_halfs, static_cast<uint64_t*>(nullptr));
+        const int rc = check_launch();
+        if (rc != MSTF_OK) return rc;
+    }
 #define MSTF_OP(WV)                                                                                                   \
     hipLaunchKernelGGL((compress_onepass_kernel<IS_VALUE, WV, SRC>), dim3((unsigned)groups), dim3(64 * WV), 0, st, xh, proj, M, kth, \
                        bmp, idx, nz_off, total_halfs, dst_off, dst_limit, overflow, reinterpret_cast<char*>(nz), cap,  \
-                       state, units, groups, spin_limit, landing)
+                       state, units, groups, spin_limit, how)
     if (W == MSTF_ONEPASS_W)
         MSTF_OP(MSTF_ONEPASS_W);
     else if (W == 2)
@@ -640,19 +644,23 @@ static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& pr
 }
 
 // Keys and values of the same tokens behind one clearing launch (status words of the keys, then of the values).
-static int launch_onepass_kv(hipStream_t st, OnepassSide k, OnepassSide v, int B, int M, uint32_t* overflow, void* ws)
+static int launch_onepass_kv(hipStream_t st, OnepassSide k, OnepassSide v, int B, int M, uint32_t* overflow, void* ws,
+                             uint64_t* status = nullptr)
 {
     const int nblk = M / 64, units = B * nblk;
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
     const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
-    k.state = reinterpret_cast<uint64_t*>(ws);
+    k.state = status ? status : reinterpret_cast<uint64_t*>(ws);
     v.state = k.state + words;
+    k.how.kept = v.how.kept = status != nullptr;
     const uint32_t spin_limit = onepass_spin_limit();
-    hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((2 * words + 255) / 256 < 256 ? (2 * words + 255) / 256 : 256)),
-                       dim3(256), 0, st, k.state, 2 * words, k.total_halfs, v.total_halfs);
-    int rc = check_launch();
-    if (rc != MSTF_OK) return rc;
+    if (!status) {
+        hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((2 * words + 255) / 256 < 256 ? (2 * words + 255) / 256 : 256)),
+                           dim3(256), 0, st, k.state, 2 * words, k.total_halfs, v.total_halfs);
+        const int rc = check_launch();
+        if (rc != MSTF_OK) return rc;
+    }
 #define MSTF_OPKV(WV)                                                                                            \
     hipLaunchKernelGGL((compress_onepass_kv_kernel<WV>), dim3(2u * (unsigned)groups), dim3(64 * WV), 0, st, k, v, M, \
                        overflow, units, groups, spin_limit)
@@ -760,7 +768,7 @@ static int append_impl(void* stream, const mstf_half* x, int B, int M, int N, in
 static int proj_impl(void* stream, const mstf_proj_source* s, int is_value, int M, int N, int kth, uint64_t* bmp,
                      uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, const uint32_t* dst_off,
                      const uint32_t* dst_limit, mstf_half* nz, uint64_t cap, uint32_t* overflow, void* ws, size_t ws_bytes,
-                     uint64_t* landing = nullptr)
+                     uint64_t* landing = nullptr, uint64_t* status = nullptr)
 {
     if (!s || !s->x || s->batch <= 0 || s->heads <= 0 || s->rows <= 0 || M < 0 || M > s->rows || kth < 0 || kth > N)
         return MSTF_EINVAL;
@@ -804,13 +812,13 @@ static int proj_impl(void* stream, const mstf_proj_source* s, int is_value, int 
         int rc;
         if (rope)
             rc = launch_onepass<false, kSrcRope>(st, nullptr, pa, B, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                                 dst_limit, overflow, nz, capacity, ws, landing);
+                                                 dst_limit, overflow, nz, capacity, ws, landing, status);
         else if (is_value)
             rc = launch_onepass<true, kSrcView>(st, nullptr, pa, B, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                                dst_limit, overflow, nz, capacity, ws, landing);
+                                                dst_limit, overflow, nz, capacity, ws, landing, status);
         else
             rc = launch_onepass<false, kSrcView>(st, nullptr, pa, B, M, kth, bmp, idx, nz_off, total_halfs, dst_off,
-                                                 dst_limit, overflow, nz, capacity, ws, landing);
+                                                 dst_limit, overflow, nz, capacity, ws, landing, status);
         if (rc != MSTF_OK) return rc;
     }
     // the tokens behind the compressed ones are only rotated
@@ -841,6 +849,19 @@ extern "C" int mstf_append_value_f16(void* stream, const mstf_half* x, int B, in
 {
     return append_impl<true>(stream, x, B, M, N, kth, bmp, idx, dst_off, dst_limit, nz, overflow, workspace,
                              workspace_bytes);
+}
+
+extern "C" size_t mstf_status_bytes(int B, int M, int sides)
+{
+    if (B <= 0 || M <= 0 || M % 64 != 0 || sides < 1) return 0;
+    return ((size_t)B * (M / 64) + 2) * (size_t)sides * sizeof(uint64_t);
+}
+int mstf::status_check(const uint64_t* status, size_t bytes, int64_t B, int M, int sides)
+{
+    if (!status) return MSTF_OK;
+    if (!aligned_to(status, 8)) return MSTF_EALIGN;
+    if (B <= 0 || B > INT32_MAX) return MSTF_EINVAL;
+    return bytes < mstf_status_bytes((int)B, M, sides) ? MSTF_EWORKSPACE : MSTF_OK;
 }
 
 extern "C" size_t mstf_compress_workspace_bytes(int B, int M, int N)
@@ -902,13 +923,15 @@ extern "C" int mstf_compress_proj_f16(void* stream, const mstf_proj_source* src,
 extern "C" int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                                             uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs,
                                             mstf_half* nz, uint64_t nz_capacity_halfs, void* workspace,
-                                            size_t workspace_bytes, int64_t* landing, int64_t* value)
+                                            size_t workspace_bytes, uint64_t* status, size_t status_bytes, int64_t* landing,
+                                            int64_t* value)
 {
-    if (M <= 0) return MSTF_EINVAL;
-    int rc = landing_ready(as_stream(stream), landing, value);
+    if (M <= 0 || !src) return MSTF_EINVAL;
+    int rc = status_check(status, status_bytes, (int64_t)src->batch * src->heads, M, 1);
+    if (rc == MSTF_OK) rc = landing_ready(as_stream(stream), landing, value);
     if (rc != MSTF_OK) return rc;
     rc = proj_impl(stream, src, is_value, M, N, kth, bmp, idx, nz_off, total_halfs, nullptr, nullptr, nz, nz_capacity_halfs,
-                   nullptr, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing));
+                   nullptr, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing), status);
     return rc != MSTF_OK ? rc : landing_wait(as_stream(stream), landing, value);
 }
 
@@ -940,7 +963,7 @@ static int compress_kv_impl(void* stream, const mstf_half* k, const mstf_half* v
                             uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off, uint64_t* k_total_halfs, mstf_half* k_nz,
                             uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
                             uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
-                            size_t workspace_bytes, uint64_t* k_landing, uint64_t* v_landing)
+                            size_t workspace_bytes, uint64_t* k_landing, uint64_t* v_landing, uint64_t* status = nullptr)
 {
     int rc = kv_side_check(k, B, M, N, kth_k, k_bmp, k_idx, k_nz);
     if (rc == MSTF_OK) rc = kv_side_check(v, B, M, N, kth_v, v_bmp, v_idx, v_nz);
@@ -951,10 +974,10 @@ static int compress_kv_impl(void* stream, const mstf_half* k, const mstf_half* v
     if (!workspace || workspace_bytes < mstf_compress_kv_workspace_bytes(B, M, N)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 256)) return MSTF_EALIGN;
     OnepassSide ks = {reinterpret_cast<const _Float16*>(k), kth_k, k_bmp, k_idx, k_nz_off, k_total_halfs, nullptr, nullptr,
-                      reinterpret_cast<char*>(k_nz), k_capacity_halfs, nullptr, k_landing};
+                      reinterpret_cast<char*>(k_nz), k_capacity_halfs, nullptr, {k_landing, 0}};
     OnepassSide vs = {reinterpret_cast<const _Float16*>(v), kth_v, v_bmp, v_idx, v_nz_off, v_total_halfs, nullptr, nullptr,
-                      reinterpret_cast<char*>(v_nz), v_capacity_halfs, nullptr, v_landing};
-    return launch_onepass_kv(as_stream(stream), ks, vs, B, M, nullptr, workspace);
+                      reinterpret_cast<char*>(v_nz), v_capacity_halfs, nullptr, {v_landing, 0}};
+    return launch_onepass_kv(as_stream(stream), ks, vs, B, M, nullptr, workspace, status);
 }
 
 extern "C" int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k,
@@ -973,20 +996,23 @@ extern "C" int mstf_compress_kv_landing_f16(void* stream, const mstf_half* k, co
                                             uint64_t* k_total_halfs, mstf_half* k_nz, uint64_t k_capacity_halfs,
                                             uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off, uint64_t* v_total_halfs,
                                             mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
-                                            size_t workspace_bytes, int64_t* landings)
+                                            size_t workspace_bytes, uint64_t* status, size_t status_bytes, int64_t* landings)
 {
-    if (!landings || !aligned_to(landings, 8)) return MSTF_EINVAL;
-    // a recorded launch would store to the words at every replay, whoever has them by then
-    bool recorded = false;
-    int rc = stream_recorded(as_stream(stream), &recorded);
+    if (!aligned_to(landings, 8)) return MSTF_EALIGN;
+    int rc = status_check(status, status_bytes, B, M, 2);
     if (rc != MSTF_OK) return rc;
-    for (int i = 0; i < 2; i++) __atomic_store_n(landings + i, recorded ? MSTF_NOT_LANDED : kLandingEmpty, __ATOMIC_RELEASE);
+    // a recorded launch would store to the words at every replay, whoever has them by then
+    bool recorded = true;
+    if (landings) rc = stream_recorded(as_stream(stream), &recorded);
+    if (rc != MSTF_OK) return rc;
+    for (int i = 0; landings && i < 2; i++)
+        __atomic_store_n(landings + i, recorded ? MSTF_NOT_LANDED : kLandingEmpty, __ATOMIC_RELEASE);
     uint64_t* l = recorded ? nullptr : reinterpret_cast<uint64_t*>(landings);
     rc = compress_kv_impl(stream, k, v, B, M, N, kth_k, kth_v, k_bmp, k_idx, k_nz_off, k_total_halfs, k_nz, k_capacity_halfs,
                           v_bmp, v_idx, v_nz_off, v_total_halfs, v_nz, v_capacity_halfs, workspace, workspace_bytes, l,
-                          l ? l + 1 : nullptr);
+                          l ? l + 1 : nullptr, status);
     if (rc != MSTF_OK)
-        for (int i = 0; i < 2; i++) __atomic_store_n(landings + i, MSTF_NOT_LANDED, __ATOMIC_RELEASE);
+        for (int i = 0; landings && i < 2; i++) __atomic_store_n(landings + i, MSTF_NOT_LANDED, __ATOMIC_RELEASE);
     return rc;
 }
 
@@ -1006,8 +1032,8 @@ extern "C" int mstf_append_kv_f16(void* stream, const mstf_half* k, const mstf_h
     if (!workspace || workspace_bytes < mstf_compress_kv_workspace_bytes(B, M, N)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 256)) return MSTF_EALIGN;
     OnepassSide ks = {reinterpret_cast<const _Float16*>(k), kth_k, k_bmp, k_idx, nullptr, nullptr, k_dst_off, k_dst_limit,
-                      reinterpret_cast<char*>(k_nz), ~0ull, nullptr, nullptr};
+                      reinterpret_cast<char*>(k_nz), ~0ull, nullptr, {nullptr, 0}};
     OnepassSide vs = {reinterpret_cast<const _Float16*>(v), kth_v, v_bmp, v_idx, nullptr, nullptr, v_dst_off, v_dst_limit,
-                      reinterpret_cast<char*>(v_nz), ~0ull, nullptr, nullptr};
+                      reinterpret_cast<char*>(v_nz), ~0ull, nullptr, {nullptr, 0}};
     return launch_onepass_kv(as_stream(stream), ks, vs, B, M, overflow, workspace);
 }

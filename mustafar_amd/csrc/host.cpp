@@ -138,6 +138,7 @@ int unlocked(F&& f)
 bool enough(const at::Tensor* ws, size_t need, bool strict) { return ws && (strict || (size_t)ws->numel() >= need); }
 PyObject* wants(size_t bytes) { return PyLong_FromSize_t(bytes); }
 size_t room(const at::Tensor* ws) { return ws ? (size_t)ws->numel() : 0; }
+size_t bytes_of(const at::Tensor* t) { return t ? (size_t)t->nbytes() : 0; }
 // least scratch memory of an attention call (ops.attention_workspace_least)
 size_t attention_least(int64_t tokens, int64_t window, int64_t rows)
 {
@@ -496,14 +497,14 @@ struct Side {
     }
 };
 
-// (k, v, kth_k, kth_v, capacity or -1, landings or 0, ws, strict) -> (bmp, idx, nz_off, total, nz) x 2
+// (k, v, kth_k, kth_v, capacity or -1, landings or 0, status, ws, strict) -> (bmp, idx, nz_off, total, nz) x 2
 PyObject* compress_kv(Args& a)
 {
     const at::Tensor &k0 = a.tensor(), &v0 = a.tensor();
     const int kth_k = a.small(), kth_v = a.small();
     const int64_t capacity = a.integer();
     int64_t* landings = static_cast<int64_t*>(a.pointer());
-    const at::Tensor* ws = a.maybe();
+    const at::Tensor *status = a.maybe(), *ws = a.maybe();
     const bool strict = a.integer() != 0;
     a.done();
     require(k0.is_cuda() && v0.is_cuda() && is_half(k0) && is_half(v0) && k0.dim() == 3 && k0.sizes() == v0.sizes(),
@@ -522,14 +523,15 @@ PyObject* compress_kv(Args& a)
                                (uint64_t)cap, ptr<uint64_t>(vs.bmp), ptr<uint32_t>(vs.idx), ptr<uint32_t>(vs.nz_off),
                                ptr<uint64_t>(vs.total), ptr<mstf_half>(vs.nz), (uint64_t)cap, ptr<void>(ws), room(ws), more...);
                  };
-                 return landings ? call(mstf_compress_kv_landing_f16, landings) : call(mstf_compress_kv_f16);
+                 return call(mstf_compress_kv_landing_f16, ptr<uint64_t>(status), bytes_of(status), landings);
              }),
-             landings ? "mstf_compress_kv_landing_f16" : "mstf_compress_kv_f16");
+             "mstf_compress_kv_landing_f16");
     return tuple_of({ks.bmp, ks.idx, ks.nz_off, ks.total, ks.nz, vs.bmp, vs.idx, vs.nz_off, vs.total, vs.nz});
 }
 
-// (x, is_value, kth, M, cos, sin, rot, capacity or -1, landing, ws, strict) -> (bmp, idx, nz_off, total, nz, size or -1).
-// Capacity -1: room for the dense rows, and the call waits for the size (M > 0; landing: address of a pinned word).
+// (x, is_value, kth, M, cos, sin, rot, capacity or -1, landing, status, ws, strict) -> (bmp, idx, nz_off, total, nz, size or -1).
+// Capacity -1: room for the dense rows, and the call waits for the size (M > 0; landing: address of a pinned word), which is
+// negative if a workgroup gave up.
 PyObject* compress_proj(Args& a)
 {
     const at::Tensor& x = a.tensor();
@@ -537,7 +539,7 @@ PyObject* compress_proj(Args& a)
     const at::Tensor *cos = a.maybe(), *sin = a.maybe(), *rot = a.maybe();
     const int64_t capacity = a.integer();
     int64_t* landing = static_cast<int64_t*>(a.pointer());
-    const at::Tensor* ws = a.maybe();
+    const at::Tensor *status = a.maybe(), *ws = a.maybe();
     const bool strict = a.integer() != 0;
     a.done();
     require(x.is_cuda() && is_half(x) && x.dim() == 4 && x.stride(3) == 1, "x: fp16 [batch, rows, heads, D] on the GPU");
@@ -572,15 +574,14 @@ PyObject* compress_proj(Args& a)
                                ptr<uint32_t>(s.nz_off), ptr<uint64_t>(s.total), ptr<mstf_half>(s.nz), (uint64_t)cap, ptr<void>(ws),
                                room(ws), more...);
                  };
-                 return sized ? call(mstf_compress_proj_sized_f16, landing, &size) : call(mstf_compress_proj_f16);
+                 return sized ? call(mstf_compress_proj_sized_f16, ptr<uint64_t>(status), bytes_of(status), landing, &size) : call(mstf_compress_proj_f16);
              }),
              sized ? "mstf_compress_proj_sized_f16" : "mstf_compress_proj_f16");
-    if (sized)
-        check_rt(size >= 0, "the compressor gave up waiting for an earlier workgroup; the packed values are incomplete");
-    return tuple_of({s.bmp, s.idx, s.nz_off, s.total, sized ? s.nz.narrow(0, 0, size) : s.nz}, PyLong_FromLongLong(size));
+    return tuple_of({s.bmp, s.idx, s.nz_off, s.total, sized && size >= 0 ? s.nz.narrow(0, 0, size) : s.nz},
+                    PyLong_FromLongLong(size));
 }
 
-// (x, is_value, bit, kth, group_size, room or None, landing or 0, ws, strict) ->
+// (x, is_value, bit, kth, group_size, room or None, landing or 0, status, ws, strict) ->
 // (bmp, tile_off, room, counts, units, scales, zeros, total).  landing: address of a pinned word - the call waits for the word
 // count, and returns it in the place of the total.
 PyObject* produce_quant(Args& a)
@@ -589,7 +590,7 @@ PyObject* produce_quant(Args& a)
     const int is_value = a.small(), bit = a.small(), kth = a.small(), gs = a.small();
     const at::Tensor* given = a.maybe();
     int64_t* landing = static_cast<int64_t*>(a.pointer());
-    const at::Tensor* ws = a.maybe();
+    const at::Tensor *status = a.maybe(), *ws = a.maybe();
     const bool strict = a.integer() != 0;
     a.done();
     require(x0.is_cuda() && x0.dim() == 3, "inputs: [B, M, N] on the GPU");
@@ -619,7 +620,7 @@ PyObject* produce_quant(Args& a)
                                ptr<uint32_t>(counts), ptr<uint32_t>(units), ptr<mstf_half>(scales), ptr<mstf_half>(zeros),
                                ptr<uint64_t>(total), ptr<uint32_t>(words), (uint64_t)cap, ptr<void>(ws), room(ws), more...);
                  };
-                 return landing ? call(mstf_compress_quant_sized, landing, &size) : call(mstf_compress_quant_grouped);
+                 return landing ? call(mstf_compress_quant_sized, ptr<uint64_t>(status), bytes_of(status), landing, &size) : call(mstf_compress_quant_grouped);
              }),
              landing ? "mstf_compress_quant_sized" : "mstf_compress_quant_grouped");
     if (landing) return tuple_of({bmp, off, words, counts, units, scales, zeros}, PyLong_FromLongLong(size));

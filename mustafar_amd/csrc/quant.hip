@@ -274,7 +274,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
     const _Float16* __restrict__ x, int M, int kth, int bit, uint64_t* __restrict__ bmp, uint32_t* __restrict__ counts,
     uint32_t* __restrict__ units, uint32_t* __restrict__ tile_off, _Float16* __restrict__ scales,
     _Float16* __restrict__ zeros, uint32_t* __restrict__ packed, uint64_t capacity_words,
-    uint64_t* __restrict__ total_words, uint64_t* state, int nunits, int groups_total, uint32_t spin_limit, uint64_t* landing)
+    uint64_t* __restrict__ total_words, uint64_t* state, int nunits, int groups_total, uint32_t spin_limit, Handover how)
 {
     // staging buffer of a half-slab, then image of half a unit's kept values (at most 64 tiles x 128 bytes), behind it
     // the 64 words that quant_words looks tiles up in
@@ -411,15 +411,14 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
             // (the unit's place is the same for the whole wavefront, and so are the addresses made from it)
             before = u64_of(__builtin_amdgcn_readfirstlane((uint32_t)before),
                             __builtin_amdgcn_readfirstlane((uint32_t)(before >> 32)));
-            if (!ok && threadIdx.x == 0) mark_gave_up(state + groups_total, total_words, nullptr);
-            if (landing && threadIdx.x == 0) {
-                if (g != groups_total - 1)
+            if (!ok && threadIdx.x == 0) mark_gave_up(state + groups_total, how.kept ? nullptr : total_words, nullptr);
+            if (how.counted()) {
+                if (g == groups_total - 1)
+                    hand_over(how, total_words, before - in_group + group_total, ok, state, groups_total, spin_limit, wave_total);
+                else if (threadIdx.x == 0)
                     count_through(state + groups_total + 1, ok);
-                else
-                    land_total(landing, before - in_group + group_total, ok, state + groups_total + 1, (uint32_t)groups_total - 1u,
-                               spin_limit);
             }
-            if (lane == 0 && unit == nunits - 1 && ok)
+            if (lane == 0 && unit == nunits - 1 && ok && !how.kept)
                 atomicMax(reinterpret_cast<unsigned long long*>(total_words), before + tot[0] + tot[1]);
             tile_off[tile0 + lane] = (uint32_t)(before + e[0]);
             tile_off[tile0 + 64 + lane] = (uint32_t)(before + tot[0] + e[1]);
@@ -459,7 +458,7 @@ template <bool IS_VALUE, bool G32>
 static int compress_quant_impl(void* stream, const mstf_half* x, int B, int M, int N, int kth, int bit, uint64_t* bmp,
                                uint32_t* tile_off, uint32_t* counts, uint32_t* units, mstf_half* scales,
                                mstf_half* zeros, uint64_t* total_words, uint32_t* packed, uint64_t cap_words, void* ws,
-                               size_t ws_bytes, uint64_t* landing)
+                               size_t ws_bytes, uint64_t* landing, uint64_t* status)
 {
     if (!x || !bmp || !tile_off || !counts || !units || !scales || !zeros || !total_words) return MSTF_EINVAL;
     if (B <= 0 || M <= 0 || N <= 0 || kth < 0 || kth > N) return MSTF_EINVAL;
@@ -487,17 +486,20 @@ static int compress_quant_impl(void* stream, const mstf_half* x, int B, int M, i
         const int units_all = B * nblk;
         const int W = nblk % 4 == 0 ? 4 : (nblk % 2 == 0 ? 2 : 1);
         const int groups = units_all / W;
-        uint64_t* state = reinterpret_cast<uint64_t*>(ws);
+        uint64_t* state = status ? status : reinterpret_cast<uint64_t*>(ws);
+        const Handover how = {landing, status != nullptr};
         const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
         const uint32_t spin_limit = onepass_spin_limit();
-        hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),
-                           dim3(256), 0, st, state, words, total_words, static_cast<uint64_t*>(nullptr));
-        if ((rc = check_launch()) != MSTF_OK) return rc;
+        if (!status) {
+            hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),
+                               dim3(256), 0, st, state, words, total_words, static_cast<uint64_t*>(nullptr));
+            if ((rc = check_launch()) != MSTF_OK) return rc;
+        }
 #define MSTF_QOP(WV)                                                                                                  \
     hipLaunchKernelGGL((quant_onepass_kernel<IS_VALUE, G32, WV>), dim3((unsigned)groups), dim3(64 * WV), 0, st, xh, M, kth, \
                        bit, bmp, counts, units, tile_off, reinterpret_cast<_Float16*>(scales),                          \
                        reinterpret_cast<_Float16*>(zeros), packed, cap_words, total_words, state, units_all, groups,    \
-                       spin_limit, landing)
+                       spin_limit, how)
         if (W == 4)
             MSTF_QOP(4);
         else if (W == 2)
@@ -535,14 +537,14 @@ template <bool IS_VALUE>
 static int compress_quant_group(int group_size, void* stream, const mstf_half* x, int B, int M, int N, int kth, int bit,
                                 uint64_t* bmp, uint32_t* tile_off, uint32_t* counts, uint32_t* units, mstf_half* scales,
                                 mstf_half* zeros, uint64_t* total_words, uint32_t* packed, uint64_t cap_words, void* ws,
-                                size_t ws_bytes, uint64_t* landing = nullptr)
+                                size_t ws_bytes, uint64_t* landing = nullptr, uint64_t* status = nullptr)
 {
     if (group_size == 64)
         return compress_quant_impl<IS_VALUE, false>(stream, x, B, M, N, kth, bit, bmp, tile_off, counts, units, scales, zeros,
-                                                    total_words, packed, cap_words, ws, ws_bytes, landing);
+                                                    total_words, packed, cap_words, ws, ws_bytes, landing, status);
     if (group_size == 32)
         return compress_quant_impl<IS_VALUE, true>(stream, x, B, M, N, kth, bit, bmp, tile_off, counts, units, scales, zeros,
-                                                   total_words, packed, cap_words, ws, ws_bytes, landing);
+                                                   total_words, packed, cap_words, ws, ws_bytes, landing, status);
     return MSTF_EUNSUPPORTED;
 }
 
@@ -581,14 +583,15 @@ extern "C" int mstf_compress_quant_sized(void* stream, const mstf_half* x, int i
                                          int group_size, uint64_t* bmp, uint32_t* tile_off, uint32_t* counts, uint32_t* units,
                                          mstf_half* scales, mstf_half* zeros, uint64_t* total_words, uint32_t* packed,
                                          uint64_t packed_capacity_words, void* workspace, size_t workspace_bytes,
-                                         int64_t* landing, int64_t* value)
+                                         uint64_t* status, size_t status_bytes, int64_t* landing, int64_t* value)
 {
     if (!packed) return MSTF_EINVAL;
     hipStream_t st = as_stream(stream);
-    int rc = landing_ready(st, landing, value);
+    int rc = status_check(status, status_bytes, B, M, 1);
+    if (rc == MSTF_OK) rc = landing_ready(st, landing, value);
     if (rc != MSTF_OK) return rc;
     rc = (is_value ? compress_quant_group<true> : compress_quant_group<false>)(
         group_size, stream, x, B, M, N, kth, bit, bmp, tile_off, counts, units, scales, zeros, total_words, packed,
-        packed_capacity_words, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing));
+        packed_capacity_words, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing), status);
     return rc != MSTF_OK ? rc : landing_wait(st, landing, value);
 }

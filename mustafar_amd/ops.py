@@ -23,6 +23,7 @@ class Workspace:
     def __init__(self, device, nbytes=1 << 20):
         self.device = torch.device(device)
         self._bufs = [torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=self.device)]
+        self._status = []       # status words of the producers, zero between two calls; the last one is in use
 
     @property
     def tensor(self):
@@ -44,6 +45,20 @@ class Workspace:
                 and torch.cuda.is_current_stream_capturing()):
             return self.tensor
         return self.reserve(nbytes)
+
+
+    def status(self, words):
+        """`words` kept status words (mstf_status_bytes) for a producer, or None where they would have to be made while the
+        stream is being captured."""
+        if not self._status or self._status[-1].numel() < words:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            self._status.append(torch.zeros(max(words, 4096), dtype=torch.int64, device=self.device))
+        return self._status[-1]
+
+    def status_spoilt(self):
+        """A producer gave up: its status words are not zero any more."""
+        self._status.append(torch.zeros(4096, dtype=torch.int64, device=self.device))
 
 
 _WS = {}
@@ -78,11 +93,11 @@ def _landing_word():
 
 class _LandingPair:
     """The pinned words that a call which returns without waiting has its two totals stored to (mstf_landing_take)."""
-    __slots__ = ("pair", "stream", "_give")
+    __slots__ = ("pair", "stream", "ws", "_give")
     NOT_LANDED = -(1 << 63) + 2
 
-    def __init__(self, pair, stream):
-        self.pair, self.stream, self._give = pair, stream, lib().mstf_landing_give
+    def __init__(self, pair, stream, ws):
+        self.pair, self.stream, self.ws, self._give = pair, stream, ws, lib().mstf_landing_give
 
     def read(self, side):
         """The total, or None where the call was recorded into a graph."""
@@ -130,9 +145,28 @@ def _call(fn, ws, device, call, *args):
     return r
 
 
+def _own_workspace(ws, device):
+    """The Workspace that keeps a producer's status words, None where the caller brought a bare buffer."""
+    if ws is None and device.type == "cuda":
+        key = (device.type, device.index, _stream())
+        ws = _WS.get(key)
+        if ws is None:
+            ws = _WS[key] = Workspace(device)
+    return ws if isinstance(ws, Workspace) and ws.device.type == device.type else None
+
+
+def gave_up(ws, what):
+    if ws is not None:
+        ws.status_spoilt()
+    raise RuntimeError(what)
+
+
 def kth_from_sparsity(sparsity, head_dim):
     """Rank of the pruning threshold: max(1, int(target_sparsity * D)) as in dh_prune_key."""
     return max(1, int(sparsity * head_dim))
+
+
+_GAVE_UP = "the compressor gave up waiting for an earlier workgroup; the packed values are incomplete"
 
 
 class CompressedKV:
@@ -157,7 +191,7 @@ class CompressedKV:
         if n is None:
             n = read_word(self.total_halfs)
         if n < 0 or n > (1 << 62):
-            raise RuntimeError("the compressor gave up waiting for an earlier workgroup; the packed values are incomplete")
+            gave_up(self._landing.ws if self._landing is not None else None, _GAVE_UP)
         return n
 
     def packed(self):
@@ -222,9 +256,11 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     k, v: [B, M, N]; capacity_halfs (default: room for the dense rows) sizes both value buffers, the totals stay on
     the device.  Returns (CompressedKV of the keys, CompressedKV of the values)."""
     pair = lib().mstf_landing_take()
-    landing = _LandingPair(pair, _stream()) if pair else None
+    own = _own_workspace(ws, k.device) if pair else None
+    landing = _LandingPair(pair, _stream(), own) if pair else None
     kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
-                                                   -1 if capacity_halfs is None else int(capacity_halfs), pair or 0)
+                                                   -1 if capacity_halfs is None else int(capacity_halfs), pair or 0,
+                                                   own.status(2 * (k.shape[0] * (k.shape[1] // 64) + 2)) if own else None)
     M, N = k.shape[1:]
     return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
@@ -259,11 +295,15 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     if cos is not None and rot is None:
         rot = x
     sized = capacity_halfs is None and M != 0
+    own = _own_workspace(ws, x.device) if sized else None
     bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
                                            rot, -1 if capacity_halfs is None else int(capacity_halfs),
-                                           _landing_word()[1] if sized else 0)
+                                           _landing_word()[1] if sized else 0,
+                                           own.status(x.shape[0] * x.shape[2] * (M // 64) + 2) if own else None)
     if M == 0:
         return None, rot
+    if sized and n < 0:
+        gave_up(own, _GAVE_UP)
     return CompressedKV(bmp, idx, nz, nz_off, M, x.shape[3], is_value, n if sized else total), rot
 
 

@@ -72,6 +72,7 @@ def test_recorded_calls_do_not_land():
         for dst, src in zip((k, v), kv(4, 512, seed)):
             dst.copy_(src)
         graph.replay()
+        assert not any(bool(s.any()) for s in ws._status)
         same(c[0]), same(c[1])
         ref = ops.compress_kv(k, v, KTH, KTH)
         assert torch.equal(c[0].packed(), ref[0].packed()) and torch.equal(c[1].packed(), ref[1].packed())
@@ -104,3 +105,33 @@ def test_a_wait_that_ran_out_lands_as_such():
                 assert "gave up" in str(e)
     finally:
         lib().mstf_test_set_spin_limit(-1)
+    for c, want in zip(ops.compress_kv(k, v, KTH, KTH), want_kv):      # behind calls whose totals nobody read, too
+        try:
+            assert torch.equal(c.packed(), want)
+        except RuntimeError as e:
+            assert "gave up" in str(e)
+    for c, want in zip(ops.compress_kv(k, v, KTH, KTH), want_kv):      # (a total that was read has brought cleared words)
+        assert torch.equal(c.packed(), want)
+
+
+@pytest.mark.parametrize("heads,tokens", [(1, 64), (3, 192), (40, 1024), (130, 2048)])
+def test_status_words_are_left_as_they_were(heads, tokens):
+    """Calls of several sizes over the same kept words, one behind the other and without a wait between them; a launch that
+    clears words in the workspace gives the same arrays."""
+    from mustafar_amd import compression_quant as cq, ops
+    k, v = kv(heads, tokens, 3)
+    ws, bare = ops.Workspace("cuda"), torch.empty(1 << 22, dtype=torch.uint8, device="cuda")
+    got = [ops.compress_kv(k, v, KTH, 10 + i, ws=ws) for i in range(6)]
+    rows = k.view(1, heads, tokens, D).transpose(1, 2)
+    part = max(64, tokens // 128 * 64)
+    for i, pair in enumerate(got):
+        ref = ops.compress_kv(k, v, KTH, 10 + i, ws=bare)
+        for a, b in zip(pair, ref):
+            assert int(a.total_halfs) == int(b.total_halfs)
+            assert all(torch.equal(x, y) for x, y in ((a.bmp, b.bmp), (a.idx, b.idx), (a.nz_off, b.nz_off), (a.packed(), b.packed())))
+        c, _ = ops.compress_proj(rows, False, KTH, part, ws=ws)
+        r, _ = ops.compress_proj(rows, False, KTH, part, ws=bare)
+        assert torch.equal(c.idx, r.idx) and torch.equal(c.nz, r.nz)
+        x, y = (cq.convert_value_batched_quant(v, 2, ws=w, kth=KTH) for w in (ws, bare))
+        assert all(torch.equal(p, q) for p, q in zip(x, y))
+    assert len(ws._status) >= 1 and not any(bool(s.any()) for s in ws._status)
