@@ -26,6 +26,8 @@ namespace mstf {
 // stream, the boundaries and the first scalar batch of the coming block are requested while the current block is
 // still being decompressed, so only the first block of a wavefront waits for memory - and folds every block's
 // (max, sum, output) into running ones before the workgroup combine.
+// WHOLE: a workgroup of sixteen wavefronts takes a whole head, the blocks of both splits, and writes the output: no merge
+// follows.  PARTS = 2 with it: up to eight blocks, each shared by two wavefronts (pair_scores).
 // SHARE (few blocks): workgroups of four wavefronts that share a block - each takes one of its key stages and one of its
 // value stages (shared_scores, shared_store) - so that the chain of dependent stages is a quarter as long; every block has a
 // split slot of its own.
@@ -52,8 +54,20 @@ constexpr int fused_wave_lds()
     constexpr int park = NM * 4 * kFusedD * 4 + 64;  // per-wave (output, max, sum) parked for the workgroup combine
     return need > park ? need : park;
 }
-template <int NM, bool MULTI, bool STEP = false, bool SHARE = false>
-__global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__((amdgpu_waves_per_eu(resident_waves(kFusedWaves * fused_wave_lds<NM>(), kFusedWaves)))) void decode_attention_kernel(
+// LDS of the WHOLE form: value buffers and tables, the query rows once, a block's weights, the scores that pairs exchange.
+template <int NM, int PARTS>
+constexpr int whole_lds()
+{
+    return kWholeWaves * kNzLds + NM * 4 * kFusedD * 2 + kWholeWaves / PARTS * NM * (4 * 64 * 2 + (PARTS == 2 ? 3 * 1024 : 0));
+}
+template <int NM, bool SHARE, bool WHOLE, int PARTS>
+constexpr int decode_lds()
+{
+    return WHOLE ? whole_lds<NM, PARTS>() : (SHARE ? kShare : kFusedWaves) * fused_wave_lds<NM>();
+}
+constexpr int decode_waves(bool share, bool whole) { return whole ? kWholeWaves : (share ? kShare : kFusedWaves); }
+template <int NM, bool MULTI, bool STEP = false, bool SHARE = false, bool WHOLE = false, int PARTS = 1>
+__global__ __launch_bounds__(decode_waves(SHARE, WHOLE) * 64) __attribute__((amdgpu_waves_per_eu(WHOLE ? 4 : resident_waves(kFusedWaves * fused_wave_lds<NM>(), kFusedWaves)))) void decode_attention_kernel(
     const uint32_t* __restrict__ k_idx, const uint32_t* __restrict__ v_idx, const uint32_t* __restrict__ k_nz_off,
     const uint32_t* __restrict__ v_nz_off, size_t tstride, const int* __restrict__ tokens_dev, int nblk, int deal,
     const uint64_t* __restrict__ k_bmp, const char* __restrict__ k_nz, const uint64_t* __restrict__ v_bmp,
@@ -80,21 +94,26 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
     }
     constexpr int kQLds = NM * 4 * D * 2;          // query rows [4*NM][D] fp16
     constexpr int kPRow = 64 * 2;                  // one row of block weights: 64 tokens fp16
-    constexpr int kWaveLds = fused_wave_lds<NM>();
-    constexpr int K = SHARE ? 1 : kKeySubs;        // key stages and value stages of a wavefront
+    constexpr int kWaveLds = WHOLE ? kNzLds : fused_wave_lds<NM>();
+    constexpr bool PAIR = WHOLE && PARTS == 2;
+    static_assert(PARTS == 1 || (PAIR && !MULTI), "two wavefronts per block: whole heads of few blocks");
+    static_assert(!WHOLE || (!STEP && !SHARE && fused_park_bytes<NM>() + NM * 2048 <= kNzLds), "room behind the parked triples");
+    static_assert(decode_lds<NM, SHARE, WHOLE, PARTS>() <= kWholeLds, "LDS of a workgroup");
+    constexpr int K = SHARE ? 1 : kKeySubs / PARTS;  // key stages and value stages of a wavefront
     constexpr int kStages = 2 * K;
     static_assert(kKeySubs == kValSubs, "as many key stages as value stages");
     static_assert(kKeySubs == kShare, "a stage of each side per wavefront of a shared block");
     static_assert(!(MULTI && SHARE), "several blocks per wavefront or several wavefronts per block");
-    constexpr int kWaves = SHARE ? kShare : kFusedWaves;
-    __shared__ __attribute__((aligned(16))) char lds[kWaves][kWaveLds];
+    __shared__ __attribute__((aligned(16))) char lds[decode_lds<NM, SHARE, WHOLE, PARTS>()];
     const int lane = lane_id();
     const int wave = wave_id();
-    const int split = (int)blockIdx.x;
+    // (WHOLE: the first eight wavefronts do what the workgroup of the first split would, the others the second's)
+    const int split = WHOLE ? (PAIR ? 0 : wave / kFusedWaves) : (int)blockIdx.x;
     const int kv = (int)blockIdx.y;
-    const int sub = SHARE ? wave : 0;                                                  // its stages of the block
-    BlockRange mine = {SHARE ? split : split * kFusedWaves + wave, 0};  // the token blocks of this wavefront
-    if constexpr (MULTI) mine = fused_blocks_of(nblk, deal, split, wave);
+    const int sub = SHARE ? wave : (PAIR ? wave & 1 : 0);               // its stages of the block
+    const int slot = PAIR ? wave >> 1 : (WHOLE ? wave % kFusedWaves : wave);
+    BlockRange mine = {SHARE ? split : split * kFusedWaves + slot, 0};  // the token blocks of this wavefront
+    if constexpr (MULTI) mine = fused_blocks_of(nblk, deal, split, slot);
     const int tb = mine.first, nb = MULTI ? mine.count : nblk - tb;     // (wave-uniform)
     const bool active = nb > 0;
     // STEP: a wavefront that also has a block of the dense window to do keeps the highest issue priority through its
@@ -108,9 +127,11 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
     }
     const int j = lane & 3;
     const size_t T = tstride;
-    char* my = lds[wave];
-    char* ql = my + kNzLds;
-    char* pl = ql + kQLds;
+    char* my = lds + wave * kWaveLds;
+    char* ql = WHOLE ? lds + kWholeWaves * kNzLds : my + kNzLds;
+    // (PAIR: both wavefronts of a block make its weights and write the same bytes before they read them)
+    char* pl = ql + kQLds + (WHOLE ? wave / PARTS * NM * 4 * kPRow : 0);
+    char* scores = lds + kWholeWaves * kNzLds + kQLds + kWholeWaves / PARTS * NM * 4 * kPRow + wave / PARTS * NM * 3 * 1024;
     const uint32_t lbase = lds_addr(my);
 
     if constexpr (STEP && SHARE) {
@@ -196,10 +217,12 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
         } else {
             const char* qsrc = reinterpret_cast<const char*>(q + (size_t)kv * groups * D);
             const uint32_t qbytes = (uint32_t)groups * D * 2u;
+            if (!WHOLE || wave == 0) {  // (WHOLE: for all, the first wavefront always has a block)
 #pragma unroll
-            for (int i = 0; i < (kQLds + 1023) / 1024; i++) {
-                const uint32_t o = (uint32_t)(i * 64 + lane) * 16u;
-                if (o < qbytes) dma16(qsrc + o, ql + i * 1024);
+                for (int i = 0; i < (kQLds + 1023) / 1024; i++) {
+                    const uint32_t o = (uint32_t)(i * 64 + lane) * 16u;
+                    if (o < qbytes) dma16(qsrc + o, ql + i * 1024);
+                }
             }
         }
         nzK = k_nz + (size_t)(uint32_t)__builtin_amdgcn_readlane(bnd, 63) * 16u;
@@ -209,7 +232,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
         // a lane multiplies tiles 4 * (lane / 32) .. + 3 of every eight (rank_device.hpp)
         const uint32_t wside = (uint32_t)(lane >> 5) * 8u;
         const uint32_t qrow = lds_addr(ql) + (uint32_t)j * D * 2u + wside + (uint32_t)(sub * K * kSubTiles * 2);
-        const uint32_t prow = lds_addr(pl) + (uint32_t)j * kPRow + wside + (uint32_t)((sub & 1) * kSubTiles * 2);
+        const uint32_t prow = lds_addr(pl) + (uint32_t)j * kPRow + wside + (uint32_t)(SHARE ? (sub & 1) * kSubTiles * 2 : 0);
         const RankConst rank = rank_const(lane);
         const RankTable table = rank_table(my + 2 * kSubBytes, lane);
 
@@ -218,6 +241,10 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
         // the coming block.
         constexpr int kBatches = kSubTiles / 8, kSideBatches = K * kBatches;
         u32x16_t cur = load_bitmaps_scalar(bmK);
+        if constexpr (WHOLE) {
+            wait_vm0_keep(touch);  // (the first stage begins with this wait anyway)
+            lds_barrier();         // the query rows are there
+        }
         // nc, woffc: stage index and byte offset of the stage's first weight from wbase, as constants (they end up in
         // immediate operands)
         auto stage_batches = [&](auto nc, const RankAddr& at, uint32_t wbase, auto woffc, uint32_t wgroup,
@@ -246,7 +273,8 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
             const int adv = (MULTI && r + 1 < nb) ? D : 0;  // tiles to the coming block of this wavefront
             f4_t acc[NM][2];          // sums of a stage
             f4_t acc_k[NM];           // scores of the block (fold_stage); SHARE: of the wavefront's stage at first
-            f4_t blk_v[2][NM];        // output of the block, half by half; SHARE: [0], the wavefront's part of its half
+            f4_t blk_v[2][NM];        // output of the block, half by half; SHARE: [0], the wavefront's part of its half; PAIR: [0]
+            f4_t stage_k[2][NM];      // PAIR: sums of the wavefront's two key stages
             float m_blk[NM], l_blk[NM];
             auto clear = [&]() {
 #pragma unroll
@@ -260,7 +288,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
             static_for<kStages>([&](auto nc) {
                 constexpr int n = decltype(nc)::value;
                 // 3, 2, 1, 0 over the key stages and again over the value stages (SHARE: one of each)
-                if constexpr (SHARE) {}
+                if constexpr (SHARE || PAIR) {}
                 else if constexpr (STEP) set_wave_priority_uniform(prio_boost | (uint32_t)(3 - n % 4));
                 else set_wave_priority(3 - n % 4);
                 wait_vm0_keep(touch);  // sub-chunk n has landed (with the query rows for the first one)
@@ -277,11 +305,18 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
                 rank_settle(at);
                 if constexpr (n < K) {
                     stage_batches(nc, at, qrow, std::integral_constant<int, n * kSubTiles * 2>{}, (uint32_t)D * 8u, acc, adv);
-                    fold_stage(acc_k, acc);
+                    if constexpr (PAIR) {
+#pragma unroll
+                        for (int m = 0; m < NM; m++) stage_k[n % 2][m] = f4_t{0.f, 0.f, 0.f, 0.f};
+                        fold_stage(stage_k[n % 2], acc);
+                    } else {
+                        fold_stage(acc_k, acc);
+                    }
                 } else {
                     if constexpr (n == K) {
                         // (the wavefront's query rows have been read: their room takes its scores)
-                        if constexpr (SHARE) shared_scores<NM>(lds[0] + kNzLds, kWaveLds, sub, lane, acc_k, acc_k);
+                        if constexpr (SHARE) shared_scores<NM>(lds + kNzLds, kWaveLds, sub, lane, acc_k, acc_k);
+                        if constexpr (PAIR) pair_scores<NM>(scores, sub, lane, stage_k, acc_k);
                         block_softmax<NM>(acc_k, sqrt_d, 64, pl, lane, m_blk, l_blk);
                         // its latency is covered by the value phase; the wait of the next stage completes it
                         if (MULTI) bnd_next = boundaries(ixK + adv, ixV + adv);
@@ -296,7 +331,7 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
             });
             if constexpr (SHARE) {
                 // (the values of the key stage, in the first buffer, have long been read)
-                shared_store<NM>(lds[0], kWaveLds, sub, lane, blk_v[0], m_blk, l_blk, groups,
+                shared_store<NM>(lds, kWaveLds, sub, lane, blk_v[0], m_blk, l_blk, groups,
                                  (size_t)kv * groups * nsplit + tb, nsplit, part_o, part_ml);
             } else if (!MULTI) {
 #pragma unroll
@@ -321,6 +356,9 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
         }
         wait_vm0();
         wait_lgkm0();
+    } else if constexpr (WHOLE) {
+        lds_barrier();  // (the barriers that the wavefronts with a block have in front of the combine)
+        if constexpr (PAIR) lds_barrier();
     } else if constexpr (SHARE) {
         if (wave == 0 && tb < blocks_room)
             store_neutral<NM>(lane, groups, (size_t)kv * groups * nsplit + tb, nsplit, part_o, part_ml);
@@ -349,45 +387,30 @@ __global__ __launch_bounds__((SHARE ? kShare : kFusedWaves) * 64) __attribute__(
             step_window_wave<NM>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, step_window_count(sw), sqrt_d, lane);
         }
     }
-    workgroup_combine<NM>(&lds[0][0], kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, split, nsplit, write_final,
-                          out, part_o, part_ml);
+    if constexpr (PAIR) {
+        combine_pairs<NM>(lds, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, out);
+    } else if constexpr (WHOLE) {
+        combine_whole_head<NM>(lds, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, out);
+    } else {
+        workgroup_combine<NM>(lds, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, split, nsplit, write_final,
+                              out, part_o, part_ml);
+    }
 }
 
 // grid = Bq, 128 threads per group: log-sum-exp combine of the token splits.  The splits are taken in runs of eight: the
 // (max, sum) pairs and the partial outputs of a run are requested together, so a run costs one memory round trip.  Group g
 // of G takes runs g, g + G, .. and folds them into running (max, output, sum) values; the groups' values meet in LDS.
 // (One group alone walked its runs one after the other: sixteen round trips at 64 k tokens of a head.)
-constexpr int kMergeRun = 8, kMergeGroups = 8;
-struct MergeSum {
-    float M, so, sl;
-};
-__device__ __forceinline__ void merge_run(MergeSum& s, const float (&m)[kMergeRun], const float (&l)[kMergeRun],
-                                          const float (&o)[kMergeRun], int valid)
-{
-    float gm = s.M;
-#pragma unroll
-    for (int u = 0; u < kMergeRun; u++)
-        if (u < valid) gm = fmaxf(gm, m[u]);
-    const float fr = s.M == -INFINITY ? 0.f : __expf(s.M - gm);
-    s.so *= fr;
-    s.sl *= fr;
-#pragma unroll
-    for (int u = 0; u < kMergeRun; u++) {
-        const float f = (u < valid && m[u] != -INFINITY) ? __expf(m[u] - gm) : 0.f;
-        s.so += f * o[u];
-        s.sl += f * l[u];
-    }
-    s.M = gm;
-}
+constexpr int kMergeGroups = 8;
 // The groups' values - in LDS, a copy of (max, output, sum) per thread - into the output row.
 typedef float MergeLds[kMergeGroups][3][128];
-__device__ __forceinline__ void merge_put(MergeLds& sh, int g, int t, const MergeSum& s)
+__device__ __forceinline__ void merge_put(MergeLds& sh, int g, int t, const Triple& s)
 {
     sh[g][0][t] = s.M;
     sh[g][1][t] = s.so;
     sh[g][2][t] = s.sl;
 }
-__device__ __forceinline__ void merge_out(const MergeSum& s, int t, size_t row, int D, _Float16* out, float* lse_out)
+__device__ __forceinline__ void merge_out(const Triple& s, int t, size_t row, int D, _Float16* out, float* lse_out)
 {
     if (t < D) out[row * D + t] = (_Float16)(s.so / s.sl);
     if (lse_out && t == 0) {
@@ -395,15 +418,15 @@ __device__ __forceinline__ void merge_out(const MergeSum& s, int t, size_t row, 
         lse_out[row * 2 + 1] = s.sl;
     }
 }
-__device__ __forceinline__ MergeSum merge_groups(const MergeLds& sh, int groups, int t)
+__device__ __forceinline__ Triple merge_groups(const MergeLds& sh, int groups, int t)
 {
-    MergeSum s = {sh[0][0][t], 0.f, 0.f};
+    Triple s = {sh[0][0][t], 0.f, 0.f};
     for (int g = 1; g < groups; g++) s.M = fmaxf(s.M, sh[g][0][t]);
     for (int g = 0; g < groups; g++) {
         const float mg = sh[g][0][t];
         const float f = mg == -INFINITY ? 0.f : __expf(mg - s.M);
-        s.so += f * sh[g][1][t];
-        s.sl += f * sh[g][2][t];
+        s.so = __builtin_fmaf(f, sh[g][1][t], s.so);
+        s.sl = __builtin_fmaf(f, sh[g][2][t], s.sl);
     }
     return s;
 }
@@ -420,7 +443,7 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_kernel(const 
     const int c = t < D ? t : D - 1;
     const float2* ml = reinterpret_cast<const float2*>(part_ml) + row * nsplit;
     const float* po = part_o + row * nsplit * D + c;
-    MergeSum s = {-INFINITY, 0.f, 0.f};
+    Triple s = {-INFINITY, 0.f, 0.f};
     for (int s0 = group * G; s0 < nsplit; s0 += groups * G) {
         float m[G], l[G], o[G];
 #pragma unroll
@@ -486,8 +509,8 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
 #pragma unroll
             for (int w = 0; w < W; w++) {
                 const float f = m[w] == -INFINITY ? 0.f : __expf(m[w] - M);
-                so += f * o[w];
-                sl += f * l[w];
+                so = __builtin_fmaf(f, o[w], so);
+                sl = __builtin_fmaf(f, l[w], sl);
             }
         } else {
             const int i = blocks + u - whole;
@@ -501,7 +524,7 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
     }
     __syncthreads();
     const int runs = (units + G - 1) / G, groups = runs < kMergeGroups ? runs : kMergeGroups;
-    MergeSum s = {-INFINITY, 0.f, 0.f};
+    Triple s = {-INFINITY, 0.f, 0.f};
     if (group < groups) {
         for (int s0 = group * G; s0 < units; s0 += groups * G) {
             float m[G], l[G], o[G];
@@ -752,6 +775,7 @@ extern "C" size_t mstf_decode_attention_workspace_bytes(int tokens, int head_dim
 struct DecodePlan {
     bool shared;
     int deal, ns, wgs;
+    bool whole = false;  // a workgroup per head, the output is final (fused_whole_head)
     int merge_blocks() const { return shared ? ns : 0; }
 };
 // pooled: the token count is in device memory, at most `tokens` - as many splits as any count needs, and the kernel works
@@ -811,8 +835,9 @@ static int decode_launch(hipStream_t st, const DecodePlan& plan, const uint64_t*
         if (plan.shared) wgs += (window_blocks(sa.win_len) + kShare - 1) / kShare;
         else if (window_blocks(sa.win_len) > ns * kFusedWaves) return MSTF_EUNSUPPORTED;
     }
+    const unsigned threads = 64 * (plan.whole ? kWholeWaves : (plan.shared ? kShare : kFusedWaves));
+    if (plan.whole) wgs = 1;
     const dim3 grid((unsigned)wgs, (unsigned)Bkv);
-    const unsigned threads = 64 * (plan.shared ? kShare : kFusedWaves);
     const char* knz = reinterpret_cast<const char*>(k_nz);
     const char* vnz = reinterpret_cast<const char*>(v_nz);
     const _Float16* qh = reinterpret_cast<const _Float16*>(q);
@@ -829,7 +854,11 @@ static int decode_launch(hipStream_t st, const DecodePlan& plan, const uint64_t*
         else if (!tokens_dev && plan.deal == kFusedWaves) MSTF_FD(NMV, false);                                        \
         else MSTF_FD(NMV, true);                                                                                      \
     } while (0)
-    if (groups <= 4) MSTF_FD_NM(1); else MSTF_FD_NM(2);
+    if (plan.whole) {
+        if (nblk <= kFusedWaves) MSTF_FD(1, false, false, false, true, 2);
+        else if (nblk <= kWholeWaves) MSTF_FD(1, false, false, false, true);
+        else MSTF_FD(1, true, false, false, true);
+    } else if (groups <= 4) MSTF_FD_NM(1); else MSTF_FD_NM(2);
 #undef MSTF_FD_NM
 #undef MSTF_FD
     return check_launch();
@@ -921,13 +950,20 @@ extern "C" int mstf_decode_attention_f16(void* stream, const uint64_t* k_bmp, co
                           workspace, workspace_bytes);
     if (rc != MSTF_OK) return rc;
     if (!aligned_to(out, 2) || (lse_out && !aligned_to(lse_out, 4))) return MSTF_EALIGN;
-    // with one split and no (max, sum) requested the kernel writes the final output itself
-    // (up to 512 tokens one launch without a merge: sharing would make it two, 10.1 -> 7.8 us from a graph but 11.1 -> 14.4
-    // launched call by call)
-    const bool one_launch = fused_nsplit(tokens) == 1 && !lse_out;
-    const DecodePlan plan = decode_plan(tokens, Bq, groups, false, 0,
-                                        !one_launch && fused_share_fits(tokens, 0, Bq, workspace_bytes));
-    const int write_final = (!plan.shared && plan.ns == 1 && !lse_out) ? 1 : 0;
+    // with one split and no (max, sum) requested, or a workgroup per head, the kernel writes the final output itself
+    DecodePlan plan = decode_plan(tokens, Bq, groups, false, 0, false);
+    const int nblk = tokens / 64, Bkv = Bq / groups;
+    const bool one_split = nblk <= kFusedWaves && !lse_out;
+    bool share = !one_split;
+    if (one_split) {
+        bool recorded = false;
+        if ((rc = stream_recorded(as_stream(stream), &recorded)) != MSTF_OK) return rc;
+        share = fused_share_one_split(nblk, Bkv, groups, recorded);
+    }
+    share = share && fused_share_fits(tokens, 0, Bq, workspace_bytes);
+    plan.whole = !lse_out && !(one_split && share) && fused_whole_head(nblk, plan.ns, Bkv, groups, true);
+    if (!plan.whole && share) plan = decode_plan(tokens, Bq, groups, false, 0, true);
+    const int write_final = plan.whole || (!plan.shared && plan.ns == 1 && !lse_out) ? 1 : 0;
     rc = decode_launch(as_stream(stream), plan, k_bmp, k_nz, k_idx, k_nz_off, v_bmp, v_nz, v_idx, v_nz_off, q, out, tokens,
                        head_dim, Bq, groups, workspace, write_final);
     if (rc != MSTF_OK || write_final) return rc;

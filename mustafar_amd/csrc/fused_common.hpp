@@ -126,6 +126,27 @@ constexpr bool fused_shares_blocks(int tokens, int Bkv, int groups, int extra = 
     return tokens <= kShareMaxBlocks * 64 && (long long)Bkv * (tokens / 64) + extra <= fused_share_launch(groups);
 }
 
+// Calls over up to eight blocks a head have no split, and their workgroups write the output.  Sharing makes the call two
+// launches: recorded into a graph, where a launch behind another takes 2 us, it is the faster form all the same up to this many
+// blocks of all heads, from five blocks a head on or with more than four query heads (fp16, 70 %, pairs or a wavefront per
+// block / shared and merged: 8 heads x 8 blocks 8.4 / 6.6 us, 64 x 8 8.9 / 8.1, 128 x 8 9.0 / 10.2; eight query heads, 8 x 4
+// 9.6 / 7.1, 64 x 8 11.2 / 9.6); launched call by call it is not (8 x 8 8.4 / 9.5).
+constexpr int kShareOneSplit = 640;
+constexpr bool fused_share_one_split(int nblk, int Bkv, int groups, bool recorded)
+{
+    return recorded && Bkv * nblk <= kShareOneSplit && (nblk > 4 || groups > 4);
+}
+// Whether a workgroup of sixteen wavefronts takes a whole head, with up to four query heads, and writes its output, so that
+// no merge follows: heads of up to eight blocks, two wavefronts per block (a wavefront per block / this: 8 heads x 1 block 7.6 /
+// 5.5 us, 8 x 4 8.0 / 6.2, 256 x 4 8.7 / 7.1, 8 x 8 8.8 / 8.4, 256 x 8 9.7 / 9.5: eight blocks keep a CU busy), and heads of two
+// splits where these are as many as fill the chip (two splits and merge / this: 256 x 16 16.4 / 14.6, 256 x 64 48.8 / 47.3,
+// 224 x 64 44.9 / 43.4, 200 x 64 41.5 / 40.2, 2 bits 256 x 64 50.5 / 48.1; but 176 x 64 41.5 / 41.9, 64 x 16 9.9 / 11.8).
+constexpr bool fused_whole_head(int nblk, int ns, int Bkv, int groups, bool pairs)
+{
+    if (groups > 4 || Bkv > 256) return false;
+    return nblk <= kFusedWaves ? pairs : ns == 2 && Bkv >= 200;
+}
+
 constexpr int window_blocks(int win_len) { return (win_len + 63) / 64; }
 // Bytes of `slots` split slots: kFusedD outputs and (max, sum) each, fp32.
 constexpr size_t fused_slot_bytes(size_t slots) { return (slots * (kFusedD + 2) * sizeof(float) + 255) / 256 * 256; }
@@ -263,10 +284,59 @@ __device__ __forceinline__ void fold_block(f4_t (&acc)[2], float& m_run, float& 
 }
 
 // Workgroup combine of the kFusedWaves blocks of a split: every wavefront parks (output[4*NM][D], max, sum) in its
-// own LDS area (`lds_base + wave * wave_stride`, at least NM*4*D*4 + 64 bytes), then one thread per (head, channel)
+// own LDS area (`lds_base + wave * wave_stride`, at least fused_park_bytes), then one thread per (head, channel)
 // folds them and writes either the final fp16 output (write_final, one split only) or the split's partial:
 //   part_o[((kv*groups + h)*nsplit + split)*D + d] (un-normalised), part_ml[..][2] = (max, sum).
 // An inactive wavefront parks (-inf, 0, 0).
+template <int NM>
+constexpr int fused_park_bytes()
+{
+    return NM * 4 * kFusedD * 4 + 64;
+}
+// (BOTH: both halves of the channels, or only half `half`, which is in acc_v[m][0])
+template <int NM, bool BOTH = true>
+__device__ __forceinline__ void park(char* area, int lane, const f4_t (&acc_v)[NM][2], const float (&m_run)[NM],
+                                     const float (&l_run)[NM], int half = 0)
+{
+    constexpr int D = kFusedD;
+    const int j = lane & 3;
+    float* po = reinterpret_cast<float*>(area);
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        if constexpr (BOTH) {
+            *reinterpret_cast<f4_t*>(po + (m * 4 + j) * D + (lane & ~3)) = acc_v[m][0];
+            *reinterpret_cast<f4_t*>(po + (m * 4 + j) * D + 64 + (lane & ~3)) = acc_v[m][1];
+        } else {
+            *reinterpret_cast<f4_t*>(po + (m * 4 + j) * D + half * 64 + (lane & ~3)) = acc_v[m][0];
+        }
+        if (lane < 4) {
+            po[NM * 4 * D + (m * 4 + j) * 2] = m_run[m];
+            po[NM * 4 * D + (m * 4 + j) * 2 + 1] = l_run[m];
+        }
+    }
+}
+struct Triple {
+    float M, so, sl;
+};
+// (head h, channel c) of kFusedWaves parked triples, stride bytes apart.
+template <int NM>
+__device__ __forceinline__ Triple combined(const char* area0, int stride, int h, int c)
+{
+    constexpr int D = kFusedD;
+    Triple t = {-INFINITY, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kFusedWaves; w++)
+        t.M = fmaxf(t.M, reinterpret_cast<const float*>(area0 + w * stride)[NM * 4 * D + h * 2]);
+#pragma unroll
+    for (int w = 0; w < kFusedWaves; w++) {
+        const float* pw = reinterpret_cast<const float*>(area0 + w * stride);
+        const float mw = pw[NM * 4 * D + h * 2];
+        const float f = mw == -INFINITY ? 0.f : __expf(mw - t.M);
+        t.so = __builtin_fmaf(f, pw[h * D + c], t.so);
+        t.sl = __builtin_fmaf(f, pw[NM * 4 * D + h * 2 + 1], t.sl);
+    }
+    return t;
+}
 template <int NM>
 __device__ __forceinline__ void workgroup_combine(char* lds_base, int wave_stride, int wave, int lane,
                                                   const f4_t (&acc_v)[NM][2], const float (&m_run)[NM],
@@ -274,46 +344,90 @@ __device__ __forceinline__ void workgroup_combine(char* lds_base, int wave_strid
                                                   int write_final, _Float16* out, float* part_o, float* part_ml)
 {
     constexpr int D = kFusedD;
-    const int j = lane & 3;
-    {
-        // (the wavefront parks its triple in its own LDS region, which only it has used so far: no barrier in front)
-        float* po = reinterpret_cast<float*>(lds_base + wave * wave_stride);
-#pragma unroll
-        for (int m = 0; m < NM; m++) {
-            *reinterpret_cast<f4_t*>(po + (m * 4 + j) * D + (lane & ~3)) = acc_v[m][0];
-            *reinterpret_cast<f4_t*>(po + (m * 4 + j) * D + 64 + (lane & ~3)) = acc_v[m][1];
-            if (lane < 4) {
-                po[NM * 4 * D + (m * 4 + j) * 2] = m_run[m];
-                po[NM * 4 * D + (m * 4 + j) * 2 + 1] = l_run[m];
-            }
-        }
-    }
+    // (the wavefront parks its triple in its own LDS region, which only it has used so far: no barrier in front)
+    park<NM>(lds_base + wave * wave_stride, lane, acc_v, m_run, l_run);
     __syncthreads();
     for (int o = (int)threadIdx.x; o < groups * D; o += kFusedWaves * 64) {
         const int h = o / D, c = o - h * D;
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < kFusedWaves; w++)
-            M = fmaxf(M, reinterpret_cast<const float*>(lds_base + w * wave_stride)[NM * 4 * D + h * 2]);
-        float so = 0.f, sl = 0.f;
-#pragma unroll
-        for (int w = 0; w < kFusedWaves; w++) {
-            const float* pw = reinterpret_cast<const float*>(lds_base + w * wave_stride);
-            const float mw = pw[NM * 4 * D + h * 2];
-            const float f = mw == -INFINITY ? 0.f : __expf(mw - M);
-            so += f * pw[h * D + c];
-            sl += f * pw[NM * 4 * D + h * 2 + 1];
-        }
+        const Triple t = combined<NM>(lds_base, wave_stride, h, c);
         const size_t row = (size_t)kv * groups + h;
         if (write_final) {
-            out[row * D + c] = (_Float16)(so / sl);
+            out[row * D + c] = (_Float16)(t.so / t.sl);
         } else {
-            part_o[(row * nsplit + split) * D + c] = so;
+            part_o[(row * nsplit + split) * D + c] = t.so;
             if (c == 0) {
-                part_ml[(row * nsplit + split) * 2] = M;
-                part_ml[(row * nsplit + split) * 2 + 1] = sl;
+                part_ml[(row * nsplit + split) * 2] = t.M;
+                part_ml[(row * nsplit + split) * 2 + 1] = t.sl;
             }
         }
+    }
+}
+
+// A run of eight splits into a running (max, output, sum) (decode_merge_kernel).
+constexpr int kMergeRun = 8;
+__device__ __forceinline__ void merge_run(Triple& s, const float (&m)[kMergeRun], const float (&l)[kMergeRun],
+                                          const float (&o)[kMergeRun], int valid)
+{
+    float gm = s.M;
+#pragma unroll
+    for (int u = 0; u < kMergeRun; u++)
+        if (u < valid) gm = fmaxf(gm, m[u]);
+    const float fr = s.M == -INFINITY ? 0.f : __expf(s.M - gm);
+    s.so *= fr;
+    s.sl *= fr;
+#pragma unroll
+    for (int u = 0; u < kMergeRun; u++) {
+        const bool there = u < valid;  // (an infinite partial of a split that is repeated must not meet the zero)
+        const float f = (there && m[u] != -INFINITY) ? __expf(m[u] - gm) : 0.f;
+        s.so = __builtin_fmaf(f, there ? o[u] : 0.f, s.so);  // (written out: the same numbers in every kernel)
+        s.sl = __builtin_fmaf(f, there ? l[u] : 0.f, s.sl);
+    }
+    s.M = gm;
+}
+
+// ---- One workgroup of sixteen wavefronts takes a whole head, and no merge follows (fused_whole_head).
+constexpr int kWholeWaves = 16;
+constexpr int kWholeLds = 160 * 1024;  // what a workgroup may have
+// Behind the parked triples of its wavefronts: both splits combined as workgroup_combine does it, and merged as
+// decode_merge_kernel does it - the same numbers bit for bit - into the output.
+template <int NM>
+__device__ __forceinline__ void combine_whole_head(char* lds_base, int stride, int wave, int lane, const f4_t (&acc_v)[NM][2],
+                                                   const float (&m_run)[NM], const float (&l_run)[NM], int kv, int groups,
+                                                   _Float16* out)
+{
+    constexpr int D = kFusedD, kHalf = kFusedWaves * 64;
+    park<NM>(lds_base + wave * stride, lane, acc_v, m_run, l_run);
+    __syncthreads();
+    const int side = (int)threadIdx.x / kHalf, first = (int)threadIdx.x % kHalf;
+    // (the second split's triples, behind three of the parked ones: max, output, sum)
+    auto other = [=](int part, int o) {
+        return reinterpret_cast<float*>(lds_base + (kFusedWaves + part) * stride + fused_park_bytes<NM>()) + o;
+    };
+    Triple mine[NM];
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        const int o = first + m * kHalf, h = o / D, c = o % D;
+        if (o >= groups * D) break;
+        mine[m] = combined<NM>(lds_base + side * kFusedWaves * stride, stride, h, c);
+        if (side == 1) *other(0, o) = mine[m].M, *other(1, o) = mine[m].so, *other(2, o) = mine[m].sl;
+    }
+    __syncthreads();
+    if (side == 1) return;
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        const int o = first + m * kHalf;
+        if (o >= groups * D) break;
+        const Triple b = {*other(0, o), *other(1, o), *other(2, o)};
+        float M[kMergeRun], l[kMergeRun], v[kMergeRun];
+#pragma unroll
+        for (int u = 0; u < kMergeRun; u++) {  // (the merge kernel repeats the last split)
+            M[u] = u == 0 ? mine[m].M : b.M;
+            l[u] = u == 0 ? mine[m].sl : b.sl;
+            v[u] = u == 0 ? mine[m].so : b.so;
+        }
+        Triple s = {-INFINITY, 0.f, 0.f};
+        merge_run(s, M, l, v, 2);
+        out[(size_t)kv * groups * D + o] = (_Float16)(s.so / s.sl);
     }
 }
 
@@ -368,6 +482,41 @@ __device__ __forceinline__ void shared_store(char* room0, int stride, int sub, i
             }
         }
     }
+}
+// Pairs of wavefronts with a half of their block's channels each (pair_scores): as workgroup_combine, final output.
+template <int NM>
+__device__ __forceinline__ void combine_pairs(char* lds_base, int stride, int wave, int lane, const f4_t (&acc_v)[NM][2],
+                                              const float (&m_run)[NM], const float (&l_run)[NM], int kv, int groups, _Float16* out)
+{
+    constexpr int D = kFusedD;
+    park<NM, false>(lds_base + wave * stride, lane, acc_v, m_run, l_run, wave & 1);
+    __syncthreads();
+    for (int o = (int)threadIdx.x; o < groups * D; o += kWholeWaves * 64) {
+        const int h = o / D, c = o % D;
+        const Triple t = combined<NM>(lds_base + (c / 64) * stride, 2 * stride, h, c);
+        out[(size_t)kv * groups * D + o] = (_Float16)(t.so / t.sl);
+    }
+}
+
+// ---- Two wavefronts share a block inside a workgroup that takes a whole head of at most eight: two key stages and a half of
+// the channels each.  The scores out of the sums of the four stages (stage[]: the wavefront's two), by way of `room` (3 KB * NM
+// of the block's own).  The barrier is the whole workgroup's: idle wavefronts wait at it too.
+template <int NM>
+__device__ __forceinline__ void pair_scores(char* room, int sub, int lane, const f4_t (&stage)[2][NM], f4_t (&acc)[NM])
+{
+    auto at = [=](int piece, int m) { return reinterpret_cast<f4_t*>(room + (piece * NM + m) * 1024 + lane * 16); };
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        if (sub == 0) {
+            *at(0, m) = stage[0][m] + stage[1][m];
+        } else {
+            *at(1, m) = stage[0][m];
+            *at(2, m) = stage[1][m];
+        }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int m = 0; m < NM; m++) acc[m] = (*at(0, m) + *at(1, m)) + *at(2, m);
 }
 // The neutral triple in the slot of a block that holds no tokens (a launch sized for more than there are); by one wavefront.
 template <int NM>

@@ -62,8 +62,14 @@ struct QuantKernargs {
     StepArgs st;
 };
 constexpr size_t kQuantStepArgsAt = offsetof(QuantKernargs, st);
-template <int NM, int BIT, bool G32, bool MULTI, bool STEP = false>
-__global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_eu(quant_occupancy<NM, BIT, G32>()))) void decode_attention_quant_kernel(
+// WHOLE: a workgroup of sixteen wavefronts takes both splits of a head and writes the output (fused_whole_head).
+template <int NM, int BIT, bool G32>
+constexpr bool quant_whole_fits()
+{
+    return NM == 1 && kWholeWaves * quant_wave_lds<NM, BIT, G32>() <= kWholeLds;
+}
+template <int NM, int BIT, bool G32, bool MULTI, bool STEP = false, bool WHOLE = false>
+__global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribute__((amdgpu_waves_per_eu(WHOLE ? 4 : quant_occupancy<NM, BIT, G32>()))) void decode_attention_quant_kernel(
     const uint32_t* __restrict__ k_off, const uint32_t* __restrict__ v_off, const uint64_t* __restrict__ k_bmp,
     const uint64_t* __restrict__ v_bmp, size_t tstride, const int* __restrict__ tokens_dev, int nblk, int deal,
     const uint32_t* k_packed, const uint32_t* k_off_dma, const uint16_t* k_scales, const uint16_t* k_zeros,
@@ -91,13 +97,16 @@ __global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_e
     constexpr int kStage = q_lds_bytes<BIT, G32>();  // image, two word buffers, two metadata buffers
     constexpr int kWaveLds = quant_wave_lds<NM, BIT, G32>();
     // one array on purpose (LDS-direct loads into several LDS objects make the compiler serialise them)
-    __shared__ __attribute__((aligned(16))) char lds_all[kFusedWaves * kWaveLds];
+    __shared__ __attribute__((aligned(16))) char lds_all[(WHOLE ? kWholeWaves : kFusedWaves) * kWaveLds];
+    static_assert(!WHOLE || (!STEP && fused_park_bytes<NM>() + NM * 2048 <= kWaveLds), "room behind the parked triples");
     const int lane = lane_id();
     const int wave = wave_id();
-    const int split = tokens_dev ? (int)blockIdx.y : (int)blockIdx.x;
+    // (WHOLE: the first eight wavefronts do what the workgroup of the first split would, the others the second's)
+    const int split = WHOLE ? wave / kFusedWaves : (tokens_dev ? (int)blockIdx.y : (int)blockIdx.x);
     const int kv = tokens_dev ? (int)blockIdx.x : (int)blockIdx.y;
-    BlockRange mine = {split * kFusedWaves + wave, 0};                // the token blocks of this wavefront
-    if constexpr (MULTI) mine = fused_blocks_of(nblk, deal, split, wave);
+    const int slot = WHOLE ? wave % kFusedWaves : wave;
+    BlockRange mine = {split * kFusedWaves + slot, 0};                // the token blocks of this wavefront
+    if constexpr (MULTI) mine = fused_blocks_of(nblk, deal, split, slot);
     const int tb = mine.first, nb = MULTI ? mine.count : nblk - tb;   // (wave-uniform)
     const bool active = nb > 0;
     const size_t T = tstride;
@@ -279,8 +288,11 @@ __global__ __launch_bounds__(kFusedWaves * 64) __attribute__((amdgpu_waves_per_e
             step_window_wave<NM, kQRow, kPRow, 8>(my, ql, pl, sw, part_o, part_ml, kv, groups, nsplit, wblk, count, sqrt_d, lane);
         }
     }
-    workgroup_combine<NM>(lds_all, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, split, nsplit, write_final, out,
-                          part_o, part_ml);
+    if constexpr (WHOLE)
+        combine_whole_head<NM>(lds_all, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, out);
+    else
+        workgroup_combine<NM>(lds_all, kWaveLds, wave, lane, acc_v, m_run, l_run, kv, groups, split, nsplit, write_final, out,
+                              part_o, part_ml);
 }
 
 template <int NM, int BIT>
@@ -290,17 +302,30 @@ static void launch_decode_quant(hipStream_t st, dim3 grid, const uint64_t* k_bmp
                                 const uint16_t* v_scales, const uint16_t* v_zeros, const _Float16* q, _Float16* out,
                                 float* part_o, float* part_ml, int tokens, int groups, int ns, int write_final, float sq,
                                 int mode, int group_size, size_t tstride, const int32_t* tokens_dev, int deal,
-                                bool one_block, const StepArgs* step)
+                                bool one_block, const StepArgs* step, bool whole)
 {
     const StepArgs sa = step ? *step : StepArgs{};
+    const unsigned threads = 64 * (whole ? kWholeWaves : kFusedWaves);
 #define MSTF_FQ_LAUNCH(...)                                                                                              \
-    hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, __VA_ARGS__>), grid, dim3(kFusedWaves * 64), 0, st, k_off, \
+    hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, __VA_ARGS__>), grid, dim3(threads), 0, st, k_off, \
                        v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales, k_zeros,   \
                        v_packed, v_off, v_scales, v_zeros, q, out, part_o, part_ml, groups, ns, write_final, sq, mode, sa)
     // With one block per wavefront the form for one where it is the faster one: 280 to 1696 blocks, 70 - 75 %, fused attention in
     // the form for several / for one: 4 bits 16.4 / 15.4 us (two groups per tile 18.4 / 17.7), 8 bits 17.8 / 17.5 (20.1 / 20.6),
     // 2 bits 14.4 / 14.6 (17.4 / 16.5; 4096 blocks, one group: 17.9 / 18.3).
     constexpr bool kMulti = quant_multi<NM>(), kOne = kMulti && BIT == 2, kOneG32 = kMulti && BIT == 8;
+    if constexpr (quant_whole_fits<NM, BIT, false>()) {
+        if (whole && group_size == 64) {
+            if (one_block) MSTF_FQ_LAUNCH(false, kOne, false, true); else MSTF_FQ_LAUNCH(false, kMulti, false, true);
+            return;
+        }
+    }
+    if constexpr (quant_whole_fits<NM, BIT, true>()) {
+        if (whole) {
+            if (one_block) MSTF_FQ_LAUNCH(true, kOneG32, false, true); else MSTF_FQ_LAUNCH(true, kMulti, false, true);
+            return;
+        }
+    }
     if (step) {  // (group_size is 64 there: quant_launch has checked it)
         if (one_block) MSTF_FQ_LAUNCH(false, kOne, true); else MSTF_FQ_LAUNCH(false, kMulti, true);
     } else if (group_size == 32) {
@@ -347,6 +372,14 @@ static int quant_resident(int groups, int bit, int group_size)
                    : bit == 4 ? (g32 ? quant_occupancy<1, 4, true>() : quant_occupancy<1, 4, false>())
                               : (g32 ? quant_occupancy<1, 8, true>() : quant_occupancy<1, 8, false>()));
 }
+// Whether sixteen wavefronts of the kernel fit a workgroup (up to four query heads).
+static bool quant_whole(int bit, int group_size)
+{
+    const bool g32 = group_size == 32;
+    return bit == 2   ? (g32 ? quant_whole_fits<1, 2, true>() : quant_whole_fits<1, 2, false>())
+           : bit == 4 ? (g32 ? quant_whole_fits<1, 4, true>() : quant_whole_fits<1, 4, false>())
+                      : (g32 ? quant_whole_fits<1, 8, true>() : quant_whole_fits<1, 8, false>());
+}
 // Split slots its launch fills for `tokens` tokens, or for any count up to that many (at most fused_nsplit(tokens), which
 // is what workspaces are sized for).  window: blocks of the dense window.
 static int quant_nsplit(int tokens, int Bkv, int groups, int bit, int group_size, int window = 0)
@@ -362,7 +395,7 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
                         const mstf_half* v_zeros, const mstf_half* q, mstf_half* out, int tokens, int head_dim, int Bq,
                         int groups, int bit, int dequant_mode, void* workspace, int ns, int nst, int write_final,
                         int group_size = 64, size_t tile_stride = 0, const int32_t* tokens_dev = nullptr,
-                        const StepArgs* step = nullptr)
+                        const StepArgs* step = nullptr, bool whole = false)
 {
     const int Bkv = Bq / groups;
     // (token count in device memory: the kernel deals the blocks out itself, from the number of workgroups that fill the chip)
@@ -375,7 +408,7 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
     // tile_stride / tokens_dev: a cache pre-allocated for `tokens` tokens that holds *tokens_dev of them (see the kernel)
     float* part_o = reinterpret_cast<float*>(workspace);
     float* part_ml = part_o + (size_t)Bq * nst * head_dim;
-    const dim3 grid = tokens_dev ? dim3((unsigned)Bkv, (unsigned)ns) : dim3((unsigned)ns, (unsigned)Bkv);
+    const dim3 grid = tokens_dev ? dim3((unsigned)Bkv, (unsigned)ns) : dim3(whole ? 1u : (unsigned)ns, (unsigned)Bkv);
     const size_t tstride = tile_stride ? tile_stride : (size_t)tokens * head_dim / 64;
     const _Float16* qh = reinterpret_cast<const _Float16*>(q);
     _Float16* oh = reinterpret_cast<_Float16*>(out);
@@ -387,7 +420,7 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
 #define MSTF_FQ(NMV, BITV)                                                                                             \
     launch_decode_quant<NMV, BITV>(st, grid, k_bmp, k_packed, k_tile_off, ks, kz, v_bmp, v_packed, v_tile_off, vs, vz, \
                                    qh, oh, part_o, part_ml, tokens, groups, nst, write_final, sq, dequant_mode, group_size, \
-                                   tstride, tokens_dev, deal, one_block, step)
+                                   tstride, tokens_dev, deal, one_block, step, whole)
     if (groups <= 4) {
         if (bit == 2) MSTF_FQ(1, 2); else if (bit == 4) MSTF_FQ(1, 4); else MSTF_FQ(1, 8);
     } else {
@@ -416,9 +449,12 @@ static int decode_attention_quant_impl(void* stream, const uint64_t* k_bmp, cons
     hipStream_t st = as_stream(stream);
     const int ns = quant_nsplit(tokens, Bq / groups, groups, bit, group_size);
     // with one split and no (max, sum) requested the kernel writes the final output itself
-    const int write_final = (ns == 1 && !lse_out) ? 1 : 0;
+    // (and with a workgroup per head)
+    const bool whole = !lse_out && quant_whole(bit, group_size) && fused_whole_head(tokens / 64, ns, Bq / groups, groups, false);
+    const int write_final = whole || (ns == 1 && !lse_out) ? 1 : 0;
     rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
-                      out, tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, ns, write_final, group_size);
+                      out, tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, ns, write_final, group_size, 0, nullptr,
+                      nullptr, whole);
     if (rc != MSTF_OK || write_final) return rc;
     return merge_splits(st, workspace, out, lse_out, ns, head_dim, Bq);
 }
