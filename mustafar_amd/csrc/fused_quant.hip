@@ -12,7 +12,6 @@
 #define MSTF_QPAD 16
 #endif
 #include "quant_device.hpp"
-#include "rank_device.hpp"
 
 namespace mstf {
 
@@ -177,6 +176,8 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
             return *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(bm + t) + touch8);
         };
 
+        const StageRank<4 * NM> rank(lbase, lane);
+
         // the query rows of this KV head: groups x D fp16, contiguous (STEP: rotated out of the projection output)
         if constexpr (STEP) {
             stage_query_rotated<kQRow>(ql, st, kv, groups, lane);
@@ -194,11 +195,9 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
         }
         uint2 touch = issue(0);
 
-        RowSums<4 * NM> sums;  // of the phase (keys, one half of the values, the other half)
+        typename StageRank<4 * NM>::Sums sums;  // of the phase (keys, one half of the values, the other half)
         const uint32_t qrow = sums.waddr(lds_addr(ql), kQRow, lane);
         const uint32_t prow = sums.waddr(lds_addr(pl), kPRow, lane);
-        const RankConst rank = rank_const(lane);
-        const uint32_t img = image_lane(lbase, lane);
 
 #pragma unroll 1
         for (int r = 0; r < (MULTI ? nb : 1); r++) {
@@ -232,7 +231,7 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                 if (n == kKeySubs) {
                     f4_t acc_k[NM];
 #pragma unroll
-                    for (int m = 0; m < NM; m++) acc_k[m] = join_halves(sums.narrow[m]);
+                    for (int m = 0; m < NM; m++) acc_k[m] = sums.joined(m);
                     sums.clear();
                     block_softmax<NM, kPRow>(acc_k, sqrt_d, 64, pl, lane, m_blk, l_blk);
                     const int adv = more ? D : 0;
@@ -244,10 +243,10 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                                         wordbuf_lds + (uint32_t)(n & 1) * F::kWordBuf, lbase, start, bits, lane, mode);
                 const uint32_t w = n < kKeySubs ? qrow + (uint32_t)n * kSubTiles * 2u
                                                 : prow + (uint32_t)(vs % kSubsPerHalf) * kSubTiles * 2u;
-                stage_img_rank(rank, bm, bits, img, w, n < kKeySubs ? 4u * kQRow : 4u * kPRow, sums);
+                rank.expand(bm, bits, w, n < kKeySubs ? 4u * kQRow : 4u * kPRow, sums);
                 if (n >= kKeySubs && vs % kSubsPerHalf == kSubsPerHalf - 1) {  // the half is complete
 #pragma unroll
-                    for (int m = 0; m < NM; m++) blk_v[m][vs / kSubsPerHalf] = join_halves(sums.narrow[m]);
+                    for (int m = 0; m < NM; m++) blk_v[m][vs / kSubsPerHalf] = sums.joined(m);
                     sums.clear();
                 }
                 wait_lgkm0();  // every read of the image and of the staged buffers is done before they are rewritten

@@ -1,7 +1,7 @@
 // Device-side building blocks of the quantised consumers (quant_spmv.hip, fused_quant.hip): staging sizes,
 // dequantisation of a staged run of tiles into an fp16 tile image in LDS, expansion of that image.
 #pragma once
-#include "rank_device.hpp"
+#include "rank_whole.hpp"
 #include "spmv_device.hpp"
 
 #ifndef MSTF_IMG_STRIDE
@@ -321,12 +321,11 @@ __device__ __forceinline__ MetaLanes meta_lanes(const uint32_t* off_dma, const u
     return m;
 }
 
-// The C operand of the address products: where the image of the lane half's first tile starts (img), in all sixteen
+// The C operand of the address products: where the image starts (of the lane half's first tile; img), in all sixteen
 // registers; the tiles behind it are immediate offsets of the gather.  Made anew for every stage by eight 64-bit moves:
 // kept, the sixteen registers would not fit beside the dequantisation's.
 __device__ __forceinline__ i32x16_t image_base(uint32_t img)
 {
-    typedef uint64_t u64x8_t __attribute__((ext_vector_type(8)));
     u64x8_t b;
     uint64_t pair = ((uint64_t)img << 32) | img;
     asm volatile("" : "+v"(pair));
@@ -334,25 +333,53 @@ __device__ __forceinline__ i32x16_t image_base(uint32_t img)
     for (int i = 0; i < 8; i++) b[i] = pair;
     return __builtin_bit_cast(i32x16_t, b);
 }
-__device__ __forceinline__ uint32_t image_lane(uint32_t img, int lane) { return img + (uint32_t)(lane >> 5) * 4u * kImgStride; }
 
-// The 32 tiles of one dequantised stage through the rank products (rank_device.hpp).  img: image_lane(); bits: bitmap of tile lane & 31; w, wgroup: see RowSums.
+// How the 32 tiles of a dequantised stage are expanded: a whole tile per LDS read for up to eight weight rows
+// (rank_whole.hpp), half of two tiles for more (rank_device.hpp).  bits: bitmap of tile lane & 31; w, wgroup: see RowSums.
 // The bitmaps of the first batch are requested behind the products and arrive while those run (nothing scalar is
 // carried across the lane-dependent branches of the dequantisation in front), the others one batch ahead.
+template <int NW, bool WIDE = wide_rows(NW)>
+struct StageRank;
 template <int NW>
-__device__ __forceinline__ void stage_img_rank(const RankConst& rank, const uint64_t* bm, uint2 bits, uint32_t img,
-                                               uint32_t w, uint32_t wgroup, RowSums<NW>& sums)
-{
-    constexpr int G = kSubTiles / 8;
-    RankAddr at = rank_addresses(rank, bits, image_base(img));
-    u32x16_t cur;
-    rank_settle_load(at, cur, bm);
-    static_for<G>([&](auto gc) {
-        constexpr int g = decltype(gc)::value;
-        u32x16_t nxt;
-        sums.template batch<(g + 1 < G), g, (g + 1) * 64, g * 8 * kImgStride, kImgStride>(cur, nxt, bm, at, w, wgroup);
-        cur = nxt;
-    });
-}
+struct StageRank<NW, true> {
+    using Sums = RowSums<NW>;
+    RankConst rank;
+    uint32_t img;
+    __device__ __forceinline__ StageRank(uint32_t image, int lane)
+        : rank(rank_const(lane)), img(image + (uint32_t)(lane >> 5) * 4u * kImgStride) {}
+    __device__ __forceinline__ void expand(const uint64_t* bm, uint2 bits, uint32_t w, uint32_t wgroup, Sums& sums) const
+    {
+        constexpr int G = kSubTiles / 8;
+        RankAddr at = rank_addresses(rank, bits, image_base(img));
+        u32x16_t cur;
+        rank_settle_load(at, cur, bm);
+        static_for<G>([&](auto gc) {
+            constexpr int g = decltype(gc)::value;
+            u32x16_t nxt;
+            sums.template batch<(g + 1 < G), g, (g + 1) * 64, g * 8 * kImgStride, kImgStride>(cur, nxt, bm, at, w, wgroup);
+            cur = nxt;
+        });
+    }
+};
+template <int NW>
+struct StageRank<NW, false> {
+    using Sums = WholeSums<NW>;
+    WholeRank rank;
+    uint32_t img;
+    __device__ __forceinline__ StageRank(uint32_t image, int lane) : rank(whole_rank(lane)), img(image) {}
+    __device__ __forceinline__ void expand(const uint64_t* bm, uint2 bits, uint32_t w, uint32_t wgroup, Sums& sums) const
+    {
+        constexpr int G = kSubTiles / 8;
+        RankAddr at = whole_addresses(rank, bits, image_base(img));
+        u64x8_t cur;
+        whole_settle_load(at, cur, bm);
+        static_for<G>([&](auto gc) {
+            constexpr int g = decltype(gc)::value;
+            u64x8_t nxt;
+            whole_batch<Sums::NM, (g + 1 < G), g, (g + 1) * 64, kImgStride>(cur, nxt, bm, at, w, w + wgroup, sums.acc);
+            cur = nxt;
+        });
+    }
+};
 
 }  // namespace mstf

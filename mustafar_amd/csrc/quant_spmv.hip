@@ -7,7 +7,7 @@
 //   2. dequantisation happens in the packed domain: one lane per packed word unpacks its 16 / 8 / 4 codes
 //      and writes the fp16 values, in rank order, into a fixed-stride tile image in LDS, so the cost is per
 //      non-zero word, not per dense position;
-//   3. the image is expanded exactly like the fp16 format (bitmap rank -> LDS gather -> MFMA, rank_device.hpp),
+//   3. the image is expanded like the fp16 format (bitmap rank -> LDS gather -> MFMA; rank_whole.hpp, rank_device.hpp),
 //      with the tile base a constant instead of idx.
 // Dequantised value = fp16( (q - zero) * scale ).  For |zero| <= 1024 this is computed with packed fp16
 // arithmetic and is the same number the reference's fp32 (dequant_mode 0) and fp16 (dequant_mode 1)
@@ -37,15 +37,14 @@ struct QCache {
 // (KV head included): tile_off / scales / zeros / bmp are flat over [Bkv, T].
 template <bool SHARED, int BIT, bool G32, int NW, class TileOf, class StageW, class WAddrOf>
 __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW stage_w, WAddrOf waddr_of, uint32_t wgroup,
-                                            const QCache& c, char* my, int lane, int mode, RowSums<NW>& sums)
+                                            const QCache& c, char* my, int lane, int mode, typename StageRank<NW>::Sums& sums)
 {
     using F = QFmt<BIT>;
     if (nsubs <= 0) return;
     const uint32_t lbase = lds_addr(my);
     char* wordbuf = my + kImgBytes;
     char* metabuf = wordbuf + 2 * F::kWordBuf;
-    const RankConst rank = rank_const(lane);
-    const uint32_t img = image_lane(lbase, lane);
+    const StageRank<NW> rank(lbase, lane);
 
     // words of the stage starting at tile t: [tile_off[t], tile_off[t + 31] + words of tile t + 31)
     auto bounds = [&](size_t t, uint32_t& s, uint32_t& e) {
@@ -117,7 +116,7 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
         }
         dequant_stage<BIT, G32>(lds_addr(metabuf) + (uint32_t)(n & 1) * kMetaBytes,
                            lds_addr(wordbuf) + (uint32_t)(n & 1) * F::kWordBuf, lbase, s_now, bits, lane, mode);
-        stage_img_rank(rank, c.bmp + t_now, bits, img, waddr_of(n), wgroup, sums);
+        rank.expand(c.bmp + t_now, bits, waddr_of(n), wgroup, sums);
         wait_lgkm0();  // every read of the image and of the staged buffers is done before they are rewritten
     }
 }
@@ -128,8 +127,8 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
 template <int NW, int BIT, bool G32>
 constexpr int key_quant_lds()
 {
-    constexpr int rows = RowSums<NW>::kRows * 128 * 2;
-    return 4 * q_lds_bytes<BIT, G32>() + (RowSums<NW>::kWide ? rows : 4 * rows);
+    constexpr int rows = StageRank<NW>::Sums::kRows * 128 * 2;
+    return 4 * q_lds_bytes<BIT, G32>() + (StageRank<NW>::Sums::kWide ? rows : 4 * rows);
 }
 template <int NW, int BIT, bool G32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_waves(key_quant_lds<NW, BIT, G32>(), 4)))) void key_spmv_quant_kernel(
@@ -137,7 +136,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
     const uint32_t* tile_off_dma, const uint16_t* scales, const uint16_t* zeros, const _Float16* Bm,
     _Float16* __restrict__ C, int Lc, int D, int nblk, int ntasks, int rows_per_kv, int row0, int mode)
 {
-    using Sums = RowSums<NW>;
+    using Sums = typename StageRank<NW>::Sums;
     constexpr bool kShared = Sums::kWide;
     constexpr int kMaxD = 128;
     constexpr int kQ = q_lds_bytes<BIT, G32>();
@@ -176,7 +175,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
         __syncthreads();
         return;
     }
-    walk_subs_q<kShared, BIT, G32>(
+    walk_subs_q<kShared, BIT, G32, NW>(
         D / kSubTiles, [=](int n) { return tile0 + (size_t)n * kSubTiles; }, stage_rows,
         [=](int n) { return Sums::advance(wrow, (uint32_t)n * kSubTiles * 2u); }, (uint32_t)D * 8u, c, my, lane, mode, sums);
     _Float16* out = C + ((size_t)kv * rows_per_kv + row0) * Lc + (size_t)tb * 64;
@@ -196,7 +195,7 @@ template <int NW, int BIT, bool G32>
 constexpr int value_quant_wave_lds()
 {
     // the rows start at a multiple of their length (64 bytes); the per-wave sums are parked in the room at the end
-    constexpr int need = ((q_lds_bytes<BIT, G32>() + 63) & ~63) + 2 * RowSums<NW>::kRows * kSubTiles * 2;
+    constexpr int need = ((q_lds_bytes<BIT, G32>() + 63) & ~63) + 2 * StageRank<NW>::Sums::kRows * kSubTiles * 2;
     return need > NW * 256 ? need : NW * 256;
 }
 template <int NW, int WAVES, int BIT, bool G32>
@@ -206,7 +205,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     _Float16* __restrict__ C, float* __restrict__ part, int Lc, int D, int nblk, int nbpw, int nsplit, int rows_per_kv,
     int row0, int mode, int nwg, uint32_t per_split)
 {
-    using Sums = RowSums<NW>;
+    using Sums = typename StageRank<NW>::Sums;
     constexpr int kWRow = kSubTiles * 2;
     constexpr int kWBuf = Sums::kRows * kWRow;
     constexpr int kQ = (q_lds_bytes<BIT, G32>() + 63) & ~63;
@@ -234,7 +233,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     constexpr int subs_per_blk = 64 / kSubTiles;
     const uint32_t wrow = Sums::waddr(lds_addr(wl), kWRow, lane);
     const size_t thead = (size_t)kv * T + (size_t)half * 64;
-    walk_subs_q<false, BIT, G32>(
+    walk_subs_q<false, BIT, G32, NW>(
         (last - first) * subs_per_blk,
         [=](int n) { return thead + (size_t)(first + n / subs_per_blk) * D + (size_t)(n % subs_per_blk) * kSubTiles; },
         [=](int n) {
