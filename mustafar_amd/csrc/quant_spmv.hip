@@ -123,14 +123,14 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
 
 // ------------------------------------------------------------------------------- key
 // One wavefront per (KV head, token block); see key_spmv_kernel (more than eight rows are shared by the workgroup, whose
-// wavefronts then work on one head).
+// wavefronts then work on one head, or, SHARE, on one block: see kKeyShareQuant).
 template <int NW, int BIT, bool G32>
 constexpr int key_quant_lds()
 {
     constexpr int rows = StageRank<NW>::Sums::kRows * 128 * 2;
     return 4 * q_lds_bytes<BIT, G32>() + (StageRank<NW>::Sums::kWide ? rows : 4 * rows);
 }
-template <int NW, int BIT, bool G32>
+template <int NW, int BIT, bool G32, bool SHARE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_waves(key_quant_lds<NW, BIT, G32>(), 4)))) void key_spmv_quant_kernel(
     const uint64_t* __restrict__ bmp, const uint32_t* packed, const uint32_t* __restrict__ tile_off,
     const uint32_t* tile_off_dma, const uint16_t* scales, const uint16_t* zeros, const _Float16* Bm,
@@ -146,14 +146,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
     const int lane = lane_id();
     const int wave = wave_id();
     const int quads = (nblk + 3) / 4;  // workgroups of a head when they may not span two
-    const int nwg = kShared ? ntasks / nblk * quads : (ntasks + 3) / 4;
+    const int nwg = SHARE ? ntasks : (kShared ? ntasks / nblk * quads : (ntasks + 3) / 4);
+    static_assert(!SHARE || (kShared && kWaveLds >= kParkShares), "rows and sums of the workgroup");
     // neighbouring token blocks on the same XCD: their packed words share cache lines
     const int wg = xcd_contiguous((int)blockIdx.x, nwg);
     if (wg >= nwg) return;  // (the whole workgroup: no barrier is left waiting)
-    const int task = wg * 4 + wave;
+    const int task = SHARE ? wg : wg * 4 + wave;
     if (!kShared && task >= ntasks) return;
-    const int kv = kShared ? wg / quads : task / nblk;
-    const int tb = kShared ? (wg - kv * quads) * 4 + wave : task - kv * nblk;
+    const int kv = kShared && !SHARE ? wg / quads : task / nblk;
+    const int tb = kShared && !SHARE ? (wg - kv * quads) * 4 + wave : task - kv * nblk;
+    const int first = SHARE ? wave : 0;  // channel stage
     const size_t T = (size_t)Lc * D / 64;
     const QCache c = {bmp, tile_off, tile_off_dma, scales, zeros, packed};
     const char* wsrc = reinterpret_cast<const char*>(Bm + ((size_t)kv * rows_per_kv + row0) * D);
@@ -162,24 +164,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
 
     Sums sums;
     sums.clear();
-    const size_t tile0 = (size_t)kv * T + (size_t)tb * D;
+    const size_t tile0 = (size_t)kv * T + (size_t)tb * D + (size_t)first * kSubTiles;
     const uint32_t rbytes = (uint32_t)D * 2u;
     const uint32_t wrow = Sums::waddr(lds_addr(wl), rbytes, lane);
     auto stage_rows = [=](int n) {
         if (n != 0) return;  // the query rows are staged once per task
         stage_key_rows<NW, 4, kShared>(wsrc, rbytes, wl, wave, lane);
     };
-    if (kShared && tb >= nblk) {  // (wave-uniform) no block left, but a share of the rows
+    if (kShared && !SHARE && tb >= nblk) {  // (wave-uniform) no block left, but a share of the rows
         stage_rows(0);
         wait_vm0();
         __syncthreads();
         return;
     }
     walk_subs_q<kShared, BIT, G32, NW>(
-        D / kSubTiles, [=](int n) { return tile0 + (size_t)n * kSubTiles; }, stage_rows,
-        [=](int n) { return Sums::advance(wrow, (uint32_t)n * kSubTiles * 2u); }, (uint32_t)D * 8u, c, my, lane, mode, sums);
+        SHARE ? 1 : D / kSubTiles, [=](int n) { return tile0 + (size_t)n * kSubTiles; }, stage_rows,
+        [=](int n) { return Sums::advance(wrow, (uint32_t)(first + n) * kSubTiles * 2u); }, (uint32_t)D * 8u, c, my, lane, mode, sums);
     _Float16* out = C + ((size_t)kv * rows_per_kv + row0) * Lc + (size_t)tb * 64;
-    if constexpr (Sums::kWide) {
+    if constexpr (SHARE) {
+        store_rows_shared(sums, lds + kRowsLds, kWaveLds, lds, out, (size_t)Lc, wave, lane);
+    } else if constexpr (Sums::kWide) {
         store_rows_wide<NW>(sums, my, out, (size_t)Lc, lane);
     } else {
         sums.each4(lane, [=](int row, int pos, const f4_t& v) {
@@ -300,19 +304,30 @@ struct QArgs {
     int group_size;  // 64: one (scale, zero) pair per tile; 32: two
 };
 
+// Whether the four wavefronts of a workgroup share a token block of a key product with more than eight rows, a channel stage
+// each, instead of taking a block each: a quarter of the chain, and as many wavefronts four times over.  1024 such workgroups
+// fit the chip; a few more still pay.  32 rows, 4 bits, 70 %, heads x blocks, a block each / shared: 1 x 1 7.06 / 3.95 us,
+// 8 x 33 7.97 / 4.88, 32 x 24 8.33 / 5.91, 32 x 33 9.33 / 8.36, 32 x 48 9.84 / 10.02, 64 x 64 13.0 / 21.0 (2 bits 6.64 / 3.89,
+// 7.43 / 4.78, 7.72 / 5.74, 8.70 / 7.91, 9.25 / 9.66, 12.5 / 20.5).
+constexpr int kKeyShareQuant = 1280;
 template <int NW, int BIT>
 static void launch_key_q(hipStream_t st, const QArgs& a, const _Float16* Bm, _Float16* C, int Lc, int D, int Bkv,
                          int rows_per_kv, int row0)
 {
     const int nblk = Lc / 64;
     const int ntasks = Bkv * nblk;
-    const int wgs = xcd_grid(wide_rows(NW) ? Bkv * ((nblk + 3) / 4) : (ntasks + 3) / 4);
-    if (a.group_size == 32)
-        hipLaunchKernelGGL((key_spmv_quant_kernel<NW, BIT, true>), dim3(wgs), dim3(256), 0, st, a.bmp, a.packed,
-                           a.tile_off, a.tile_off, a.scales, a.zeros, Bm, C, Lc, D, nblk, ntasks, rows_per_kv, row0, a.mode);
-    else
-        hipLaunchKernelGGL((key_spmv_quant_kernel<NW, BIT, false>), dim3(wgs), dim3(256), 0, st, a.bmp, a.packed,
-                           a.tile_off, a.tile_off, a.scales, a.zeros, Bm, C, Lc, D, nblk, ntasks, rows_per_kv, row0, a.mode);
+    const bool share = wide_rows(NW) && D == 128 && ntasks <= kKeyShareQuant;
+    const int wgs = xcd_grid(share ? ntasks : (wide_rows(NW) ? Bkv * ((nblk + 3) / 4) : (ntasks + 3) / 4));
+#define MSTF_KQ_LAUNCH(G32, SHARE)                                                                                            \
+    hipLaunchKernelGGL((key_spmv_quant_kernel<NW, BIT, G32, SHARE>), dim3(wgs), dim3(256), 0, st, a.bmp, a.packed, a.tile_off, \
+                       a.tile_off, a.scales, a.zeros, Bm, C, Lc, D, nblk, ntasks, rows_per_kv, row0, a.mode)
+    constexpr bool kShare = wide_rows(NW);
+    if (a.group_size == 32) {
+        if (share) MSTF_KQ_LAUNCH(true, kShare); else MSTF_KQ_LAUNCH(true, false);
+    } else {
+        if (share) MSTF_KQ_LAUNCH(false, kShare); else MSTF_KQ_LAUNCH(false, false);
+    }
+#undef MSTF_KQ_LAUNCH
 }
 template <int NW>
 static void launch_key_q_bit(int bit, hipStream_t st, const QArgs& a, const _Float16* Bm, _Float16* C, int Lc, int D,

@@ -409,6 +409,53 @@ __device__ __forceinline__ void store_rows_wide(const RowSums<NW, FOLD>& sums, c
     }
 }
 
+// The four wavefronts of a workgroup took a channel stage each of one token block: adds their sums of more than eight rows,
+// in the order of the stages, and stores them as store_rows_wide does.  Wavefront w adds up the positions 8 w .. 8 w + 7 of
+// both halves and parks the others at its `my` (6 KB, its reads are over; the others' are at area + i * bytes); the fp16
+// rows pass through `room` (4 KB that no wavefront reads any more behind the first barrier).
+constexpr int kParkShares = 3 * 2 * 1024;
+template <int NW, bool FOLD>
+__device__ __forceinline__ void store_rows_shared(const RowSums<NW, FOLD>& sums, char* area, int bytes, char* room, _Float16* out,
+                                                  size_t stride, int wave, int lane)
+{
+    static_assert(NW % 8 == 0 && wide_rows(NW), "eight rows per store instruction");
+    const uint32_t mine = lds_addr(area) + (uint32_t)(wave * bytes) + (uint32_t)lane * 16u;
+    f4_t own[2];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const f4_t v = {sums.wide[p][4 * r], sums.wide[p][4 * r + 1], sums.wide[p][4 * r + 2], sums.wide[p][4 * r + 3]};
+            if (r == wave)
+                own[p] = v;
+            else  // (slot r, or r - 1 behind the wavefront's own)
+                *(MSTF_LDS f4_t*)(uintptr_t)(mine + (uint32_t)((r - (r > wave ? 1 : 0)) * 2 + p) * 1024u) = v;
+        }
+    __syncthreads();
+    f4_t sum[2];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const uint32_t slot = (uint32_t)((wave - (wave > i ? 1 : 0)) * 2 + p) * 1024u;
+            const f4_t v = i == wave ? own[p]
+                                     : *(MSTF_LDS const f4_t*)(uintptr_t)(lds_addr(area) + (uint32_t)(i * bytes) + slot + (uint32_t)lane * 16u);
+            sum[p] = i == 0 ? v : sum[p] + v;
+        }
+    const uint32_t base = lds_addr(room);
+    const uint32_t row = (uint32_t)lane & 31u;
+#pragma unroll
+    for (int p = 0; p < 2; p++)  // (pieces as in store_rows_wide)
+        *(MSTF_LDS h4_t*)(uintptr_t)(base + row * 128u + (((uint32_t)(4 * p + wave) ^ (row & 7u)) * 16u) +
+                                     (uint32_t)(lane >> 5) * 8u) = round_h4(sum[p]);
+    __syncthreads();
+    if (wave < NW / 8) {
+        const uint32_t piece = (uint32_t)lane & 7u, sub = (uint32_t)lane >> 3, at = (uint32_t)wave * 8u + sub;
+        const u32x4_t v = *(MSTF_LDS const u32x4_t*)(uintptr_t)(base + at * 128u + ((piece ^ sub) * 16u));
+        *reinterpret_cast<u32x4_t*>(out + (size_t)at * stride + piece * 8u) = v;
+    }
+}
+
 // Requests the weights of the 32 tiles of a stage for more than eight rows of a value product: 64 bytes each of rows
 // `stride` apart into [row][32] at dst, the sixteen-byte pieces where weight_swizzle wants them.  Sixteen rows per
 // instruction; with four bytes a lane the sixteen instructions a stage took kept a CU's address unit busy as well

@@ -3,8 +3,9 @@
 //
 // In rank_device.hpp a register of the address products holds the same half of two tiles, so that an exec mask is put
 // together from two 32-bit pieces and the lane halves' sums have to be joined.  Here the rows of a product are the two halves
-// of sixteen tiles - row 8 g + 4 P + j for half P of a tile - so that a register holds a tile whole, lane = element: one 64-bit reversal sets its exec mask, two products (three there) make the addresses of 32 tiles, and nothing is
-// joined.  A product sums over 64 bits: the elements of the row's own half in front of the column's position (lanes 0 .. 31),
+// of sixteen tiles - row 8 g + 4 P + j for half P of a tile - so that a register holds a tile whole, lane = element: one
+// 64-bit reversal sets its exec mask, two products (three there) make the addresses of 32 tiles, and nothing is joined.
+// A product sums over 64 bits: the elements of the row's own half in front of the column's position (lanes 0 .. 31),
 // and for the second half of a tile all of the first (lanes 32 .. 63; masked off for the first half).
 // The bits are 4-bit floats and the sums 32-bit floats below the normal range, whose bits are the integer they hold: with the
 // products' unit at twice the smallest 32-bit float every bit adds 2 to the LDS byte address in C, all of it exact.  (Where the

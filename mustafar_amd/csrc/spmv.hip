@@ -23,7 +23,8 @@ namespace mstf {
 // One wavefront per (KV head, token block): walks the D/32 channel sub-chunks of the block.
 // C[(kv*rows + row0 + n)*Lc + token] = sum_d K[token][d] * Bm[(kv*rows + row0 + n)*D + d],  n < NW.
 // LDS: per wavefront the value double buffer and the table of the tiles' addresses, and the query rows - one copy per
-// wavefront of at most eight rows, one for the workgroup of more, whose WAVES wavefronts then work on blocks of one head.
+// wavefront of at most eight rows, one for the workgroup of more, whose WAVES wavefronts then work on blocks of one head or,
+// SHARE, on one block (kKeyShare).
 // With four of them three workgroups fit a CU (three wavefronts per SIMD), with eight two (four per SIMD): key_waves().
 template <int NW, int WAVES>
 constexpr int key_lds()
@@ -31,7 +32,7 @@ constexpr int key_lds()
     constexpr int rows = RowSums<NW>::kRows * 128 * 2;
     return WAVES * kNzLds + (RowSums<NW>::kWide ? rows : WAVES * rows);
 }
-template <int NW, int WAVES>
+template <int NW, int WAVES, bool SHARE>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resident_waves(key_lds<NW, WAVES>(), WAVES)))) void key_spmv_kernel(
     const uint64_t* __restrict__ bmp, const char* __restrict__ nz, const uint32_t* __restrict__ idx,
     const uint32_t* __restrict__ nz_off, const _Float16* __restrict__ Bm, _Float16* __restrict__ C, int Lc, int D, int nblk,
@@ -47,10 +48,12 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     const int lane = lane_id();
     const int wave = wave_id();
     const int wgs = (nblk + WAVES - 1) / WAVES;  // workgroups of a head when they may not span two
-    const int task = (int)blockIdx.x * WAVES + wave;
+    static_assert(!SHARE || (kShared && WAVES == 4 && kWaveLds >= kParkShares), "rows and sums of the workgroup");
+    const int task = SHARE ? (int)blockIdx.x : (int)blockIdx.x * WAVES + wave;
     if (!kShared && task >= ntasks) return;
-    const int kv = kShared ? (int)blockIdx.x / wgs : task / nblk;
-    const int tb = kShared ? ((int)blockIdx.x - kv * wgs) * WAVES + wave : task - kv * nblk;
+    const int kv = kShared && !SHARE ? (int)blockIdx.x / wgs : task / nblk;
+    const int tb = kShared && !SHARE ? ((int)blockIdx.x - kv * wgs) * WAVES + wave : task - kv * nblk;
+    const int first = SHARE ? wave : 0;  // channel stage
     const size_t T = (size_t)Lc * D / 64;
     const uint64_t* bmk = bmp + (size_t)kv * T;
     const uint32_t* ixk = idx + (size_t)kv * (T + 1);
@@ -61,24 +64,26 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
 
     Sums sums;
     sums.clear();
-    const size_t tile0 = (size_t)tb * D;
+    const size_t tile0 = (size_t)tb * D + (size_t)first * kSubTiles;
     const uint32_t rbytes = (uint32_t)D * 2u;
     const uint32_t wrow = Sums::waddr(lds_addr(wl), rbytes, lane);
     auto stage_rows = [=](int n) {
         if (n != 0) return;  // the query rows are staged once per task
         stage_key_rows<NW, WAVES, kShared>(wsrc, rbytes, wl, wave, lane);
     };
-    if (kShared && tb >= nblk) {  // (wave-uniform) no block left, but a share of the rows
+    if (kShared && !SHARE && tb >= nblk) {  // (wave-uniform) no block left, but a share of the rows
         stage_rows(0);
         wait_vm0();
         __syncthreads();
         return;
     }
     walk_subs<kShared>(
-        D / kSubTiles, [=](int n) { return tile0 + (size_t)n * kSubTiles; }, stage_rows,
-        [=](int n) { return Sums::advance(wrow, (uint32_t)n * kSubTiles * 2u); }, (uint32_t)D * 8u, bmk, ixk, nzk, my, lane, sums);
+        SHARE ? 1 : D / kSubTiles, [=](int n) { return tile0 + (size_t)n * kSubTiles; }, stage_rows,
+        [=](int n) { return Sums::advance(wrow, (uint32_t)(first + n) * kSubTiles * 2u); }, (uint32_t)D * 8u, bmk, ixk, nzk, my, lane, sums);
     _Float16* out = C + ((size_t)kv * bm_rows_per_kv + row0) * Lc + (size_t)tb * 64;
-    if constexpr (Sums::kWide) {
+    if constexpr (SHARE) {
+        store_rows_shared(sums, lds + kRowsLds, kWaveLds, lds, out, (size_t)Lc, wave, lane);
+    } else if constexpr (Sums::kWide) {
         store_rows_wide<NW>(sums, my, out, (size_t)Lc, lane);
     } else {
         sums.each4(lane, [=](int row, int pos, const f4_t& v) {
@@ -299,15 +304,19 @@ static int key_waves(int nblk, int Bkv)
     const int fours = (nblk + 3) / 4, eights = (nblk + 7) / 8;
     return (long)Bkv * fours > 768 && 2 * fours > 3 * eights ? 8 : 4;
 }
-template <int NW, int WAVES>
+// Blocks up to which the four wavefronts of a workgroup share a block of more than eight rows, a channel stage each, instead of
+// taking a block each: the workgroups that fit the chip.  32 rows, 70 %, heads x blocks, a block each / shared: 1 x 1 5.41 /
+// 3.48 us, 8 x 33 6.12 / 4.25, 32 x 24 7.12 / 6.03, 32 x 33 7.67 / 8.82, 64 x 64 11.6 / 22.2.
+constexpr int kKeyShare = 768;
+template <int NW, int WAVES, bool SHARE = false>
 static void launch_key_waves(hipStream_t st, const uint64_t* bmp, const char* nz, const uint32_t* idx,
                              const uint32_t* nz_off, const _Float16* Bm, _Float16* C, int Lc, int D, int Bkv,
                              int rows_per_kv, int row0)
 {
     const int nblk = Lc / 64;
     const int ntasks = Bkv * nblk;
-    const int wgs = wide_rows(NW) ? Bkv * ((nblk + WAVES - 1) / WAVES) : (ntasks + WAVES - 1) / WAVES;
-    hipLaunchKernelGGL((key_spmv_kernel<NW, WAVES>), dim3(wgs), dim3(WAVES * 64), 0, st, bmp, nz, idx, nz_off, Bm, C, Lc, D,
+    const int wgs = SHARE ? ntasks : (wide_rows(NW) ? Bkv * ((nblk + WAVES - 1) / WAVES) : (ntasks + WAVES - 1) / WAVES);
+    hipLaunchKernelGGL((key_spmv_kernel<NW, WAVES, SHARE>), dim3(wgs), dim3(WAVES * 64), 0, st, bmp, nz, idx, nz_off, Bm, C, Lc, D,
                        nblk, ntasks, rows_per_kv, row0);
 }
 template <int NW>
@@ -316,6 +325,8 @@ static void launch_key(hipStream_t st, const uint64_t* bmp, const char* nz, cons
                        int row0)
 {
     if constexpr (wide_rows(NW)) {
+        if (D == 128 && Bkv * (Lc / 64) <= kKeyShare)
+            return launch_key_waves<NW, 4, true>(st, bmp, nz, idx, nz_off, Bm, C, Lc, D, Bkv, rows_per_kv, row0);
         if (key_waves<NW>(Lc / 64, Bkv) == 8)
             return launch_key_waves<NW, 8>(st, bmp, nz, idx, nz_off, Bm, C, Lc, D, Bkv, rows_per_kv, row0);
     }
