@@ -20,7 +20,7 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, si
     own = ops._own_workspace(ws, inputs.device) if sized else None
     out = ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),
                     int(group_size), room, ops._landing_word()[1] if sized else 0,
-                    own.status(inputs.shape[0] * (inputs.shape[1] // 64) + 2) if own else None)
+                    own.status(ops.status_words(inputs.shape[0] * (inputs.shape[1] // 64))) if own else None)
     if sized and out[-1] < 0:
         ops.gave_up(own, _GAVE_UP)
     return out

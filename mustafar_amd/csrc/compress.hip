@@ -332,7 +332,7 @@ __global__ __launch_bounds__(64) void compress_scatter_kernel(const _Float16* __
 // workgroup that gives up writes no values and marks the call itself (mark_gave_up): the flag word behind the
 // workgroup words, *total_halfs raised to all ones (packed layout: the last workgroup raises it to the sum with the
 // same atomic maximum, so the order of the two does not matter) and bit 1 of *overflow (pooled layout).
-// onepass_init_kernel clears the words and *total_halfs before the launch.
+// onepass_init_kernel clears the words and *total_halfs before the launch, unless the words are kept (Handover).
 __device__ __forceinline__ void stream_image(uint32_t img, uint32_t bytes, char* dst, int lane)
 {
     for (uint32_t o = (uint32_t)lane * 16u; o < bytes; o += 1024u)
@@ -470,7 +470,8 @@ __device__ __forceinline__ void onepass_workgroup(
         ok = ok && bases[w][2] != 0ull;
     }
     if (!ok && threadIdx.x == 0) mark_gave_up(gave_up, how.kept ? nullptr : total_halfs, overflow);
-    if (how.counted() && g != groups_total - 1 && threadIdx.x == 0) count_through(state + groups_total + 1, ok);
+    if (how.counted() && g != groups_total - 1 && threadIdx.x == 0) 
+        count_through(counter_of(how, state, groups_total, g), ok);
     const uint32_t base = (uint32_t)in_head + in_group;
     const uint32_t end = base + total;
 
@@ -620,8 +621,9 @@ static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& pr
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
     uint64_t* state = status ? status : reinterpret_cast<uint64_t*>(ws);
-    const Handover how = {landing, status != nullptr};
-    const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
+    const int counters = status ? kCounters : counters_within(compress_ws_bytes(B, M) / 8, groups);
+    const Handover how = {landing, status != nullptr, counters};
+    const int words = status_words(groups, counters);
     const uint32_t spin_limit = onepass_spin_limit();
     if (!status) {
         hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),
@@ -650,10 +652,12 @@ static int launch_onepass_kv(hipStream_t st, OnepassSide k, OnepassSide v, int B
     const int nblk = M / 64, units = B * nblk;
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
-    const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
+    const int counters = status ? kCounters : counters_within(compress_ws_bytes(B, M) / 8, groups);  // (a side's half of ws)
+    const int words = status_words(groups, counters);
     k.state = status ? status : reinterpret_cast<uint64_t*>(ws);
     v.state = k.state + words;
     k.how.kept = v.how.kept = status != nullptr;
+    k.how.counters = v.how.counters = counters;
     const uint32_t spin_limit = onepass_spin_limit();
     if (!status) {
         hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((2 * words + 255) / 256 < 256 ? (2 * words + 255) / 256 : 256)),
@@ -854,7 +858,7 @@ extern "C" int mstf_append_value_f16(void* stream, const mstf_half* x, int B, in
 extern "C" size_t mstf_status_bytes(int B, int M, int sides)
 {
     if (B <= 0 || M <= 0 || M % 64 != 0 || sides < 1) return 0;
-    return ((size_t)B * (M / 64) + 2) * (size_t)sides * sizeof(uint64_t);
+    return ((size_t)B * (M / 64) + status_words(0, kCounters)) * (size_t)sides * sizeof(uint64_t);
 }
 int mstf::status_check(const uint64_t* status, size_t bytes, int64_t B, int M, int sides)
 {

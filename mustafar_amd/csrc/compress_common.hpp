@@ -594,7 +594,7 @@ __device__ __forceinline__ void compact_half(const uint32_t (&r)[64], const uint
 }
 
 // ------------------------------------------------------------------------------- one-pass ordering
-// Status words of the one-pass producers (compress.hip describes the protocol): cleared by onepass_init_kernel,
+// Status words of the one-pass producers (compress.hip describes the protocol): cleared by onepass_init_kernel or kept clear (Handover),
 // one word per workgroup = bit 63 | total, published with an agent-scope store, polled by the workgroups behind.
 constexpr uint32_t kSpinLimit = 1u << 20;  // the default of onepass_spin_limit() (runtime.hip)
 // The limit the launchers pass: kSpinLimit unless mstf_test_set_spin_limit (runtime.hip) lowered it - a test's way
@@ -643,7 +643,7 @@ constexpr uint64_t kWordReady = 1ull << 63;
 // stream: with a launch that fetches the word behind the kernel, the GPU stood idle from the kernel's end until the host
 // had seen the word and made that next call (keys and values of 128 heads x 256 tokens, both sizes read: 52.8 -> 44.7 us a
 // pass; 2-bit codes of 64 heads x 4096, two calls: 132 -> 120; two calls from the projection, 128 x 4096: 183 -> 178).  Certain means that no workgroup gave up its wait: every workgroup that is
-// through counts itself in a word behind the flag word (failures in the upper half), and the last one waits for all of them.
+// through counts itself in words behind the flag word (failures in the upper half), and the last one waits for all of them.
 // (Counted in their status words, which the others poll, the waits of all became longer: 77 -> 84 us, 128 heads x 4096 tokens.)
 __device__ __forceinline__ void count_through(uint64_t* counter, bool ok)
 {
@@ -656,37 +656,60 @@ __device__ __forceinline__ void count_through(uint64_t* counter, bool ok)
 //             compressors from the projection, 128 x 4096, 158.6 -> 153.5).  The last workgroup clears them when the others are through,
 //             and writes the total; a wait that ran out leaves the flag word set, and with it the total of this launch and of
 //             every one behind it is all ones until the caller brings cleared words again.
+//   counters: in how many words the workgroups count themselves, a power of two; word i stands kCounterStep words behind word
+//             i - 1, in a cache line of its own.  Adding to one word takes the chip 7 ns each time: 4500 workgroups of one wavefront
+//             (60 heads x 4800 tokens from the projection) took 82 us with one word, 52 without counting.
+constexpr int kCounters = 16, kCounterStep = 16;
 struct Handover {
     uint64_t* landing;
     int kept;
+    int counters;
     __device__ __forceinline__ bool counted() const { return landing != nullptr || kept != 0; }
 };
+// Status words, flag word and counters of a launch of `groups` workgroups.
+constexpr int status_words(int groups, int counters) { return groups + 2 + (counters - 1) * kCounterStep; }
+// The counters that `room` words leave space for.
+inline int counters_within(size_t room, int groups)
+{
+    int n = kCounters;
+    while (n > 1 && (size_t)status_words(groups, n) > room) n /= 2;
+    return n;
+}
+__device__ __forceinline__ uint64_t* counter_of(const Handover& how, uint64_t* state, int groups, int g)
+{
+    return state + groups + 1 + (g & (how.counters - 1)) * kCounterStep;
+}
 // By the last workgroup of a launch whose workgroups count themselves, all its threads: waits until the others are through and
 // hands the total over, all ones if a wait ran out.  ok: whether its own waits ended.  state: the `groups` status words, the
-// flag word and the counter; total_out: the caller's total (kept).
+// flag word and the counters; total_out: the caller's total (kept).
 __device__ __forceinline__ void hand_over(const Handover& how, uint64_t* total_out, uint64_t total, bool ok, uint64_t* state,
                                           int groups, uint32_t spin_limit, uint32_t* room)
 {
-    if (threadIdx.x == 0) {
-        uint64_t through = agent_load(state + groups + 1);
+    if (threadIdx.x < 64) {
+        const bool reads = (int)threadIdx.x < how.counters;
+        const uint64_t* mine = counter_of(how, state, groups, reads ? (int)threadIdx.x : 0);
+        auto counted = [&]() { return wave_sum_u64(reads ? agent_load(mine) : 0ull); };
+        uint64_t through = counted();
         const uint32_t others = (uint32_t)groups - 1u;
         for (uint32_t polls = 0; (uint32_t)through != others && polls < spin_limit; polls++) {
             __builtin_amdgcn_s_sleep(1);
-            through = agent_load(state + groups + 1);
+            through = counted();
         }
         const bool all = (uint32_t)through == others;
-        if (!all && how.kept) agent_store(state + groups, 1ull);  // (words are still in use: they cannot be cleared)
-        ok = ok && through == others && agent_load(state + groups) == 0ull;
-        const uint64_t v = ok ? total : ~0ull;
-        if (how.kept) *total_out = v;
-        if (how.landing) __hip_atomic_store(how.landing, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        *room = all ? 1u : 0u;
+        if (threadIdx.x == 0) {
+            if (!all && how.kept) agent_store(state + groups, 1ull);  // (words are still in use: they cannot be cleared)
+            ok = ok && through == others && agent_load(state + groups) == 0ull;
+            const uint64_t v = ok ? total : ~0ull;
+            if (how.kept) *total_out = v;
+            if (how.landing) __hip_atomic_store(how.landing, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            *room = all ? 1u : 0u;
+        }
     }
     if (!how.kept) return;
     __syncthreads();
     if (*room == 0u) return;
     for (int i = (int)threadIdx.x; i < groups; i += (int)blockDim.x) agent_store(state + i, 0ull);
-    if (threadIdx.x == 0) agent_store(state + groups + 1, 0ull);
+    if ((int)threadIdx.x < how.counters) agent_store(counter_of(how, state, groups, (int)threadIdx.x), 0ull);
 }
 
 // This wavefront's share of the wait for state[first .. g): the windows of 64 words number `wave`, wave + W, ...,

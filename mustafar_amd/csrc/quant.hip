@@ -416,7 +416,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                 if (g == groups_total - 1)
                     hand_over(how, total_words, before - in_group + group_total, ok, state, groups_total, spin_limit, wave_total);
                 else if (threadIdx.x == 0)
-                    count_through(state + groups_total + 1, ok);
+                    count_through(counter_of(how, state, groups_total, g), ok);
             }
             if (lane == 0 && unit == nunits - 1 && ok && !how.kept)
                 atomicMax(reinterpret_cast<unsigned long long*>(total_words), before + tot[0] + tot[1]);
@@ -487,8 +487,9 @@ static int compress_quant_impl(void* stream, const mstf_half* x, int B, int M, i
         const int W = nblk % 4 == 0 ? 4 : (nblk % 2 == 0 ? 2 : 1);
         const int groups = units_all / W;
         uint64_t* state = status ? status : reinterpret_cast<uint64_t*>(ws);
-        const Handover how = {landing, status != nullptr};
-        const int words = groups + 2;  // (the flag word, and the count of the workgroups that are through)
+        const int counters = status ? kCounters : counters_within(quant_ws_bytes(B, M) / 8, groups);
+        const Handover how = {landing, status != nullptr, counters};
+        const int words = status_words(groups, counters);
         const uint32_t spin_limit = onepass_spin_limit();
         if (!status) {
             hipLaunchKernelGGL(onepass_init_kernel, dim3((unsigned)((words + 255) / 256 < 256 ? (words + 255) / 256 : 256)),

@@ -61,6 +61,11 @@ class Workspace:
         self._status.append(torch.zeros(4096, dtype=torch.int64, device=self.device))
 
 
+def status_words(units, sides=1):
+    """mstf_status_bytes in words, of a producer's call over `units` blocks a side."""
+    return sides * (units + 242)
+
+
 _WS = {}
 
 
@@ -260,7 +265,7 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     landing = _LandingPair(pair, _stream(), own) if pair else None
     kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
                                                    -1 if capacity_halfs is None else int(capacity_halfs), pair or 0,
-                                                   own.status(2 * (k.shape[0] * (k.shape[1] // 64) + 2)) if own else None)
+                                                   own.status(status_words(k.shape[0] * (k.shape[1] // 64), 2)) if own else None)
     M, N = k.shape[1:]
     return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
@@ -299,7 +304,7 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
                                            rot, -1 if capacity_halfs is None else int(capacity_halfs),
                                            _landing_word()[1] if sized else 0,
-                                           own.status(x.shape[0] * x.shape[2] * (M // 64) + 2) if own else None)
+                                           own.status(status_words(x.shape[0] * x.shape[2] * (M // 64))) if own else None)
     if M == 0:
         return None, rot
     if sized and n < 0:

@@ -114,7 +114,7 @@ def test_a_wait_that_ran_out_lands_as_such():
         assert torch.equal(c.packed(), want)
 
 
-@pytest.mark.parametrize("heads,tokens", [(1, 64), (3, 192), (40, 1024), (130, 2048)])
+@pytest.mark.parametrize("heads,tokens", [(1, 64), (3, 192), (40, 1024), (130, 2048), (33, 3264)])
 def test_status_words_are_left_as_they_were(heads, tokens):
     """Calls of several sizes over the same kept words, one behind the other and without a wait between them; a launch that
     clears words in the workspace gives the same arrays."""

@@ -84,3 +84,10 @@ def test_scratch_memory(tokens):
     lse = torch.empty((8, 2), device="cuda")
     assert ops.decode_attention(ck, cv, q, 4, out=out, lse=lse) is not None
     assert torch.equal(out, ops.decode_attention(ck, cv, q, 4)) and bool((lse[:, 1] > 0).all())
+
+
+@pytest.mark.parametrize("heads,tokens,sides", [(1, 64, 1), (3, 192, 2), (60, 4800, 1), (128, 4096, 2)])
+def test_status_words(heads, tokens, sides):
+    from mustafar_amd import ops
+    from mustafar_amd._lib import lib
+    assert 8 * ops.status_words(heads * (tokens // 64), sides) == lib().mstf_status_bytes(heads, tokens, sides)
