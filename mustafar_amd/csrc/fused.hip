@@ -547,7 +547,7 @@ __global__ __launch_bounds__(128 * kMergeGroups) void decode_merge_blocks_kernel
                     o[k] = po[(size_t)i * D];
                 }
             }
-            merge_run(s, m, l, o, units - s0);
+            merge_run(s, m, l, o, units - s0, units == 1);
         }
     }
     if (groups > 1) {

@@ -366,7 +366,7 @@ __device__ __forceinline__ void workgroup_combine(char* lds_base, int wave_strid
 // A run of eight splits into a running (max, output, sum) (decode_merge_kernel).
 constexpr int kMergeRun = 8;
 __device__ __forceinline__ void merge_run(Triple& s, const float (&m)[kMergeRun], const float (&l)[kMergeRun],
-                                          const float (&o)[kMergeRun], int valid)
+                                          const float (&o)[kMergeRun], int valid, bool alone = false)
 {
     float gm = s.M;
 #pragma unroll
@@ -377,10 +377,11 @@ __device__ __forceinline__ void merge_run(Triple& s, const float (&m)[kMergeRun]
     s.sl *= fr;
 #pragma unroll
     for (int u = 0; u < kMergeRun; u++) {
-        const bool there = u < valid;  // (an infinite partial of a split that is repeated must not meet the zero)
+        const bool there = u < valid;
         const float f = (there && m[u] != -INFINITY) ? __expf(m[u] - gm) : 0.f;
-        s.so = __builtin_fmaf(f, there ? o[u] : 0.f, s.so);  // (written out: the same numbers in every kernel)
-        s.sl = __builtin_fmaf(f, there ? l[u] : 0.f, s.sl);
+        // (alone: one split, which no merge would follow without sharing; its infinite outputs must not meet the zero)
+        s.so = __builtin_fmaf(f, there || !alone ? o[u] : 0.f, s.so);  // (written out: the same numbers in every kernel)
+        s.sl = __builtin_fmaf(f, there || !alone ? l[u] : 0.f, s.sl);
     }
     s.M = gm;
 }
