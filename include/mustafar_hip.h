@@ -67,8 +67,8 @@ int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* 
 #define MSTF_NOT_LANDED (INT64_MIN + 2)
 /* status (those calls; null: none): mstf_status_bytes(B, M, sides) bytes of device memory, 8-byte aligned, that hold zeros when
  * the call begins and are used by nothing else meanwhile; the call leaves zeros, so that the next one may have them as they are
- * (without, a launch in front clears words in the workspace).  After a total of all ones they have to be cleared.  sides: 2 for
- * keys and values in one call. */
+ * (without, a launch in front clears words in the workspace).  After a total of all ones they have to be cleared: until then the
+ * total of every call that is given them is all ones, whatever its size.  sides: 2 for keys and values in one call. */
 size_t mstf_status_bytes(int B, int M, int sides);
 int64_t* mstf_landing_take(void);
 void mstf_landing_give(int64_t* pair);

@@ -329,8 +329,8 @@ __global__ __launch_bounds__(64) void compress_scatter_kernel(const _Float16* __
 // trip, until every word is set, and adds them up; the others wait at the barrier.
 // A workgroup publishes its total before it waits for anything and waits only for workgroups of a lower index, which
 // the dispatcher has started before it: every wait ends.  The waits are bounded all the same (kSpinLimit polls); a
-// workgroup that gives up writes no values and marks the call itself (mark_gave_up): the flag word behind the
-// workgroup words, *total_halfs raised to all ones (packed layout: the last workgroup raises it to the sum with the
+// workgroup that gives up writes no values and marks the call itself (mark_gave_up): the flag word of the
+// launch, *total_halfs raised to all ones (packed layout: the last workgroup raises it to the sum with the
 // same atomic maximum, so the order of the two does not matter) and bit 1 of *overflow (pooled layout).
 // onepass_init_kernel clears the words and *total_halfs before the launch, unless the words are kept (Handover).
 __device__ __forceinline__ void stream_image(uint32_t img, uint32_t bytes, char* dst, int lane)
@@ -386,7 +386,6 @@ __device__ __forceinline__ void onepass_workgroup(
     const int wave = wave_id();
     const int nblk = M / 64;
     const size_t T = (size_t)M * kD / 64;
-    uint64_t* gave_up = state + groups_total;
     const int u = g * W + wave;  // all W units are of one head and exist: W divides nblk
     const int b = u / nblk, tb = u - b * nblk;
     uint32_t* buf = bufs[wave];
@@ -469,8 +468,8 @@ __device__ __forceinline__ void onepass_workgroup(
         in_head += bases[w][1];
         ok = ok && bases[w][2] != 0ull;
     }
-    if (!ok && threadIdx.x == 0) mark_gave_up(gave_up, how.kept ? nullptr : total_halfs, overflow);
-    if (how.counted() && g != groups_total - 1 && threadIdx.x == 0) 
+    if (!ok && threadIdx.x == 0) mark_gave_up(how.flag, how.kept ? nullptr : total_halfs, overflow);
+    if (how.counted() && g != groups_total - 1 && threadIdx.x == 0)
         count_through(counter_of(how, state, groups_total, g), ok);
     const uint32_t base = (uint32_t)in_head + in_group;
     const uint32_t end = base + total;
@@ -620,9 +619,9 @@ static int launch_onepass(hipStream_t st, const _Float16* xh, const ProjArgs& pr
 #endif
     const int W = nblk % MSTF_ONEPASS_W == 0 ? MSTF_ONEPASS_W : (nblk % 2 == 0 ? 2 : 1);
     const int groups = units / W;
-    uint64_t* state = status ? status : reinterpret_cast<uint64_t*>(ws);
+    uint64_t* state = status ? status + kKeptHead : reinterpret_cast<uint64_t*>(ws);
     const int counters = status ? kCounters : counters_within(compress_ws_bytes(B, M) / 8, groups);
-    const Handover how = {landing, status != nullptr, counters};
+    const Handover how = {landing, status ? status : state + groups, status != nullptr, counters};
     const int words = status_words(groups, counters);
     const uint32_t spin_limit = onepass_spin_limit();
     if (!status) {
@@ -654,8 +653,10 @@ static int launch_onepass_kv(hipStream_t st, OnepassSide k, OnepassSide v, int B
     const int groups = units / W;
     const int counters = status ? kCounters : counters_within(compress_ws_bytes(B, M) / 8, groups);  // (a side's half of ws)
     const int words = status_words(groups, counters);
-    k.state = status ? status : reinterpret_cast<uint64_t*>(ws);
+    k.state = status ? status + kKeptHead : reinterpret_cast<uint64_t*>(ws);
     v.state = k.state + words;
+    k.how.flag = status ? status : k.state + groups;
+    v.how.flag = status ? status : v.state + groups;
     k.how.kept = v.how.kept = status != nullptr;
     k.how.counters = v.how.counters = counters;
     const uint32_t spin_limit = onepass_spin_limit();
@@ -858,7 +859,7 @@ extern "C" int mstf_append_value_f16(void* stream, const mstf_half* x, int B, in
 extern "C" size_t mstf_status_bytes(int B, int M, int sides)
 {
     if (B <= 0 || M <= 0 || M % 64 != 0 || sides < 1) return 0;
-    return ((size_t)B * (M / 64) + status_words(0, kCounters)) * (size_t)sides * sizeof(uint64_t);
+    return (kKeptHead + ((size_t)B * (M / 64) + status_words(0, kCounters)) * (size_t)sides) * sizeof(uint64_t);
 }
 int mstf::status_check(const uint64_t* status, size_t bytes, int64_t B, int M, int sides)
 {
@@ -978,9 +979,9 @@ static int compress_kv_impl(void* stream, const mstf_half* k, const mstf_half* v
     if (!workspace || workspace_bytes < mstf_compress_kv_workspace_bytes(B, M, N)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 256)) return MSTF_EALIGN;
     OnepassSide ks = {reinterpret_cast<const _Float16*>(k), kth_k, k_bmp, k_idx, k_nz_off, k_total_halfs, nullptr, nullptr,
-                      reinterpret_cast<char*>(k_nz), k_capacity_halfs, nullptr, {k_landing, 0}};
+                      reinterpret_cast<char*>(k_nz), k_capacity_halfs, nullptr, {k_landing}};
     OnepassSide vs = {reinterpret_cast<const _Float16*>(v), kth_v, v_bmp, v_idx, v_nz_off, v_total_halfs, nullptr, nullptr,
-                      reinterpret_cast<char*>(v_nz), v_capacity_halfs, nullptr, {v_landing, 0}};
+                      reinterpret_cast<char*>(v_nz), v_capacity_halfs, nullptr, {v_landing}};
     return launch_onepass_kv(as_stream(stream), ks, vs, B, M, nullptr, workspace, status);
 }
 
@@ -1036,8 +1037,8 @@ extern "C" int mstf_append_kv_f16(void* stream, const mstf_half* k, const mstf_h
     if (!workspace || workspace_bytes < mstf_compress_kv_workspace_bytes(B, M, N)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 256)) return MSTF_EALIGN;
     OnepassSide ks = {reinterpret_cast<const _Float16*>(k), kth_k, k_bmp, k_idx, nullptr, nullptr, k_dst_off, k_dst_limit,
-                      reinterpret_cast<char*>(k_nz), ~0ull, nullptr, {nullptr, 0}};
+                      reinterpret_cast<char*>(k_nz), ~0ull, nullptr, {nullptr}};
     OnepassSide vs = {reinterpret_cast<const _Float16*>(v), kth_v, v_bmp, v_idx, nullptr, nullptr, v_dst_off, v_dst_limit,
-                      reinterpret_cast<char*>(v_nz), ~0ull, nullptr, {nullptr, 0}};
+                      reinterpret_cast<char*>(v_nz), ~0ull, nullptr, {nullptr}};
     return launch_onepass_kv(as_stream(stream), ks, vs, B, M, overflow, workspace);
 }

@@ -594,7 +594,8 @@ __device__ __forceinline__ void compact_half(const uint32_t (&r)[64], const uint
 }
 
 // ------------------------------------------------------------------------------- one-pass ordering
-// Status words of the one-pass producers (compress.hip describes the protocol): cleared by onepass_init_kernel or kept clear (Handover),
+// Status words of the one-pass producers (compress.hip describes the protocol): cleared by onepass_init_kernel or kept clear
+// (Handover),
 // one word per workgroup = bit 63 | total, published with an agent-scope store, polled by the workgroups behind.
 constexpr uint32_t kSpinLimit = 1u << 20;  // the default of onepass_spin_limit() (runtime.hip)
 // The limit the launchers pass: kSpinLimit unless mstf_test_set_spin_limit (runtime.hip) lowered it - a test's way
@@ -613,7 +614,7 @@ static __global__ __launch_bounds__(256) void onepass_init_kernel(uint64_t* __re
         if (total2) *total2 = 0ull;
     }
 }
-// The marker of a workgroup whose wait ran out, from one thread: the flag word behind the status words, all ones in
+// The marker of a workgroup whose wait ran out, from one thread: the launch's flag word (Handover), all ones in
 // the caller's total (compress contract) or bit 1 of the caller's sticky flag (append contract).
 constexpr uint32_t kFlagOverflow = 1u, kFlagGaveUp = 2u;
 __device__ __forceinline__ void mark_gave_up(uint64_t* flag_word, uint64_t* total, uint32_t* sticky)
@@ -651,22 +652,28 @@ __device__ __forceinline__ void count_through(uint64_t* counter, bool ok)
 }
 // How the total of a launch is handed over.
 //   landing : the word in pinned host memory, or null
+//   flag    : set by a workgroup whose wait ran out.  The word behind the status words, or, where these are kept, the first of
+//             the caller's words, in the same place for launches of any size and for both sides of a launch: what a launch
+//             that gave up leaves behind are ready words at places that the next one, of another size, takes for its own
+//             totals, flag or counters.
 //   kept    : the status words were zero when the launch began and are left zero, so that no launch clears them in front of
 //             it (a pass: keys and values of 128 heads x 256 tokens 34.4 -> 31.8 us, two 2-bit producers of 64 heads x 4096 100 -> 96.7, two
 //             compressors from the projection, 128 x 4096, 158.6 -> 153.5).  The last workgroup clears them when the others are through,
-//             and writes the total; a wait that ran out leaves the flag word set, and with it the total of this launch and of
-//             every one behind it is all ones until the caller brings cleared words again.
+//             and writes the total; a wait that ran out leaves the flag word set and other words as they are, and the total of
+//             this launch and of every one behind it is all ones until the caller brings cleared words again.
 //   counters: in how many words the workgroups count themselves, a power of two; word i stands kCounterStep words behind word
 //             i - 1, in a cache line of its own.  Adding to one word takes the chip 7 ns each time: 4500 workgroups of one wavefront
 //             (60 heads x 4800 tokens from the projection) took 82 us with one word, 52 without counting.
 constexpr int kCounters = 16, kCounterStep = 16;
+constexpr int kKeptHead = 16;  // kept words: the flag, in a cache line of its own, then the status words of each side
 struct Handover {
     uint64_t* landing;
+    uint64_t* flag;
     int kept;
     int counters;
     __device__ __forceinline__ bool counted() const { return landing != nullptr || kept != 0; }
 };
-// Status words, flag word and counters of a launch of `groups` workgroups.
+// Status words, flag word (unused where the words are kept) and counters of a launch of `groups` workgroups.
 constexpr int status_words(int groups, int counters) { return groups + 2 + (counters - 1) * kCounterStep; }
 // The counters that `room` words leave space for.
 inline int counters_within(size_t room, int groups)
@@ -680,8 +687,8 @@ __device__ __forceinline__ uint64_t* counter_of(const Handover& how, uint64_t* s
     return state + groups + 1 + (g & (how.counters - 1)) * kCounterStep;
 }
 // By the last workgroup of a launch whose workgroups count themselves, all its threads: waits until the others are through and
-// hands the total over, all ones if a wait ran out.  ok: whether its own waits ended.  state: the `groups` status words, the
-// flag word and the counters; total_out: the caller's total (kept).
+// hands the total over, all ones if a wait ran out.  ok: whether its own waits ended.  state: the `groups` status words, a
+// word, and the counters; total_out: the caller's total (kept).
 __device__ __forceinline__ void hand_over(const Handover& how, uint64_t* total_out, uint64_t total, bool ok, uint64_t* state,
                                           int groups, uint32_t spin_limit, uint32_t* room)
 {
@@ -689,16 +696,18 @@ __device__ __forceinline__ void hand_over(const Handover& how, uint64_t* total_o
         const bool reads = (int)threadIdx.x < how.counters;
         const uint64_t* mine = counter_of(how, state, groups, reads ? (int)threadIdx.x : 0);
         auto counted = [&]() { return wave_sum_u64(reads ? agent_load(mine) : 0ull); };
+        // (a flag that is up already, by an earlier launch perhaps: the counters may never come to what they should)
+        const bool flagged = agent_load(how.flag) != 0ull;
         uint64_t through = counted();
         const uint32_t others = (uint32_t)groups - 1u;
-        for (uint32_t polls = 0; (uint32_t)through != others && polls < spin_limit; polls++) {
+        for (uint32_t polls = 0; (uint32_t)through != others && !flagged && polls < spin_limit; polls++) {
             __builtin_amdgcn_s_sleep(1);
             through = counted();
         }
-        const bool all = (uint32_t)through == others;
+        const bool all = (uint32_t)through == others && !flagged;
         if (threadIdx.x == 0) {
-            if (!all && how.kept) agent_store(state + groups, 1ull);  // (words are still in use: they cannot be cleared)
-            ok = ok && through == others && agent_load(state + groups) == 0ull;
+            if (!all && how.kept) agent_store(how.flag, 1ull);  // (words are still in use: they cannot be cleared)
+            ok = ok && all && through == others && agent_load(how.flag) == 0ull;
             const uint64_t v = ok ? total : ~0ull;
             if (how.kept) *total_out = v;
             if (how.landing) __hip_atomic_store(how.landing, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

@@ -411,7 +411,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
             // (the unit's place is the same for the whole wavefront, and so are the addresses made from it)
             before = u64_of(__builtin_amdgcn_readfirstlane((uint32_t)before),
                             __builtin_amdgcn_readfirstlane((uint32_t)(before >> 32)));
-            if (!ok && threadIdx.x == 0) mark_gave_up(state + groups_total, how.kept ? nullptr : total_words, nullptr);
+            if (!ok && threadIdx.x == 0) mark_gave_up(how.flag, how.kept ? nullptr : total_words, nullptr);
             if (how.counted()) {
                 if (g == groups_total - 1)
                     hand_over(how, total_words, before - in_group + group_total, ok, state, groups_total, spin_limit, wave_total);
@@ -486,9 +486,9 @@ static int compress_quant_impl(void* stream, const mstf_half* x, int B, int M, i
         const int units_all = B * nblk;
         const int W = nblk % 4 == 0 ? 4 : (nblk % 2 == 0 ? 2 : 1);
         const int groups = units_all / W;
-        uint64_t* state = status ? status : reinterpret_cast<uint64_t*>(ws);
+        uint64_t* state = status ? status + kKeptHead : reinterpret_cast<uint64_t*>(ws);
         const int counters = status ? kCounters : counters_within(quant_ws_bytes(B, M) / 8, groups);
-        const Handover how = {landing, status != nullptr, counters};
+        const Handover how = {landing, status ? status : state + groups, status != nullptr, counters};
         const int words = status_words(groups, counters);
         const uint32_t spin_limit = onepass_spin_limit();
         if (!status) {

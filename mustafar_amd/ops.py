@@ -63,7 +63,7 @@ class Workspace:
 
 def status_words(units, sides=1):
     """mstf_status_bytes in words, of a producer's call over `units` blocks a side."""
-    return sides * (units + 242)
+    return 16 + sides * (units + 242)
 
 
 _WS = {}
