@@ -148,7 +148,8 @@ int mstf_compress_kv_f16(void* stream, const mstf_half* k, const mstf_half* v, i
                          uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,
                          uint64_t* v_total_halfs, mstf_half* v_nz, uint64_t v_capacity_halfs, void* workspace,
                          size_t workspace_bytes);
-/* The same with a pair of landings (mstf_landing_take; null: none) - keys' total, values' total - and kept status words. */
+/* The same with a pair of landings (mstf_landing_take; null: none) - keys' total, values' total - and kept status words.
+ * Recorded into a graph it uses neither: the launch that clears words in the workspace is part of the graph. */
 int mstf_compress_kv_landing_f16(void* stream, const mstf_half* k, const mstf_half* v, int B, int M, int N, int kth_k, int kth_v,
                                  uint64_t* k_bmp, uint32_t* k_idx, uint32_t* k_nz_off, uint64_t* k_total_halfs, mstf_half* k_nz,
                                  uint64_t k_capacity_halfs, uint64_t* v_bmp, uint32_t* v_idx, uint32_t* v_nz_off,

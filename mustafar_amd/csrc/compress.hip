@@ -1006,10 +1006,12 @@ extern "C" int mstf_compress_kv_landing_f16(void* stream, const mstf_half* k, co
     if (!aligned_to(landings, 8)) return MSTF_EALIGN;
     int rc = status_check(status, status_bytes, B, M, 2);
     if (rc != MSTF_OK) return rc;
-    // a recorded launch would store to the words at every replay, whoever has them by then
+    // a recorded launch would store to the landings at every replay, whoever has them by then, and nobody could bring it
+    // cleared status words behind a replay, or another call, that gave up
     bool recorded = true;
-    if (landings) rc = stream_recorded(as_stream(stream), &recorded);
+    if (landings || status) rc = stream_recorded(as_stream(stream), &recorded);
     if (rc != MSTF_OK) return rc;
+    if (recorded) status = nullptr;
     for (int i = 0; landings && i < 2; i++)
         __atomic_store_n(landings + i, recorded ? MSTF_NOT_LANDED : kLandingEmpty, __ATOMIC_RELEASE);
     uint64_t* l = recorded ? nullptr : reinterpret_cast<uint64_t*>(landings);

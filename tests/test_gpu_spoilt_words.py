@@ -75,3 +75,22 @@ def test_calls_of_other_sizes_behind_a_give_up(spoiling):
                 assert "gave up" in str(e)
         want = cq.convert_value_batched_quant(inputs[3][1], 2, ws=bare, kth=KTH)
         assert all(torch.equal(a, b) for a, b in zip(out, want))
+
+
+@pytest.mark.parametrize("heads,tokens", [(1, 192), (12, 1024), (64, 4800)])
+def test_a_recorded_call_clears_its_own_words(heads, tokens):
+    """Behind a call that gave up over the words of the same Workspace a graph's replays are exact, every one."""
+    from mustafar_amd import ops
+    k, v = kv(heads, tokens, 5)
+    ws = ops.Workspace("cuda", 1 << 22)
+    want = ops.compress_kv(k, v, KTH, 10, ws=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c = ops.compress_kv(k, v, KTH, 10, ws=ws)
+    for _ in range(3):
+        spoil(ws, 60, 4800)
+        for t in c[0].bmp, c[0].idx, c[0].nz, c[1].bmp, c[1].idx, c[1].nz:
+            t.zero_()
+        graph.replay()
+        assert all([exact(g, w) for g, w in zip(c, want)])
