@@ -18,11 +18,11 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, si
     as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host.
     sized: the total as an int instead."""
     own = ops._own_workspace(ws, inputs.device) if sized else None
+    words = own.status(ops.status_words(inputs.shape[0] * (inputs.shape[1] // 64))) if own else None
     out = ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),
-                    int(group_size), room, ops._landing_word()[1] if sized else 0,
-                    own.status(ops.status_words(inputs.shape[0] * (inputs.shape[1] // 64))) if own else None)
+                    int(group_size), room, ops._landing_word()[1] if sized else 0, words)
     if sized and out[-1] < 0:
-        ops.gave_up(own, _GAVE_UP)
+        ops.gave_up(own, words, _GAVE_UP)
     return out
 
 

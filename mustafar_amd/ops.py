@@ -24,6 +24,7 @@ class Workspace:
         self.device = torch.device(device)
         self._bufs = [torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=self.device)]
         self._status = []       # status words of the producers, zero between two calls; the last one is in use
+        self._spoilt = False    # the last one is not zero any more
 
     @property
     def tensor(self):
@@ -46,19 +47,21 @@ class Workspace:
             return self.tensor
         return self.reserve(nbytes)
 
-
     def status(self, words):
-        """`words` kept status words (mstf_status_bytes) for a producer, or None where they would have to be made while the
-        stream is being captured."""
-        if not self._status or self._status[-1].numel() < words:
+        """`words` kept status words (mstf_status_bytes) for a producer on the current stream, or None where they would have
+        to be made while it is being captured."""
+        if self._spoilt or not self._status or self._status[-1].numel() < words:
             if torch.cuda.is_current_stream_capturing():
                 return None
             self._status.append(torch.zeros(max(words, 4096), dtype=torch.int64, device=self.device))
+            self._spoilt = False
         return self._status[-1]
 
-    def status_spoilt(self):
-        """A producer gave up: its status words are not zero any more."""
-        self._status.append(torch.zeros(4096, dtype=torch.int64, device=self.device))
+    def status_spoilt(self, words):
+        """A producer gave up over these words: they are not zero any more.  The next producer makes others, cleared on its own
+        stream, which need not be the one that this is called on."""
+        if self._status and self._status[-1] is words:
+            self._spoilt = True
 
 
 def status_words(units, sides=1):
@@ -98,11 +101,11 @@ def _landing_word():
 
 class _LandingPair:
     """The pinned words that a call which returns without waiting has its two totals stored to (mstf_landing_take)."""
-    __slots__ = ("pair", "stream", "ws", "_give")
+    __slots__ = ("pair", "stream", "ws", "words", "_give")
     NOT_LANDED = -(1 << 63) + 2
 
-    def __init__(self, pair, stream, ws):
-        self.pair, self.stream, self.ws, self._give = pair, stream, ws, lib().mstf_landing_give
+    def __init__(self, pair, stream, ws, words):
+        self.pair, self.stream, self.ws, self.words, self._give = pair, stream, ws, words, lib().mstf_landing_give
 
     def read(self, side):
         """The total, or None where the call was recorded into a graph."""
@@ -160,9 +163,9 @@ def _own_workspace(ws, device):
     return ws if isinstance(ws, Workspace) and ws.device.type == device.type else None
 
 
-def gave_up(ws, what):
+def gave_up(ws, words, what):
     if ws is not None:
-        ws.status_spoilt()
+        ws.status_spoilt(words)
     raise RuntimeError(what)
 
 
@@ -196,7 +199,8 @@ class CompressedKV:
         if n is None:
             n = read_word(self.total_halfs)
         if n < 0 or n > (1 << 62):
-            gave_up(self._landing.ws if self._landing is not None else None, _GAVE_UP)
+            own = self._landing
+            gave_up(own and own.ws, own and own.words, _GAVE_UP)
         return n
 
     def packed(self):
@@ -262,10 +266,10 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     the device.  Returns (CompressedKV of the keys, CompressedKV of the values)."""
     pair = lib().mstf_landing_take()
     own = _own_workspace(ws, k.device) if pair else None
-    landing = _LandingPair(pair, _stream(), own) if pair else None
+    words = own.status(status_words(k.shape[0] * (k.shape[1] // 64), 2)) if own else None
+    landing = _LandingPair(pair, _stream(), own, words) if pair else None
     kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
-                                                   -1 if capacity_halfs is None else int(capacity_halfs), pair or 0,
-                                                   own.status(status_words(k.shape[0] * (k.shape[1] // 64), 2)) if own else None)
+                                                   -1 if capacity_halfs is None else int(capacity_halfs), pair or 0, words)
     M, N = k.shape[1:]
     return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
@@ -301,14 +305,14 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
         rot = x
     sized = capacity_halfs is None and M != 0
     own = _own_workspace(ws, x.device) if sized else None
+    words = own.status(status_words(x.shape[0] * x.shape[2] * (M // 64))) if own else None
     bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
                                            rot, -1 if capacity_halfs is None else int(capacity_halfs),
-                                           _landing_word()[1] if sized else 0,
-                                           own.status(status_words(x.shape[0] * x.shape[2] * (M // 64))) if own else None)
+                                           _landing_word()[1] if sized else 0, words)
     if M == 0:
         return None, rot
     if sized and n < 0:
-        gave_up(own, _GAVE_UP)
+        gave_up(own, words, _GAVE_UP)
     return CompressedKV(bmp, idx, nz, nz_off, M, x.shape[3], is_value, n if sized else total), rot
 
 

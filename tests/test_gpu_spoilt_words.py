@@ -94,3 +94,26 @@ def test_a_recorded_call_clears_its_own_words(heads, tokens):
             t.zero_()
         graph.replay()
         assert all([exact(g, w) for g, w in zip(c, want)])
+
+
+def test_cleared_words_come_on_the_stream_that_uses_them():
+    """The read that finds a give-up may be made on another, busy stream: the next call does not wait for that one."""
+    from mustafar_amd import ops
+    k, v = kv(12, 1024, 6)
+    ws = ops.Workspace("cuda", 1 << 22)
+    want = ops.compress_kv(k, v, KTH, 10, ws=torch.empty(1 << 22, dtype=torch.uint8, device="cuda"))
+    spoil(ws, 60, 4800)
+    c = ops.compress_kv(k, v, KTH, 10, ws=ws)
+    torch.cuda.synchronize()
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(other):
+        # what such words hold in front of their clearing: the ready mark and a total
+        used = [torch.full((4096,), -(1 << 63) + 64, dtype=torch.int64, device="cuda") for _ in range(8)]
+        torch.cuda.synchronize()
+        del used
+        torch.cuda._sleep(int(2e8))
+        with pytest.raises(RuntimeError, match="gave up"):
+            c[0].packed()
+    got = ops.compress_kv(k, v, KTH, 10, ws=ws)
+    assert all([exact(g, w) for g, w in zip(got, want)])
+    torch.cuda.synchronize()
