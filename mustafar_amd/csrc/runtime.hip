@@ -157,7 +157,8 @@ extern "C" int mstf_landing_wait(void* stream, const int64_t* landing, int64_t* 
 // ------------------------------------------------------------------ landings of calls that are not waited for
 // Pairs of words in one block of pinned memory, made with the first of them and kept: 1024 pairs, so that a program that holds
 // on to more results than that finds none free and reads its totals by mstf_read_word.  A pair that is given back while its
-// kernel has yet to store to it stays away from the others until it has.
+// kernel has yet to store to it stays away from the others until it has.  The first call may be one that is being recorded: the
+// allocation is no part of what is recorded, and a failure leaves no error for the launch behind it to find.
 namespace mstf {
 static std::mutex g_landing_lock;
 static int64_t* g_landing_block = nullptr;
@@ -172,9 +173,16 @@ extern "C" int64_t* mstf_landing_take(void)
     using namespace mstf;
     std::lock_guard<std::mutex> hold(g_landing_lock);
     if (!g_landing_block) {
+        if (g_landing_failed) return nullptr;
         void* p = nullptr;
-        if (g_landing_failed || hipHostMalloc(&p, kLandingPairs * 2 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
-            g_landing_failed = true;
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (of this thread, for this call alone)
+        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        const hipError_t e = hipHostMalloc(&p, kLandingPairs * 2 * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped);
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            // (refused because of a capture somewhere: asked again by the next call)
+            g_landing_failed = e != hipErrorStreamCaptureUnsupported && e != hipErrorStreamCaptureImplicit;
             return nullptr;
         }
         g_landing_block = static_cast<int64_t*>(p);
