@@ -61,7 +61,8 @@ int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* 
 /* Totals that a producer's kernel stores to pinned host memory itself, before its values are all out (the calls ..._sized and
  * ..._landing_f16 below): known on the host without a launch behind the kernel and a wait for its end.
  * mstf_landing_take: a pair of such words for a call that returns without waiting; null when none is free (the caller then
- * uses the call without landings).  mstf_landing_give hands it back, at any time, from any thread.
+ * uses the call without landings).  mstf_landing_give hands it back, at any time, from any thread; what is no pair, or not out,
+ * is left alone.
  * mstf_landing_wait: waits for a word's value; MSTF_NOT_LANDED: the call was recorded into a graph or refused, and the total is
  * in device memory only.  All ones: a workgroup gave up waiting. */
 #define MSTF_NOT_LANDED (INT64_MIN + 2)

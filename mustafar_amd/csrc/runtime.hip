@@ -165,6 +165,7 @@ static int64_t* g_landing_block = nullptr;
 static bool g_landing_failed = false;
 constexpr int kLandingPairs = 1024;
 static uint16_t g_landing_free[kLandingPairs];  // a ring: the one that was given back first is the first to be taken
+static bool g_landing_taken[kLandingPairs];
 static int g_landing_head = 0, g_landing_count = 0;
 }  // namespace mstf
 
@@ -193,11 +194,13 @@ extern "C" int64_t* mstf_landing_take(void)
         g_landing_count = kLandingPairs;
     }
     if (g_landing_count == 0) return nullptr;
-    int64_t* pair = g_landing_block + 2 * g_landing_free[g_landing_head];
+    const uint16_t at = g_landing_free[g_landing_head];
+    int64_t* pair = g_landing_block + 2 * at;
     for (int i = 0; i < 2; i++)
         if (__atomic_load_n(pair + i, __ATOMIC_ACQUIRE) == kLandingEmpty) return nullptr;  // (and those behind it are younger)
     g_landing_head = (g_landing_head + 1) % kLandingPairs;
     g_landing_count--;
+    g_landing_taken[at] = true;
     return pair;
 }
 
@@ -206,6 +209,9 @@ extern "C" void mstf_landing_give(int64_t* pair)
     using namespace mstf;
     std::lock_guard<std::mutex> hold(g_landing_lock);
     if (!pair || !g_landing_block || pair < g_landing_block || pair >= g_landing_block + 2 * kLandingPairs) return;
-    g_landing_free[(g_landing_head + g_landing_count) % kLandingPairs] = (uint16_t)((pair - g_landing_block) / 2);
+    const uint16_t at = (uint16_t)((pair - g_landing_block) / 2);
+    if (pair != g_landing_block + 2 * at || !g_landing_taken[at]) return;  // no pair, or not out
+    g_landing_taken[at] = false;
+    g_landing_free[(g_landing_head + g_landing_count) % kLandingPairs] = at;
     g_landing_count++;
 }

@@ -6,6 +6,7 @@ packed size when the caller did not provide a capacity.
 import ctypes
 import math
 import threading
+import weakref
 
 import torch
 
@@ -105,13 +106,19 @@ class _LandingPair:
     NOT_LANDED = -(1 << 63) + 2
 
     def __init__(self, pair, stream, ws, words):
-        self.pair, self.stream, self.ws, self.words, self._give = pair, stream, ws, words, lib().mstf_landing_give
+        self.pair, self.stream, self._give = pair, stream, lib().mstf_landing_give
+        self.ws, self.words = ws and weakref.ref(ws), words
 
     def read(self, side):
         """The total, or None where the call was recorded into a graph."""
-        own = _landing_word()
-        check(lib().mstf_landing_wait(self.stream, self.pair + 8 * side, own[3]), "mstf_landing_wait")
-        return None if own[2].value == self.NOT_LANDED else own[2].value
+        value = ctypes.c_int64()
+        check(lib().mstf_landing_wait(self.stream, self.pair + 8 * side, ctypes.addressof(value)), "mstf_landing_wait")
+        return None if value.value == self.NOT_LANDED else value.value
+
+    def spoilt(self):
+        ws = self.ws and self.ws()
+        if ws is not None:
+            ws.status_spoilt(self.words)
 
     def __del__(self):
         self._give(self.pair)
@@ -182,11 +189,18 @@ class CompressedKV:
 
     bmp int64 [B, T], idx int32 [B, T+1], nz fp16 flat, nz_off int32 [B] (16-byte units)."""
 
+    _landing = None     # _LandingPair that gets the total too; given back once the total is read
+    _used = None        # the total, from there
+
     def __init__(self, bmp, idx, nz, nz_off, tokens, head_dim, is_value, total_halfs=None, landing=None):
         self.bmp, self.idx, self.nz, self.nz_off = bmp, idx, nz, nz_off
         self.tokens, self.head_dim, self.is_value = tokens, head_dim, is_value
         self.total_halfs = total_halfs
-        self._landing = landing     # _LandingPair that gets the total too
+        self._landing = landing
+
+    def __getstate__(self):
+        # a copy has the total from its own tensor (total_halfs): the words that it landed in go with the call
+        return {name: value for name, value in self.__dict__.items() if name != "_landing"}
 
     @property
     def heads(self):
@@ -195,12 +209,20 @@ class CompressedKV:
     def used_halfs(self):
         """Number of fp16 values in use (reads the device-side total once).  The one-pass compressor reports a wait that
         ran out - which the dispatch order rules out - as a total of all ones: that raises here."""
-        n = self._landing.read(int(self.is_value)) if self._landing is not None else None
-        if n is None:
+        if self._used is not None:
+            return self._used
+        landing = self._landing
+        n = landing.read(int(self.is_value)) if landing is not None else None
+        landed = n is not None
+        if not landed:
             n = read_word(self.total_halfs)
         if n < 0 or n > (1 << 62):
-            own = self._landing
-            gave_up(own and own.ws, own and own.words, _GAVE_UP)
+            if landed:
+                landing.spoilt()
+            raise RuntimeError(_GAVE_UP)
+        self._landing = None
+        if landed:
+            self._used = n
         return n
 
     def packed(self):

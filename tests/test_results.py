@@ -1,0 +1,103 @@
+"""Results of the producers as objects: copied, saved, and done with the words that their totals landed in (ops.CompressedKV)."""
+import copy
+import ctypes
+import gc
+import io
+import pickle
+import weakref
+
+import pytest
+import torch
+
+
+def landed(total, ws=None, words=None):
+    """A result of values whose total landed in two words, and the words."""
+    from mustafar_amd import ops
+    pair = (ctypes.c_int64 * 2)(7, total)
+    landing = ops._LandingPair(ctypes.addressof(pair), 0, ws, words)
+    c = ops.CompressedKV(torch.arange(2).view(1, 2), torch.tensor([[0, 1, 2]], dtype=torch.int32), torch.ones(16, dtype=torch.float16),
+                         torch.zeros(1, dtype=torch.int32), 64, 128, True, torch.tensor([max(total, -1)]), landing)
+    return c, pair
+
+
+@pytest.mark.parametrize("read_first", [False, True])
+def test_results_are_copied_and_saved(read_first):
+    c, pair = landed(8)
+    if read_first:
+        assert c.used_halfs() == 8
+    file = io.BytesIO()
+    torch.save(c, file)
+    file.seek(0)
+    for other in (copy.copy(c), copy.deepcopy(c), pickle.loads(pickle.dumps(c)), torch.load(file, weights_only=False)):
+        assert torch.equal(other.bmp, c.bmp) and torch.equal(other.nz, c.nz) and other.is_value and other.tokens == 64
+        assert other.used_halfs() == 8 and other.packed().numel() == 8 and other.nbytes() == c.nbytes()
+    assert c.used_halfs() == 8
+
+
+def test_a_result_saved_without_the_attribute():
+    from mustafar_amd import ops
+    c = ops.CompressedKV.__new__(ops.CompressedKV)
+    c.__dict__.update(bmp=None, idx=None, nz=torch.ones(8), nz_off=None, tokens=64, head_dim=128, is_value=False,
+                      total_halfs=torch.tensor([4]))
+    assert c.used_halfs() == 4
+
+
+def test_a_known_total_gives_the_words_back_and_holds_no_workspace():
+    from mustafar_amd import ops
+    ws = ops.Workspace("cpu", 256)
+    ws._status.append(torch.zeros(8, dtype=torch.int64))
+    c, pair = landed(8, ws, ws._status[-1])
+    landing, alive = c._landing, weakref.ref(ws)
+    given = []
+    landing._give = given.append
+    del landing
+    assert c.used_halfs() == 8 and given == [ctypes.addressof(pair)]
+    pair[1] = 5                                     # another call's by now
+    assert c.used_halfs() == 8
+    c, pair = landed(8, ws, ws._status[-1])
+    del ws
+    gc.collect()
+    assert alive() is None and c.used_halfs() == 8
+
+
+def test_a_give_up_marks_the_words_that_the_call_had():
+    from mustafar_amd import ops
+    ws = ops.Workspace("cpu", 256)
+    ws._status.append(torch.zeros(8, dtype=torch.int64))
+    c, pair = landed(-1, ws, ws._status[-1])
+    old, pair2 = landed(-1, ws, torch.zeros(8, dtype=torch.int64))
+    for bad, spoils in ((old, False), (c, True)):
+        with pytest.raises(RuntimeError, match="gave up"):
+            bad.packed()
+        assert ws._spoilt == spoils
+
+
+@pytest.mark.gpu
+def test_a_pair_is_given_back_once():
+    from mustafar_amd._lib import lib
+    L = lib()
+    pair = L.mstf_landing_take()
+    for p in (pair, pair, pair + 8, pair + 4):      # twice, and what is no pair
+        L.mstf_landing_give(p)
+    held = []
+    while True:
+        p = L.mstf_landing_take()
+        if not p:
+            break
+        held.append(p)
+        assert len(held) <= 1024
+    assert len(set(held)) == len(held) and pair in held
+    for p in held:
+        L.mstf_landing_give(p)
+
+
+@pytest.mark.gpu
+def test_more_results_than_pairs():
+    from mustafar_amd import ops
+    x = torch.randn((1, 64, 128), device="cuda", dtype=torch.float16)
+    results = []
+    for _ in range(1100):
+        c = ops.compress_kv(x, x, 89, 89, capacity_halfs=4096)
+        assert c[0]._landing is not None
+        assert all(side.used_halfs() == int(side.total_halfs) for side in c)    # (keys' and values' tiles are padded each on their own)
+        results.append(c)
