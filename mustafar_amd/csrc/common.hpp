@@ -114,10 +114,12 @@ inline int check_launch()
 }
 
 // A call's word in pinned host memory (runtime.hip).  ready: the word is told apart from every result, unless the stream is
-// being captured, which is refused (a recorded kernel would store to it at every replay).  wait: watches it, then the stream.
+// being captured, which is refused (a recorded kernel would store to it at every replay).  wait: watches it, then the stream;
+// for a total (no total is the word of landing_ready) it is an error if the stream is done and nothing has come.
 constexpr int64_t kLandingEmpty = INT64_MIN + 1;
 int landing_ready(hipStream_t st, int64_t* landing, const int64_t* value);
 int landing_wait(hipStream_t st, const int64_t* landing, int64_t* value);
+int total_wait(hipStream_t st, const int64_t* landing, int64_t* value);
 int stream_recorded(hipStream_t st, bool* recorded);
 // Kept status words of a producer (mstf_status_bytes; null: none), compress.hip.
 int status_check(const uint64_t* status, size_t bytes, int64_t B, int M, int sides);

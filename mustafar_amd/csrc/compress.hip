@@ -937,7 +937,7 @@ extern "C" int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source
     if (rc != MSTF_OK) return rc;
     rc = proj_impl(stream, src, is_value, M, N, kth, bmp, idx, nz_off, total_halfs, nullptr, nullptr, nz, nz_capacity_halfs,
                    nullptr, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing), status);
-    return rc != MSTF_OK ? rc : landing_wait(as_stream(stream), landing, value);
+    return rc != MSTF_OK ? rc : total_wait(as_stream(stream), landing, value);
 }
 
 extern "C" int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,

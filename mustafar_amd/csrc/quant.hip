@@ -594,5 +594,5 @@ extern "C" int mstf_compress_quant_sized(void* stream, const mstf_half* x, int i
     rc = (is_value ? compress_quant_group<true> : compress_quant_group<false>)(
         group_size, stream, x, B, M, N, kth, bit, bmp, tile_off, counts, units, scales, zeros, total_words, packed,
         packed_capacity_words, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing), status);
-    return rc != MSTF_OK ? rc : landing_wait(st, landing, value);
+    return rc != MSTF_OK ? rc : total_wait(st, landing, value);
 }

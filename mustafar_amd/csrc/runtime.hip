@@ -135,6 +135,14 @@ int mstf::landing_wait(hipStream_t st, const int64_t* landing, int64_t* value)
     return MSTF_OK;
 }
 
+int mstf::total_wait(hipStream_t st, const int64_t* landing, int64_t* value)
+{
+    const int rc = landing_wait(st, landing, value);
+    if (rc != MSTF_OK || *value != kLandingEmpty) return rc;
+    set_last_hip_error((int)hipErrorNotReady);  // the stream is done and nothing has come
+    return MSTF_ELAUNCH;
+}
+
 extern "C" int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* value)
 {
     if (!src || !landing || !value) return MSTF_EINVAL;
@@ -151,7 +159,7 @@ extern "C" int mstf_landing_wait(void* stream, const int64_t* landing, int64_t* 
 {
     if (!landing || !value) return MSTF_EINVAL;
     if (!mstf::aligned_to(landing, 8)) return MSTF_EALIGN;
-    return mstf::landing_wait(mstf::as_stream(stream), landing, value);
+    return mstf::total_wait(mstf::as_stream(stream), landing, value);
 }
 
 // ------------------------------------------------------------------ landings of calls that are not waited for

@@ -102,18 +102,23 @@ def _landing_word():
 
 class _LandingPair:
     """The pinned words that a call which returns without waiting has its two totals stored to (mstf_landing_take)."""
-    __slots__ = ("pair", "stream", "ws", "words", "_give")
-    NOT_LANDED = -(1 << 63) + 2
+    __slots__ = ("pair", "stream", "device", "ws", "words", "_give")
+    EMPTY, NOT_LANDED = -(1 << 63) + 1, -(1 << 63) + 2
 
-    def __init__(self, pair, stream, ws, words):
-        self.pair, self.stream, self._give = pair, stream, lib().mstf_landing_give
+    def __init__(self, pair, stream, ws, words, device=None):
+        """device: the one that was current at the call, which `stream` is a handle of."""
+        self.pair, self.stream, self.device, self._give = pair, stream, device, lib().mstf_landing_give
         self.ws, self.words = ws and weakref.ref(ws), words
 
     def read(self, side):
         """The total, or None where the call was recorded into a graph."""
-        value = ctypes.c_int64()
-        check(lib().mstf_landing_wait(self.stream, self.pair + 8 * side, ctypes.addressof(value)), "mstf_landing_wait")
-        return None if value.value == self.NOT_LANDED else value.value
+        value = ctypes.c_int64.from_address(self.pair + 8 * side).value
+        if value == self.EMPTY:
+            own = ctypes.c_int64()
+            with torch.cuda.device(self.device):    # (a default stream's handle is the same on every device)
+                check(lib().mstf_landing_wait(self.stream, self.pair + 8 * side, ctypes.addressof(own)), "mstf_landing_wait")
+            value = own.value
+        return None if value == self.NOT_LANDED else value
 
     def spoilt(self):
         ws = self.ws and self.ws()
@@ -161,7 +166,10 @@ def _call(fn, ws, device, call, *args):
 
 
 def _own_workspace(ws, device):
-    """The Workspace that keeps a producer's status words, None where the caller brought a bare buffer."""
+    """The Workspace that keeps a producer's status words, None where the caller brought a bare buffer or tensors of another
+    device than the current one, on whose stream the words are cleared and the launch goes."""
+    if device.type == "cuda" and device.index != torch._C._cuda_getDevice():
+        return None
     if ws is None and device.type == "cuda":
         key = (device.type, device.index, _stream())
         ws = _WS.get(key)
@@ -289,7 +297,7 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     pair = lib().mstf_landing_take()
     own = _own_workspace(ws, k.device) if pair else None
     words = own.status(status_words(k.shape[0] * (k.shape[1] // 64), 2)) if own else None
-    landing = _LandingPair(pair, _stream(), own, words) if pair else None
+    landing = _LandingPair(pair, _stream(), own, words, torch._C._cuda_getDevice()) if pair else None
     kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
                                                    -1 if capacity_halfs is None else int(capacity_halfs), pair or 0, words)
     M, N = k.shape[1:]

@@ -72,6 +72,53 @@ def test_a_give_up_marks_the_words_that_the_call_had():
         assert ws._spoilt == spoils
 
 
+def test_a_total_is_waited_for_on_the_device_of_its_call(monkeypatch):
+    from mustafar_amd import ops
+    c, pair = landed(8)
+    c._landing.device, current = 3, [0]
+
+    class Device:
+        def __init__(self, index):
+            self.index = index
+
+        def __enter__(self):
+            current.append(self.index)
+
+        def __exit__(self, *e):
+            current.pop()
+
+    class Library:
+        def mstf_landing_wait(self, stream, word, value):
+            assert current[-1] == 3 and word == ctypes.addressof(pair) + 8
+            ctypes.c_int64.from_address(value).value = 8
+            return 0
+
+    pair[1] = ops._LandingPair.EMPTY
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(ops, "lib", Library)
+    assert c.used_halfs() == 8 and current == [0]
+
+
+def test_status_words_stay_with_the_current_device(monkeypatch):
+    from mustafar_amd import ops
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    ws = ops.Workspace("cpu", 256)
+    monkeypatch.setattr(ws, "device", torch.device("cuda", 1))
+    assert ops._own_workspace(ws, torch.device("cuda", 1)) is None
+    assert ops._own_workspace(ws, torch.device("cuda", 0)) is ws
+
+
+@pytest.mark.gpu
+def test_a_word_that_never_comes_is_an_error():
+    from mustafar_amd import ops
+    from mustafar_amd._lib import lib
+    word, value = torch.empty(1, dtype=torch.int64, pin_memory=True), ctypes.c_int64()
+    word[0] = ops._LandingPair.EMPTY
+    assert lib().mstf_landing_wait(ops._stream(), word.data_ptr(), ctypes.addressof(value)) == -5
+    word[0] = 6
+    assert lib().mstf_landing_wait(ops._stream(), word.data_ptr(), ctypes.addressof(value)) == 0 and value.value == 6
+
+
 @pytest.mark.gpu
 def test_a_pair_is_given_back_once():
     from mustafar_amd._lib import lib
