@@ -257,13 +257,13 @@ __global__ __launch_bounds__(decode_waves(SHARE, WHOLE) * 64) __attribute__((amd
                 constexpr int wo = woff + g * 16;
                 u32x16_t nxt;
                 if constexpr (g1 < kSideBatches)
-                    rank_batch<NM, true, g, g1 * 64, wo>(cur, nxt, bmK, at, wbase, wbase + wgroup, acc);
+                    rank_batch<NM, true, g, g1 * 64, 0, 0, wo>(cur, nxt, bmK, at, wbase, wbase + wgroup, acc);
                 else if constexpr (g1 < 2 * kSideBatches)
-                    rank_batch<NM, true, g, (g1 - kSideBatches) * 64, wo>(cur, nxt, bmV, at, wbase, wbase + wgroup, acc);
+                    rank_batch<NM, true, g, (g1 - kSideBatches) * 64, 0, 0, wo>(cur, nxt, bmV, at, wbase, wbase + wgroup, acc);
                 else if constexpr (MULTI)
-                    rank_batch<NM, true, g, 0, wo>(cur, nxt, bmK + adv, at, wbase, wbase + wgroup, acc);
+                    rank_batch<NM, true, g, 0, 0, 0, wo>(cur, nxt, bmK + adv, at, wbase, wbase + wgroup, acc);
                 else
-                    rank_batch<NM, false, g, 0, wo>(cur, nxt, bmK, at, wbase, wbase + wgroup, acc);
+                    rank_batch<NM, false, g, 0, 0, 0, wo>(cur, nxt, bmK, at, wbase, wbase + wgroup, acc);
                 cur = nxt;
             });
         };

@@ -176,7 +176,7 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
             return *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(bm + t) + touch8);
         };
 
-        const StageRank<4 * NM> rank(lbase, lane);
+        const StageRank<4 * NM, false> rank(lbase, lane);
 
         // the query rows of this KV head: groups x D fp16, contiguous (STEP: rotated out of the projection output)
         if constexpr (STEP) {
@@ -195,7 +195,7 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
         }
         uint2 touch = issue(0);
 
-        typename StageRank<4 * NM>::Sums sums;  // of the phase (keys, one half of the values, the other half)
+        typename StageRank<4 * NM, false>::Sums sums;  // of the phase (keys, one half of the values, the other half)
         const uint32_t qrow = sums.waddr(lds_addr(ql), kQRow, lane);
         const uint32_t prow = sums.waddr(lds_addr(pl), kPRow, lane);
 

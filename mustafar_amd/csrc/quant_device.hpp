@@ -334,11 +334,15 @@ __device__ __forceinline__ i32x16_t image_base(uint32_t img)
     return __builtin_bit_cast(i32x16_t, b);
 }
 
-// How the 32 tiles of a dequantised stage are expanded: a whole tile per LDS read for up to eight weight rows
-// (rank_whole.hpp), half of two tiles for more (rank_device.hpp).  bits: bitmap of tile lane & 31; w, wgroup: see RowSums.
+// How the 32 tiles of a dequantised stage are expanded: half of two tiles per LDS read (HALVES, rank_device.hpp), as for more
+// than eight weight rows always, or a whole tile (rank_whole.hpp).  bits: bitmap of tile lane & 31; w, wgroup: see RowSums.
+// With whole tiles a batch has fewer scalar instructions but twice as many reads of weights: less where the scalar unit's share
+// is on the way of the vector unit's, as in the fused kernels, more where a wavefront waits for its own reads, as in the key
+// products (us, 70 %, halves / whole: 256 heads x 4096 tokens, keys, 2 bits, four rows 32.6 / 33.3, eight 33.6 / 37.5; 4 bits 33.5
+// / 34.5, 35.6 / 39.5; 32 x 1024, 4 bits, eight rows 7.61 / 8.15).  The value products: value_whole (quant_spmv.hip).
 // The bitmaps of the first batch are requested behind the products and arrive while those run (nothing scalar is
 // carried across the lane-dependent branches of the dequantisation in front), the others one batch ahead.
-template <int NW, bool WIDE = wide_rows(NW)>
+template <int NW, bool HALVES>
 struct StageRank;
 template <int NW>
 struct StageRank<NW, true> {

@@ -35,16 +35,16 @@ struct QCache {
 
 // Walks `nsubs` stages of 32 tiles with a two-deep pipeline (see walk_subs).  Tile indices are global
 // (KV head included): tile_off / scales / zeros / bmp are flat over [Bkv, T].
-template <bool SHARED, int BIT, bool G32, int NW, class TileOf, class StageW, class WAddrOf>
+template <bool SHARED, int BIT, bool G32, class Rank, class TileOf, class StageW, class WAddrOf>
 __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW stage_w, WAddrOf waddr_of, uint32_t wgroup,
-                                            const QCache& c, char* my, int lane, int mode, typename StageRank<NW>::Sums& sums)
+                                            const QCache& c, char* my, int lane, int mode, typename Rank::Sums& sums)
 {
     using F = QFmt<BIT>;
     if (nsubs <= 0) return;
     const uint32_t lbase = lds_addr(my);
     char* wordbuf = my + kImgBytes;
     char* metabuf = wordbuf + 2 * F::kWordBuf;
-    const StageRank<NW> rank(lbase, lane);
+    const Rank rank(lbase, lane);
 
     // words of the stage starting at tile t: [tile_off[t], tile_off[t + 31] + words of tile t + 31)
     auto bounds = [&](size_t t, uint32_t& s, uint32_t& e) {
@@ -127,8 +127,8 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
 template <int NW, int BIT, bool G32>
 constexpr int key_quant_lds()
 {
-    constexpr int rows = StageRank<NW>::Sums::kRows * 128 * 2;
-    return 4 * q_lds_bytes<BIT, G32>() + (StageRank<NW>::Sums::kWide ? rows : 4 * rows);
+    constexpr int rows = RowSums<NW>::kRows * 128 * 2;
+    return 4 * q_lds_bytes<BIT, G32>() + (RowSums<NW>::kWide ? rows : 4 * rows);
 }
 template <int NW, int BIT, bool G32, bool SHARE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_waves(key_quant_lds<NW, BIT, G32>(), 4)))) void key_spmv_quant_kernel(
@@ -136,7 +136,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
     const uint32_t* tile_off_dma, const uint16_t* scales, const uint16_t* zeros, const _Float16* Bm,
     _Float16* __restrict__ C, int Lc, int D, int nblk, int ntasks, int rows_per_kv, int row0, int mode)
 {
-    using Sums = typename StageRank<NW>::Sums;
+    using Rank = StageRank<NW, true>;
+    using Sums = typename Rank::Sums;
     constexpr bool kShared = Sums::kWide;
     constexpr int kMaxD = 128;
     constexpr int kQ = q_lds_bytes<BIT, G32>();
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
         __syncthreads();
         return;
     }
-    walk_subs_q<kShared, BIT, G32, NW>(
+    walk_subs_q<kShared, BIT, G32, Rank>(
         SHARE ? 1 : D / kSubTiles, [=](int n) { return tile0 + (size_t)n * kSubTiles; }, stage_rows,
         [=](int n) { return Sums::advance(wrow, (uint32_t)(first + n) * kSubTiles * 2u); }, (uint32_t)D * 8u, c, my, lane, mode, sums);
     _Float16* out = C + ((size_t)kv * rows_per_kv + row0) * Lc + (size_t)tb * 64;
@@ -199,17 +200,19 @@ template <int NW, int BIT, bool G32>
 constexpr int value_quant_wave_lds()
 {
     // the rows start at a multiple of their length (64 bytes); the per-wave sums are parked in the room at the end
-    constexpr int need = ((q_lds_bytes<BIT, G32>() + 63) & ~63) + 2 * StageRank<NW>::Sums::kRows * kSubTiles * 2;
+    constexpr int need = ((q_lds_bytes<BIT, G32>() + 63) & ~63) + 2 * RowSums<NW>::kRows * kSubTiles * 2;
     return need > NW * 256 ? need : NW * 256;
 }
-template <int NW, int WAVES, int BIT, bool G32>
+template <int NW, int WAVES, int BIT, bool G32, bool WHOLE>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resident_waves(WAVES * value_quant_wave_lds<NW, BIT, G32>(), WAVES)))) void value_spmv_quant_kernel(
     const uint64_t* __restrict__ bmp, const uint32_t* packed, const uint32_t* __restrict__ tile_off,
     const uint32_t* tile_off_dma, const uint16_t* scales, const uint16_t* zeros, const _Float16* P,
     _Float16* __restrict__ C, float* __restrict__ part, int Lc, int D, int nblk, int nbpw, int nsplit, int rows_per_kv,
     int row0, int mode, int nwg, uint32_t per_split)
 {
-    using Sums = typename StageRank<NW>::Sums;
+    using Rank = StageRank<NW, !WHOLE>;
+    using Sums = typename Rank::Sums;
+    static_assert(Sums::kRows == RowSums<NW>::kRows, "LDS of a wavefront");
     constexpr int kWRow = kSubTiles * 2;
     constexpr int kWBuf = Sums::kRows * kWRow;
     constexpr int kQ = (q_lds_bytes<BIT, G32>() + 63) & ~63;
@@ -237,7 +240,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     constexpr int subs_per_blk = 64 / kSubTiles;
     const uint32_t wrow = Sums::waddr(lds_addr(wl), kWRow, lane);
     const size_t thead = (size_t)kv * T + (size_t)half * 64;
-    walk_subs_q<false, BIT, G32, NW>(
+    walk_subs_q<false, BIT, G32, Rank>(
         (last - first) * subs_per_blk,
         [=](int n) { return thead + (size_t)(first + n / subs_per_blk) * D + (size_t)(n % subs_per_blk) * kSubTiles; },
         [=](int n) {
@@ -341,19 +344,28 @@ static void launch_key_q_bit(int bit, hipStream_t st, const QArgs& a, const _Flo
         launch_key_q<NW, 8>(st, a, Bm, C, Lc, D, Bkv, rows_per_kv, row0);
 }
 
+// Whether a value product of up to eight rows reads whole tiles (StageRank): with more blocks of all heads than this there is more
+// than one to a wavefront all over the chip.  70 %, heads x blocks, whole / halves, over rows 1, 4 and 8, 2, 4 and 8 bits, one
+// group per tile or two: 256 x 64 0.96 - 1.00 (4 bits, four rows 29.4 -> 28.3 us), 64 x 256 0.96 - 1.01, 40 x 256 0.97 - 1.01; but
+// 128 x 64 0.98 - 1.05, 256 x 32 0.99 - 1.06, 32 x 256 0.98 - 1.05, 256 x 16 0.99 - 1.07, 32 x 16 1.00 - 1.04.
+static bool value_whole(int nw, int nblk, int Bkv) { return !wide_rows(nw) && (long long)Bkv * nblk > 8192; }
 template <int NW, int WAVES, int BIT>
 static void launch_value_q(hipStream_t st, const ValuePlan& pl, const QArgs& a, const _Float16* P, _Float16* C,
                            float* part, int Lc, int D, int Bkv, int rows_per_kv, int row0)
 {
     const int nwg = pl.nsplit * (D / 64) * Bkv;
-    if (a.group_size == 32)
-        hipLaunchKernelGGL((value_spmv_quant_kernel<NW, WAVES, BIT, true>), dim3(xcd_grid(nwg)), dim3(WAVES * 64), 0,
-                           st, a.bmp, a.packed, a.tile_off, a.tile_off, a.scales, a.zeros, P, C, part, Lc, D, Lc / 64,
-                           pl.nbpw, pl.nsplit, rows_per_kv, row0, a.mode, nwg, split_inverse(pl.nsplit));
-    else
-        hipLaunchKernelGGL((value_spmv_quant_kernel<NW, WAVES, BIT, false>), dim3(xcd_grid(nwg)), dim3(WAVES * 64), 0,
-                           st, a.bmp, a.packed, a.tile_off, a.tile_off, a.scales, a.zeros, P, C, part, Lc, D, Lc / 64,
-                           pl.nbpw, pl.nsplit, rows_per_kv, row0, a.mode, nwg, split_inverse(pl.nsplit));
+    const bool whole = value_whole(NW, Lc / 64, Bkv);
+#define MSTF_VQ_LAUNCH(G32, WHOLE)                                                                                           \
+    hipLaunchKernelGGL((value_spmv_quant_kernel<NW, WAVES, BIT, G32, WHOLE>), dim3(xcd_grid(nwg)), dim3(WAVES * 64), 0, st, \
+                       a.bmp, a.packed, a.tile_off, a.tile_off, a.scales, a.zeros, P, C, part, Lc, D, Lc / 64, pl.nbpw,       \
+                       pl.nsplit, rows_per_kv, row0, a.mode, nwg, split_inverse(pl.nsplit))
+    constexpr bool kWhole = !wide_rows(NW);
+    if (a.group_size == 32) {
+        if (whole) MSTF_VQ_LAUNCH(true, kWhole); else MSTF_VQ_LAUNCH(true, false);
+    } else {
+        if (whole) MSTF_VQ_LAUNCH(false, kWhole); else MSTF_VQ_LAUNCH(false, false);
+    }
+#undef MSTF_VQ_LAUNCH
 }
 template <int NW, int WAVES>
 static void launch_value_q_bit(int bit, hipStream_t st, const ValuePlan& pl, const QArgs& a, const _Float16* P,

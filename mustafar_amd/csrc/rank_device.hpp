@@ -172,16 +172,16 @@ __device__ __forceinline__ RankTable rank_table(const char* room, int lane)
 // packs - and an infinite weight makes a NaN of a tile's neighbour as it does of an absent element, 0 x inf.  Eight: the
 // pairs are merged first, two vector instructions for two products less; only absent elements meet a zero then.
 //   mv      : the batch's eight bitmaps;  PREFETCH: those of the coming batch are requested at nbm + BOFF bytes
+//   I0, IS  : immediate offset of the batch's first tile and bytes between two tiles (0, 0: `a` holds full addresses)
 //   wa, wb  : LDS address of w[lane & 3][4 * (lane >> 5)] of the first tile of the stage, for the accumulators 0 .. 3
 //             and (NM = 2) 4 .. 7;  WOFF: + bytes to the batch's first tile
 // Two products of one accumulator are at least two instructions apart, and the statement ends
 // with the wait states that an ordinary vector instruction needs before it may read a sum.
-template <int NM, bool PREFETCH, int G, int BOFF, int WOFF>
+template <int NM, bool PREFETCH, int G, int BOFF, int I0, int IS, int WOFF>
 __device__ __forceinline__ void rank_batch(const u32x16_t& mv, u32x16_t& nxt, const uint64_t* nbm, const RankAddr& a,
                                            uint32_t wa, uint32_t wb, f4_t (&acc)[NM][2])
 {
     static_assert(NM == 1 || NM == 2, "four or eight accumulators");
-    constexpr int I0 = 0, IS = 0;  // (`a` holds full addresses)
     u32x2_t w, w2;
 #define MSTF_RM(ACC, A, W) "v_mfma_f32_4x4x4_16b_f16 %[" ACC "], " A ", %[" W "], %[" ACC "]\n\t"
 #define MSTF_RONE                                                                                                     \
@@ -228,8 +228,7 @@ __device__ __forceinline__ void rank_batch(const u32x16_t& mv, u32x16_t& nxt, co
 // Batch G into the 32 accumulators of acc[P] by one 32x32x8 product per half P: the result layout of the address
 // products is also the A layout of that shape (row = position, the lane half's four tiles the k index).  The two
 // registers of a pair are merged first (one vector instruction per two reads), since the product, not the vector unit,
-// bounds this form.  wa: LDS address of w[lane & 31][8 G + 4 * (lane >> 5)];  I0, IS: immediate offset of the batch's first
-// tile and bytes between two tiles (0, 0: `a` holds full addresses).
+// bounds this form.  wa: LDS address of w[lane & 31][8 G + 4 * (lane >> 5)].
 template <bool PREFETCH, int G, int BOFF, int I0, int IS>
 __device__ __forceinline__ void rank_batch_wide(const u32x16_t& mv, u32x16_t& nxt, const uint64_t* nbm, const RankAddr& a,
                                                 uint32_t wa, f16x_t (&acc)[2])
@@ -346,10 +345,8 @@ struct RowSums {
     {
         if constexpr (kWide)
             rank_batch_wide<PREFETCH, G, BOFF, I0, IS>(mv, nxt, nbm, a, w ^ (uint32_t)(G * 16), wide);
-        else {
-            static_assert(I0 == 0 && IS == 0, "full addresses");
-            rank_batch<NM, PREFETCH, G, BOFF, G * 16>(mv, nxt, nbm, a, w, w + wgroup, narrow);
-        }
+        else
+            rank_batch<NM, PREFETCH, G, BOFF, I0, IS, G * 16>(mv, nxt, nbm, a, w, w + wgroup, narrow);
     }
     __device__ __forceinline__ void stage_done()
     {

@@ -1,5 +1,5 @@
-// Expansion of bitmap tiles a whole tile per LDS read, for images of tiles at a fixed stride (quant_device.hpp) and up to eight
-// weight rows.
+// Expansion of bitmap tiles a whole tile per LDS read, for images of tiles at a fixed stride and up to eight weight rows: the
+// quantised fused kernels and value products over many blocks (quant_device.hpp, StageRank).
 //
 // In rank_device.hpp a register of the address products holds the same half of two tiles, so that an exec mask is put
 // together from two 32-bit pieces and the lane halves' sums have to be joined.  Here the rows of a product are the two halves
