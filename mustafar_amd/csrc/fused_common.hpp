@@ -130,17 +130,24 @@ constexpr bool fused_shares_blocks(int tokens, int Bkv, int groups, int extra = 
 // launches: recorded into a graph, where a launch behind another takes 2 us, it is the faster form all the same up to this many
 // blocks of all heads, from five blocks a head on or with more than four query heads (fp16, 70 %, pairs or a wavefront per
 // block / shared and merged: 8 heads x 8 blocks 8.4 / 6.6 us, 64 x 8 8.9 / 8.1, 128 x 8 9.0 / 10.2; eight query heads, 8 x 4
-// 9.6 / 7.1, 64 x 8 11.2 / 9.6); launched call by call it is not (8 x 8 8.4 / 9.5).
+// 9.6 / 7.1, 64 x 8 11.2 / 9.6); launched call by call it is not (8 x 8 8.4 / 9.5).  With more than four query heads the
+// rows that the merge has to launch for outweigh few blocks a head (recorded, eight query heads: 128 x 1 9.04 / 8.24, 256 x 1 9.31 /
+// 9.80, 128 x 2 9.43 / 8.93, 160 x 2 9.46 / 10.00, 96 x 3 9.60 / 9.40, 128 x 3 9.71 / 9.93, 96 x 4 10.16 / 9.47, 160 x 4 10.25 / 10.98;
+// but 80 x 8 11.3 / 10.9; five: 256 x 1 9.24 / 8.96, 160 x 2 9.34 / 9.49), unless there are more heads than workgroups fit the
+// chip at once (five, 512 x 1 17.2 / 11.5).
 constexpr int kShareOneSplit = 640;
 constexpr bool fused_share_one_split(int nblk, int Bkv, int groups, bool recorded)
 {
-    return recorded && Bkv * nblk <= kShareOneSplit && (nblk > 4 || groups > 4);
+    if (!recorded || Bkv * nblk > kShareOneSplit) return false;
+    if (nblk > 4 || groups <= 4) return nblk > 4;
+    return Bkv > 256 || (nblk == 1 ? Bkv * groups <= 1280 : Bkv <= (nblk == 2 ? 128 : 112));
 }
 // Whether a workgroup of sixteen wavefronts takes a whole head, with up to four query heads, and writes its output, so that
 // no merge follows: heads of up to eight blocks, two wavefronts per block (a wavefront per block / this: 8 heads x 1 block 7.6 /
 // 5.5 us, 8 x 4 8.0 / 6.2, 256 x 4 8.7 / 7.1, 8 x 8 8.8 / 8.4, 256 x 8 9.7 / 9.5: eight blocks keep a CU busy), and heads of two
 // splits where these are as many as fill the chip (two splits and merge / this: 256 x 16 16.4 / 14.6, 256 x 64 48.8 / 47.3,
-// 224 x 64 44.9 / 43.4, 200 x 64 41.5 / 40.2, 2 bits 256 x 64 50.5 / 48.1; but 176 x 64 41.5 / 41.9, 64 x 16 9.9 / 11.8).
+// 224 x 64 44.9 / 43.4, 200 x 64 41.5 / 40.2, 2 bits 256 x 64 50.5 / 48.1; but 176 x 64 41.5 / 41.9, 64 x 16 9.9 / 11.8), with one
+// to four query heads alike, and longer heads no slower (200 and 256 x 128: from 0.96 to 1.03 of the two splits', by the card).
 constexpr bool fused_whole_head(int nblk, int ns, int Bkv, int groups, bool pairs)
 {
     if (groups > 4 || Bkv > 256) return false;

@@ -87,3 +87,9 @@ def test_recorded_calls_give_the_same_numbers(heads, groups, blocks):
             q.copy_(torch.randn(q.shape, generator=g, device="cuda", dtype=torch.float16))
             graph.replay()
             assert torch.equal(o.view(torch.int16), ops.decode_attention(ck, cv, q, groups, ws=ws).view(torch.int16))
+
+
+@pytest.mark.parametrize("heads,groups,blocks", [(160, 8, 1), (161, 8, 1), (112, 5, 3), (113, 5, 3), (128, 8, 5), (129, 8, 5), (128, 5, 2),
+                                                 (129, 5, 2), (257, 5, 2), (640, 5, 1), (641, 5, 1)])
+def test_recorded_calls_at_the_lines_of_their_rule(heads, groups, blocks):
+    test_recorded_calls_give_the_same_numbers(heads, groups, blocks)
