@@ -17,6 +17,7 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, si
     default: a fresh buffer with room for the worst case.  Returns the per-tile arrays, the buffer and the word total
     as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host.
     sized: the total as an int instead."""
+    assert inputs.dim() == 3
     own = ops._own_workspace(ws, inputs.device) if sized else None
     words = own.status(ops.status_words(inputs.shape[0] * (inputs.shape[1] // 64))) if own else None
     out = ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),

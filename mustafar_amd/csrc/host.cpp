@@ -409,6 +409,7 @@ PyObject* key_formulation_quant(Args& a)
 {
     const at::Tensor* s[7];
     for (int i = 0; i < 7; i++) s[i] = i == 3 || i == 4 ? a.maybe() : &a.tensor();
+    if (!s[3]) s[4] = nullptr;  // (units come with counts or not at all)
     const at::Tensor& B = a.tensor();
     const int M = a.small(), K = a.small(), Bq = a.small(), groups = a.small(), bit = a.small(), cap = a.small(), mode = a.small();
     a.done();

@@ -289,17 +289,28 @@ def compress(x, is_value, kth=0, capacity_halfs=None, ws=None):
     return CompressedKV(bmp, idx, nz, nz_off, M, N, is_value, total)
 
 
+def _capacity(capacity_halfs):
+    """The capacity argument of a native call (-1: none given)."""
+    if capacity_halfs is None:
+        return -1
+    if int(capacity_halfs) < 0:
+        raise RuntimeError("capacity_halfs must not be negative")
+    return int(capacity_halfs)
+
+
 def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     """compress(k, False, kth_k) and compress(v, True, kth_v) of the same tokens in one launch (mstf_compress_kv_f16):
     identical outputs, less time - a launch of both sides runs less in lockstep than two launches of one side each.
     k, v: [B, M, N]; capacity_halfs (default: room for the dense rows) sizes both value buffers, the totals stay on
     the device.  Returns (CompressedKV of the keys, CompressedKV of the values)."""
+    assert k.dim() == 3
+    capacity = _capacity(capacity_halfs)
     pair = lib().mstf_landing_take()
     own = _own_workspace(ws, k.device) if pair else None
     words = own.status(status_words(k.shape[0] * (k.shape[1] // 64), 2)) if own else None
     landing = _LandingPair(pair, _stream(), own, words, torch._C._cuda_getDevice()) if pair else None
     kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
-                                                   -1 if capacity_halfs is None else int(capacity_halfs), pair or 0, words)
+                                                   capacity, pair or 0, words)
     M, N = k.shape[1:]
     return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
@@ -331,13 +342,15 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     """Prune and compress the first M tokens of x [batch, rows, heads, 128] where the projection left them, the keys
     rotated first when cos / sin are given (all rows are rotated and written to rot).  Heads are numbered
     batch * heads + head.  Returns (CompressedKV, rot)."""
+    assert x.dim() == 4
     if cos is not None and rot is None:
         rot = x
+    capacity = _capacity(capacity_halfs)
     sized = capacity_halfs is None and M != 0
     own = _own_workspace(ws, x.device) if sized else None
     words = own.status(status_words(x.shape[0] * x.shape[2] * (M // 64))) if own else None
     bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
-                                           rot, -1 if capacity_halfs is None else int(capacity_halfs),
+                                           rot, capacity,
                                            _landing_word()[1] if sized else 0, words)
     if M == 0:
         return None, rot
