@@ -21,11 +21,13 @@ class Workspace:
     keeps the old buffers alive (a captured graph may still point at them), and growing while the current stream is
     being captured is an error - unless it holds the least that an attention call does with, if slower."""
 
+    _status = ()        # status words of the producers, zero between two calls; the last ones are in use
+    _spoilt = False     # the last ones are not zero any more
+
     def __init__(self, device, nbytes=1 << 20):
         self.device = torch.device(device)
         self._bufs = [torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=self.device)]
-        self._status = []       # status words of the producers, zero between two calls; the last one is in use
-        self._spoilt = False    # the last one is not zero any more
+        self._status = []
 
     @property
     def tensor(self):
@@ -54,7 +56,7 @@ class Workspace:
         if self._spoilt or not self._status or self._status[-1].numel() < words:
             if torch.cuda.is_current_stream_capturing():
                 return None
-            self._status.append(torch.zeros(max(words, 4096), dtype=torch.int64, device=self.device))
+            self._status = [*self._status, torch.zeros(max(words, 4096), dtype=torch.int64, device=self.device)]
             self._spoilt = False
         return self._status[-1]
 
@@ -112,13 +114,20 @@ class _LandingPair:
 
     def read(self, side):
         """The total, or None where the call was recorded into a graph."""
-        value = ctypes.c_int64.from_address(self.pair + 8 * side).value
+        at = self.pair + 8 * side
+        value = ctypes.c_int64.from_address(at).value
         if value == self.EMPTY:
-            own = ctypes.c_int64()
-            with torch.cuda.device(self.device):    # (a default stream's handle is the same on every device)
-                check(lib().mstf_landing_wait(self.stream, self.pair + 8 * side, ctypes.addressof(own)), "mstf_landing_wait")
-            value = own.value
+            if self.device == torch._C._cuda_getDevice():
+                value = self._wait(at)
+            else:
+                with torch.cuda.device(self.device):    # (a default stream's handle is the same on every device)
+                    value = self._wait(at)
         return None if value == self.NOT_LANDED else value
+
+    def _wait(self, at):
+        value = ctypes.c_int64()
+        check(lib().mstf_landing_wait(self.stream, at, ctypes.addressof(value)), "mstf_landing_wait")
+        return value.value
 
     def spoilt(self):
         ws = self.ws and self.ws()
@@ -168,14 +177,14 @@ def _call(fn, ws, device, call, *args):
 def _own_workspace(ws, device):
     """The Workspace that keeps a producer's status words, None where the caller brought a bare buffer or tensors of another
     device than the current one, on whose stream the words are cleared and the launch goes."""
-    if device.type == "cuda" and device.index != torch._C._cuda_getDevice():
+    if device.type != "cuda" or device.index != torch._C._cuda_getDevice():
         return None
-    if ws is None and device.type == "cuda":
-        key = (device.type, device.index, _stream())
+    if ws is None:
+        key = ("cuda", device.index, _stream())
         ws = _WS.get(key)
         if ws is None:
             ws = _WS[key] = Workspace(device)
-    return ws if isinstance(ws, Workspace) and ws.device.type == device.type else None
+    return ws if isinstance(ws, Workspace) and ws.device.type == "cuda" else None
 
 
 def gave_up(ws, words, what):
@@ -290,12 +299,10 @@ def compress(x, is_value, kth=0, capacity_halfs=None, ws=None):
 
 
 def _capacity(capacity_halfs):
-    """The capacity argument of a native call (-1: none given)."""
-    if capacity_halfs is None:
-        return -1
-    if int(capacity_halfs) < 0:
+    capacity = int(capacity_halfs)
+    if capacity < 0:    # (-1 is 'none given' to the native calls)
         raise RuntimeError("capacity_halfs must not be negative")
-    return int(capacity_halfs)
+    return capacity
 
 
 def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
@@ -304,14 +311,14 @@ def compress_kv(k, v, kth_k=0, kth_v=0, capacity_halfs=None, ws=None):
     k, v: [B, M, N]; capacity_halfs (default: room for the dense rows) sizes both value buffers, the totals stay on
     the device.  Returns (CompressedKV of the keys, CompressedKV of the values)."""
     assert k.dim() == 3
-    capacity = _capacity(capacity_halfs)
+    B, M, N = k.shape
+    capacity = -1 if capacity_halfs is None else _capacity(capacity_halfs)
     pair = lib().mstf_landing_take()
     own = _own_workspace(ws, k.device) if pair else None
-    words = own.status(status_words(k.shape[0] * (k.shape[1] // 64), 2)) if own else None
+    words = own.status(status_words(B * (M // 64), 2)) if own else None
     landing = _LandingPair(pair, _stream(), own, words, torch._C._cuda_getDevice()) if pair else None
     kb, ki, ko, kt, kn, vb, vi, vo, vt, vn = _call(host().compress_kv, ws, k.device, None, k, v, int(kth_k), int(kth_v),
                                                    capacity, pair or 0, words)
-    M, N = k.shape[1:]
     return (CompressedKV(kb, ki, kn, ko, M, N, False, kt, landing), CompressedKV(vb, vi, vn, vo, M, N, True, vt, landing))
 
 
@@ -345,7 +352,7 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     assert x.dim() == 4
     if cos is not None and rot is None:
         rot = x
-    capacity = _capacity(capacity_halfs)
+    capacity = -1 if capacity_halfs is None else _capacity(capacity_halfs)
     sized = capacity_halfs is None and M != 0
     own = _own_workspace(ws, x.device) if sized else None
     words = own.status(status_words(x.shape[0] * x.shape[2] * (M // 64))) if own else None

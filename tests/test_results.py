@@ -42,6 +42,18 @@ def test_a_result_saved_without_the_attribute():
     assert c.used_halfs() == 4
 
 
+def test_workspaces_are_saved_and_read_back():
+    from mustafar_amd import ops
+    ws = ops.Workspace("cpu", 512)
+    for old in (False, True):
+        if old:                                     # saved before it held status words
+            del ws._status
+        other = pickle.loads(pickle.dumps(ws))
+        assert other.tensor.numel() == 512 and not other._spoilt and len(other._status) == 0
+        other.status_spoilt(None)
+        assert copy.deepcopy(ws).tensor.numel() == 512
+
+
 def test_a_known_total_gives_the_words_back_and_holds_no_workspace():
     from mustafar_amd import ops
     ws = ops.Workspace("cpu", 256)
@@ -95,6 +107,7 @@ def test_a_total_is_waited_for_on_the_device_of_its_call(monkeypatch):
 
     pair[1] = ops._LandingPair.EMPTY
     monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current[-1], raising=False)
     monkeypatch.setattr(ops, "lib", Library)
     assert c.used_halfs() == 8 and current == [0]
 
