@@ -664,7 +664,7 @@ __device__ __forceinline__ void count_through(uint64_t* counter, bool ok)
 //   counters: in how many words the workgroups count themselves, a power of two; word i stands kCounterStep words behind word
 //             i - 1, in a cache line of its own.  Adding to one word takes the chip 7 ns each time: 4500 workgroups of one wavefront
 //             (60 heads x 4800 tokens from the projection) took 82 us with one word, 52 without counting.
-constexpr int kCounters = 16, kCounterStep = 16;
+constexpr int kCounters = 16, kCounterStep = 16;  // (fewer than a wavefront's lanes: the last ones look at the flag)
 constexpr int kKeptHead = 16;  // kept words: the flag, in a cache line of its own, then the status words of each side
 struct Handover {
     uint64_t* landing;
@@ -693,22 +693,27 @@ __device__ __forceinline__ void hand_over(const Handover& how, uint64_t* total_o
                                           int groups, uint32_t spin_limit, uint32_t* room)
 {
     if (threadIdx.x < 64) {
+        // The counters and, in the other lanes, the flag: by an earlier launch, since which the words are not what they should
+        // be.  (A workgroup of this one that gave up has counted itself as a failure.)
         const bool reads = (int)threadIdx.x < how.counters;
-        const uint64_t* mine = counter_of(how, state, groups, reads ? (int)threadIdx.x : 0);
-        auto counted = [&]() { return wave_sum_u64(reads ? agent_load(mine) : 0ull); };
-        // (a flag that is up already, by an earlier launch perhaps: the counters may never come to what they should)
-        const bool flagged = agent_load(how.flag) != 0ull;
-        uint64_t through = counted();
+        const uint64_t* mine = reads ? counter_of(how, state, groups, (int)threadIdx.x) : how.flag;
+        uint64_t through;
+        bool flagged;
+        auto look = [&]() {
+            const uint64_t v = agent_load(mine);
+            flagged = __ballot(!reads && v != 0ull) != 0ull;
+            through = wave_sum_u64(reads ? v : 0ull);
+        };
+        look();
         const uint32_t others = (uint32_t)groups - 1u;
         for (uint32_t polls = 0; (uint32_t)through != others && !flagged && polls < spin_limit; polls++) {
             __builtin_amdgcn_s_sleep(1);
-            through = counted();
+            look();
         }
         const bool all = (uint32_t)through == others && !flagged;
         if (threadIdx.x == 0) {
             if (!all && how.kept) agent_store(how.flag, 1ull);  // (words are still in use: they cannot be cleared)
-            ok = ok && all && through == others && agent_load(how.flag) == 0ull;
-            const uint64_t v = ok ? total : ~0ull;
+            const uint64_t v = ok && all && through == others ? total : ~0ull;
             if (how.kept) *total_out = v;
             if (how.landing) __hip_atomic_store(how.landing, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             *room = all ? 1u : 0u;
