@@ -3,11 +3,12 @@
  *
  * Conventions for every entry point
  *   - all data pointers are DEVICE pointers; `stream` is a hipStream_t passed as void*
- *     (NULL = the default stream); launches are asynchronous, nothing here synchronises;
+ *     (NULL = the default stream); launches are asynchronous and nothing here waits for the GPU, except mstf_read_word,
+ *     mstf_landing_wait and the calls ..._sized, which wait for a number (see there);
  *   - fp16 buffers are IEEE binary16 (`mstf_half` = raw 16-bit pattern);
  *   - inputs are borrowed and never modified; outputs are caller-allocated;
- *   - nothing allocates: scratch memory comes in through `workspace` (size from the
- *     matching *_workspace_bytes query, 256-byte aligned);
+ *   - nothing allocates (mstf_landing_take: 16 KB of pinned host memory, once a process): scratch memory comes in through
+ *     `workspace` (size from the matching *_workspace_bytes query, 256-byte aligned);
  *   - the return value is MSTF_OK or a negative MSTF_E* code (never an exception);
  *     mstf_strerror() names it; a failed launch also records the HIP error, readable
  *     with mstf_last_hip_error().
@@ -53,13 +54,13 @@ int mstf_version(void);
  * practically impossible case that the xor of all data read by a workgroup hits a fixed constant).  Timing it gives the
  * plain-read time of a buffer of that size on the box at hand. */
 int mstf_probe_read(void* stream, const void* src, size_t bytes, uint32_t* sink, int workgroups);
-/* The 64-bit word at src (device memory) on the host, once the work in front of it on `stream` is done: the one call here
- * that waits for the GPU.  A kernel of one thread writes it to `landing`, 8 bytes of pinned host memory that no other call
+/* The 64-bit word at src (device memory) on the host, once the work in front of it on `stream` is done.  A kernel of one thread writes it to `landing`, 8 bytes of pinned host memory that no other call
  * uses meanwhile and that keep what they are given when the call fails; the caller's thread watches for it there.
  * Refused (MSTF_ELAUNCH) while the stream is being captured.  landing and value: host pointers. */
 int mstf_read_word(void* stream, const int64_t* src, int64_t* landing, int64_t* value);
 /* Totals that a producer's kernel stores to pinned host memory itself, before its values are all out (the calls ..._sized and
- * ..._landing_f16 below): known on the host without a launch behind the kernel and a wait for its end.
+ * ..._landing_f16 below): known on the host without a launch behind the kernel and a wait for its end.  The outputs are complete
+ * in the order of the stream, as behind every call here, not when the total is known.
  * mstf_landing_take: a pair of such words for a call that returns without waiting; null when none is free (the caller then
  * uses the call without landings).  mstf_landing_give hands it back, at any time, from any thread; what is no pair, or not out,
  * is left alone.

@@ -3,7 +3,9 @@ convert_value_batched_quant :425-529): same arguments and return tuples.  The re
 2-bit codes; `bit` is exposed here as an extra keyword (2, 4 or 8; capacity = 32 // bit), and `group_size`
 (64 = one scale / zero pair per tile as in the reference; 32 = two, scales and zeros then [B, T, 2]).
 
-inputs: [B, M, N] fp16 on the GPU, already pruned (or pruned here: `kth`), M % 64 == 0.
+inputs: [B, M, N] fp16 on the GPU, already pruned (or pruned here: `kth`), M % 64 == 0.  The converters wait for the size of
+the packed words and copy these out by a launch behind that, as the reference does: results are complete in the order of the
+current stream.
 """
 import torch
 

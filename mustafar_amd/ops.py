@@ -1,7 +1,9 @@
 """Zero-copy device path: fused prune+compress into a flat cache, SpMVs with one row per head.
 
-Everything stays on the device; the only host synchronisation is the optional read-back of the
-packed size when the caller did not provide a capacity.
+Everything stays on the device, in the order of the current stream; the host waits for a packed size where the caller did
+not provide a capacity or asks for it, and for nothing else.  Such a size may be there before the kernel has stored its last
+values: a result that another stream is to use, or an input that another stream may write to or free, waits for this one as with
+any torch call (an event recorded, or wait_stream called, after the call).
 """
 import ctypes
 import math
@@ -224,8 +226,9 @@ class CompressedKV:
         return self.bmp.shape[0]
 
     def used_halfs(self):
-        """Number of fp16 values in use (reads the device-side total once).  The one-pass compressor reports a wait that
-        ran out - which the dispatch order rules out - as a total of all ones: that raises here."""
+        """Number of fp16 values in use (the total is read once; the values themselves may be on their way yet, see above).
+        The one-pass compressor reports a wait that ran out - which the dispatch order rules out - as a total of all ones:
+        that raises here."""
         if self._used is not None:
             return self._used
         landing = self._landing
@@ -243,7 +246,7 @@ class CompressedKV:
         return n
 
     def packed(self):
-        """The used part of the flat value buffer (needs the host-side size)."""
+        """The used part of the flat value buffer (needs the host-side size), complete in the order of the call's stream."""
         return self.nz[:self.used_halfs()]
 
     def nbytes(self):
@@ -265,8 +268,8 @@ def prune_rows(x, kth, out=None):
 def compress(x, is_value, kth=0, capacity_halfs=None, ws=None):
     """Prune (kth > 0) and compress x [B, M, N] into the bitmap format.
 
-    With capacity_halfs=None the packed size is read back once (like the reference's .item());
-    with a capacity the call is fully asynchronous and `total_halfs` stays on the device."""
+    With capacity_halfs=None the packed size is read back once (like the reference's .item()) and the values are stored by
+    a launch behind that; with a capacity nothing is waited for and `total_halfs` stays on the device."""
     assert x.is_cuda and x.dtype == torch.float16 and x.dim() == 3
     x = x.contiguous()
     B, M, N = x.shape
@@ -348,7 +351,8 @@ def proj_source(x, cos=None, sin=None, rot=None):
 def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_halfs=None, ws=None):
     """Prune and compress the first M tokens of x [batch, rows, heads, 128] where the projection left them, the keys
     rotated first when cos / sin are given (all rows are rotated and written to rot).  Heads are numbered
-    batch * heads + head.  Returns (CompressedKV, rot)."""
+    batch * heads + head.  Returns (CompressedKV, rot); without a capacity it waits for the size, not for the last values
+    and rotated rows."""
     assert x.dim() == 4
     if cos is not None and rot is None:
         rot = x
