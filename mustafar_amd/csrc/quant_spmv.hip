@@ -311,7 +311,8 @@ struct QArgs {
 // each, instead of taking a block each: a quarter of the chain, and as many wavefronts four times over.  1024 such workgroups
 // fit the chip; a few more still pay.  32 rows, 4 bits, 70 %, heads x blocks, a block each / shared: 1 x 1 7.06 / 3.95 us,
 // 8 x 33 7.97 / 4.88, 32 x 24 8.33 / 5.91, 32 x 33 9.33 / 8.36, 32 x 48 9.84 / 10.02, 64 x 64 13.0 / 21.0 (2 bits 6.64 / 3.89,
-// 7.43 / 4.78, 7.72 / 5.74, 8.70 / 7.91, 9.25 / 9.66, 12.5 / 20.5).
+// 7.43 / 4.78, 7.72 / 5.74, 8.70 / 7.91, 9.25 / 9.66, 12.5 / 20.5).  Up to the line no call of 16, 24 or 32 rows, 2, 4 or 8 bits, one
+// group per tile or two, is slower for it (32 x 40, 8 bits, 32 rows 10.85 / 10.57).
 constexpr int kKeyShareQuant = 1280;
 template <int NW, int BIT>
 static void launch_key_q(hipStream_t st, const QArgs& a, const _Float16* Bm, _Float16* C, int Lc, int D, int Bkv,

@@ -306,7 +306,8 @@ static int key_waves(int nblk, int Bkv)
 }
 // Blocks up to which the four wavefronts of a workgroup share a block of more than eight rows, a channel stage each, instead of
 // taking a block each: the workgroups that fit the chip.  32 rows, 70 %, heads x blocks, a block each / shared: 1 x 1 5.41 /
-// 3.48 us, 8 x 33 6.12 / 4.25, 32 x 24 7.12 / 6.03, 32 x 33 7.67 / 8.82, 64 x 64 11.6 / 22.2.
+// 3.48 us, 8 x 33 6.12 / 4.25, 32 x 24 7.12 / 6.03, 32 x 33 7.67 / 8.82, 64 x 64 11.6 / 22.2; sixteen rows gain as much, and 24
+// (a pass of sixteen and one of eight) 4 - 9 % up to the line.
 constexpr int kKeyShare = 768;
 template <int NW, int WAVES, bool SHARE = false>
 static void launch_key_waves(hipStream_t st, const uint64_t* bmp, const char* nz, const uint32_t* idx,

@@ -33,5 +33,5 @@ print("replayed", flush=True)
 
 
 def test_the_first_call_is_recorded():
-    r = subprocess.run([sys.executable, "-u", "-c", CHILD], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    r = subprocess.run([sys.executable, "-u", "-c", CHILD], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
     assert r.returncode == 0 and "replayed" in r.stdout, r.stdout[-2000:]
