@@ -58,7 +58,10 @@ class Workspace:
         if self._spoilt or not self._status or self._status[-1].numel() < words:
             if torch.cuda.is_current_stream_capturing():
                 return None
-            self._status = [*self._status, torch.zeros(max(words, 4096), dtype=torch.int64, device=self.device)]
+            # (as the words before them at least, twice that if they were too few: all of them together are bounded)
+            last = self._status[-1].numel() if self._status else 0
+            room = max(words, 4096, last if words <= last else 2 * last)
+            self._status = [*self._status, torch.zeros(room, dtype=torch.int64, device=self.device)]
             self._spoilt = False
         return self._status[-1]
 

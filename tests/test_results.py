@@ -54,6 +54,19 @@ def test_workspaces_are_saved_and_read_back():
         assert copy.deepcopy(ws).tensor.numel() == 512
 
 
+def test_status_words_of_growing_calls_are_bounded(monkeypatch):
+    from mustafar_amd import ops
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ws = ops.Workspace("cpu", 256)
+    for words in range(64, 60000, 64):
+        t = ws.status(words)
+        assert t.numel() >= words and t is ws._status[-1]
+    assert sum(t.numel() for t in ws._status) <= 4 * 60000
+    before = len(ws._status)
+    ws.status_spoilt(ws._status[-1])
+    assert ws.status(64).numel() >= 59968 and len(ws._status) == before + 1 and ws.status(59968) is ws._status[-1]
+
+
 def test_a_known_total_gives_the_words_back_and_holds_no_workspace():
     from mustafar_amd import ops
     ws = ops.Workspace("cpu", 256)
