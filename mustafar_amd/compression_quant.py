@@ -20,8 +20,9 @@ def _produce(inputs, is_value, bit, kth=0, group_size=64, ws=None, room=None, si
     as a device tensor (all ones should a wait of the one-pass producer have run out) - nothing is read on the host.
     sized: the total as an int instead."""
     assert inputs.dim() == 3
+    B, M, _ = inputs.shape
     own = ops._own_workspace(ws, inputs.device) if sized else None
-    words = own.status(ops.status_words(inputs.shape[0] * (inputs.shape[1] // 64))) if own else None
+    words = own.status(ops.status_words(B * (M // 64))) if own else None
     out = ops._call(host().produce_quant, ws, inputs.device, None, inputs, int(bool(is_value)), int(bit), int(kth),
                     int(group_size), room, ops._landing_word()[1] if sized else 0, words)
     if sized and out[-1] < 0:

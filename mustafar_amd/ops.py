@@ -357,12 +357,13 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     batch * heads + head.  Returns (CompressedKV, rot); without a capacity it waits for the size, not for the last values
     and rotated rows."""
     assert x.dim() == 4
+    batch, _, heads, N = x.shape
     if cos is not None and rot is None:
         rot = x
     capacity = -1 if capacity_halfs is None else _capacity(capacity_halfs)
     sized = capacity_halfs is None and M != 0
     own = _own_workspace(ws, x.device) if sized else None
-    words = own.status(status_words(x.shape[0] * x.shape[2] * (M // 64))) if own else None
+    words = own.status(status_words(batch * heads * (M // 64))) if own else None
     bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
                                            rot, capacity,
                                            _landing_word()[1] if sized else 0, words)
@@ -370,7 +371,7 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
         return None, rot
     if sized and n < 0:
         gave_up(own, words, _GAVE_UP)
-    return CompressedKV(bmp, idx, nz, nz_off, M, x.shape[3], is_value, n if sized else total), rot
+    return CompressedKV(bmp, idx, nz, nz_off, M, N, is_value, n if sized else total), rot
 
 
 def key_spmv(ck, q, groups, n_rows=1, out=None):
