@@ -275,19 +275,27 @@ __device__ __forceinline__ void block_softmax(const f4_t (&acc_k)[NM], float sqr
     }
 }
 
-// Folds a block's (max, sum, output) into the running one of the wavefront (lane 4b+j: head j in every register).
+// Folds a block's (max, sum, output) into the running one of the wavefront (lane 4b+j: head j in every register).  In two
+// steps: what the running output and the block's are worth beside each other follows from the maxima, before the block's is there.
+struct Folded {
+    float fa, fb;
+    __device__ __forceinline__ Folded(float& m_run, float& l_run, float m_blk, float l_blk)
+    {
+        const float mn = fmaxf(m_run, m_blk);
+        fa = m_run == -INFINITY ? 0.f : __expf(m_run - mn);
+        fb = m_blk == -INFINITY ? 0.f : __expf(m_blk - mn);
+        l_run = l_run * fa + l_blk * fb;
+        m_run = mn;
+    }
+};
 __device__ __forceinline__ void fold_block(f4_t (&acc)[2], float& m_run, float& l_run, const f4_t (&blk)[2], float m_blk,
                                            float l_blk)
 {
-    const float mn = fmaxf(m_run, m_blk);
-    const float fa = m_run == -INFINITY ? 0.f : __expf(m_run - mn);
-    const float fb = m_blk == -INFINITY ? 0.f : __expf(m_blk - mn);
+    const Folded f(m_run, l_run, m_blk, l_blk);
 #pragma unroll
     for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) acc[h][c] = acc[h][c] * fa + blk[h][c] * fb;
-    l_run = l_run * fa + l_blk * fb;
-    m_run = mn;
+        for (int c = 0; c < 4; c++) acc[h][c] = acc[h][c] * f.fa + blk[h][c] * f.fb;
 }
 
 // Workgroup combine of the kFusedWaves blocks of a split: every wavefront parks (output[4*NM][D], max, sum) in its

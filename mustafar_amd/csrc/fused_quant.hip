@@ -20,12 +20,17 @@ namespace mstf {
 // Rows of the query and of the block weights sit 16 bytes further apart than their length: the four rows that the lanes
 // of a group read together then start in different LDS banks.
 constexpr int kQuantQRow = kFusedD * 2 + MSTF_QPAD;
-constexpr int kQuantPRow = 64 * 2 + MSTF_QPAD;
+// (Block weights as far apart as query rows where the LDS has room: the lanes' places in both are then one register.)
+template <int NM>
+constexpr int quant_prow()
+{
+    return NM == 1 ? kQuantQRow : 64 * 2 + MSTF_QPAD;
+}
 template <int NM, int BIT, bool G32>
 constexpr int quant_wave_lds()
 {
     // image, two word buffers, two metadata buffers; query rows; block weights; or the parked triple at the end
-    constexpr int need = q_lds_bytes<BIT, G32>() + NM * 4 * (kQuantQRow + kQuantPRow);
+    constexpr int need = q_lds_bytes<BIT, G32>() + NM * 4 * (kQuantQRow + quant_prow<NM>());
     constexpr int park = NM * 4 * kFusedD * 4 + 64;
     return need > park ? need : park;
 }
@@ -90,7 +95,7 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
         if (MULTI) deal = fused_deal(nblk, fused_splits(nblk, fused_fill_unpack(deal)));
     }
     constexpr int D = kFusedD;
-    constexpr int kQRow = kQuantQRow, kPRow = kQuantPRow;
+    constexpr int kQRow = kQuantQRow, kPRow = quant_prow<NM>();
     constexpr int kQLds = NM * 4 * kQRow;
     constexpr int kMetaBytes = meta_bytes<G32>();
     constexpr int kStage = q_lds_bytes<BIT, G32>();  // image, two word buffers, two metadata buffers
@@ -157,7 +162,8 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
         MetaLanes metaK = meta_lanes<G32>(k_off_dma + tile0, k_scales + tile0 * kPairs, k_zeros + tile0 * kPairs, bmK, lane);
         MetaLanes metaV = meta_lanes<G32>(v_off_dma + tile0, v_scales + tile0 * kPairs, v_zeros + tile0 * kPairs, bmV, lane);
         const uint32_t lane4 = (uint32_t)lane * 4u;
-        const uint32_t touch8 = (uint32_t)(lane & (kSubTiles - 1)) * 8u;
+        using Rank = StageRank<4 * NM, BIT, G32, false>;
+        const uint32_t bits_at = Rank::bits_at(lane);
         const uint32_t wordbuf_lds = lds_addr(wordbuf);
         auto start_of = [&](int n) { return (uint32_t)__builtin_amdgcn_readlane(bnd, n < kKeySubs ? n : 16 + n - kKeySubs); };
         auto end_of = [&](int n) { return (uint32_t)__builtin_amdgcn_readlane(bnd, n < kKeySubs ? n + 1 : 17 + n - kKeySubs); };
@@ -172,11 +178,11 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                                                 wordbuf_lds + (uint32_t)(n & 1) * F::kWordBuf, (uint32_t)lane, lane4);
             // metadata: lanes 0..31 the word offsets, 32..47 the scales, 48..63 the zero-points (two per lane)
             meta_issue_next<G32>(n < kKeySubs ? metaK : metaV, metabuf + (n & 1) * kMetaBytes);
-            // the stage's bitmaps: lane l holds the one of tile l & 31 (and the scalar loads of the expansion find them in L2)
-            return *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(bm + t) + touch8);
+            // the stage's bitmaps (and the scalar loads of the expansion find them in L2)
+            return Rank::bits_load(bm + t, bits_at);
         };
 
-        const StageRank<4 * NM, false> rank(lbase, lane);
+        Rank rank(lds_addr(metabuf), wordbuf_lds, lbase, lane);
 
         // the query rows of this KV head: groups x D fp16, contiguous (STEP: rotated out of the projection output)
         if constexpr (STEP) {
@@ -195,26 +201,24 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
         }
         uint2 touch = issue(0);
 
-        typename StageRank<4 * NM, false>::Sums sums;  // of the phase (keys, one half of the values, the other half)
+        typename Rank::Sums sums;  // of the phase (keys, one half of the values, the other half)
         const uint32_t qrow = sums.waddr(lds_addr(ql), kQRow, lane);
-        const uint32_t prow = sums.waddr(lds_addr(pl), kPRow, lane);
+        const uint32_t prow = kPRow == kQRow ? qrow + (uint32_t)kQLds : sums.waddr(lds_addr(pl), kPRow, lane);
 
 #pragma unroll 1
         for (int r = 0; r < (MULTI ? nb : 1); r++) {
             const bool more = MULTI && r + 1 < nb;
-            f4_t blk_v[NM][2];
-            float m_blk[NM], l_blk[NM];
+            float fb[NM];
             Raw coming;
             uint32_t bnd_next = bnd;
-            sums.clear();
-#pragma unroll
-            for (int n = 0; n < kKeySubs + kValSubs; n++) {
+            static_for<kKeySubs + kValSubs>([&](auto nc) {
+                constexpr int n = decltype(nc)::value;
                 // 3, 2, 1, 0 over the key stages and again over the value stages (keeping the wavefronts that also take a
                 // block of the dense window at 3, as the fp16 kernel does, measured slower here)
                 set_wave_priority(3 - n % 4);
                 asm volatile("s_waitcnt vmcnt(0)" : "+v"(touch.x), "+v"(touch.y)::"memory");  // stage n has landed
-                const uint2 bits = touch;  // lane l: bitmap l & 31 of stage n
-                const uint32_t start = start_of(n);
+                const uint2 bits = touch;
+                const uint32_t start = start_of(n), end = end_of(n);
                 const uint64_t* bm = (n < kKeySubs ? bmK : bmV) + (n < kKeySubs ? n : n - kKeySubs) * kSubTiles;
                 if (n + 1 < kKeySubs + kValSubs) {
                     touch = issue(n + 1);
@@ -232,36 +236,45 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                     f4_t acc_k[NM];
 #pragma unroll
                     for (int m = 0; m < NM; m++) acc_k[m] = sums.joined(m);
-                    sums.clear();
+                    float m_blk[NM], l_blk[NM];
                     block_softmax<NM, kPRow>(acc_k, sqrt_d, 64, pl, lane, m_blk, l_blk);
+                    // (the fold of the block begins here, so that nothing of it waits in registers beside the running output)
+#pragma unroll
+                    for (int m = 0; m < NM; m++) {
+                        if constexpr (MULTI) {
+                            const Folded f(m_run[m], l_run[m], m_blk[m], l_blk[m]);
+                            fb[m] = f.fb;
+#pragma unroll
+                            for (int h = 0; h < 2; h++)
+#pragma unroll
+                                for (int c = 0; c < 4; c++) acc_v[m][h][c] *= f.fa;
+                        } else {
+                            m_run[m] = m_blk[m];
+                            l_run[m] = l_blk[m];
+                        }
+                    }
                     const int adv = more ? D : 0;
                     if (MULTI) coming = bounds_of(offK + adv, offV + adv, bmK + adv, bmV + adv);
                 }
-                const int vs = n - kKeySubs;  // value stage: half = vs / 2, tokens (vs % 2) * 32..
+                constexpr int vs = n - kKeySubs;  // value stage: half = vs / 2, tokens (vs % 2) * 32..
                 constexpr int kSubsPerHalf = 64 / kSubTiles;
-                dequant_stage<BIT, G32>(lds_addr(metabuf) + (uint32_t)(n & 1) * kMetaBytes,
-                                        wordbuf_lds + (uint32_t)(n & 1) * F::kWordBuf, lbase, start, bits, lane, mode);
                 const uint32_t w = n < kKeySubs ? qrow + (uint32_t)n * kSubTiles * 2u
                                                 : prow + (uint32_t)(vs % kSubsPerHalf) * kSubTiles * 2u;
-                rank.expand(bm, bits, w, n < kKeySubs ? 4u * kQRow : 4u * kPRow, sums);
+                const StageAt here = {lds_addr(metabuf), wordbuf_lds, (uint32_t)(n & 1) * kMetaBytes, (uint32_t)(n & 1) * F::kWordBuf,
+                                      start, end};
+                constexpr bool kStarts = n == 0 || n == kKeySubs || n == kKeySubs + kSubsPerHalf;
+                rank.template stage<kStarts>(here, bm, bits, w, n < kKeySubs ? 4u * kQRow : 4u * kPRow, sums, lane, mode);
                 if (n >= kKeySubs && vs % kSubsPerHalf == kSubsPerHalf - 1) {  // the half is complete
 #pragma unroll
-                    for (int m = 0; m < NM; m++) blk_v[m][vs / kSubsPerHalf] = sums.joined(m);
-                    sums.clear();
+                    for (int m = 0; m < NM; m++) {
+                        const f4_t blk = sums.joined(m);
+                        f4_t& out_v = acc_v[m][vs / kSubsPerHalf];
+#pragma unroll
+                        for (int c = 0; c < 4; c++) out_v[c] = MULTI ? out_v[c] + blk[c] * fb[m] : blk[c];
+                    }
                 }
                 wait_lgkm0();  // every read of the image and of the staged buffers is done before they are rewritten
-            }
-#pragma unroll
-            for (int m = 0; m < NM; m++) {
-                if (MULTI) {
-                    fold_block(acc_v[m], m_run[m], l_run[m], blk_v[m], m_blk[m], l_blk[m]);
-                } else {
-                    acc_v[m][0] = blk_v[m][0];
-                    acc_v[m][1] = blk_v[m][1];
-                    m_run[m] = m_blk[m];
-                    l_run[m] = l_blk[m];
-                }
-            }
+            });
         }
     }
     if constexpr (STEP) {

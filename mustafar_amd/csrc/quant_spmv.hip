@@ -44,7 +44,6 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
     const uint32_t lbase = lds_addr(my);
     char* wordbuf = my + kImgBytes;
     char* metabuf = wordbuf + 2 * F::kWordBuf;
-    const Rank rank(lbase, lane);
 
     // words of the stage starting at tile t: [tile_off[t], tile_off[t + 31] + words of tile t + 31)
     auto bounds = [&](size_t t, uint32_t& s, uint32_t& e) {
@@ -55,8 +54,9 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
     constexpr int kMetaBytes = meta_bytes<G32>();
     const MetaLanes meta = meta_lanes<G32>(c.off_dma, c.scales, c.zeros, c.bmp, lane);
     const uint32_t lane4 = (uint32_t)lane * 4u;
-    const uint32_t touch8 = (uint32_t)(lane & (kSubTiles - 1)) * 8u;
+    const uint32_t bits_at = Rank::bits_at(lane);
     const uint32_t wordbuf_lds = lds_addr(wordbuf);
+    Rank rank(lds_addr(metabuf), wordbuf_lds, lbase, lane);
     auto uni = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
     // (no lane-dependent branches in the word and metadata loads: exec set by hand, clamped touch address)
     auto issue = [&](int n, size_t t, uint32_t s, uint32_t e) {
@@ -68,8 +68,8 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
         // when a tile has two (scale, zero) pairs
         meta_issue<G32>(meta, (uint32_t)t, metabuf + (n & 1) * kMetaBytes);
         stage_w(n);
-        // the stage's bitmaps: lane l holds the one of tile l & 31 (and the scalar loads of the expansion find them in L2)
-        return *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(c.bmp + t) + touch8);
+        // the stage's bitmaps (and the scalar loads of the expansion find them in L2)
+        return Rank::bits_load(c.bmp + t, bits_at);
     };
 
     size_t t_cur = tile_of(0), t_nxt = nsubs > 1 ? tile_of(1) : t_cur;
@@ -101,7 +101,7 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
                      : "+v"(touch.x), "+v"(touch.y), "+v"(bnd.off), "+v"(bnd.last.x), "+v"(bnd.last.y)::"memory");
         const uint2 bits = touch;
         const size_t t_now = t_cur;
-        const uint32_t s_now = s_cur;
+        const uint32_t s_now = s_cur, e_now = e_cur;
         if (n + 1 < nsubs) {
             t_cur = t_nxt;
             const uint32_t words = ((uint32_t)__builtin_popcount(bnd.last.x) + (uint32_t)__builtin_popcount(bnd.last.y) +
@@ -114,9 +114,8 @@ __device__ __forceinline__ void walk_subs_q(int nsubs, TileOf tile_of, StageW st
                 bnd = bounds_of(t_nxt);
             }
         }
-        dequant_stage<BIT, G32>(lds_addr(metabuf) + (uint32_t)(n & 1) * kMetaBytes,
-                           lds_addr(wordbuf) + (uint32_t)(n & 1) * F::kWordBuf, lbase, s_now, bits, lane, mode);
-        rank.expand(c.bmp + t_now, bits, waddr_of(n), wgroup, sums);
+        const StageAt here = {lds_addr(metabuf), wordbuf_lds, (uint32_t)(n & 1) * kMetaBytes, (uint32_t)(n & 1) * F::kWordBuf, s_now, e_now};
+        rank.stage(here, c.bmp + t_now, bits, waddr_of(n), wgroup, sums, lane, mode);
         wait_lgkm0();  // every read of the image and of the staged buffers is done before they are rewritten
     }
 }
@@ -136,7 +135,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(resident_wa
     const uint32_t* tile_off_dma, const uint16_t* scales, const uint16_t* zeros, const _Float16* Bm,
     _Float16* __restrict__ C, int Lc, int D, int nblk, int ntasks, int rows_per_kv, int row0, int mode)
 {
-    using Rank = StageRank<NW, true>;
+    using Rank = StageRank<NW, BIT, G32, true>;
     using Sums = typename Rank::Sums;
     constexpr bool kShared = Sums::kWide;
     constexpr int kMaxD = 128;
@@ -210,7 +209,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(resi
     _Float16* __restrict__ C, float* __restrict__ part, int Lc, int D, int nblk, int nbpw, int nsplit, int rows_per_kv,
     int row0, int mode, int nwg, uint32_t per_split)
 {
-    using Rank = StageRank<NW, !WHOLE>;
+    using Rank = StageRank<NW, BIT, G32, !WHOLE>;
     using Sums = typename Rank::Sums;
     static_assert(Sums::kRows == RowSums<NW>::kRows, "LDS of a wavefront");
     constexpr int kWRow = kSubTiles * 2;
