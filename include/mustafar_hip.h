@@ -200,6 +200,12 @@ int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source* src, int 
                                  uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, mstf_half* nz,
                                  uint64_t nz_capacity_halfs, void* workspace, size_t workspace_bytes, uint64_t* status,
                                  size_t status_bytes, int64_t* landing, int64_t* value);
+/* The same (M > 0) without a wait: the total comes to one of a pair of landings (mstf_landing_take), to be read with
+ * mstf_landing_wait.  Refused (MSTF_ELAUNCH) while the stream is being captured. */
+int mstf_compress_proj_landing_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
+                                   uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs, mstf_half* nz,
+                                   uint64_t nz_capacity_halfs, void* workspace, size_t workspace_bytes, uint64_t* status,
+                                   size_t status_bytes, int64_t* landing);
 int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                          uint64_t* bmp, uint32_t* idx, const uint32_t* dst_off, const uint32_t* dst_limit,
                          mstf_half* nz, uint32_t* overflow, void* workspace, size_t workspace_bytes);

@@ -61,6 +61,7 @@ SIGNATURES = {
                                 _vp, _sz]),
     "mstf_compress_proj_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _sz]),
     "mstf_compress_proj_sized_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _sz, _vp, _sz, _vp, _vp]),
+    "mstf_compress_proj_landing_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _u64, _vp, _sz, _vp, _sz, _vp]),
     "mstf_append_proj_f16": (_i, [_vp, _ps, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz]),
     "mstf_key_spmv_f16": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i]),
     "mstf_value_spmv_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),

@@ -482,6 +482,8 @@ class SparseKVCache:
                 self.k, self.v = ck, cv
         K, V = kx.transpose(1, 2), vx.transpose(1, 2)
         self._prefill_window(K, V, Lc)
+        if self.max_tokens == 0 and Lc > 0:     # cut to size, or an error where a wait ran out, behind all launches
+            self.k.nz, self.v.nz
         return K, V
 
     def prefill(self, K, V):

@@ -940,6 +940,21 @@ extern "C" int mstf_compress_proj_sized_f16(void* stream, const mstf_proj_source
     return rc != MSTF_OK ? rc : total_wait(as_stream(stream), landing, value);
 }
 
+extern "C" int mstf_compress_proj_landing_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
+                                              uint64_t* bmp, uint32_t* idx, uint32_t* nz_off, uint64_t* total_halfs,
+                                              mstf_half* nz, uint64_t nz_capacity_halfs, void* workspace,
+                                              size_t workspace_bytes, uint64_t* status, size_t status_bytes, int64_t* landing)
+{
+    if (M <= 0 || !src) return MSTF_EINVAL;
+    int rc = status_check(status, status_bytes, (int64_t)src->batch * src->heads, M, 1);
+    if (rc == MSTF_OK) rc = landing_ready(as_stream(stream), landing, landing);
+    if (rc != MSTF_OK) return rc;
+    rc = proj_impl(stream, src, is_value, M, N, kth, bmp, idx, nz_off, total_halfs, nullptr, nullptr, nz, nz_capacity_halfs,
+                   nullptr, workspace, workspace_bytes, reinterpret_cast<uint64_t*>(landing), status);
+    if (rc != MSTF_OK) __atomic_store_n(landing, MSTF_NOT_LANDED, __ATOMIC_RELEASE);
+    return rc;
+}
+
 extern "C" int mstf_append_proj_f16(void* stream, const mstf_proj_source* src, int is_value, int M, int N, int kth,
                                     uint64_t* bmp, uint32_t* idx, const uint32_t* dst_off, const uint32_t* dst_limit,
                                     mstf_half* nz, uint32_t* overflow, void* workspace, size_t workspace_bytes)

@@ -530,9 +530,9 @@ PyObject* compress_kv(Args& a)
     return tuple_of({ks.bmp, ks.idx, ks.nz_off, ks.total, ks.nz, vs.bmp, vs.idx, vs.nz_off, vs.total, vs.nz});
 }
 
-// (x, is_value, kth, M, cos, sin, rot, capacity or -1, landing, status, ws, strict) -> (bmp, idx, nz_off, total, nz, size or -1).
-// Capacity -1: room for the dense rows, and the call waits for the size (M > 0; landing: address of a pinned word), which is
-// negative if a workgroup gave up.
+// (x, is_value, kth, M, cos, sin, rot, capacity or -1, landing, waits, status, ws, strict) -> (bmp, idx, nz_off, total, nz, size or -1).
+// Capacity -1: room for the dense rows, and the size comes to the landing (M > 0; address of a pinned word).  waits: the call waits
+// for it, and returns the values cut to size; negative if a workgroup gave up.
 PyObject* compress_proj(Args& a)
 {
     const at::Tensor& x = a.tensor();
@@ -540,6 +540,7 @@ PyObject* compress_proj(Args& a)
     const at::Tensor *cos = a.maybe(), *sin = a.maybe(), *rot = a.maybe();
     const int64_t capacity = a.integer();
     int64_t* landing = static_cast<int64_t*>(a.pointer());
+    const bool waits = a.integer() != 0;
     const at::Tensor *status = a.maybe(), *ws = a.maybe();
     const bool strict = a.integer() != 0;
     a.done();
@@ -575,9 +576,11 @@ PyObject* compress_proj(Args& a)
                                ptr<uint32_t>(s.nz_off), ptr<uint64_t>(s.total), ptr<mstf_half>(s.nz), (uint64_t)cap, ptr<void>(ws),
                                room(ws), more...);
                  };
-                 return sized ? call(mstf_compress_proj_sized_f16, ptr<uint64_t>(status), bytes_of(status), landing, &size) : call(mstf_compress_proj_f16);
+                 if (!sized) return call(mstf_compress_proj_f16);
+                 return waits ? call(mstf_compress_proj_sized_f16, ptr<uint64_t>(status), bytes_of(status), landing, &size)
+                              : call(mstf_compress_proj_landing_f16, ptr<uint64_t>(status), bytes_of(status), landing);
              }),
-             sized ? "mstf_compress_proj_sized_f16" : "mstf_compress_proj_f16");
+             !sized ? "mstf_compress_proj_f16" : (waits ? "mstf_compress_proj_sized_f16" : "mstf_compress_proj_landing_f16"));
     return tuple_of({s.bmp, s.idx, s.nz_off, s.total, sized && size >= 0 ? s.nz.narrow(0, 0, size) : s.nz},
                     PyLong_FromLongLong(size));
 }
