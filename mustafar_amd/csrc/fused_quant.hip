@@ -72,8 +72,13 @@ constexpr bool quant_whole_fits()
 {
     return NM == 1 && kWholeWaves * quant_wave_lds<NM, BIT, G32>() <= kWholeLds;
 }
-template <int NM, int BIT, bool G32, bool MULTI, bool STEP = false, bool WHOLE = false>
-__global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribute__((amdgpu_waves_per_eu(WHOLE ? 4 : quant_occupancy<NM, BIT, G32>()))) void decode_attention_quant_kernel(
+// SHARE (few blocks): workgroups of four wavefronts that share a block, a key stage and a value stage each (shared_scores,
+// shared_store, fused_common.hpp); every block has a split slot then.  FOLDED: the sums of a stage start at zero and are added up in
+// the order of the stages, as the wavefronts that share a block do it - the same numbers bit for bit - for a call that would share
+// blocks and has no room for a slot per block.
+constexpr int quant_waves(bool share, bool whole) { return whole ? kWholeWaves : (share ? kShare : kFusedWaves); }
+template <int NM, int BIT, bool G32, bool MULTI, bool STEP = false, bool WHOLE = false, bool SHARE = false, bool FOLDED = false>
+__global__ __launch_bounds__(quant_waves(SHARE, WHOLE) * 64) __attribute__((amdgpu_waves_per_eu(WHOLE ? 4 : quant_occupancy<NM, BIT, G32>()))) void decode_attention_quant_kernel(
     const uint32_t* __restrict__ k_off, const uint32_t* __restrict__ v_off, const uint64_t* __restrict__ k_bmp,
     const uint64_t* __restrict__ v_bmp, size_t tstride, const int* __restrict__ tokens_dev, int nblk, int deal,
     const uint32_t* k_packed, const uint32_t* k_off_dma, const uint16_t* k_scales, const uint16_t* k_zeros,
@@ -101,7 +106,9 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
     constexpr int kStage = q_lds_bytes<BIT, G32>();  // image, two word buffers, two metadata buffers
     constexpr int kWaveLds = quant_wave_lds<NM, BIT, G32>();
     // one array on purpose (LDS-direct loads into several LDS objects make the compiler serialise them)
-    __shared__ __attribute__((aligned(16))) char lds_all[(WHOLE ? kWholeWaves : kFusedWaves) * kWaveLds];
+    __shared__ __attribute__((aligned(16))) char lds_all[quant_waves(SHARE, WHOLE) * kWaveLds];
+    static_assert(!SHARE || (!MULTI && !STEP && !WHOLE && kKeySubs == kShare), "a stage of each side per wavefront of a shared block");
+    static_assert(!SHARE || (kQLds >= NM * 1024 && kImgBytes >= NM * 1024), "room for the sums that the wavefronts exchange");
     static_assert(!WHOLE || (!STEP && fused_park_bytes<NM>() + NM * 2048 <= kWaveLds), "room behind the parked triples");
     const int lane = lane_id();
     const int wave = wave_id();
@@ -109,7 +116,8 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
     const int split = WHOLE ? wave / kFusedWaves : (tokens_dev ? (int)blockIdx.y : (int)blockIdx.x);
     const int kv = tokens_dev ? (int)blockIdx.x : (int)blockIdx.y;
     const int slot = WHOLE ? wave % kFusedWaves : wave;
-    BlockRange mine = {split * kFusedWaves + slot, 0};                // the token blocks of this wavefront
+    const int sub = SHARE ? wave : 0;                                 // its stages of the block
+    BlockRange mine = {SHARE ? split : split * kFusedWaves + slot, 0};  // the token blocks of this wavefront
     if constexpr (MULTI) mine = fused_blocks_of(nblk, deal, split, slot);
     const int tb = mine.first, nb = MULTI ? mine.count : nblk - tb;   // (wave-uniform)
     const bool active = nb > 0;
@@ -159,8 +167,9 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
             return r.off + (bnd_l == kKeySubs ? words : 0u);
         };
         uint32_t bnd = bound(bounds_of(offK, offV, bmK, bmV));
-        MetaLanes metaK = meta_lanes<G32>(k_off_dma + tile0, k_scales + tile0 * kPairs, k_zeros + tile0 * kPairs, bmK, lane);
-        MetaLanes metaV = meta_lanes<G32>(v_off_dma + tile0, v_scales + tile0 * kPairs, v_zeros + tile0 * kPairs, bmV, lane);
+        const size_t tile1 = tile0 + (size_t)sub * kSubTiles;
+        MetaLanes metaK = meta_lanes<G32>(k_off_dma + tile1, k_scales + tile1 * kPairs, k_zeros + tile1 * kPairs, k_bmp + tile1, lane);
+        MetaLanes metaV = meta_lanes<G32>(v_off_dma + tile1, v_scales + tile1 * kPairs, v_zeros + tile1 * kPairs, v_bmp + tile1, lane);
         const uint32_t lane4 = (uint32_t)lane * 4u;
         using Rank = StageRank<4 * NM, BIT, G32, false>;
         const uint32_t bits_at = Rank::bits_at(lane);
@@ -199,16 +208,51 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                 *reinterpret_cast<uint4*>(ql + row * kQRow + (lane & 15) * 16) = v;
             }
         }
-        uint2 touch = issue(0);
-
         typename Rank::Sums sums;  // of the phase (keys, one half of the values, the other half)
         const uint32_t qrow = sums.waddr(lds_addr(ql), kQRow, lane);
         const uint32_t prow = kPRow == kQRow ? qrow + (uint32_t)kQLds : sums.waddr(lds_addr(pl), kPRow, lane);
+        if constexpr (SHARE) {
+            // Both stages are requested at once: one round trip behind the boundaries'.
+            const uint64_t* bm[2] = {k_bmp + tile1, v_bmp + tile1};
+            uint32_t start[2], end[2];
+            uint2 bits[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                start[i] = (uint32_t)__builtin_amdgcn_readlane((int)bnd, 16 * i + sub);
+                end[i] = (uint32_t)__builtin_amdgcn_readlane((int)bnd, 16 * i + sub + 1);
+                uint32_t nw = end[i] - start[i];
+                nw = nw > (uint32_t)F::kWordsMax ? (uint32_t)F::kWordsMax : nw;  // never true for a well-formed cache
+                words_issue_flat<F::kWordsMax / 64>((i == 0 ? k_packed : v_packed) + start[i], nw,
+                                                    wordbuf_lds + (uint32_t)i * F::kWordBuf, (uint32_t)lane, lane4);
+                meta_issue_next<G32>(i == 0 ? metaK : metaV, metabuf + i * kMetaBytes);
+                bits[i] = Rank::bits_load(bm[i], bits_at);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(bits[0].x), "+v"(bits[0].y), "+v"(bits[1].x), "+v"(bits[1].y)::"memory");
+            f4_t part[NM], acc_k[NM];
+            float m_blk[NM], l_blk[NM];
+            auto stage = [&](int i, uint32_t w, uint32_t wgroup) {
+                const StageAt here = {lds_addr(metabuf), wordbuf_lds, (uint32_t)i * kMetaBytes, (uint32_t)i * F::kWordBuf, start[i],
+                                      end[i]};
+                rank.template stage<true>(here, bm[i], bits[i], w, wgroup, sums, lane, mode);
+#pragma unroll
+                for (int m = 0; m < NM; m++) part[m] = sums.joined(m);
+                wait_lgkm0();
+            };
+            stage(0, qrow + (uint32_t)(sub * kSubTiles * 2), 4u * kQRow);
+            shared_scores<NM>(lds_all + kStage, kWaveLds, sub, lane, part, acc_k);  // (the query rows have been read)
+            block_softmax<NM, kPRow>(acc_k, sqrt_d, 64, pl, lane, m_blk, l_blk);
+            stage(1, prow + (uint32_t)((sub & 1) * kSubTiles * 2), 4u * kPRow);
+            shared_store<NM>(lds_all, kWaveLds, sub, lane, part, m_blk, l_blk, groups, (size_t)kv * groups * nsplit + tb, nsplit,
+                             part_o, part_ml);  // (the image has been read, and only by this wavefront)
+            return;
+        }
+        uint2 touch = issue(0);
 
 #pragma unroll 1
         for (int r = 0; r < (MULTI ? nb : 1); r++) {
             const bool more = MULTI && r + 1 < nb;
             float fb[NM];
+            f4_t acc_k[NM], blk[NM];  // scores; a half of the block's output
             Raw coming;
             uint32_t bnd_next = bnd;
             static_for<kKeySubs + kValSubs>([&](auto nc) {
@@ -233,9 +277,10 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                     }
                 }
                 if (n == kKeySubs) {
-                    f4_t acc_k[NM];
+                    if constexpr (!FOLDED) {
 #pragma unroll
-                    for (int m = 0; m < NM; m++) acc_k[m] = sums.joined(m);
+                        for (int m = 0; m < NM; m++) acc_k[m] = sums.joined(m);
+                    }
                     float m_blk[NM], l_blk[NM];
                     block_softmax<NM, kPRow>(acc_k, sqrt_d, 64, pl, lane, m_blk, l_blk);
                     // (the fold of the block begins here, so that nothing of it waits in registers beside the running output)
@@ -262,15 +307,23 @@ __global__ __launch_bounds__((WHOLE ? kWholeWaves : kFusedWaves) * 64) __attribu
                                                 : prow + (uint32_t)(vs % kSubsPerHalf) * kSubTiles * 2u;
                 const StageAt here = {lds_addr(metabuf), wordbuf_lds, (uint32_t)(n & 1) * kMetaBytes, (uint32_t)(n & 1) * F::kWordBuf,
                                       start, end};
-                constexpr bool kStarts = n == 0 || n == kKeySubs || n == kKeySubs + kSubsPerHalf;
+                constexpr bool kStarts = FOLDED || n == 0 || n == kKeySubs || n == kKeySubs + kSubsPerHalf;
                 rank.template stage<kStarts>(here, bm, bits, w, n < kKeySubs ? 4u * kQRow : 4u * kPRow, sums, lane, mode);
+                if constexpr (FOLDED) {
+                    f4_t(&to)[NM] = n < kKeySubs ? acc_k : blk;
+#pragma unroll
+                    for (int m = 0; m < NM; m++) {
+                        if constexpr (n == 0 || (n >= kKeySubs && vs % kSubsPerHalf == 0)) to[m] = sums.joined(m);
+                        else to[m] += sums.joined(m);
+                    }
+                }
                 if (n >= kKeySubs && vs % kSubsPerHalf == kSubsPerHalf - 1) {  // the half is complete
 #pragma unroll
                     for (int m = 0; m < NM; m++) {
-                        const f4_t blk = sums.joined(m);
+                        if constexpr (!FOLDED) blk[m] = sums.joined(m);
                         f4_t& out_v = acc_v[m][vs / kSubsPerHalf];
 #pragma unroll
-                        for (int c = 0; c < 4; c++) out_v[c] = MULTI ? out_v[c] + blk[c] * fb[m] : blk[c];
+                        for (int c = 0; c < 4; c++) out_v[c] = MULTI ? out_v[c] + blk[m][c] * fb[m] : blk[m][c];
                     }
                 }
                 wait_lgkm0();  // every read of the image and of the staged buffers is done before they are rewritten
@@ -314,10 +367,10 @@ static void launch_decode_quant(hipStream_t st, dim3 grid, const uint64_t* k_bmp
                                 const uint16_t* v_scales, const uint16_t* v_zeros, const _Float16* q, _Float16* out,
                                 float* part_o, float* part_ml, int tokens, int groups, int ns, int write_final, float sq,
                                 int mode, int group_size, size_t tstride, const int32_t* tokens_dev, int deal,
-                                bool one_block, const StepArgs* step, bool whole)
+                                bool one_block, const StepArgs* step, bool whole, bool shared, bool folded)
 {
     const StepArgs sa = step ? *step : StepArgs{};
-    const unsigned threads = 64 * (whole ? kWholeWaves : kFusedWaves);
+    const unsigned threads = 64 * (unsigned)quant_waves(shared, whole);
 #define MSTF_FQ_LAUNCH(...)                                                                                              \
     hipLaunchKernelGGL((decode_attention_quant_kernel<NM, BIT, __VA_ARGS__>), grid, dim3(threads), 0, st, k_off, \
                        v_off, k_bmp, v_bmp, tstride, tokens_dev, tokens / 64, deal, k_packed, k_off, k_scales, k_zeros,   \
@@ -326,6 +379,15 @@ static void launch_decode_quant(hipStream_t st, dim3 grid, const uint64_t* k_bmp
     // the form for several / for one: 4 bits 16.4 / 15.4 us (two groups per tile 18.4 / 17.7), 8 bits 17.8 / 17.5 (20.1 / 20.6),
     // 2 bits 14.4 / 14.6 (17.4 / 16.5; 4096 blocks, one group: 17.9 / 18.3).
     constexpr bool kMulti = quant_multi<NM>(), kOne = kMulti && BIT == 2, kOneG32 = kMulti && BIT == 8;
+    if (shared) {
+        if (group_size == 32) MSTF_FQ_LAUNCH(true, false, false, false, true); else MSTF_FQ_LAUNCH(false, false, false, false, true);
+        return;
+    }
+    if (folded) {  // (so few blocks that no wavefront has more than one)
+        if (group_size == 32) MSTF_FQ_LAUNCH(true, false, false, false, false, true);
+        else MSTF_FQ_LAUNCH(false, false, false, false, false, true);
+        return;
+    }
     if constexpr (quant_whole_fits<NM, BIT, false>()) {
         if (whole && group_size == 64) {
             if (one_block) MSTF_FQ_LAUNCH(false, kOne, false, true); else MSTF_FQ_LAUNCH(false, kMulti, false, true);
@@ -407,7 +469,7 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
                         const mstf_half* v_zeros, const mstf_half* q, mstf_half* out, int tokens, int head_dim, int Bq,
                         int groups, int bit, int dequant_mode, void* workspace, int ns, int nst, int write_final,
                         int group_size = 64, size_t tile_stride = 0, const int32_t* tokens_dev = nullptr,
-                        const StepArgs* step = nullptr, bool whole = false)
+                        const StepArgs* step = nullptr, bool whole = false, bool shared = false, bool folded = false)
 {
     const int Bkv = Bq / groups;
     // (token count in device memory: the kernel deals the blocks out itself, from the number of workgroups that fill the chip)
@@ -432,7 +494,7 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
 #define MSTF_FQ(NMV, BITV)                                                                                             \
     launch_decode_quant<NMV, BITV>(st, grid, k_bmp, k_packed, k_tile_off, ks, kz, v_bmp, v_packed, v_tile_off, vs, vz, \
                                    qh, oh, part_o, part_ml, tokens, groups, nst, write_final, sq, dequant_mode, group_size, \
-                                   tstride, tokens_dev, deal, one_block, step, whole)
+                                   tstride, tokens_dev, deal, one_block, step, whole, shared, folded)
     if (groups <= 4) {
         if (bit == 2) MSTF_FQ(1, 2); else if (bit == 4) MSTF_FQ(1, 4); else MSTF_FQ(1, 8);
     } else {
@@ -459,16 +521,23 @@ static int decode_attention_quant_impl(void* stream, const uint64_t* k_bmp, cons
     if (!workspace || workspace_bytes < fused_workspace_need(tokens, 0, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
-    const int ns = quant_nsplit(tokens, Bq / groups, groups, bit, group_size);
+    // Few blocks are shared, also where one split would leave no merge to launch behind it: with half a dozen stages' arithmetic
+    // less in a wavefront's chain the two launches are the faster form, call by call and recorded alike (us, 70 %, a wavefront per block /
+    // shared; recorded unless said: 2 bits, 8 heads x 2 blocks 12.2 / 9.1, call by call 10.9 / 10.3, 8 x 8 13.2 / 9.1, 12.0 / 10.5, 8 x 16
+    // 15.3 / 9.2, 24 x 32 15.3 / 11.8, 16 x 64 15.5 / 13.5, 8 x 128 15.8 / 15.1, eight query heads 8 x 16 16.8 / 10.1, 96 x 8 and 8 x 96 17.3 / 14.8;
+    // 8 bits, two groups, eight query heads 22.3 / 11.5).  The rule is the fp16 kernel's; at its most blocks the forms are alike.
+    const bool few = fused_shares_blocks(tokens, Bq / groups, groups);
+    const bool shared = few && fused_share_fits(tokens, 0, Bq, workspace_bytes);
+    const int ns = shared ? tokens / 64 : quant_nsplit(tokens, Bq / groups, groups, bit, group_size);
     // with one split and no (max, sum) requested the kernel writes the final output itself
     // (and with a workgroup per head)
-    const bool whole = !lse_out && quant_whole(bit, group_size) && fused_whole_head(tokens / 64, ns, Bq / groups, groups, false);
-    const int write_final = whole || (ns == 1 && !lse_out) ? 1 : 0;
+    const bool whole = !shared && !lse_out && quant_whole(bit, group_size) && fused_whole_head(tokens / 64, ns, Bq / groups, groups, false);
+    const int write_final = whole || (!shared && ns == 1 && !lse_out) ? 1 : 0;
     rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
                       out, tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, ns, write_final, group_size, 0, nullptr,
-                      nullptr, whole);
+                      nullptr, whole, shared, few && !shared);
     if (rc != MSTF_OK || write_final) return rc;
-    return merge_splits(st, workspace, out, lse_out, ns, head_dim, Bq);
+    return merge_splits(st, workspace, out, lse_out, ns, head_dim, Bq, shared ? ns : 0);
 }
 
 extern "C" int mstf_decode_attention_quant(void* stream, const uint64_t* k_bmp, const uint32_t* k_packed,

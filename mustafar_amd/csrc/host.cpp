@@ -206,7 +206,7 @@ PyObject* decode_attention_quant(Args& a)
     a.done();
     const int D = as_int(q.size(-1)), Bq = as_int(q.numel() / D);
     const int tokens = as_int(s[0]->size(1) * 64 / D);
-    const size_t need = attention_least(tokens, 0, Bq);
+    const size_t need = groups > 0 ? mstf_decode_attention_workspace_bytes(tokens, D, Bq, groups) : attention_least(tokens, 0, Bq);
     if (!enough(ws, need, strict)) return wants(need);
     const int gs = group_size_of(*s[0], *s[3], *s[4]);
     check_rt(group_size_of(*s[5], *s[8], *s[9]) == gs, "key side and value side must use the same group size.");
