@@ -678,9 +678,6 @@ class QuantSparseKVCache(SparseKVCache):
         self.bit, self.dequant_mode = bit, dequant_mode
         # self.k / self.v: 7-element lists [bitmaps, tile_offsets, packed, counts, units, scales, zeros]
 
-    def _step_workspace_bytes(self, tokens, rows):
-        return ops.attention_workspace_least(tokens, self.residual_length + CHUNK, rows)
-
     def _step_device(self, q_in, k_in, v_in, cos, sin):
         from . import mustafar_package_quant as mpq
         return mpq.decode_step_quant_pool(self.k_pool, self.v_pool, q_in, k_in, v_in, self._kbuf, self._vbuf,
@@ -701,7 +698,9 @@ class QuantSparseKVCache(SparseKVCache):
         """As SparseKVCache.prefill_proj for the rotation - the keys are rotated in place by the compressor's kernel,
         in the projection's own layout - while the quantised producer, which takes contiguous rows like the
         reference's, goes through prefill on the transposed views."""
-        ws = self._workspace(kx.device, kx.shape[0] * kx.shape[2], kx.shape[1] // 64 * 64)
+        L = kx.shape[1]     # (the most room is not the longest context's: see fused_shares_blocks, csrc/fused_common.hpp)
+        Lc = ((L - self.residual_length) // CHUNK) * CHUNK if L > self.residual_length else 0
+        ws = self._workspace(kx.device, kx.shape[0] * kx.shape[2], Lc)
         ops.compress_proj(kx, False, self.kth_k, 0, cos, sin, ws=ws)      # M = 0: rotation only
         K, V = kx.transpose(1, 2), vx.transpose(1, 2)
         self.prefill(K, V)

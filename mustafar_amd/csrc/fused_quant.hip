@@ -92,6 +92,7 @@ __global__ __launch_bounds__(quant_waves(SHARE, WHOLE) * 64) __attribute__((amdg
     // pre-allocated for more.  tokens_dev (nullable): the number of cached tokens is read from device memory, at most
     // nblk blocks of it; the launch is then sized for the capacity.
     using F = QFmt<BIT>;
+    const int blocks_room = nblk;  // (SHARE: split slots of blocks)
     if (tokens_dev) {
         const int valid = *tokens_dev / 64;
         nblk = valid < nblk ? valid : nblk;
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(quant_waves(SHARE, WHOLE) * 64) __attribute__((amdg
     constexpr int kWaveLds = quant_wave_lds<NM, BIT, G32>();
     // one array on purpose (LDS-direct loads into several LDS objects make the compiler serialise them)
     __shared__ __attribute__((aligned(16))) char lds_all[quant_waves(SHARE, WHOLE) * kWaveLds];
-    static_assert(!SHARE || (!MULTI && !STEP && !WHOLE && kKeySubs == kShare), "a stage of each side per wavefront of a shared block");
+    static_assert(!SHARE || (!MULTI && !WHOLE && kKeySubs == kShare), "a stage of each side per wavefront of a shared block");
     static_assert(!SHARE || (kQLds >= NM * 1024 && kImgBytes >= NM * 1024), "room for the sums that the wavefronts exchange");
     static_assert(!WHOLE || (!STEP && fused_park_bytes<NM>() + NM * 2048 <= kWaveLds), "room behind the parked triples");
     const int lane = lane_id();
@@ -128,6 +129,26 @@ __global__ __launch_bounds__(quant_waves(SHARE, WHOLE) * 64) __attribute__((amdg
     char* ql = my + kStage;
     char* pl = ql + kQLds;
     const uint32_t lbase = lds_addr(my);
+
+    if constexpr (STEP && SHARE) {
+        // (the blocks of the dense window get workgroups of their own behind the splits, see decode_attention_kernel)
+        if (split >= st.wg0) {
+            const int wblk = (split - st.wg0) * kShare + wave;
+            if (wblk < (st.win_len + 63) / 64) {
+                stage_query_rotated<kQRow>(ql, st, kv, groups, lane);
+                step_window_wave<NM, kQRow, kPRow, 8>(my, ql, pl, st, part_o, part_ml, kv, groups, nsplit, wblk, step_window_count(st),
+                                                      sqrt_d, lane);
+            }
+            return;  // (the whole workgroup: no barrier is left waiting)
+        }
+    }
+    if constexpr (SHARE) {
+        if (!active) {  // (wave-uniform, and the same for the workgroup)
+            if (wave == 0 && tb < blocks_room)
+                store_neutral<NM>(lane, groups, (size_t)kv * groups * nsplit + tb, nsplit, part_o, part_ml);
+            return;
+        }
+    }
 
     f4_t acc_v[NM][2];
     float m_run[NM], l_run[NM];
@@ -330,7 +351,7 @@ __global__ __launch_bounds__(quant_waves(SHARE, WHOLE) * 64) __attribute__((amdg
             });
         }
     }
-    if constexpr (STEP) {
+    if constexpr (STEP && !SHARE) {
         // The dense window: block i goes to wavefront number i / ns of split i % ns, behind its compressed block (see
         // decode_attention_kernel); the value rows pass through the room of the tile image, eight at a time.  The
         // step's arguments are fetched again here, through a pointer the compiler cannot see through, so that they
@@ -380,11 +401,14 @@ static void launch_decode_quant(hipStream_t st, dim3 grid, const uint64_t* k_bmp
     // 2 bits 14.4 / 14.6 (17.4 / 16.5; 4096 blocks, one group: 17.9 / 18.3).
     constexpr bool kMulti = quant_multi<NM>(), kOne = kMulti && BIT == 2, kOneG32 = kMulti && BIT == 8;
     if (shared) {
-        if (group_size == 32) MSTF_FQ_LAUNCH(true, false, false, false, true); else MSTF_FQ_LAUNCH(false, false, false, false, true);
+        if (step) MSTF_FQ_LAUNCH(false, false, true, false, true);
+        else if (group_size == 32) MSTF_FQ_LAUNCH(true, false, false, false, true);
+        else MSTF_FQ_LAUNCH(false, false, false, false, true);
         return;
     }
     if (folded) {  // (so few blocks that no wavefront has more than one)
-        if (group_size == 32) MSTF_FQ_LAUNCH(true, false, false, false, false, true);
+        if (step) MSTF_FQ_LAUNCH(false, false, true, false, false, true);
+        else if (group_size == 32) MSTF_FQ_LAUNCH(true, false, false, false, false, true);
         else MSTF_FQ_LAUNCH(false, false, false, false, false, true);
         return;
     }
@@ -461,6 +485,28 @@ static int quant_nsplit(int tokens, int Bkv, int groups, int bit, int group_size
     return fused_splits_step(tokens / 64, fused_fill(Bkv, quant_resident(groups, bit, group_size)), window);
 }
 
+// How a launch takes its blocks: shared by four wavefronts, a split slot each, where they are few; without room for those slots
+// (folded) the same numbers come from a wavefront per block.  window: tokens of the dense window behind them.
+// Shared also where one split would leave no merge to launch behind it: with three quarters of the stages gone from a wavefront's
+// chain the two launches are the faster form, call by call and recorded alike (us, 70 %, a wavefront per block / shared; recorded
+// unless said: 2 bits, 8 heads x 2 blocks 12.2 / 9.1, call by call 10.9 / 10.3, 8 x 8 13.2 / 9.1, 12.0 / 10.5, 8 x 16 15.3 / 9.2, 24 x 32
+// 15.3 / 11.8, 16 x 64 15.5 / 13.5, 8 x 128 15.8 / 15.1, eight query heads 8 x 16 16.8 / 10.1, 8 x 96 17.3 / 14.8; 8 bits, two groups, eight
+// query heads 22.3 / 11.5; a step with a window of 300: 2 bits 8 x 8 21.6 / 11.7, 24 x 32 19.8 / 15.6, 8 bits 8 x 60 23.3 / 15.0).  The rule is
+// the fp16 kernel's (fused_shares_blocks); at its most blocks the forms are alike.
+struct QuantPlan {
+    bool shared, folded;
+    int ns;
+    int merge_blocks() const { return shared ? ns : 0; }
+};
+static QuantPlan quant_plan(int tokens, int Bq, int groups, int bit, int group_size, int window, int window_in_launch,
+                            size_t workspace_bytes)
+{
+    const int Bkv = Bq / groups;
+    const bool few = fused_shares_blocks(tokens, Bkv, groups, Bkv * ((window_blocks(window) + kShare - 1) / kShare));
+    if (few && fused_share_fits(tokens, window, Bq, workspace_bytes)) return {true, false, tokens / 64};
+    return {false, few, quant_nsplit(tokens, Bkv, groups, bit, group_size, window_blocks(window_in_launch))};
+}
+
 // The quantised kernel over the compressed tokens: fills split slots 0 .. ns-1 (ns: quant_nsplit) of a workspace
 // with nst slots per query row (or writes the final output when write_final).
 static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k_packed, const uint32_t* k_tile_off,
@@ -478,11 +524,15 @@ static int quant_launch(hipStream_t st, const uint64_t* k_bmp, const uint32_t* k
     // no wavefront has more than one block (and none has with fewer tokens, should their number be in device memory)
     const bool one_block = fused_splits(tokens / 64, fill) == fused_nsplit(tokens);
     // step: the launch is a whole decode step; its window blocks are dealt out over the wavefronts of a head
-    if (step && (group_size != 64 || window_blocks(step->win_len) > ns * kFusedWaves)) return MSTF_EUNSUPPORTED;
+    // (or get workgroups of their own behind those of shared blocks, which a call may go without: they take no longer windows)
+    const int window = step ? window_blocks(step->win_len) : 0;
+    const int walks = shared && step ? quant_nsplit(tokens, Bkv, groups, bit, group_size, window) : ns;
+    if (step && (group_size != 64 || window > walks * kFusedWaves)) return MSTF_EUNSUPPORTED;
+    const int wgs = ns + (shared ? (window + kShare - 1) / kShare : 0);
     // tile_stride / tokens_dev: a cache pre-allocated for `tokens` tokens that holds *tokens_dev of them (see the kernel)
     float* part_o = reinterpret_cast<float*>(workspace);
     float* part_ml = part_o + (size_t)Bq * nst * head_dim;
-    const dim3 grid = tokens_dev ? dim3((unsigned)Bkv, (unsigned)ns) : dim3(whole ? 1u : (unsigned)ns, (unsigned)Bkv);
+    const dim3 grid = tokens_dev ? dim3((unsigned)Bkv, (unsigned)wgs) : dim3(whole ? 1u : (unsigned)wgs, (unsigned)Bkv);
     const size_t tstride = tile_stride ? tile_stride : (size_t)tokens * head_dim / 64;
     const _Float16* qh = reinterpret_cast<const _Float16*>(q);
     _Float16* oh = reinterpret_cast<_Float16*>(out);
@@ -521,23 +571,17 @@ static int decode_attention_quant_impl(void* stream, const uint64_t* k_bmp, cons
     if (!workspace || workspace_bytes < fused_workspace_need(tokens, 0, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
-    // Few blocks are shared, also where one split would leave no merge to launch behind it: with half a dozen stages' arithmetic
-    // less in a wavefront's chain the two launches are the faster form, call by call and recorded alike (us, 70 %, a wavefront per block /
-    // shared; recorded unless said: 2 bits, 8 heads x 2 blocks 12.2 / 9.1, call by call 10.9 / 10.3, 8 x 8 13.2 / 9.1, 12.0 / 10.5, 8 x 16
-    // 15.3 / 9.2, 24 x 32 15.3 / 11.8, 16 x 64 15.5 / 13.5, 8 x 128 15.8 / 15.1, eight query heads 8 x 16 16.8 / 10.1, 96 x 8 and 8 x 96 17.3 / 14.8;
-    // 8 bits, two groups, eight query heads 22.3 / 11.5).  The rule is the fp16 kernel's; at its most blocks the forms are alike.
-    const bool few = fused_shares_blocks(tokens, Bq / groups, groups);
-    const bool shared = few && fused_share_fits(tokens, 0, Bq, workspace_bytes);
-    const int ns = shared ? tokens / 64 : quant_nsplit(tokens, Bq / groups, groups, bit, group_size);
+    const QuantPlan plan = quant_plan(tokens, Bq, groups, bit, group_size, 0, 0, workspace_bytes);
+    const int ns = plan.ns;
     // with one split and no (max, sum) requested the kernel writes the final output itself
     // (and with a workgroup per head)
-    const bool whole = !shared && !lse_out && quant_whole(bit, group_size) && fused_whole_head(tokens / 64, ns, Bq / groups, groups, false);
-    const int write_final = whole || (!shared && ns == 1 && !lse_out) ? 1 : 0;
+    const bool whole = !plan.shared && !lse_out && quant_whole(bit, group_size) && fused_whole_head(tokens / 64, ns, Bq / groups, groups, false);
+    const int write_final = whole || (!plan.shared && ns == 1 && !lse_out) ? 1 : 0;
     rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
                       out, tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, ns, write_final, group_size, 0, nullptr,
-                      nullptr, whole, shared, few && !shared);
+                      nullptr, whole, plan.shared, plan.folded);
     if (rc != MSTF_OK || write_final) return rc;
-    return merge_splits(st, workspace, out, lse_out, ns, head_dim, Bq, shared ? ns : 0);
+    return merge_splits(st, workspace, out, lse_out, ns, head_dim, Bq, plan.merge_blocks());
 }
 
 extern "C" int mstf_decode_attention_quant(void* stream, const uint64_t* k_bmp, const uint32_t* k_packed,
@@ -586,23 +630,25 @@ extern "C" int mstf_decode_attention_window_quant(
     if (!workspace || workspace_bytes < fused_workspace_need(tokens, win_len, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
-    int rc, ns = 0;
+    int rc;
+    QuantPlan plan = {false, false, 0};
     if (tokens > 0) {
         rc = quant_check(k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
                          tokens, head_dim, Bq, groups, bit, capacity, dequant_mode);
         if (rc != MSTF_OK) return rc;
-        ns = quant_nsplit(tokens, Bq / groups, groups, bit, 64);
+        plan = quant_plan(tokens, Bq, groups, bit, 64, win_len, 0, workspace_bytes);
     }
-    const int nst = ns + window_blocks(win_len);
+    const int ns = plan.ns, nst = ns + window_blocks(win_len);
     if (tokens > 0) {
         rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales,
-                          v_zeros, q, nullptr, tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, nst, 0);
+                          v_zeros, q, nullptr, tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, nst, 0, 64, 0, nullptr,
+                          nullptr, false, plan.shared, plan.folded);
         if (rc != MSTF_OK) return rc;
     }
     if ((rc = window_launch(st, k_win, v_win, q, workspace, win_len, win_len_dev, win_stride, head_dim, Bq, groups, nst,
                             ns)) != MSTF_OK)
         return rc;
-    return merge_splits(st, workspace, out, lse_out, nst, head_dim, Bq);
+    return merge_splits(st, workspace, out, lse_out, nst, head_dim, Bq, plan.merge_blocks());
 }
 
 extern "C" int mstf_decode_attention_window_quant_pool(
@@ -630,15 +676,16 @@ extern "C" int mstf_decode_attention_window_quant_pool(
                          max_tokens, head_dim, Bq, groups, bit, capacity, dequant_mode);
     if (rc != MSTF_OK) return rc;
     const int wblk = window_blocks(win_len);
-    const int ns = quant_nsplit(max_tokens, Bq / groups, groups, bit, 64, wblk), nst = ns + wblk;
+    const QuantPlan plan = quant_plan(max_tokens, Bq, groups, bit, 64, win_len, win_len, workspace_bytes);
+    const int ns = plan.ns, nst = ns + wblk;
     rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
                       nullptr, max_tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, nst, 0, 64,
-                      (size_t)tile_capacity, tokens_dev);
+                      (size_t)tile_capacity, tokens_dev, nullptr, false, plan.shared, plan.folded);
     if (rc != MSTF_OK) return rc;
     if ((rc = window_launch(st, k_win, v_win, q, workspace, win_len, win_len_dev, win_stride, head_dim, Bq, groups, nst,
                             ns)) != MSTF_OK)
         return rc;
-    return merge_splits(st, workspace, out, lse_out, nst, head_dim, Bq);
+    return merge_splits(st, workspace, out, lse_out, nst, head_dim, Bq, plan.merge_blocks());
 }
 
 extern "C" int mstf_decode_step_quant_pool(
@@ -675,7 +722,8 @@ extern "C" int mstf_decode_step_quant_pool(
     if (rc != MSTF_OK) return rc;
     hipStream_t st = as_stream(stream);
     const int wblk = window_blocks(win_len);
-    const int ns = quant_nsplit(max_tokens, Bq / groups, groups, bit, 64, wblk), nst = ns + wblk;
+    const QuantPlan plan = quant_plan(max_tokens, Bq, groups, bit, 64, win_len, win_len, workspace_bytes);
+    const int ns = plan.ns, nst = ns + wblk;
     StepArgs sa = {};
     sa.q_in = reinterpret_cast<const _Float16*>(q_in);
     sa.k_in = reinterpret_cast<const _Float16*>(k_in);
@@ -694,9 +742,10 @@ extern "C" int mstf_decode_step_quant_pool(
     sa.win_stride = win_stride;
     sa.n_kv = n_kv;
     sa.ns = ns;
+    sa.wg0 = ns;
     rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros,
                       q_in, nullptr, max_tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, nst, 0, 64,
-                      (size_t)tile_capacity, tokens_dev, &sa);
+                      (size_t)tile_capacity, tokens_dev, &sa, false, plan.shared, plan.folded);
     if (rc != MSTF_OK) return rc;
-    return merge_splits(st, workspace, out, lse_out, nst, head_dim, Bq);
+    return merge_splits(st, workspace, out, lse_out, nst, head_dim, Bq, plan.merge_blocks());
 }

@@ -302,7 +302,7 @@ PyObject* decode_step_quant(Args& a)
     for (auto& t : s) t = &a.tensor();
     const Step e(a);
     a.done();
-    const size_t need = attention_least(e.max_tokens, e.win_len, e.Bq);
+    const size_t need = mstf_decode_attention_window_workspace_bytes(e.max_tokens, e.win_len, e.D, e.Bq, e.n_q / e.n_kv);
     if (!enough(e.ws, need, e.strict)) return wants(need);
     check_rt(bit > 0, "bit must be positive");
     at::Tensor o = e.output();

@@ -85,6 +85,11 @@ def decode_attention_quant(key_side, value_side, q, num_key_value_groups, bit, d
                      int(num_key_value_groups), int(bit), int(dequant_mode), out, lse)
 
 
+def _window_workspace(q, tokens, win_len, rows, groups, ws):
+    best = lib().mstf_decode_attention_window_workspace_bytes(tokens, win_len, q.shape[-1], rows, groups)
+    return ops.workspace(q.device, best or ops.attention_workspace_least(tokens, win_len, rows), ws, (tokens, win_len, rows))
+
+
 def decode_attention_window_quant(key_side, value_side, q, k_win, v_win, win_len, num_key_value_groups, bit,
                                   dequant_mode=0, out=None, lse=None, win_len_dev=None, ws=None):
     """The whole attention of a decode step over [quantised compressed tokens | dense window] in three launches
@@ -107,7 +112,7 @@ def decode_attention_window_quant(key_side, value_side, q, k_win, v_win, win_len
                 vo.data_ptr(), vs.data_ptr(), vz.data_ptr()]
     else:
         tokens, ptrs = 0, [None] * 10
-    ws = ops.workspace(q.device, ops.attention_workspace_least(tokens, int(win_len), Bq), ws)
+    ws = _window_workspace(q, tokens, int(win_len), Bq, int(num_key_value_groups), ws)
     check(L.mstf_decode_attention_window_quant(
         ops._stream(), *ptrs, q.contiguous().data_ptr(), k_win.data_ptr(), v_win.data_ptr(),
         int(win_len), win_len_dev.data_ptr() if win_len_dev is not None else None, int(k_win.shape[1]), o.data_ptr(),
@@ -128,7 +133,7 @@ def decode_attention_window_quant_pool(k_pool, v_pool, q, k_win, v_win, win_len,
     Bq = q.numel() // D
     L = lib()
     o = torch.empty((Bq, D), dtype=torch.float16, device=q.device) if out is None else out
-    ws = ops.workspace(q.device, ops.attention_workspace_least(k_pool.max_tokens, int(win_len), Bq), ws)
+    ws = _window_workspace(q, k_pool.max_tokens, int(win_len), Bq, int(num_key_value_groups), ws)
     ptrs = []
     for p in (k_pool, v_pool):
         ptrs += [p.bmp_store.data_ptr(), p.packed.data_ptr(), p.off_store.data_ptr(), p.scales_store.data_ptr(),

@@ -66,3 +66,32 @@ def dequantised(side, tokens, is_value, bit):
     if not is_value:
         return x.transpose(2, 3).reshape(H, tokens, D)
     return x.view(H, tokens // 64, 2, 64, 64).transpose(2, 3).reshape(H, tokens, D)
+
+
+@pytest.mark.parametrize("bit", [2, 4, 8])
+@pytest.mark.parametrize("heads,groups,tokens,window", [(4, 4, 768, 60), (2, 8, 256, 100), (64, 4, 1024, 1), (61, 4, 1024, 130)])
+def test_step_and_windows_without_room(bit, heads, groups, tokens, window):
+    """A step over pools, with room for a slot per block and without: the same numbers, and those of append and attention apart.
+    64 heads of 16 blocks and a window block each are one workgroup too many for the shared form, 61 too few heads for that."""
+    from mustafar_amd import mustafar_package_quant as mq, ops
+    from mustafar_amd.cache import QuantSparseKVCache
+    g = torch.Generator(device="cuda").manual_seed(tokens + bit)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda", dtype=torch.float16)  # noqa: E731
+    K, V = rand(1, heads, tokens + window, D), rand(1, heads, tokens + window, D)
+    cache = QuantSparseKVCache(groups, D, 0.7, 0.7, window, bit=bit, window_kernel=True, max_tokens=tokens + 256)
+    cache.prefill(K, V)
+    q, k, v = rand(1, heads * groups * D), rand(1, heads * D), rand(1, heads * D)
+    rows, win = heads * groups, cache._kbuf.shape[1]
+    length = torch.tensor([window + 1], dtype=torch.int32, device="cuda")
+    outs = []
+    for room in (ops.attention_workspace_least(tokens + 256, win, rows), 16 << 20):
+        kw, vw = cache._kbuf.clone(), cache._vbuf.clone()
+        for step in (True, False):
+            ws = torch.empty(room, dtype=torch.uint8, device="cuda")
+            if step:
+                outs.append(mq.decode_step_quant_pool(cache.k_pool, cache.v_pool, q, k, v, kw, vw, win, win_len_dev=length, ws=ws))
+            else:
+                outs.append(mq.decode_attention_window_quant_pool(cache.k_pool, cache.v_pool, q.view(rows, D), kw, vw, win, groups,
+                                                                  win_len_dev=length, ws=ws))
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    assert outs[0].isfinite().all()
