@@ -466,6 +466,7 @@ class SparseKVCache:
         attention (models/llama_mustafar_kernel.py:373-374, 531-560 in one pass over K and one over V)."""
         bs, L, n_kv, D = kx.shape
         Lc = ((L - self.residual_length) // CHUNK) * CHUNK if L > self.residual_length else 0
+        sized = None
         if self.max_tokens > 0:
             if self.k_pool is None:
                 self._make_pools(bs * n_kv, D, kx.device)
@@ -479,11 +480,12 @@ class SparseKVCache:
             ck, _ = ops.compress_proj(kx, False, self.kth_k, Lc, cos, sin, ws=ws)
             if Lc > 0:
                 cv, _ = ops.compress_proj(vx, True, self.kth_v, Lc, ws=ws)
-                self.k, self.v = ck, cv
+
+                def sized():
+                    ck.nz, cv.nz
+                    self.k, self.v = ck, cv
         K, V = kx.transpose(1, 2), vx.transpose(1, 2)
-        self._prefill_window(K, V, Lc)
-        if self.max_tokens == 0 and Lc > 0:     # cut to size, or an error where a wait ran out, behind all launches
-            self.k.nz, self.v.nz
+        self._prefill_window(K, V, Lc, sized)
         return K, V
 
     def prefill(self, K, V):
@@ -494,29 +496,35 @@ class SparseKVCache:
             self._grow(K[:, :, :Lc].contiguous(), V[:, :, :Lc].contiguous())
         self._prefill_window(K, V, Lc)
 
-    def _prefill_window(self, K, V, Lc):
+    def _prefill_window(self, K, V, Lc, sized=None):
+        """sized: called behind the launches and in front of everything that says the cache is filled (it may raise)."""
         L = K.shape[2]
-        self.compressed_length, self.kv_len = Lc, L
+        wlen = L - Lc
         if self.window_kernel:
             bs, n_kv, _, D = K.shape
             if self.max_tokens > 0 and self.k_pool is None:
                 # nothing compressed yet: the (empty) pools exist from the start, so the attention call never changes form
                 self._make_pools(bs * n_kv, D, K.device)
             self._workspace(K.device, bs * n_kv, Lc)
-            cap = max(self.residual_length + CHUNK, L - Lc)   # the window never holds more before a chunk leaves
-            self._kbuf = torch.empty((bs * n_kv, cap, D), dtype=torch.float16, device=K.device)
-            self._vbuf = torch.empty_like(self._kbuf)
-            self._wlen = L - Lc
-            self._wlen_dev = torch.full((1,), self._wlen, dtype=torch.int32, device=K.device)   # valid rows
+            cap = max(self.residual_length + CHUNK, wlen)   # the window never holds more before a chunk leaves
+            kbuf = torch.empty((bs * n_kv, cap, D), dtype=torch.float16, device=K.device)
+            vbuf = torch.empty_like(kbuf)
+            wlen_dev = torch.full((1,), wlen, dtype=torch.int32, device=K.device)   # valid rows
+            wovf = torch.zeros((1,), dtype=torch.int32, device=K.device)   # set by an append past the buffer
+            kbuf[:, :wlen] = K[:, :, Lc:].reshape(bs * n_kv, wlen, D)
+            vbuf[:, :wlen] = V[:, :, Lc:].reshape(bs * n_kv, wlen, D)
+        else:
+            k_win, v_win = K[:, :, Lc:].contiguous().clone(), V[:, :, Lc:].contiguous().clone()
+        if sized is not None:
+            sized()
+        self.compressed_length, self.kv_len = Lc, L
+        if self.window_kernel:
+            self._kbuf, self._vbuf, self._wlen, self._wlen_dev, self._wovf = kbuf, vbuf, wlen, wlen_dev, wovf
             self._owns_clock, self._clock_shared = True, False
-            self._wovf = torch.zeros((1,), dtype=torch.int32, device=K.device)   # set by an append past the buffer
-            self._kbuf[:, :self._wlen] = K[:, :, Lc:].reshape(bs * n_kv, self._wlen, D)
-            self._vbuf[:, :self._wlen] = V[:, :, Lc:].reshape(bs * n_kv, self._wlen, D)
             self._shape = (bs, n_kv, D)
             self._window_views()
-            return
-        self.k_win = K[:, :, Lc:].contiguous().clone()
-        self.v_win = V[:, :, Lc:].contiguous().clone()
+        else:
+            self.k_win, self.v_win = k_win, v_win
 
     def _window_views(self):
         bs, n_kv, D = self._shape
