@@ -477,13 +477,13 @@ class SparseKVCache:
                 self._pool_views()
         else:
             ws = self._workspace(kx.device, bs * n_kv, Lc)
-            ck, _ = ops.compress_proj(kx, False, self.kth_k, Lc, cos, sin, ws=ws)
             if Lc > 0:
-                cv, _ = ops.compress_proj(vx, True, self.kth_v, Lc, ws=ws)
+                settle = ops.compress_proj_both(kx, vx, self.kth_k, self.kth_v, Lc, cos, sin, ws=ws)
 
                 def sized():
-                    ck.nz, cv.nz
-                    self.k, self.v = ck, cv
+                    self.k, self.v = settle()
+            else:
+                ops.compress_proj(kx, False, self.kth_k, 0, cos, sin, ws=ws)
         K, V = kx.transpose(1, 2), vx.transpose(1, 2)
         self._prefill_window(K, V, Lc, sized)
         return K, V

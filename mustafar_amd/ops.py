@@ -203,20 +203,20 @@ def kth_from_sparsity(sparsity, head_dim):
     return max(1, int(sparsity * head_dim))
 
 
+def _gave_up(total):
+    return not 0 <= total <= 1 << 62
+
+
 _GAVE_UP = "the compressor gave up waiting for an earlier workgroup; the packed values are incomplete"
 
 
 class CompressedKV:
     """One side (K or V) of the compressed cache, flat on the device.
 
-    bmp int64 [B, T], idx int32 [B, T+1], nz fp16 flat, nz_off int32 [B] (16-byte units).
-
-    A call that cuts nz to size may return before that is known (`cut`): nz and total_halfs are then made, and waited for, when they
-    are first asked for."""
+    bmp int64 [B, T], idx int32 [B, T+1], nz fp16 flat, nz_off int32 [B] (16-byte units)."""
 
     _landing = None     # _LandingPair that gets the total too; given back once the total is read
     _used = None        # the total, from there
-    _uncut = None       # (values, total) of a call whose size has not been asked for
 
     def __init__(self, bmp, idx, nz, nz_off, tokens, head_dim, is_value, total_halfs=None, landing=None):
         self.bmp, self.idx, self.nz, self.nz_off = bmp, idx, nz, nz_off
@@ -224,25 +224,8 @@ class CompressedKV:
         self.total_halfs = total_halfs
         self._landing = landing
 
-    @classmethod
-    def cut(cls, bmp, idx, nz, nz_off, tokens, head_dim, is_value, total, landing):
-        c = cls(bmp, idx, nz, nz_off, tokens, head_dim, is_value, total, landing)
-        del c.nz, c.total_halfs
-        c._uncut = (nz, total)
-        return c
-
-    def __getattr__(self, name):    # (of attributes that are not there)
-        if name not in ("nz", "total_halfs") or self._uncut is None:
-            raise AttributeError(name)
-        nz, total = self._uncut
-        n = self._size(total)
-        self.nz, self.total_halfs, self._used, self._uncut = nz[:n], n, n, None
-        return self.__dict__[name]
-
     def __getstate__(self):
         # a copy has the total from its own tensor (total_halfs): the words that it landed in go with the call
-        if self._uncut is not None:
-            self.nz
         return {name: value for name, value in self.__dict__.items() if name != "_landing"}
 
     @property
@@ -253,25 +236,20 @@ class CompressedKV:
         """Number of fp16 values in use (the total is read once; the values themselves may be on their way yet, see above).
         The one-pass compressor reports a wait that ran out - which the dispatch order rules out - as a total of all ones:
         that raises here."""
-        if self._used is None and self._uncut is not None:
-            self.nz
+        landing = self._landing     # (in front of _used, which is set before this one goes: another thread may be between the two)
         if self._used is not None:
             return self._used
-        return self._size(self.total_halfs)
-
-    def _size(self, total):
-        landing = self._landing
         n = landing.read(int(self.is_value)) if landing is not None else None
         landed = n is not None
         if not landed:
-            n = read_word(total)
-        if n < 0 or n > (1 << 62):
+            n = read_word(self.total_halfs)
+        if _gave_up(n):
             if landed:
                 landing.spoilt()
             raise RuntimeError(_GAVE_UP)
-        self._landing = None
         if landed:
             self._used = n
+        self._landing = None
         return n
 
     def packed(self):
@@ -380,9 +358,8 @@ def proj_source(x, cos=None, sin=None, rot=None):
 def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_halfs=None, ws=None):
     """Prune and compress the first M tokens of x [batch, rows, heads, 128] where the projection left them, the keys
     rotated first when cos / sin are given (all rows are rotated and written to rot).  Heads are numbered
-    batch * heads + head.  Returns (CompressedKV, rot); without a capacity the values are cut to size, and whoever asks for nz,
-    total_halfs, packed() or a copy first waits for that - not the call, behind which the next one can go out (keys and values of 16
-    prompts of 4096 tokens, 8 heads each: two waits of the host, 18 us each, between and behind kernels of 82 and 39 us)."""
+    batch * heads + head.  Returns (CompressedKV, rot); without a capacity it waits for the size, not for the last values
+    and rotated rows."""
     assert x.dim() == 4
     batch, _, heads, N = x.shape
     if cos is not None and rot is None:
@@ -391,19 +368,39 @@ def compress_proj(x, is_value, kth, M, cos=None, sin=None, rot=None, capacity_ha
     sized = capacity_halfs is None and M != 0
     own = _own_workspace(ws, x.device) if sized else None
     words = own.status(status_words(batch * heads * (M // 64))) if own else None
-    device = torch._C._cuda_getDevice() if sized and x.is_cuda else None
-    pair = lib().mstf_landing_take() if sized and x.is_cuda and x.device.index == device else None
-    landing = _LandingPair(pair, _stream(), own, words, device) if pair else None
-    word = pair + 8 * int(bool(is_value)) if pair else (_landing_word()[1] if sized else 0)
     bmp, idx, nz_off, total, nz, n = _call(host().compress_proj, ws, x.device, None, x, int(is_value), int(kth), int(M), cos, sin,
-                                           rot, capacity, word, int(landing is None), words)
+                                           rot, capacity, _landing_word()[1] if sized else 0, 1, words)
     if M == 0:
         return None, rot
-    if landing is not None:
-        return CompressedKV.cut(bmp, idx, nz, nz_off, M, N, bool(is_value), total, landing), rot
     if sized and n < 0:
         gave_up(own, words, _GAVE_UP)
     return CompressedKV(bmp, idx, nz, nz_off, M, N, is_value, n if sized else total), rot
+
+
+def compress_proj_both(kx, vx, kth_k, kth_v, M, cos, sin, ws=None):
+    """compress_proj of the keys, rotated in place, and of the values of the same tokens (M > 0), for a caller who wants both: the
+    second launch goes out while the first one runs, not behind a wait for its size.  Returns a function to be called
+    once, behind the caller's other launches, which waits for both sizes and returns the two CompressedKV, or raises."""
+    assert kx.dim() == 4 and vx.dim() == 4 and M > 0
+    device = torch._C._cuda_getDevice() if kx.is_cuda else None
+    pair = lib().mstf_landing_take() if kx.is_cuda and kx.device.index == device and vx.device == kx.device else None
+    if not pair:
+        both = compress_proj(kx, False, kth_k, M, cos, sin, ws=ws)[0], compress_proj(vx, True, kth_v, M, ws=ws)[0]
+        return lambda: both
+    own = _own_workspace(ws, kx.device)
+    words = own.status(status_words(max(x.shape[0] * x.shape[2] for x in (kx, vx)) * (M // 64))) if own else None
+    landing = _LandingPair(pair, _stream(), own, words, device)
+    sides = [_call(host().compress_proj, ws, x.device, None, x, side, int(kth), int(M), *rope, -1, pair + 8 * side, 0, words)
+             for side, (x, kth, rope) in enumerate(((kx, kth_k, (cos, sin, kx)), (vx, kth_v, (None,) * 3)))]
+
+    def settle():
+        sizes = [landing.read(side) for side in (0, 1)]
+        if any(map(_gave_up, sizes)):
+            landing.spoilt()
+            raise RuntimeError(_GAVE_UP)
+        return tuple(CompressedKV(bmp, idx, nz[:n], nz_off, M, x.shape[3], bool(side), n)
+                     for side, (n, x, (bmp, idx, nz_off, _, nz, _)) in enumerate(zip(sizes, (kx, vx), sides)))
+    return settle
 
 
 def key_spmv(ck, q, groups, n_rows=1, out=None):
