@@ -485,25 +485,54 @@ static int quant_nsplit(int tokens, int Bkv, int groups, int bit, int group_size
     return fused_splits_step(tokens / 64, fused_fill(Bkv, quant_resident(groups, bit, group_size)), window);
 }
 
-// How a launch takes its blocks: shared by four wavefronts, a split slot each, where they are few; without room for those slots
-// (folded) the same numbers come from a wavefront per block.  window: tokens of the dense window behind them.
-// Shared also where one split would leave no merge to launch behind it: with three quarters of the stages gone from a wavefront's
-// chain the two launches are the faster form, call by call and recorded alike (us, 70 %, a wavefront per block / shared; recorded
-// unless said: 2 bits, 8 heads x 2 blocks 12.2 / 9.1, call by call 10.9 / 10.3, 8 x 8 13.2 / 9.1, 12.0 / 10.5, 8 x 16 15.3 / 9.2, 24 x 32
+// KV heads whose blocks, up to eight of each, the chip holds at once with a wavefront per block: its workgroups of kFusedWaves.
+static int quant_heads_at_once(int groups, int bit, int group_size)
+{
+    if (groups <= 4) return quant_resident(groups, bit, group_size) / kFusedWaves;
+    const bool g32 = group_size == 32;
+    return 1024 / kFusedWaves * (bit == 2   ? (g32 ? quant_occupancy<2, 2, true>() : quant_occupancy<2, 2, false>())
+                                 : bit == 4 ? (g32 ? quant_occupancy<2, 4, true>() : quant_occupancy<2, 4, false>())
+                                            : (g32 ? quant_occupancy<2, 8, true>() : quant_occupancy<2, 8, false>()));
+}
+// Whether four wavefronts share a block, where blocks are few (fused_shares_blocks).  merged: the call has splits to merge
+// without that too: a window, or (max, sum) asked for.
+// Nearly always, also where one split would leave no merge to launch behind it: with three quarters of the stages gone from a
+// wavefront's chain the two launches are the faster form, call by call and recorded alike (us, 70 %, a wavefront per block / shared;
+// recorded unless said: 2 bits, 8 heads x 2 blocks 12.2 / 9.1, call by call 10.9 / 10.3, 8 x 8 13.2 / 9.1, 12.0 / 10.5, 8 x 16 15.3 / 9.2, 24 x 32
 // 15.3 / 11.8, 16 x 64 15.5 / 13.5, 8 x 128 15.8 / 15.1, eight query heads 8 x 16 16.8 / 10.1, 8 x 96 17.3 / 14.8; 8 bits, two groups, eight
-// query heads 22.3 / 11.5; a step with a window of 300: 2 bits 8 x 8 21.6 / 11.7, 24 x 32 19.8 / 15.6, 8 bits 8 x 60 23.3 / 15.0).  The rule is
-// the fp16 kernel's (fused_shares_blocks); at its most blocks the forms are alike.
+// query heads 22.3 / 11.5; a step with a window of 300: 2 bits 8 x 8 21.6 / 11.7, 24 x 32 19.8 / 15.6, 8 bits 8 x 60 23.3 / 15.0).
+// Not for many heads of one to four blocks that are all there at once anyway: workgroups of all blocks come one behind the other then,
+// and the merge launches for every query row.  The more query heads and the fewer bits, the sooner that is so (a wavefront
+// per block / shared: 2 bits, four query heads 256 x 4 10.9 / 11.7, 448 x 2 11.7 / 12.2, but 192 x 4 10.8 / 10.4; eight 512 x 1 12.2 / 14.2, 384 x 1
+// 12.2 / 12.4, 256 x 3 12.0 / 13.2, 192 x 3 11.9 / 12.3, but 128 x 4 12.0 / 10.3, 160 x 3 11.8 / 10.8; 8 bits, four 256 x 4 14.1 / 14.9; 4 bits, eight
+// 256 x 3 13.2 / 13.6, 192 x 3 12.9 / 12.7; a 2-bit step of 384 heads of one block, eight query heads, window of 256 23.1 / 25.6), while heads for
+// which the chip has no room at once gain by a factor (8 bits, 300 x 1 24.3 / 9.9).
+static bool quant_shares(int tokens, int Bkv, int groups, int bit, int group_size, int window, bool merged)
+{
+    const int nblk = tokens / 64, wgs = Bkv * (nblk + (window_blocks(window) + kShare - 1) / kShare);
+    if (nblk > 4 || Bkv > quant_heads_at_once(groups, bit, group_size)) return true;
+    if (merged) return nblk > 1 || bit > 2 || window_blocks(window) < 4 || groups * wgs < 4608;
+    if (groups <= 4) return bit == 4 || wgs <= 768 || groups == 1 || (groups == 2 && bit == 2);
+    if (bit == 8 || (group_size == 32 && (bit == 4 || nblk > 1))) return true;
+    const bool least = bit == 2 && group_size == 64;
+    const int most = least ? 4096 : 5376;  // query heads x blocks
+    return nblk == 1 ? 3 * groups * wgs < 2 * most : groups * wgs <= most && (!least || wgs <= 640);
+}
+// How a launch takes its blocks: shared by four wavefronts, a split slot each, where they are few; without room for those slots, or
+// where the shared form is the slower one (folded), the same numbers come from a wavefront per block.  window: tokens of the dense
+// window behind them.
 struct QuantPlan {
     bool shared, folded;
     int ns;
     int merge_blocks() const { return shared ? ns : 0; }
 };
 static QuantPlan quant_plan(int tokens, int Bq, int groups, int bit, int group_size, int window, int window_in_launch,
-                            size_t workspace_bytes)
+                            bool merged, size_t workspace_bytes)
 {
     const int Bkv = Bq / groups;
     const bool few = fused_shares_blocks(tokens, Bkv, groups, Bkv * ((window_blocks(window) + kShare - 1) / kShare));
-    if (few && fused_share_fits(tokens, window, Bq, workspace_bytes)) return {true, false, tokens / 64};
+    if (few && quant_shares(tokens, Bkv, groups, bit, group_size, window, merged) && fused_share_fits(tokens, window, Bq, workspace_bytes))
+        return {true, false, tokens / 64};
     return {false, few, quant_nsplit(tokens, Bkv, groups, bit, group_size, window_blocks(window_in_launch))};
 }
 
@@ -571,7 +600,7 @@ static int decode_attention_quant_impl(void* stream, const uint64_t* k_bmp, cons
     if (!workspace || workspace_bytes < fused_workspace_need(tokens, 0, Bq)) return MSTF_EWORKSPACE;
     if (!aligned_to(workspace, 16)) return MSTF_EALIGN;
     hipStream_t st = as_stream(stream);
-    const QuantPlan plan = quant_plan(tokens, Bq, groups, bit, group_size, 0, 0, workspace_bytes);
+    const QuantPlan plan = quant_plan(tokens, Bq, groups, bit, group_size, 0, 0, lse_out || tokens > kFusedWaves * 64, workspace_bytes);
     const int ns = plan.ns;
     // with one split and no (max, sum) requested the kernel writes the final output itself
     // (and with a workgroup per head)
@@ -636,7 +665,7 @@ extern "C" int mstf_decode_attention_window_quant(
         rc = quant_check(k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
                          tokens, head_dim, Bq, groups, bit, capacity, dequant_mode);
         if (rc != MSTF_OK) return rc;
-        plan = quant_plan(tokens, Bq, groups, bit, 64, win_len, 0, workspace_bytes);
+        plan = quant_plan(tokens, Bq, groups, bit, 64, win_len, 0, true, workspace_bytes);
     }
     const int ns = plan.ns, nst = ns + window_blocks(win_len);
     if (tokens > 0) {
@@ -676,7 +705,7 @@ extern "C" int mstf_decode_attention_window_quant_pool(
                          max_tokens, head_dim, Bq, groups, bit, capacity, dequant_mode);
     if (rc != MSTF_OK) return rc;
     const int wblk = window_blocks(win_len);
-    const QuantPlan plan = quant_plan(max_tokens, Bq, groups, bit, 64, win_len, win_len, workspace_bytes);
+    const QuantPlan plan = quant_plan(max_tokens, Bq, groups, bit, 64, win_len, win_len, true, workspace_bytes);
     const int ns = plan.ns, nst = ns + wblk;
     rc = quant_launch(st, k_bmp, k_packed, k_tile_off, k_scales, k_zeros, v_bmp, v_packed, v_tile_off, v_scales, v_zeros, q,
                       nullptr, max_tokens, head_dim, Bq, groups, bit, dequant_mode, workspace, ns, nst, 0, 64,
@@ -722,7 +751,7 @@ extern "C" int mstf_decode_step_quant_pool(
     if (rc != MSTF_OK) return rc;
     hipStream_t st = as_stream(stream);
     const int wblk = window_blocks(win_len);
-    const QuantPlan plan = quant_plan(max_tokens, Bq, groups, bit, 64, win_len, win_len, workspace_bytes);
+    const QuantPlan plan = quant_plan(max_tokens, Bq, groups, bit, 64, win_len, win_len, true, workspace_bytes);
     const int ns = plan.ns, nst = ns + wblk;
     StepArgs sa = {};
     sa.q_in = reinterpret_cast<const _Float16*>(q_in);
