@@ -532,18 +532,15 @@ struct StageRank<NW, BIT, G32, false> {
             if (direct == 0u) clear_zeros(lane);
             direct = kDirectMax;
             const uint2 pair = dequant_halves<BIT, G32>(at, s, lt, (uint32_t)kWholeZeros, false, lane, mode);
-            whole_stage<Sums::NM, kImgStride, FIRST>(rank, lt.mask != 0ull ? whole_without(bits, lt.tiles(), lane) : bits, image, w,
-                                                     w + wgroup, sums.acc);
+            static_assert(Sums::NM == 1, "four rows");
+            whole_stage<kImgStride, FIRST>(rank, lt.mask != 0ull ? whole_without(bits, lt.tiles(), lane) : bits, image, w, sums.acc[0]);
             for (uint64_t left = lt.mask; left != 0ull; left &= left - 1ull) {
                 const uint32_t bit = (uint32_t)__builtin_ctzll(left), tl = bit / LongTiles<BIT>::kLanes;
                 const uint64_t there = lanes_of(whole_bitmap(bits, tl));
                 const _Float16 v = dequant_long<BIT, G32>(s, lt, pair, bit, rank_below(there), mode);
                 const uint32_t x = select_lane(there, (uint32_t)as_u16(v), 0u);
-    #pragma unroll
-                for (int m = 0; m < Sums::NM; m++) {
-                    const uint32_t wt = lds_load_u16(w + (uint32_t)m * wgroup + tl * 2u);
-                    sums.acc[m][0] = __builtin_amdgcn_mfma_f32_4x4x4f16(as_h4(x, 0u), as_h4(wt, 0u), sums.acc[m][0], 0, 0, 0);
-                }
+                const uint32_t wt = lds_load_u16(w + tl * 2u);
+                sums.acc[0][0] = __builtin_amdgcn_mfma_f32_4x4x4f16(as_h4(x, 0u), as_h4(wt, 0u), sums.acc[0][0], 0, 0, 0);
             }
         }
     }

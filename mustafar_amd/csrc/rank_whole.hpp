@@ -109,9 +109,8 @@ __device__ __forceinline__ uint32_t whole_base(uint32_t image)
 // gather into the register of each address, all lanes active, and the 4x4x4 products, in one statement on fixed registers.  Eight
 // gathers are in flight while the products of the eight in front of them run, and nothing is scalar: under exec masks, eight tiles
 // at a time, a wavefront waited for its own reads and for the masks of the coming tiles.
-// v[96:111], v[112:127]: addresses, then values, of the two products; v87, v[88:95]: the products' scales and rows, then the weights of two batches
-// (eight rows: v[80:95]).
-//   wa, wb : LDS address of w[lane & 3][0] of the first tile of the stage, for the accumulators 0 .. 3 and (NM = 2) 4 .. 7
+// v[96:111], v[112:127]: addresses, then values, of the two products; v87, v[88:95]: the products' scales and rows, then the weights of two batches.
+//   wa : LDS address of w[lane & 3][0] of the first tile of the stage (up to four rows)
 #define MSTF_SG(H, R, T) "ds_read_u16" H " v" R ", v" R " offset:%[is]*" T "\n\t"
 #define MSTF_SQUAD(R0, R1, R2, R3, T0, T1, T2, T3)                                                                  \
     MSTF_SG("", R0, T0) MSTF_SG("", R1, T2) MSTF_SG("_d16_hi", R2, T1) MSTF_SG("_d16_hi", R3, T3)
@@ -143,21 +142,13 @@ __device__ __forceinline__ uint32_t whole_base(uint32_t image)
     MSTF_SM0("p0", A0, W0) MSTF_SM0("p1", B0, W1) MSTF_SM("p0", A1, W0) "s_nop 0\n\t" MSTF_SM("p1", B1, W1)
 #define MSTF_SONE(A0, A1, B0, B1, W0, W1)                                                                           \
     MSTF_SM("p0", A0, W0) MSTF_SM("p1", B0, W1) MSTF_SM("p0", A1, W0) "s_nop 0\n\t" MSTF_SM("p1", B1, W1)
-// (eight rows: the pairs merged first, half the products)
-#define MSTF_SOR(D, S) "v_or_b32 " D ", " D ", " S "\n\t"
-#define MSTF_STWO(A, A2, A3, A4, B, B2, B3, B4, PA, PB, WA0, WA1, WB0, WB1)                                         \
-    MSTF_SOR(A, A3) MSTF_SOR(A2, A4) MSTF_SOR(B, B3) MSTF_SOR(B2, B4) "s_nop 1\n\t"                                 \
-    MSTF_SM("p0", PA, WA0) MSTF_SM("q0", PA, WB0) MSTF_SM("p1", PB, WA1) MSTF_SM("q1", PB, WB1)
 #define MSTF_SREGS                                                                                                  \
     "v87", "v88", "v89", "v90", "v91", "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104", "v105", "v106", "v107", "v108", "v109", "v110", "v111", "v112",  \
         "v113", "v114", "v115", "v116", "v117", "v118", "v119", "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127"
-template <int NM, int IS, bool FIRST>
-__device__ __forceinline__ void whole_stage(const WholeRank& c, uint2 bits, uint32_t image, uint32_t wa, uint32_t wb, f4_t (&acc)[NM][2])
+template <int IS, bool FIRST>
+__device__ __forceinline__ void whole_stage(const WholeRank& c, uint2 bits, uint32_t image, uint32_t wa, f4_t (&acc)[2])
 {
-    static_assert(NM == 1 || NM == 2, "four or eight accumulators");
     const uint64_t base = (uint64_t)image << 32 | image;
-    if constexpr (FIRST && NM == 2) acc[0][0] = acc[0][1] = acc[1][0] = acc[1][1] = f4_t{0.f, 0.f, 0.f, 0.f};
-    if constexpr (NM == 1) {
 #define MSTF_SSTAGE(M0)                                                                                             \
     MSTF_SADDRS MSTF_SW("wa", "v[88:91]", "0") MSTF_SG0 MSTF_SW("wa", "v[92:95]", "16")                                \
     MSTF_SG1 "s_waitcnt lgkmcnt(9)\n\t" M0("v[96:97]", "v[98:99]", "v[112:113]", "v[114:115]", "v[88:89]", "v[90:91]")  \
@@ -169,34 +160,16 @@ __device__ __forceinline__ void whole_stage(const WholeRank& c, uint2 bits, uint
 #define MSTF_SIN                                                                                                    \
     [x] "v"(bits.x), [y] "v"(bits.y), [one] "v"(c.one), [f] "v"(c.factor), [base] "s"(base),         \
         [sc] "i"(kWholeScales), [wa] "v"(wa), [is] "i"(IS)
-        if constexpr (FIRST)
-            asm volatile(MSTF_SSTAGE(MSTF_SONE0) : [p0] "=&v"(acc[0][0]), [p1] "=&v"(acc[0][1]) : MSTF_SIN : MSTF_SREGS, "memory");
-        else
-            asm volatile(MSTF_SSTAGE(MSTF_SONE) : [p0] "+v"(acc[0][0]), [p1] "+v"(acc[0][1]) : MSTF_SIN : MSTF_SREGS, "memory");
-    } else {
-        asm volatile(MSTF_SADDRS MSTF_SW("wa", "v[80:83]", "0") MSTF_SW("wb", "v[84:87]", "0") MSTF_SG0
-                     MSTF_SW("wa", "v[88:91]", "16") MSTF_SW("wb", "v[92:95]", "16") MSTF_SG1 "s_waitcnt lgkmcnt(10)\n\t"
-                     MSTF_STWO("v96", "v97", "v98", "v99", "v112", "v113", "v114", "v115", "v[96:97]", "v[112:113]", "v[80:81]", "v[82:83]",
-                               "v[84:85]", "v[86:87]")
-                     MSTF_SW("wa", "v[80:83]", "32") MSTF_SW("wb", "v[84:87]", "32") MSTF_SG2 "s_waitcnt lgkmcnt(10)\n\t"
-                     MSTF_STWO("v100", "v101", "v102", "v103", "v116", "v117", "v118", "v119", "v[100:101]", "v[116:117]", "v[88:89]", "v[90:91]",
-                               "v[92:93]", "v[94:95]")
-                     MSTF_SW("wa", "v[88:91]", "48") MSTF_SW("wb", "v[92:95]", "48") MSTF_SG3 "s_waitcnt lgkmcnt(10)\n\t"
-                     MSTF_STWO("v104", "v105", "v106", "v107", "v120", "v121", "v122", "v123", "v[104:105]", "v[120:121]", "v[80:81]", "v[82:83]",
-                               "v[84:85]", "v[86:87]")
-                     "s_waitcnt lgkmcnt(0)\n\t"
-                     MSTF_STWO("v108", "v109", "v110", "v111", "v124", "v125", "v126", "v127", "v[108:109]", "v[124:125]", "v[88:89]", "v[90:91]",
-                               "v[92:93]", "v[94:95]") "s_nop 4"
-                     : [p0] "+v"(acc[0][0]), [p1] "+v"(acc[0][1]), [q0] "+v"(acc[1][0]), [q1] "+v"(acc[1][1])
-                     : [x] "v"(bits.x), [y] "v"(bits.y), [one] "v"(c.one), [f] "v"(c.factor), [base] "s"(base),
-                       [sc] "i"(kWholeScales), [wa] "v"(wa), [wb] "v"(wb), [is] "i"(IS)
-                     : "v80", "v81", "v82", "v83", "v84", "v85", "v86", MSTF_SREGS, "memory");
-    }
+    if constexpr (FIRST)
+        asm volatile(MSTF_SSTAGE(MSTF_SONE0) : [p0] "=&v"(acc[0]), [p1] "=&v"(acc[1]) : MSTF_SIN : MSTF_SREGS, "memory");
+    else
+        asm volatile(MSTF_SSTAGE(MSTF_SONE) : [p0] "+v"(acc[0]), [p1] "+v"(acc[1]) : MSTF_SIN : MSTF_SREGS, "memory");
 }
 
 // The same for tiles of any number of survivors, without zeros in the image, under the tiles' masks: eight tiles at a time, each
 // read under its bitmap into cleared registers, the bitmaps from scalar loads one batch ahead.  bm: of the first tile.
 // v[96:127]: addresses; v[88:95]: values; v[84:87] (and v[80:83], eight rows): weights; s[64:79], s[80:95]: bitmaps.
+//   wa, wb : LDS address of w[lane & 3][0] of the first tile of the stage, for the accumulators 0 .. 3 and (NM = 2) 4 .. 7
 #define MSTF_XG(H, R, A, M, T) "s_brev_b64 exec, s[" M "]\n\tds_read_u16" H " " R ", " A " offset:%[is]*" T "\n\t"
 #define MSTF_XCLEAR "v_mov_b64 v[88:89], 0\n\tv_mov_b64 v[90:91], 0\n\tv_mov_b64 v[92:93], 0\n\tv_mov_b64 v[94:95], 0\n\t"
 #define MSTF_XGATHER(M0, M1, M2, M3, M4, M5, M6, M7, A0, A1, A2, A3, B0, B1, B2, B3, T0, T1, T2, T3, T4, T5, T6, T7)  \
@@ -217,6 +190,8 @@ __device__ __forceinline__ void whole_stage(const WholeRank& c, uint2 bits, uint
     "s_waitcnt lgkmcnt(4)\n\t" MSTF_SM("p0", "v[88:89]", "v[84:85]") "s_waitcnt lgkmcnt(0)\n\t"                       \
     MSTF_SM("p1", "v[92:93]", "v[86:87]") MSTF_SM("p0", "v[90:91]", "v[84:85]") "s_nop 0\n\t"                         \
     MSTF_SM("p1", "v[94:95]", "v[86:87]") "s_nop 4\n\t"
+// (eight rows: the pairs merged first, half the products)
+#define MSTF_SOR(D, S) "v_or_b32 " D ", " D ", " S "\n\t"
 #define MSTF_XTWO                                                                                                   \
     "s_waitcnt lgkmcnt(4)\n\t" MSTF_SOR("v88", "v90") MSTF_SOR("v89", "v91") "s_nop 1\n\t"                           \
     MSTF_SM("p0", "v[88:89]", "v[84:85]") MSTF_SM("q0", "v[88:89]", "v[80:81]") "s_waitcnt lgkmcnt(0)\n\t"           \
