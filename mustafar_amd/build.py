@@ -8,8 +8,11 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmustafar_hip.so")
 HOST = os.path.join(HERE, "_host.so")
 SOURCES = ["runtime.hip", "spmv.hip", "compress.hip", "quant.hip", "quant_spmv.hip", "fused.hip", "fused_quant.hip", "window_append.hip"]
+# SRAM-ECC on, as it always is on this chip: a load into the upper half of a register then clears the lower half, which gathers
+# into the registers of their own addresses rely on (csrc/rank_whole.hpp).  A device without it refuses the library.
+ARCH = "gfx950:sramecc+"
 FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-shared",
     # packed-fp32 VALU forms are kept out of the generated code on purpose
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # the leading kernel arguments (up to fourteen 32-bit words) arrive in scalar registers with the wavefront
@@ -44,7 +47,7 @@ def build(verbose=False):
 
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
         results = list(pool.map(compile_one, sources()))
-    link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + [o for o, _ in results]
+    link = [hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", LIB] + [o for o, _ in results]
     res = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout)

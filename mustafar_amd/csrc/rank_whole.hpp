@@ -109,6 +109,8 @@ __device__ __forceinline__ uint32_t whole_base(uint32_t image)
 // gather into the register of each address, all lanes active, and the 4x4x4 products, in one statement on fixed registers.  Eight
 // gathers are in flight while the products of the eight in front of them run, and nothing is scalar: under exec masks, eight tiles
 // at a time, a wavefront waited for its own reads and for the masks of the coming tiles.
+// A gather into an upper half clears the lower one, where the tile's address was: so it is with SRAM-ECC on, for which alone this library
+// is built (build.py).  With the half kept, address bits would be multiplied by a weight.
 // v[96:111], v[112:127]: addresses, then values, of the two products; v87, v[88:95]: the products' scales and rows, then the weights of two batches.
 //   wa : LDS address of w[lane & 3][0] of the first tile of the stage (up to four rows)
 #define MSTF_SG(H, R, T) "ds_read_u16" H " v" R ", v" R " offset:%[is]*" T "\n\t"
