@@ -1,8 +1,8 @@
 """Four wavefronts per block in the fused attention over codes (SHARE, csrc/fused_quant.hip): on both sides of the sizes where the
 launch takes that form (1024 blocks of all heads, 768 with more than four query heads, 128 of a head), one block a head, with and
-without (max, sum), and with a workspace that has no room for a slot per block, where the call goes without.  Reference: the
-three operators over the same codes; the bound is the one of scores rounded to fp16 in front of the softmax.  The forms add up
-the same products in another order, so they agree within that bound too."""
+without (max, sum), and with a workspace that has no room for a slot per block, where the call goes without.  The forms add
+the same products up in the same order: they give the same numbers, bit for bit, wherever the call is one that may share.  Reference:
+the three operators over the same codes; the bound is the one of scores rounded to fp16 in front of the softmax."""
 import pytest
 import torch
 
@@ -45,6 +45,9 @@ def check(bit, group_size, heads, groups, blocks):
     for o in (got, with_lse, alone):
         err = (o.float() - want).abs().amax(-1) / want.abs().amax(-1)
         assert float(err.max()) < 2e-3
+    assert torch.equal(got, with_lse)
+    if blocks <= 128 and heads * blocks <= (1024 if groups <= 4 else 768):
+        assert torch.equal(got, alone)
     assert torch.allclose(lse[:, 0], (s / D ** 0.5).float().amax(-1).view(-1), atol=2e-2)
 
 
@@ -95,3 +98,25 @@ def test_step_and_windows_without_room(bit, heads, groups, tokens, window):
                                                                   win_len_dev=length, ws=ws))
     assert all(torch.equal(o, outs[0]) for o in outs[1:])
     assert outs[0].isfinite().all()
+
+
+@pytest.mark.parametrize("bit", [2, 4, 8])
+@pytest.mark.parametrize("heads,groups,blocks,window", [(3, 4, 1, 1), (8, 4, 9, 300), (2, 8, 16, 65), (96, 8, 2, 512), (5, 1, 0, 70)])
+def test_window_calls_without_room(bit, heads, groups, blocks, window):
+    """decode_attention_window_quant, with room for a slot per block and with the least workspace: the same numbers."""
+    from mustafar_amd import compression_quant as cq, mustafar_package_quant as mq, ops
+    g = torch.Generator(device="cuda").manual_seed(heads * blocks + bit)
+    tokens, rows = blocks * 64, heads * groups
+    k = v = None
+    if blocks:
+        K, V = (torch.randn((heads, tokens, D), generator=g, device="cuda", dtype=torch.float16) for _ in range(2))
+        k = cq.convert_key_batched_quant(K, True, bit, kth=89 if bit < 8 else 40)
+        v = cq.convert_value_batched_quant(V, bit, kth=89 if bit < 8 else 40)
+    q = 0.25 * torch.randn((rows, D), generator=g, device="cuda", dtype=torch.float16)
+    kw, vw = (torch.randn((heads, window, D), generator=g, device="cuda", dtype=torch.float16) for _ in range(2))
+    outs, lses = [], []
+    for room in (ops.attention_workspace_least(tokens, window, rows), 64 << 20):
+        lses.append(torch.empty((rows, 2), device="cuda"))
+        ws = torch.empty(room, dtype=torch.uint8, device="cuda")
+        outs.append(mq.decode_attention_window_quant(k, v, q, kw, vw, window, groups, bit, lse=lses[-1], ws=ws))
+    assert torch.equal(*outs) and torch.equal(*lses) and outs[0].isfinite().all()
