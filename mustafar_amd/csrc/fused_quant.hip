@@ -519,8 +519,11 @@ static bool quant_shares(int tokens, int Bkv, int groups, int bit, int group_siz
     return nblk == 1 ? 3 * groups * wgs < 2 * most : groups * wgs <= most && (!least || wgs <= 640);
 }
 // How a launch takes its blocks: shared by four wavefronts, a split slot each, where they are few; without room for those slots, or
-// where the shared form is the slower one (folded), the same numbers come from a wavefront per block.  window: tokens of the dense
-// window behind them.
+// where the shared form is the slower one (folded), the same numbers come from a wavefront per block, in no more time than from sums
+// that run through the stages (8 heads x 16 blocks, running / folded: 2 / 4 / 8 bits 13.4 / 14.6 / 16.5, 12.4 / 14.5 / 16.4; eight query heads
+// 15.1 / 16.1 / 18.1, 15.2 / 16.0 / 17.9) but with 2 bits, two groups and more than four query heads, whose folded form spills registers (16.9,
+// 17.8; the half of the output that is done parked in LDS, the metadata's addresses made late or anew: three to eleven still spill).
+// window: tokens of the dense window behind them.
 struct QuantPlan {
     bool shared, folded;
     int ns;
